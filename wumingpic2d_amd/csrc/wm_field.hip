@@ -706,9 +706,10 @@ int wm_k_bc_phi(wm_ctx *ctx, double *phi, int l) {
   return WM_OK;
 }
 
+// Two partial sums per workgroup and component: the CG sweeps launch
+// ceil(nx / CGB) workgroups per row, the preconditioner one per tile.
 size_t wm_cg_partials(int nx, int ny) {
-  const size_t n = (size_t)nx * ny;
-  return 3 * 2 * std::max((size_t)wm_cdiv((long long)n, CGB), (size_t)wm_pc_dot_tiles(nx, ny));
+  return 3 * 2 * std::max((size_t)wm_cdiv(nx, CGB) * ny, (size_t)wm_pc_dot_tiles(nx, ny));
 }
 
 // Flexible CG with the learned preconditioner from the warm start in df;
