@@ -181,6 +181,16 @@ int ensure_stage(wm_ctx *ctx, size_t elems) {
   return WM_OK;
 }
 
+// particle_y's mover lists (the host-array entry point's alone).
+int ensure_mover_lists(wm_ctx *ctx) {
+  if (ctx->mvid_dn) return WM_OK;
+  const size_t ms = (size_t)nseg_of(ctx) * ctx->mcap;
+  if (!ctx->mv_up.uz) WM_TRY(alloc_bank(ctx, ctx->mv_up, ms));
+  if (!ctx->mv_dn.uz) WM_TRY(alloc_bank(ctx, ctx->mv_dn, ms));
+  if (!ctx->mvid_up) WM_TRY(dmalloc(ctx, &ctx->mvid_up, ms));
+  return dmalloc(ctx, &ctx->mvid_dn, ms);
+}
+
 // Upload the active records (cnt[seg] per segment) of a reference-layout
 // particle array into bank `b` and the current ID array.
 int upload_particles(wm_ctx *ctx, const double *up, const int *cnt_host, int b) {
@@ -201,6 +211,7 @@ int upload_particles(wm_ctx *ctx, const double *up, const int *cnt_host, int b) 
     w = std::max(w, cnt_host[s]);
   }
   w = std::max(w, 1);
+  ctx->perm_valid = false;                 // rows as given
   const size_t elems = (size_t)nseg * w * g.ndim;
   WM_TRY(ensure_stage(ctx, elems));
   std::vector<double> h(elems);
@@ -483,6 +494,7 @@ int check_bounds(wm_ctx *ctx, int nxs, int nxe) {
 
 // ------------------------------------------ the state row by row (restart I/O)
 int wm_state_np2(wm_ctx *ctx, int *np2_host) {
+  WM_TRY(wm_order_apply(ctx));
   if (ctx->form == WM_FORM_FP32) {
     WM_TRY(wm_settle_movers(ctx));
     WM_TRY(wm_k_bin_rows(ctx));
@@ -500,6 +512,7 @@ int wm_rows_out(wm_ctx *ctx, int s0, int s1, int w, double *h) {
   if (ctx->form == WM_FORM_FP32) {
     WM_TRY(wm_k_bins_to_stage(ctx, s0, s1 - s0, w));
   } else {
+    WM_TRY(wm_order_apply(ctx));
     const size_t off = (size_t)s0 * ctx->cap;
     const PBank &A = ctx->bank[0];
     const PBank B{A.x + off, A.y + off, A.ux + off, A.uy + off, A.uz + off};
@@ -537,6 +550,7 @@ int wm_rows_in(wm_ctx *ctx, int s0, int s1, int w, const int *cnt_host, const do
 
 int wm_rows_begin(wm_ctx *ctx) {
   WM_TRY(wm_alloc_device(ctx));
+  ctx->perm_valid = false;
   if (ctx->form == WM_FORM_FP32) WM_TRY(fresh_bins(ctx));
   // a restarted run begins as a fresh process does: the CG warm start df is
   // zero (field.f90:105-119)
@@ -665,15 +679,23 @@ int wm_alloc_device(wm_ctx *ctx) {
     WM_TRY(dmalloc(ctx, &ctx->nhole, nseg));
     WM_TRY(dmalloc(ctx, &ctx->nup, nseg));
     WM_TRY(dmalloc(ctx, &ctx->ndn, nseg));
-    WM_TRY(alloc_bank(ctx, ctx->mv_up, ms));
-    WM_TRY(alloc_bank(ctx, ctx->mv_dn, ms));
-    WM_TRY(dmalloc(ctx, &ctx->mvid_up, ms));
-    WM_TRY(dmalloc(ctx, &ctx->mvid_dn, ms));
-    ctx->ytiles = wm_cdiv(ctx->cap, 64);
-    WM_TRY(dmalloc(ctx, &ctx->ytmask, (size_t)nseg * ctx->ytiles));
-    WM_TRY(dmalloc(ctx, &ctx->ytpre, (size_t)nseg * ctx->ytiles));
-    WM_TRY(dmalloc(ctx, &ctx->yhist, (size_t)nseg * g.nx));
-    WM_HIP(hipMemsetAsync(ctx->yhist, 0, sizeof(int) * (size_t)nseg * g.nx, ctx->stream));
+    // the row order between steps
+    WM_TRY(dmalloc(ctx, &ctx->perm, slots));
+    WM_TRY(dmalloc(ctx, &ctx->code, slots));
+    WM_TRY(dmalloc(ctx, &ctx->kind, (size_t)nseg * g.nx));
+    WM_TRY(dmalloc(ctx, &ctx->farcnt, (size_t)nseg * g.nx));
+    WM_TRY(dmalloc(ctx, &ctx->far, nseg));
+    WM_TRY(dmalloc(ctx, &ctx->lup, ms));
+    WM_TRY(dmalloc(ctx, &ctx->ldn, ms));
+    WM_TRY(dmalloc(ctx, &ctx->disp, 2 * ms));
+    WM_TRY(dmalloc(ctx, &ctx->dstart, (size_t)nseg * (g.nx + 1)));
+    WM_TRY(dmalloc(ctx, &ctx->cumnew, (size_t)nseg * (g.nx + 1)));
+    WM_TRY(dmalloc(ctx, &ctx->nold, nseg));
+    WM_TRY(dmalloc(ctx, &ctx->rowok, nseg));
+    WM_HIP(hipMemsetAsync(ctx->perm, 0, sizeof(unsigned) * slots, ctx->stream));
+    WM_HIP(hipMemsetAsync(ctx->farcnt, 0, sizeof(int) * (size_t)nseg * g.nx, ctx->stream));
+    WM_HIP(hipMemsetAsync(ctx->far, 0, sizeof(int) * nseg, ctx->stream));
+    WM_HIP(hipMemsetAsync(ctx->cumnew, 0, sizeof(int) * (size_t)nseg * (g.nx + 1), ctx->stream));
   }
 
   FieldGeom &fg = ctx->fg;
@@ -798,8 +820,9 @@ int wm_destroy(wm_ctx *ctx) {
                   ctx->bstart, ctx->pcnt, ctx->mfill[0], ctx->mfill[1], ctx->rowpend,
                   ctx->fstat, ctx->relay_ctl, ctx->relay_blocks, ctx->blkflag, ctx->relay_segs,
                   ctx->segflag, ctx->rws.q, ctx->rws.uz, ctx->rws_id, ctx->rws_bs,
-                  ctx->spill_l, ctx->spill_p, ctx->spill_q, ctx->sfill, ctx->ytmask,
-                  ctx->ytpre, ctx->yhist};
+                  ctx->spill_l, ctx->spill_p, ctx->spill_q, ctx->sfill, ctx->perm, ctx->code,
+                  ctx->kind, ctx->farcnt, ctx->far, ctx->lup, ctx->ldn, ctx->disp, ctx->dstart,
+                  ctx->cumnew, ctx->nold, ctx->rowok};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   wm_pc_free(ctx);
@@ -1021,7 +1044,8 @@ int wm_bcp_particle_y(wm_ctx *ctx, double *up, int *np2) {
   WM_TRY(upload_particles(ctx, up, np2, 0));
   const int nseg = nseg_of(ctx);
   WM_HIP(hipMemcpyAsync(ctx->np2, np2, sizeof(int) * nseg, hipMemcpyHostToDevice, ctx->stream));
-  WM_TRY(wm_k_particle_y(ctx, 0, 0));
+  WM_TRY(ensure_mover_lists(ctx));
+  WM_TRY(wm_k_particle_y(ctx, 0));
   WM_TRY(wm_check_derr(ctx, "boundary_periodic__particle_y"));
   std::vector<int> n2(nseg);
   WM_HIP(hipMemcpyAsync(n2.data(), ctx->np2, sizeof(int) * nseg, hipMemcpyDeviceToHost, ctx->stream));
@@ -1266,6 +1290,7 @@ int wm_state_download(wm_ctx *ctx, double *up, int *np2, int *cumcnt, double *uf
     WM_TRY(wm_settle_movers(ctx));
     WM_TRY(wm_k_bin_rows(ctx));
   }
+  if (up) WM_TRY(wm_order_apply(ctx));
   std::vector<int> n2(nseg);
   WM_HIP(hipMemcpyAsync(n2.data(), ctx->np2, sizeof(int) * nseg, hipMemcpyDeviceToHost, ctx->stream));
   if (cumcnt)
@@ -1290,6 +1315,7 @@ int wm_state_init_weibel(wm_ctx *ctx, uint64_t seed, int ppc, double vth, double
     WM_TRY(fresh_bins(ctx));
     WM_TRY(wm_k_init_weibel(ctx, seed, ppc, vth, udrift));
   } else {
+    ctx->perm_valid = false;
     WM_TRY(wm_k_init_weibel(ctx, seed, ppc, vth, udrift));
     // stable by cell within each row: the order of sort__bucket
     WM_TRY(wm_k_sort(ctx, 1, 0));
@@ -1345,23 +1371,16 @@ int wm_step(wm_ctx *ctx, int nsteps) {
       WM_TRY(wm_relayout(ctx));
       WM_HIP(hipEventRecord(e[7], ctx->stream));
     } else {
-      // The particle boundaries and the sort (app.f90:104-106) read only the
-      // pushed particles, and the field solve (app.f90:103) only the current
-      // and the fields: they run concurrently, the particles on the second
-      // stream, and the next step waits for both.
-      WM_TRY(wm_k_push_deposit(ctx, 0, 1));
+      // The row order (particle_y and the sort, app.f90:105-106) reads only
+      // what the push left, and the field solve (app.f90:103) only the
+      // current and the fields: they run concurrently, the order on the
+      // second stream, and the next step waits for both.
+      WM_TRY(wm_k_push_step(ctx));
       WM_HIP(hipEventRecord(e[2], ctx->stream));
       WM_HIP(hipStreamWaitEvent(ctx->stream2, e[2], 0));
       StreamSwap on2(ctx, ctx->stream2);
       WM_HIP(hipEventRecord(e[5], ctx->stream));
-      {
-        // app.f90:104-105 (x fused into y pass 1): the periodic wrap, the
-        // reconnection's walls (proj/reconnection/app.f90:104), or none
-        // (the shock's edges came with the push, proj/shock/app.f90:113)
-        const int xmode = ctx->bcf == WM_BC_PERIODIC ? 1 : ctx->bcf == WM_BC_RECONNECTION ? 2 : 0;
-        // app.f90:105-106: pass 1, then pass 2 fused with the sort
-        WM_TRY(wm_k_particle_y_sort(ctx, 1, 0, xmode, e[6]));
-      }
+      WM_TRY(wm_k_order(ctx, e[6]));
       WM_HIP(hipEventRecord(e[7], ctx->stream));
     }
     WM_TRY(f32 ? wm_k_deposit_gather32(ctx) : wm_k_deposit_gather(ctx));
@@ -1373,7 +1392,7 @@ int wm_step(wm_ctx *ctx, int nsteps) {
     WM_HIP(hipEventRecord(e[8], ctx->stream));
     WM_HIP(hipEventSynchronize(e[8]));
     // phases: [0..3] on the first stream (e0..e4), [4] particle boundaries
-    // (e5..e6) and [5] sort (e6..e7) on the second (FP64; in the FP32 form
+    // (e5..e6) and [5] the places (e6..e7) on the second (FP64; in the FP32 form
     // the push holds them, and [4] is the fill check, [5] the re-layout)
     const int from[WM_NPHASE] = {0, 1, 2, 3, 5, 6}, to[WM_NPHASE] = {1, 2, 3, 4, 6, 7};
     for (int k = 0; k < WM_NPHASE; ++k) {
@@ -1468,6 +1487,7 @@ int wm_moments(wm_ctx *ctx, double *mom) {
     return WM_ERR_NOT_INIT;
   }
   if (ctx->form == WM_FORM_FP32) WM_TRY(wm_settle_movers(ctx));
+  WM_TRY(wm_order_apply(ctx));
   hipEvent_t *e = ctx->ev + 20;
   WM_HIP(hipEventRecord(e[0], ctx->stream));
   WM_TRY(wm_k_moments(ctx, true));

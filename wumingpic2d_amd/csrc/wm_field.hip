@@ -888,7 +888,8 @@ int wm_k_energy(wm_ctx *ctx, int bank, double *out) {
     WM_TRY(wm_k_energy_kin32(ctx, bank, part, nchunk));
   else
     hipLaunchKernelGGL(k_energy_kin, dim3(nchunk, nseg), dim3(256), 0, ctx->stream, g.ny,
-                       ctx->cap, g.nsp, ctx->np2, ctx->bank[bank].ux, ctx->bank[bank].uy,
+                       ctx->cap, g.nsp, ctx->perm_valid ? ctx->nold : ctx->np2,   // any order will do
+                       ctx->bank[bank].ux, ctx->bank[bank].uy,
                        ctx->bank[bank].uz, g.c, part, nchunk);
   hipLaunchKernelGGL(k_energy_fld, dim3(g.ny), dim3(256), 0, ctx->stream, ctx->fg, ctx->uf,
                      part + (size_t)nseg * nchunk);

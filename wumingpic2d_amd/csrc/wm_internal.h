@@ -16,7 +16,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
+#include <algorithm>
 #include <string>
+#include <utility>
 
 #include "../../include/wmpic.h"
 #include "wm_records.h"
@@ -168,18 +170,26 @@ struct wm_ctx {
   int *np2 = nullptr;      // [nseg]
   int *cumcnt = nullptr;   // [nseg*(nx+1)]
 
-  // particle_y workspace
+  // particle_y workspace (the mover lists: host-array entry point, on first use)
   int *hole = nullptr;     // [nseg*2*mcap]
   int *nhole = nullptr, *nup = nullptr, *ndn = nullptr;  // [nseg]
   PBank mv_up{}, mv_dn{};
   int64_t *mvid_up = nullptr, *mvid_dn = nullptr;
-  // the resident step's fused pass 2 + sort: per tile of 64 slots of a row
-  // segment, pass 1's leaver mask and the holes before the tile; per
-  // segment, the histogram of the cells the row holds after pass 2
-  unsigned long long *ytmask = nullptr;   // [nseg*ytiles]
-  int *ytpre = nullptr;                   // [nseg*ytiles]
-  int *yhist = nullptr;                   // [nseg*nx], zero between steps
-  int ytiles = 0;
+  // The resident step's row order (wm_order.hip).  With perm_valid, bank 0
+  // holds the last push's output in the slots it read its particles from
+  // (nold per segment), and slot k of a row is the particle at index
+  // perm[seg * cap + k] of its species' plane (row * cap + slot); np2, cumcnt
+  // and the IDs are the ordered rows'.
+  bool perm_valid = false;
+  unsigned *perm = nullptr;      // [nseg*cap]
+  uint16_t *code = nullptr;      // [nseg*cap] the push's code per particle (wm_order.h)
+  int4 *kind = nullptr;          // [nseg*nx] moves out of a cell by kind
+  int *farcnt = nullptr, *far = nullptr;   // [nseg*nx], [nseg]; zero between steps
+  uint2 *lup = nullptr, *ldn = nullptr;    // [nseg*mcap] a row's leavers
+  uint2 *disp = nullptr;         // [nseg*2*mcap] displaced particles by new cell
+  int *dstart = nullptr;         // [nseg*(nx+1)]
+  int *cumnew = nullptr;         // [nseg*(nx+1)] the other cumcnt
+  int *nold = nullptr, *rowok = nullptr;   // [nseg]
 
   // fields
   FieldGeom fg{};
@@ -288,7 +298,7 @@ int wm_report_derr(wm_ctx *ctx, int h, const char *where);
 int wm_k_cell_fields(wm_ctx *ctx);
 int wm_k_push(wm_ctx *ctx, int src, int dst);
 int wm_k_deposit(wm_ctx *ctx, int oldb, int newb);
-int wm_k_push_deposit(wm_ctx *ctx, int src, int dst);
+int wm_k_push_step(wm_ctx *ctx);   // the resident step's: push, deposit, particle_x, codes
 int wm_k_deposit_gather(wm_ctx *ctx);
 // Fields (wm_field.hip)
 int wm_k_bc_curre(wm_ctx *ctx, double *uj);
@@ -299,12 +309,11 @@ int wm_k_field_solve(wm_ctx *ctx);   // RHS .. uf += df (after the current is re
 int wm_k_energy(wm_ctx *ctx, int bank, double *out_host);
 // Particle boundaries (wm_bc.hip)
 int wm_k_particle_x(wm_ctx *ctx, int bank);
-// xmode: 0 y only, 1 with the periodic x wrap fused, 2 with the walls' mirrors fused
-int wm_k_particle_y(wm_ctx *ctx, int bank, int xmode);
-// The resident step's particle_y and sort: pass 1, then pass 2 fused with
-// the sort, from bank src into bank dst (the ID arrays follow); mid is
-// recorded between the two
-int wm_k_particle_y_sort(wm_ctx *ctx, int src, int dst, int xmode, hipEvent_t mid);
+int wm_k_particle_y(wm_ctx *ctx, int bank);
+// The resident step's particle_y and sort, as the order of the rows in
+// bank 0; mid is recorded before the last kernel (wm_order.hip)
+int wm_k_order(wm_ctx *ctx, hipEvent_t mid);
+int wm_order_apply(wm_ctx *ctx);   // bank 0 in that order, if one is pending
 int wm_k_injection(wm_ctx *ctx, int bank, double u0);   // boundary_shock__injection
 double wm_injection_xend(const wm_ctx *ctx, double u0);
 // Sort (wm_sort.hip)

@@ -21,6 +21,8 @@
 // kernel sums in a fixed order, so the deposit is deterministic (no
 // floating-point atomics).
 #include "wm_internal.h"
+#include "wm_edges.h"
+#include "wm_order.h"
 
 namespace {
 
@@ -30,18 +32,36 @@ constexpr int TW = CHUNK + 2;         // push tile width (halo 1)
 constexpr int DW = CHUNK + 4;         // deposit tile width (halo 2)
 constexpr int TILE = 5 * DW * 3;      // doubles per deposit tile
 constexpr int NACC = 65;              // Jx 4x5 + Jy 5x4 + Jz 5x5
-constexpr int MCAP = 16;              // a cell's movers listed in LDS per species
+constexpr int MCAP = 24;              // a cell's movers listed in LDS at a time
 
 struct PP {                           // particle-kernel parameters
   int nx, ny, nxgs, nys, nsp, cap, nchunk;
   double d_delx, delt, c, qc_scale;   // qc_scale = delx / delt
+  double ic2;                         // 1 / c^2
   double q[WM_MAXSP], r[WM_MAXSP];
   // the shock's injection edge, applied to the pushed particle before its
   // current (proj/shock/app.f90:112-114): inj, nxs, the left mirror point
   // 2 (nxs+1) delx, xend and u0 (boundary_shock.f90:266-294)
   int inj, xs;
   double delx, wl, xend, u0;
+  // the resident step's particle boundaries, applied as the particle is
+  // stored: xmode 1 the periodic wrap, 2 the walls' mirrors, 0 neither
+  int xmode, xe;
+  double spanx, spany, wr;
 };
+
+// What the resident step's push leaves for the row order (wm_order.h).
+struct Order {
+  const unsigned *perm;          // the rows' order now: species-plane index per slot
+  uint16_t *code;                // per slot
+  int4 *kind;                    // per cell: to the left, staying, to the right, others
+  int *farcnt, *far;             // particles more than one cell away: per new cell; rows with any
+};
+
+// Where the kernel reads its particles: the slots themselves, or through
+// Order::perm with 32-bit byte offsets into the species' plane (planes below
+// 4 GB) or 64-bit ones.
+enum { SRC_SLOT = 0, SRC_PERM32 = 1, SRC_PERM64 = 2 };
 
 __device__ inline void injection_edge(double &x, double &ux, double &uy, double &uz,
                                       const PP &P) {
@@ -265,17 +285,11 @@ __device__ inline double group_sum(double v) {
 }
 
 // Contribution of one component of a cell's crossing particles, combined
-// over the group and added by lane 0 to cellbuf.  The cell's first MCAP
-// movers of the species come from its LDS list L (x0, y0, x1, y1, q v_z;
-// lane sub takes entries sub, sub + GROUP, ...); a mover past them from the
-// lane's own mask (bit m = the lane's m-th particle from ka, the state read
-// back from the banks); particles beyond the mask are re-examined.
+// over the group and added by lane 0 to cellbuf: the cell's LDS list L (x0,
+// y0, x1, y1, q v_z), lane sub taking entries sub, sub + GROUP, ...
 template <int C>
-__device__ inline void crossing_pass(double *cb, int sub, const double *L, int nl,
-                                     unsigned long long mask, int ka, int ke, size_t base,
-                                     const double *xa, const double *ya, const double *xb,
-                                     const double *yb, const double *uxb, const double *uyb,
-                                     const double *uzb, int i, int j, double q, const PP &P) {
+__device__ inline void crossing_pass(double *cb, int sub, const double *L, int nl, int i, int j,
+                                     double q, const PP &P) {
   constexpr int N = C == 2 ? 25 : 20;
   double acc[N];
 #pragma unroll
@@ -286,26 +300,6 @@ __device__ inline void crossing_pass(double *cb, int sub, const double *L, int n
     make_move(m, L[e], L[MCAP + e], L[2 * MCAP + e], L[3 * MCAP + e], i, j, P);
     stencil<C>(acc, m, qc, L[4 * MCAP + e]);
   }
-  auto one = [&](int k, bool known) {
-    const size_t p = base + (size_t)k;
-    Move m;
-    const double x1 = xb[p], y1 = yb[p];
-    const bool cross = (int)(x1 * P.d_delx) != i || (int)(y1 * P.d_delx) != j;
-    if (!known && !cross) return;
-    make_move(m, xa[p], ya[p], x1, y1, i, j, P);
-    double qv = 0.0;
-    if (C == 2) {
-      const double ux = uxb[p], uy = uyb[p], uz = uzb[p];
-      qv = q * (uz / sqrt(1.0 + (ux * ux + uy * uy + uz * uz) / (P.c * P.c)));
-    }
-    stencil<C>(acc, m, qc, qv);
-  };
-  while (mask) {
-    const int m = __ffsll((long long)mask) - 1;
-    mask &= mask - 1;
-    one(ka + sub + GROUP * m, true);
-  }
-  for (int k = ka + sub + GROUP * 64; k < ke; k += GROUP) one(k, false);
   const int off = C == 0 ? 0 : (C == 1 ? 20 : 40);
 #pragma unroll
   for (int k = 0; k < N; ++k) {
@@ -324,6 +318,8 @@ __device__ inline void seg_st(double *seg, int k, double v) {
   *(double *)((char *)seg + (unsigned)k * 8u) = v;
 }
 
+// The push alone or the deposit alone, of rows in place (the host-array entry
+// points); the resident step's kernel is k_push_step below.
 template <bool PUSH, bool DEPOSIT>
 __global__ __launch_bounds__(256, 3) void k_particle(
     PP P, const int *__restrict__ cumcnt,
@@ -337,9 +333,9 @@ __global__ __launch_bounds__(256, 3) void k_particle(
     double *__restrict__ part, int *__restrict__ derr) {
   __shared__ double T[PUSH ? 6 * 3 * TW : 1];
   __shared__ double cellbuf[DEPOSIT ? CHUNK * NACC : 1];
-  // per cell: its first MCAP movers of the species in hand, as
-  // [x0 | y0 | x1 | y1 | q v_z][entry], so that their full stencils need not
-  // read the banks again (their lines are gone from L2 by then)
+  // per cell: up to MCAP of its movers, as [x0 | y0 | x1 | y1 | q v_z][entry],
+  // so that their full stencils need not read the banks again (their lines
+  // are gone from L2 by then)
   __shared__ double mvl[DEPOSIT ? CHUNK * 5 * MCAP : 1];
   const int chunk = blockIdx.x;
   const int jl = blockIdx.y;                 // row j = nys + jl
@@ -361,7 +357,7 @@ __global__ __launch_bounds__(256, 3) void k_particle(
 #pragma unroll
     for (int k = 0; k < 27; ++k) core[k] = 0.0;
   }
-  bool ok = true;
+  int bad = 0;
   if (g < ncell) {
     for (int s = 0; s < P.nsp; ++s) {
       const size_t seg = (size_t)s * P.ny + jl;
@@ -372,124 +368,118 @@ __global__ __launch_bounds__(256, 3) void k_particle(
       const double fac1 = q / r * 0.5 * P.delt;
       const double txxx = fac1 * fac1;
       const double fac2 = q * P.delt / r;
-      unsigned long long mask = 0ULL;
-      if (kb >= ke) continue;                  // no particle of species s here
       // windows of 2 GROUP consecutive particles start at the 2 GROUP
       // boundary at or below the cell's first particle, so that each array's
       // load is one aligned 128-byte line for the group; lane sub takes the
-      // window's particles sub and GROUP + sub, in that order (the order of
-      // GROUP-particle windows, m counting them from ka)
+      // window's particles sub and GROUP + sub, in that order
       const int ka = kb - kb % (2 * GROUP);
-      // segment bases: the same for the whole workgroup, 32-bit indices below
+      // bases: the same for the whole workgroup, 32-bit indices below
       const double *Xa = xa + base, *Ya = ya + base;
       const double *Uxa = uxa + base, *Uya = uya + base, *Uza = uza + base;
       double *Xb = xb + base, *Yb = yb + base;
       double *Uxb = uxb + base, *Uyb = uyb + base, *Uzb = uzb + base;
-      int mcnt = 0;                            // the cell's movers so far (lane 0's is kept)
-      // particle k (the lane's m-th): pushed and stored, its stay-in-cell
-      // stencil added; a crossing one returns true with its deposit inputs
-      auto one = [&](int k, int m, double x0, double y0, double cux, double cuy, double cuz,
-                     double &x1, double &y1, double &qv) {
+      int mcnt = 0;                            // the list's entries (lane 0's is kept)
+      // particle k: pushed and stored, its stay-in-cell stencil added; a
+      // crossing one returns true with its deposit inputs
+      auto one = [&](int k, double x0, double y0, double cux, double cuy, double cuz, double &x1,
+                     double &y1, double &qv) {
         if (k < kb || k >= ke) return false;   // before or after the cell
         double ux, uy, uz, ig = 0.0;
         // keep the 54 tile values in LDS instead of hoisting them into
         // registers for the whole cell loop (occupancy)
         __asm__ volatile("" ::: "memory");
+        int i2, j2;
         if (PUSH) {
           PushOut o = boris(T, g, x0, y0, cux, cuy, cuz, i, j, P, fac1, txxx, fac2);
-          if (P.inj) injection_edge(o.x, o.ux, o.uy, o.uz, P);
+          x1 = o.x; y1 = o.y; ux = o.ux; uy = o.uy; uz = o.uz; ig = o.ig;
+          i2 = (int)(x1 * P.d_delx);
+          j2 = (int)(y1 * P.d_delx);
           seg_st(Xb, k, o.x); seg_st(Yb, k, o.y);
           seg_st(Uxb, k, o.ux); seg_st(Uyb, k, o.uy); seg_st(Uzb, k, o.uz);
-          x1 = o.x; y1 = o.y; ux = o.ux; uy = o.uy; uz = o.uz; ig = o.ig;
         } else {
           x1 = seg_ld(Xb, k); y1 = seg_ld(Yb, k);
           ux = seg_ld(Uxb, k); uy = seg_ld(Uyb, k); uz = seg_ld(Uzb, k);
+          i2 = (int)(x1 * P.d_delx);
+          j2 = (int)(y1 * P.d_delx);
         }
         if (DEPOSIT) {
-          const int i2 = (int)(x1 * P.d_delx), j2 = (int)(y1 * P.d_delx);
-          // field.f90:270's v_z = u_z / gamma; the fused kernel reuses the
-          // push's 1 / gamma of the same u (a product instead of a
-          // quotient: within an ulp), except where the shock's injection
-          // edge may have reflected the pushed u
-          const double gvz = PUSH && !P.inj
-                                 ? uz * ig
-                                 : uz / sqrt(1.0 + (ux * ux + uy * uy + uz * uz) / (P.c * P.c));
+          // v_z = u_z / gamma, field.f90:270
+          const double gvz = PUSH ? uz * ig
+                                  : uz / sqrt(1.0 + (ux * ux + uy * uy + uz * uz) / (P.c * P.c));
           if (i2 == i && j2 == j) {
             stencil_core(core, x0, y0, x1, y1, gvz, i, j, q, P);
           } else {
-            ok = ok && (i2 - i >= -1 && i2 - i <= 1 && j2 - j >= -1 && j2 - j <= 1);
+            if (!(i2 - i >= -1 && i2 - i <= 1 && j2 - j >= -1 && j2 - j <= 1)) bad |= DERR_JUMP;
             qv = q * gvz;
-            return m < 64;                     // later ones: re-examined from the banks
+            return true;
           }
         }
         return false;
       };
       // a crossing particle goes to the cell's LDS list in (window, lane)
-      // order, ranked by a ballot over the group (lane 0 of the group runs
-      // every window any of its lanes runs); past MCAP to the lane's mask
-      auto record = [&](bool cross, int m, double x0, double y0, double x1, double y1,
-                        double qv) {
+      // order, ranked by a ballot over the group
+      auto record = [&](bool cross, double x0, double y0, double x1, double y1, double qv) {
         const unsigned gb = (unsigned)(__ballot(cross) >> (GROUP * wg)) & 0xFFu;
         if (cross) {
           const int e = mcnt + __popc(gb & ((1u << sub) - 1u));
-          if (e < MCAP) {
-            L[e] = x0;
-            L[MCAP + e] = y0;
-            L[2 * MCAP + e] = x1;
-            L[3 * MCAP + e] = y1;
-            L[4 * MCAP + e] = qv;
-          } else {
-            mask |= 1ULL << m;
-          }
+          L[e] = x0;
+          L[MCAP + e] = y0;
+          L[2 * MCAP + e] = x1;
+          L[3 * MCAP + e] = y1;
+          L[4 * MCAP + e] = qv;
         }
         mcnt += __popc(gb);
       };
-      for (int m = 0, k = ka + sub; k < ke; k += 2 * GROUP, m += 2) {
-        // both halves' loads issued together, each index clamped into the
-        // cell's particles (a lane outside them reads a neighbour and idles)
-        const int kA = min(max(k, kb), ke - 1), kB = min(max(k + GROUP, kb), ke - 1);
-        const double xA = seg_ld(Xa, kA), yA = seg_ld(Ya, kA);
-        const double xB = seg_ld(Xa, kB), yB = seg_ld(Ya, kB);
-        double uxA = 0, uyA = 0, uzA = 0, uxB = 0, uyB = 0, uzB = 0;
-        if (PUSH) {
-          uxA = seg_ld(Uxa, kA); uyA = seg_ld(Uya, kA); uzA = seg_ld(Uza, kA);
-          uxB = seg_ld(Uxa, kB); uyB = seg_ld(Uya, kB); uzB = seg_ld(Uza, kB);
+      bool more = kb < ke;
+      int k = (more ? ka : ke) + sub;
+      // a pass over the cell's windows until the cell ends or some cell's
+      // list could overflow in the next window (then the lists are deposited
+      // and the pass goes on): the same for the wavefront
+      while (__ballot(more) != 0ULL) {
+        for (; k - sub < ke && __ballot(mcnt > MCAP - 2 * GROUP) == 0ULL; k += 2 * GROUP) {
+          // both halves' loads issued together, each index clamped into the
+          // cell's particles (a lane outside them reads a neighbour and idles)
+          const int kA = min(max(k, kb), ke - 1), kB = min(max(k + GROUP, kb), ke - 1);
+          const double xA = seg_ld(Xa, kA), yA = seg_ld(Ya, kA);
+          const double xB = seg_ld(Xa, kB), yB = seg_ld(Ya, kB);
+          double uxA = 0, uyA = 0, uzA = 0, uxB = 0, uyB = 0, uzB = 0;
+          if (PUSH) {
+            uxA = seg_ld(Uxa, kA); uyA = seg_ld(Uya, kA); uzA = seg_ld(Uza, kA);
+            uxB = seg_ld(Uxa, kB); uyB = seg_ld(Uya, kB); uzB = seg_ld(Uza, kB);
+          }
+          // one particle at a time: interleaving the two would need twice the
+          // registers of one push and deposit
+          double x1, y1, qv = 0.0;
+          bool cr = one(k, xA, yA, uxA, uyA, uzA, x1, y1, qv);
+          if (DEPOSIT) record(cr, xA, yA, x1, y1, qv);
+          __builtin_amdgcn_sched_barrier(0);
+          cr = one(k + GROUP, xB, yB, uxB, uyB, uzB, x1, y1, qv);
+          if (DEPOSIT) record(cr, xB, yB, x1, y1, qv);
         }
-        // one particle at a time: interleaving the two would need twice the
-        // registers of one push and deposit
-        double x1, y1, qv = 0.0;
-        bool cr = one(k, m, xA, yA, uxA, uyA, uzA, x1, y1, qv);
-        if (DEPOSIT) record(cr, m, xA, yA, x1, y1, qv);
-        __builtin_amdgcn_sched_barrier(0);
-        cr = one(k + GROUP, m + 1, xB, yB, uxB, uyB, uzB, x1, y1, qv);
-        if (DEPOSIT) record(cr, m + 1, xB, yB, x1, y1, qv);
-      }
-      if (DEPOSIT) {
-        // add the stay-in-cell stencils of this species over the 8 lanes
+        more = k - sub < ke;
+        if (DEPOSIT) {
+          // add the stay-in-cell stencils of this species over the 8 lanes
 #pragma unroll
-        for (int c = 0; c < 27; ++c) {
-          const double v = group_sum(core[c]);
-          core[c] = 0.0;
-          if (sub == 0) cb[core_slot(c)] += v;
+          for (int c = 0; c < 27; ++c) {
+            const double v = group_sum(core[c]);
+            core[c] = 0.0;
+            if (sub == 0) cb[core_slot(c)] += v;
+          }
+          __builtin_amdgcn_wave_barrier();     // the group reads what its lanes listed
+          const int nl = __shfl(mcnt, 0, GROUP);
+          if (__ballot(nl > 0)) {
+            // cell-crossing particles: full 5x5 stencils, one component at a time
+            crossing_pass<0>(cb, sub, L, nl, i, j, q, P);
+            crossing_pass<1>(cb, sub, L, nl, i, j, q, P);
+            crossing_pass<2>(cb, sub, L, nl, i, j, q, P);
+          }
+          __builtin_amdgcn_wave_barrier();     // the list is read before it is filled again
+          mcnt = 0;
         }
       }
-      mcnt = __shfl(mcnt, 0, GROUP);
-      __builtin_amdgcn_wave_barrier();         // the group reads what its lanes listed
-      const int nl = DEPOSIT ? min(mcnt, MCAP) : 0;
-      if (DEPOSIT && __ballot(nl > 0 || mask != 0ULL || ke - ka > GROUP * 64)) {
-        // cell-crossing particles: full 5x5 stencils, one component at a time
-        // (the banks' new state stream-ordered after this lane's own writes)
-        crossing_pass<0>(cb, sub, L, nl, mask, ka, ke, base, xa, ya, xb, yb, uxb, uyb, uzb, i, j,
-                         q, P);
-        crossing_pass<1>(cb, sub, L, nl, mask, ka, ke, base, xa, ya, xb, yb, uxb, uyb, uzb, i, j,
-                         q, P);
-        crossing_pass<2>(cb, sub, L, nl, mask, ka, ke, base, xa, ya, xb, yb, uxb, uyb, uzb, i, j,
-                         q, P);
-      }
-      __builtin_amdgcn_wave_barrier();         // the list is read before the next species
     }
   }
-  if (!ok) atomicOr(derr, DERR_JUMP);
+  if (bad) atomicOr(derr, bad);
   if (DEPOSIT) {
     __syncthreads();
     // assemble the workgroup tile [b][t][comp] in a fixed order
@@ -503,6 +493,446 @@ __global__ __launch_bounds__(256, 3) void k_particle(
       for (int gg = glo; gg <= ghi; ++gg) sum += acc_at(cellbuf + gg * NACC, comp, t - gg, b);
       out[e] = sum;
     }
+  }
+}
+
+// ------------------------------------------------ the resident step's push
+// Push, particle_x, Esirkepov deposit and the row order's inputs in one pass
+// over the particles: read through the pending order (Order::perm), written
+// sorted, 40 bytes each way, plus 4 bytes of index and 2 of code.
+//
+// The decomposition is k_particle's, a group of 8 lanes per cell, with steps
+// of 8 consecutive particles (one per lane) from the 8-particle boundary at
+// or below the cell's first: a step's five loads were issued during the step
+// before it, its index one more step ahead.  Steps of 16 (two per lane) left
+// a third of the lanes idle at 64 particles per cell (a wavefront's eight
+// cells step together), steps of 8 leave a fifth.
+//
+// Per cell, over all species: 21 stay-in-cell stencil values per lane
+// (wm: of the 27 values of the 3 x 3 cores, Jx's last column and Jy's last
+// row carry the sum of all three shape changes, which is zero), and a list of
+// the crossing particles in LDS, whose full stencils are summed at the end,
+// or whenever some cell's list could overflow in the next step.
+//
+// The TSC gather of particle.f90:107-129 inside a cell is a biquadratic in
+// the in-cell offsets: nine coefficients per field and cell (LDS), 8 FMAs a
+// field.
+constexpr int MLC = 16;               // a cell's listed movers
+constexpr int CFN = 10;               // doubles per field and cell (9 coefficients, padded)
+constexpr int NCORE = 21;
+
+// w-(o) = 1/2 - o + o^2/2, w0(o) = 1/2 + o - o^2, w+(o) = o^2/2:
+// sum_ab T(a, b) w_a(ox) w_b(oy) = sum_ij C_ij ox^i oy^j, C row i at 3 i.
+__device__ inline void cell_coeffs(double *cf, const double *Tk) {
+  double R[3][3];
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    const double m = Tk[b * TW], z = Tk[b * TW + 1], p = Tk[b * TW + 2];
+    R[b][0] = 0.5 * (m + z);
+    R[b][1] = z - m;
+    R[b][2] = 0.5 * ((m - z) + (p - z));
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    cf[3 * i] = 0.5 * (R[0][i] + R[1][i]);
+    cf[3 * i + 1] = R[1][i] - R[0][i];
+    cf[3 * i + 2] = 0.5 * ((R[0][i] - R[1][i]) + (R[2][i] - R[1][i]));
+  }
+}
+
+// 1 / sqrt(a), a > 0 normal: the hardware's estimate (to about 2^-23) and two
+// Newton steps in FMAs, within an ulp.
+__device__ inline double rsqrt64(double a) {
+  double y = __builtin_amdgcn_rsq(a);
+  double h = 0.5 * y;
+  double e = fma(-a * y, h, 0.5);      // 1/2 - a y^2 / 2
+  y = fma(y, e, y);
+  h = 0.5 * y;
+  const double g = a * y;              // sqrt(a) to twice the estimate's bits
+  e = fma(-g, h, 0.5);
+  return fma(y, e, y);
+}
+
+__device__ inline PushOut boris_coeffs(const double2 *cf, double ox, double oy, double x, double y,
+                                       double ux, double uy, double uz, const PP &P, double fac1,
+                                       double txxx, double fac2) {
+  double f[6];
+#pragma unroll
+  for (int kk = 0; kk < 6; ++kk) {
+    const int k = (kk + 3) % 6;
+    const double2 a = cf[5 * k], b = cf[5 * k + 1], c = cf[5 * k + 2], d = cf[5 * k + 3],
+                  e = cf[5 * k + 4];
+    const double r0 = fma(oy, fma(oy, b.x, a.y), a.x);
+    const double r1 = fma(oy, fma(oy, c.y, c.x), b.y);
+    const double r2 = fma(oy, fma(oy, e.x, d.y), d.x);
+    f[k] = fma(ox, fma(ox, r2, r1), r0);
+    __asm__ volatile("" ::: "memory");   // one field's coefficients in registers at a time
+  }
+  const double bpx = f[0], bpy = f[1], bpz = f[2];
+  const double epx = f[3], epy = f[4], epz = f[5];
+  // particle.f90:131-161
+  double uvm1 = ux + fac1 * epx;
+  double uvm2 = uy + fac1 * epy;
+  double uvm3 = uz + fac1 * epz;
+  const double g2 = P.c * P.c + uvm1 * uvm1 + uvm2 * uvm2 + uvm3 * uvm3;
+  const double igam = rsqrt64(g2);
+  const double g1 = g2 * igam, gam = fma(fma(-g1, g1, g2), 0.5 * igam, g1);   // sqrt(g2)
+  const double fac1r = fac1 * igam;
+  const double fac2r = fac2 / (gam + txxx * (bpx * bpx + bpy * bpy + bpz * bpz) * igam);
+  const double uvm4 = uvm1 + fac1r * (uvm2 * bpz - uvm3 * bpy);
+  const double uvm5 = uvm2 + fac1r * (uvm3 * bpx - uvm1 * bpz);
+  const double uvm6 = uvm3 + fac1r * (uvm1 * bpy - uvm2 * bpx);
+  uvm1 = uvm1 + fac2r * (uvm5 * bpz - uvm6 * bpy);
+  uvm2 = uvm2 + fac2r * (uvm6 * bpx - uvm4 * bpz);
+  uvm3 = uvm3 + fac2r * (uvm4 * bpy - uvm5 * bpx);
+  PushOut o;
+  o.ux = uvm1 + fac1 * epx;
+  o.uy = uvm2 + fac1 * epy;
+  o.uz = uvm3 + fac1 * epz;
+  const double ig = rsqrt64(1.0 + (o.ux * o.ux + o.uy * o.uy + o.uz * o.uz) * P.ic2);
+  o.x = x + o.ux * P.delt * ig;
+  o.y = y + o.uy * P.delt * ig;
+  o.ig = ig;
+  return o;
+}
+
+// Weights at the cell's -1, 0, +1 neighbours for the old offset o0 and their
+// change to o1 in the same cell, taken directly: d+ = (o1 - o0)(o1 + o0) / 2,
+// d- = (o1 - o0)(o1 + o0 - 2) / 2, d0 = -(d- + d+).
+__device__ inline void shape_delta(double o0, double o1, double *s, double *d) {
+  const double t = 1.0 - o0;
+  s[0] = (0.5 * t) * t;
+  s[2] = (0.5 * o0) * o0;
+  s[1] = (1.0 - s[0]) - s[2];
+  const double hd = 0.5 * (o1 - o0), sg = o1 + o0;
+  d[2] = hd * sg;
+  d[0] = hd * (sg - 2.0);
+  d[1] = -(d[0] + d[2]);
+}
+
+// A particle that stays in its cell: Jx (a < 2, b < 3) at 0..5, Jy (a < 3,
+// b < 2) at 6..11, Jz (3 x 3) at 12..20.  Jx and Jy weigh -q dx/dt times the
+// running sum of the shape changes: -qc d-, then qc d+ (their sum is zero).
+// Jz's s0x s0y + dx s0y / 2 + s0x dy / 2 + dx dy / 3 is X Y + dx dy / 12 with
+// X = s0x + dx / 2, Y = s0y + dy / 2.
+__device__ inline void core_add(double *core, double ox0, double oy0, double ox1, double oy1,
+                                double qc, double qv) {
+  double sx[3], sy[3], dx[3], dy[3], X[3], Y[3];
+  shape_delta(ox0, ox1, sx, dx);
+  shape_delta(oy0, oy1, sy, dy);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    X[k] = fma(0.5, dx[k], sx[k]);
+    Y[k] = fma(0.5, dy[k], sy[k]);
+  }
+  const double wx0 = -(qc * dx[0]), wx1 = qc * dx[2];
+  const double wy0 = -(qc * dy[0]), wy1 = qc * dy[2];
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    core[b] = fma(wx0, Y[b], core[b]);
+    core[3 + b] = fma(wx1, Y[b], core[3 + b]);
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    core[6 + 2 * a] = fma(X[a], wy0, core[6 + 2 * a]);
+    core[7 + 2 * a] = fma(X[a], wy1, core[7 + 2 * a]);
+  }
+  const double qv12 = qv * (1.0 / 12.0);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const double za = qv * X[a], zb = qv12 * dx[a];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      double &c = core[12 + a * 3 + b];
+      c = fma(za, Y[b], c);
+      c = fma(zb, dy[b], c);
+    }
+  }
+}
+
+// Slot of core value e in the 65-value cell layout of acc_at().
+__device__ inline int core_at(int e) {
+  if (e < 6) return (1 + e / 3) * 5 + 1 + e % 3;                 // Jx: tile column 2 + a
+  if (e < 12) return 20 + (1 + (e - 6) / 2) * 4 + 1 + (e - 6) % 2;   // Jy: tile row 2 + b
+  return 40 + (1 + (e - 12) / 3) * 5 + 1 + (e - 12) % 3;
+}
+
+template <int CTRL>
+__device__ inline double dpp_f64(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
+}
+
+// Sums of M values over the 8 lanes of a group, by halving: in each of three
+// exchanges a lane keeps one half of the values and adds its partner's share
+// of them (partners: the mirrored lane, then lane xor 2, then lane xor 1).
+// Lane sub ends with the sums of values slot .. slot + M / 8 - 1 in v[0..],
+// slot = (sub >> 2) M / 2 + (sub >> 1 & 1) M / 4 + (sub & 1) M / 8.  About 6
+// instructions a value against 12 for a butterfly of each and one lane
+// writing them all.
+template <int M, int CTRL>
+__device__ inline void halve(double *v, bool up) {
+#pragma unroll
+  for (int e = 0; e < M / 2; ++e) {
+    const double a = v[e], b = v[M / 2 + e];
+    const double keep = up ? b : a, give = up ? a : b;
+    v[e] = keep + dpp_f64<CTRL>(give);
+  }
+}
+template <int M>
+__device__ inline int group_sums(double *v, int sub) {
+  static_assert(M % 8 == 0, "three halvings");
+  halve<M, 0x141>(v, sub & 4);           // row_half_mirror: lane 7 - sub
+  halve<M / 2, 0x4E>(v, sub & 2);        // quad_perm [2,3,0,1]
+  halve<M / 4, 0xB1>(v, sub & 1);        // quad_perm [1,0,3,2]
+  return ((sub >> 2) & 1) * (M / 2) + ((sub >> 1) & 1) * (M / 4) + (sub & 1) * (M / 8);
+}
+
+// One current component of a cell's listed movers, added to its sums.
+template <int C>
+__device__ inline void mover_pass(double *cb, int sub, const double *L, const uint8_t *Ls, int nl,
+                                  int i, int j, const PP &P) {
+  constexpr int N = C == 2 ? 25 : 20, M = C == 2 ? 32 : 24;
+  double acc[M];
+#pragma unroll
+  for (int k = 0; k < M; ++k) acc[k] = 0.0;
+  for (int e = sub; e < nl; e += GROUP) {
+    Move m;
+    make_move(m, L[e], L[MLC + e], L[2 * MLC + e], L[3 * MLC + e], i, j, P);
+    stencil<C>(acc, m, P.q[Ls[e]] * P.qc_scale, L[4 * MLC + e]);
+  }
+  const int off = C == 0 ? 0 : (C == 1 ? 20 : 40), s0 = group_sums<M>(acc, sub);
+#pragma unroll
+  for (int k = 0; k < M / 8; ++k)
+    if (s0 + k < N) cb[off + s0 + k] += acc[k];
+}
+
+struct Part {
+  double x, y, ux, uy, uz;
+};
+
+template <int SRC>
+__global__ __launch_bounds__(256, 3) void k_push_step(PP P, const int *__restrict__ cumcnt,
+                                                      const double *__restrict__ tmp, int TX,
+                                                      size_t tps, Rec64 A, Rec64 B, Order O,
+                                                      double *__restrict__ part,
+                                                      int *__restrict__ derr) {
+  __shared__ __attribute__((aligned(16))) double CF[CHUNK * 6 * CFN];
+  __shared__ double cellbuf[CHUNK * NACC];
+  // the movers' lists [x0 | y0 | x1 | y1 | q v_z][entry] per cell; before
+  // them, the chunk's cell-centred fields
+  __shared__ double mvl[CHUNK * 5 * MLC];
+  __shared__ uint8_t mvs[CHUNK * MLC];       // the entries' species
+  __shared__ int mk[CHUNK * 4];              // moves out of a cell: left, right, others
+  static_assert(6 * 3 * TW <= CHUNK * 5 * MLC, "the fields fit the lists' space");
+  double *T = mvl;
+  const int chunk = blockIdx.x;
+  const int jl = blockIdx.y;                 // row j = nys + jl
+  const int j = P.nys + jl;
+  const int i0 = P.nxgs + chunk * CHUNK;
+  const int ncell = min(CHUNK, P.nx - chunk * CHUNK);
+  load_tmp_tile(T, tmp, TX, tps, jl, chunk * CHUNK, min(TW, ncell + 2));
+  for (int e = threadIdx.x; e < CHUNK * NACC; e += 256) cellbuf[e] = 0.0;
+  __syncthreads();
+  if (threadIdx.x < CHUNK * 6) {
+    const int c = threadIdx.x % CHUNK, k = threadIdx.x / CHUNK;
+    cell_coeffs(CF + (c * 6 + k) * CFN, T + k * 3 * TW + c);
+  }
+  __syncthreads();
+  const int g = threadIdx.x / GROUP;
+  const int sub = threadIdx.x % GROUP;
+  const int il = chunk * CHUNK + g, i = i0 + g;
+  double *cb = cellbuf + g * NACC;
+  double *L = mvl + g * 5 * MLC;
+  uint8_t *Ls = mvs + g * MLC;
+  const double2 *cf = (const double2 *)(CF + g * 6 * CFN);
+  const int wg = (threadIdx.x & 63) / GROUP;   // the group's place in its wavefront
+  int bad = 0;
+  if (g < ncell) {
+    double core[24];
+    int mcnt = 0;                              // the list's entries
+    int kb = 0, ke = 0, k = 0;
+    unsigned pn = 0;                           // the source of the step after next's particle
+    Part nxt{};                                // the next step's particle
+    const double *Xa = nullptr, *Ya = nullptr, *Uxa = nullptr, *Uya = nullptr, *Uza = nullptr;
+    const unsigned *Pm = nullptr;
+    auto src = [&](int q) {
+      q = min(max(q, kb), ke - 1);
+      return SRC == SRC_SLOT ? (unsigned)q : Pm[q];
+    };
+    auto load = [&](unsigned p) {
+      if (SRC == SRC_PERM64)
+        return Part{Xa[(size_t)p], Ya[(size_t)p], Uxa[(size_t)p], Uya[(size_t)p], Uza[(size_t)p]};
+      return Part{seg_ld(Xa, (int)p), seg_ld(Ya, (int)p), seg_ld(Uxa, (int)p), seg_ld(Uya, (int)p),
+                  seg_ld(Uza, (int)p)};
+    };
+    bool fresh = true, empty = true;
+    for (int s = 0;;) {
+      if (empty) {
+#pragma unroll
+        for (int e = 0; e < 24; ++e) core[e] = 0.0;
+        empty = false;
+      }
+      const size_t seg = (size_t)s * P.ny + jl, base = seg * (size_t)P.cap;
+      const double q = P.q[s], r = P.r[s];
+      const double fac1 = q / r * 0.5 * P.delt;
+      const double txxx = fac1 * fac1;
+      const double fac2 = q * P.delt / r;
+      const double qc = q * P.qc_scale;
+      if (fresh) {
+        const int *cc = cumcnt + seg * (size_t)(P.nx + 1) + il;
+        kb = max(0, cc[0]);
+        ke = min(P.cap, cc[1]);
+        if (kb >= ke) ke = kb;
+        k = kb - kb % GROUP + sub;
+        const size_t sb = SRC == SRC_SLOT ? base : (size_t)s * P.ny * (size_t)P.cap;
+        Xa = A.x + sb;
+        Ya = A.y + sb;
+        Uxa = A.ux + sb;
+        Uya = A.uy + sb;
+        Uza = A.uz + sb;
+        Pm = O.perm + base;
+        if (sub < 4) mk[g * 4 + sub] = 0;
+        if (kb == ke) k = ke + sub;
+        fresh = false;
+      }
+      if (k - sub < ke) {
+        nxt = load(src(k));
+        pn = src(k + GROUP);
+      }
+      double *Xb = B.x + base, *Yb = B.y + base;
+      double *Uxb = B.ux + base, *Uyb = B.uy + base, *Uzb = B.uz + base;
+      uint16_t *Cd = O.code + base;
+      for (; k - sub < ke && __ballot(mcnt > MLC - GROUP) == 0ULL; k += GROUP) {
+        const Part c = nxt;
+        nxt = load(pn);
+        pn = src(k + 2 * GROUP);
+        bool cross = false;
+        double qv = 0.0, x1 = 0.0, y1 = 0.0;
+        if (k >= kb && k < ke) {
+          const double ox = c.x * P.d_delx - i, oy = c.y * P.d_delx - j;
+          PushOut o = boris_coeffs(cf, ox, oy, c.x, c.y, c.ux, c.uy, c.uz, P, fac1, txxx, fac2);
+          if (P.inj) injection_edge(o.x, o.ux, o.uy, o.uz, P);
+          x1 = o.x;
+          y1 = o.y;
+          const int i2 = (int)(x1 * P.d_delx), j2 = (int)(y1 * P.d_delx);
+          cross = i2 != i || j2 != j;
+          // field.f90:270's v_z = u_z / gamma with the push's 1 / gamma of the
+          // same u, except where the shock's injection edge may have
+          // reflected it
+          const double gvz = !P.inj ? o.uz * o.ig
+                                    : o.uz / sqrt(1.0 + (o.ux * o.ux + o.uy * o.uy + o.uz * o.uz) /
+                                                            (P.c * P.c));
+          qv = q * gvz;
+          if (!cross) core_add(core, ox, oy, x1 * P.d_delx - i, y1 * P.d_delx - j, qc, qv);
+          unsigned cd = (unsigned)il << 2;
+          if (cross || P.xmode == 2) {
+            // particle_x and particle_y of the stored state (the deposit takes
+            // the unwrapped one), as boundary_periodic.f90 and the wall
+            // families' particle_x write them
+            if (!(i2 - i >= -1 && i2 - i <= 1)) bad |= DERR_JUMP;
+            int inew = i2;
+            if (P.xmode == 1) {
+              if (i2 < P.nxgs) o.x = wm_edges::add_rd(o.x, P.spanx);
+              else if (i2 >= P.nxgs + P.nx) o.x = wm_edges::add_rd(o.x, -P.spanx);
+              inew = (int)o.x;
+            } else if (P.xmode == 2) {
+              const bool lo = i2 < P.xs + 1, hi = i2 >= P.xe - 1;
+              if (lo || hi) {
+                o.x = (lo ? P.wl : P.wr) - o.x;
+                o.ux = -o.ux;
+                o.uy = -o.uy;
+                o.uz = -o.uz;
+                inew = (int)o.x;
+              }
+            }
+            const int d = j2 - j;
+            if (j2 < P.nys) o.y = wm_edges::add_rd(o.y, P.spany);
+            else if (j2 >= P.nys + P.ny) o.y = wm_edges::add_rd(o.y, -P.spany);
+            int cn = inew - P.nxgs;
+            if (cn < 0 || cn >= P.nx) {
+              bad |= DERR_RANGE;
+              cn = min(max(cn, 0), P.nx - 1);
+            }
+            if (d < -1 || d > 1) bad |= DERR_JUMP;
+            int dc = cn - il;
+            if (P.xmode == 1) dc = dc == P.nx - 1 ? -1 : (dc == 1 - P.nx ? 1 : dc);
+            const bool out = d == 1 || d == -1, far = !out && (dc < -1 || dc > 1);
+            cd = (unsigned)cn << 2 | (out ? (d == 1 ? WM_CODE_UP : WM_CODE_DOWN)
+                                          : (far ? WM_CODE_FAR : WM_CODE_STAY));
+            if (far) {                         // (a wall's mirror from a cell beyond it)
+              atomicAdd(O.farcnt + seg * P.nx + cn, 1);
+              O.far[seg] = 1;
+            }
+            if (out || dc != 0) atomicAdd(&mk[g * 4 + (out || far ? 2 : (dc < 0 ? 0 : 1))], 1);
+          }
+          Cd[k] = (uint16_t)cd;
+          seg_st(Xb, k, o.x);
+          seg_st(Yb, k, o.y);
+          seg_st(Uxb, k, o.ux);
+          seg_st(Uyb, k, o.uy);
+          seg_st(Uzb, k, o.uz);
+        }
+        // a crossing particle goes to the cell's list in (step, lane) order,
+        // ranked by a ballot over the group
+        const unsigned gb = (unsigned)(__ballot(cross) >> (GROUP * wg)) & 0xFFu;
+        if (cross) {
+          const int e = mcnt + __popc(gb & ((1u << sub) - 1u));
+          L[e] = c.x;
+          L[MLC + e] = c.y;
+          L[2 * MLC + e] = x1;
+          L[3 * MLC + e] = y1;
+          L[4 * MLC + e] = qv;
+          Ls[e] = (uint8_t)s;
+        }
+        mcnt += __popc(gb);
+      }
+      if (__ballot(k - sub < ke) == 0ULL) {    // every cell's particles of this species are done
+        __builtin_amdgcn_wave_barrier();
+        if (sub == 0) {
+          const int l = mk[g * 4], rr = mk[g * 4 + 1], o = mk[g * 4 + 2];
+          O.kind[seg * P.nx + il] = make_int4(l, ke - kb - l - rr - o, rr, o);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (++s < P.nsp) {
+          fresh = true;
+          continue;
+        }
+      }
+      // the cell's sums so far (its accumulators are free for the lists then)
+      {
+        const int s0 = group_sums<24>(core, sub);
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (s0 + e < NCORE) cb[core_at(s0 + e)] += core[e];
+        empty = true;
+      }
+      __builtin_amdgcn_wave_barrier();         // the group reads what its lanes listed
+      if (__ballot(mcnt > 0)) {
+        // full 5x5 stencils, one component at a time
+        mover_pass<0>(cb, sub, L, Ls, mcnt, i, j, P);
+        mover_pass<1>(cb, sub, L, Ls, mcnt, i, j, P);
+        mover_pass<2>(cb, sub, L, Ls, mcnt, i, j, P);
+        mcnt = 0;
+      }
+      __builtin_amdgcn_wave_barrier();         // the list is read before it is filled again
+      if (s == P.nsp) break;
+    }
+  }
+  if (bad) atomicOr(derr, bad);
+  __syncthreads();
+  // assemble the workgroup tile [b][t][comp] in a fixed order
+  double *out = part + ((size_t)jl * P.nchunk + chunk) * TILE;
+  for (int e = threadIdx.x; e < TILE; e += 256) {
+    const int comp = e % 3;
+    const int t = (e / 3) % DW;
+    const int b = e / (3 * DW);
+    double sum = 0.0;
+    const int glo = max(0, t - 4), ghi = min(ncell - 1, t);
+    for (int gg = glo; gg <= ghi; ++gg) sum += acc_at(cellbuf + gg * NACC, comp, t - gg, b);
+    out[e] = sum;
   }
 }
 
@@ -564,6 +994,7 @@ PP make_pp(const wm_ctx *ctx) {
   P.d_delx = 1.0 / g.delx;
   P.delt = g.delt;
   P.c = g.c;
+  P.ic2 = 1.0 / (g.c * g.c);
   P.qc_scale = g.delx * (1.0 / g.delt);
   for (int s = 0; s < WM_MAXSP; ++s) {
     P.q[s] = s < g.nsp ? g.q[s] : 0.0;
@@ -575,23 +1006,22 @@ PP make_pp(const wm_ctx *ctx) {
   P.wl = 2.0 * (P.xs + 1) * g.delx;
   P.xend = 0.0;
   P.u0 = 0.0;
+  P.xmode = 0;
+  P.xe = ctx->xe > 0 ? ctx->xe : g.nxge;
+  P.spanx = (double)(g.nxge - g.nxgs + 1) * g.delx;
+  P.spany = (double)(g.nyge - g.nygs + 1) * g.delx;
+  P.wr = 2.0 * (P.xe - 1) * g.delx;
   return P;
 }
 
 template <bool PUSH, bool DEP>
-int launch_particle(wm_ctx *ctx, int a, int b, bool inj = false) {
-  PP P = make_pp(ctx);
-  if (inj) {
-    P.inj = 1;
-    P.u0 = ctx->u0;
-    P.xend = wm_injection_xend(ctx, ctx->u0);
-  }
-  dim3 grid(P.nchunk, P.ny);
+int launch_particle(wm_ctx *ctx, int a, int b) {
+  const PP P = make_pp(ctx);
   const int TX = ctx->g.nx + 2;
   const size_t tps = (size_t)TX * (size_t)(ctx->g.ny + 2);
   const PBank &A = ctx->bank[a];
   const PBank &B = ctx->bank[b];
-  hipLaunchKernelGGL((k_particle<PUSH, DEP>), grid, dim3(256), 0, ctx->stream, P,
+  hipLaunchKernelGGL((k_particle<PUSH, DEP>), dim3(P.nchunk, P.ny), dim3(256), 0, ctx->stream, P,
                      ctx->cumcnt, ctx->tmp, TX, tps, A.x, A.y, A.ux, A.uy, A.uz,
                      B.x, B.y, B.ux, B.uy, B.uz, ctx->dep_part, ctx->derr);
   WM_HIP(hipGetLastError());
@@ -615,10 +1045,31 @@ int wm_k_cell_fields(wm_ctx *ctx) {
 
 int wm_k_push(wm_ctx *ctx, int src, int dst) { return launch_particle<true, false>(ctx, src, dst); }
 int wm_k_deposit(wm_ctx *ctx, int oldb, int newb) { return launch_particle<false, true>(ctx, oldb, newb); }
-// The device-resident shock step fuses its injection edge between the push
-// and the current.
-int wm_k_push_deposit(wm_ctx *ctx, int src, int dst) {
-  return launch_particle<true, true>(ctx, src, dst, ctx->bcf == WM_BC_SHOCK);
+// The resident step's push, from bank 0 (read in its order, if one is
+// pending) into bank 1, which becomes bank 0: the shock's injection edge
+// before the current, the periodic wrap or the reconnection's walls
+// (app.f90:104-105, proj/reconnection/app.f90:104; the shock has neither,
+// proj/shock/app.f90:113) as it is stored.
+int wm_k_push_step(wm_ctx *ctx) {
+  PP P = make_pp(ctx);
+  if (ctx->bcf == WM_BC_SHOCK) {
+    P.inj = 1;
+    P.u0 = ctx->u0;
+    P.xend = wm_injection_xend(ctx, ctx->u0);
+  }
+  P.xmode = ctx->bcf == WM_BC_PERIODIC ? 1 : ctx->bcf == WM_BC_RECONNECTION ? 2 : 0;
+  const int TX = ctx->g.nx + 2;
+  const size_t tps = (size_t)TX * (size_t)(ctx->g.ny + 2);
+  const Order O{ctx->perm, ctx->code, ctx->kind, ctx->farcnt, ctx->far};
+  // a species' plane below 4 GB is addressed by 32-bit byte offsets
+  auto kernel = !ctx->perm_valid                              ? k_push_step<SRC_SLOT>
+                : (size_t)P.ny * P.cap <= (size_t)1 << 29 ? k_push_step<SRC_PERM32>
+                                                              : k_push_step<SRC_PERM64>;
+  hipLaunchKernelGGL(kernel, dim3(P.nchunk, P.ny), dim3(256), 0, ctx->stream, P, ctx->cumcnt,
+                     ctx->tmp, TX, tps, ctx->bank[0], ctx->bank[1], O, ctx->dep_part, ctx->derr);
+  WM_HIP(hipGetLastError());
+  std::swap(ctx->bank[0], ctx->bank[1]);
+  return WM_OK;
 }
 
 int wm_k_deposit_gather(wm_ctx *ctx) {
