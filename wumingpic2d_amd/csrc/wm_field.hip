@@ -15,6 +15,7 @@
 // the last workgroup sums the partials in a fixed order and performs the
 // scalar update of the reference on the device.
 #include "wm_internal.h"
+#include "wm_solve.h"
 
 #include <math.h>
 
@@ -22,22 +23,7 @@ namespace {
 
 constexpr double PI = 3.141592653589793115997963468544185161590576171875;  // field.f90:13
 
-struct FC {      // field constants, field.f90:53-57
-  double f1, f2, f3, f4, f5, gfac, delt;
-};
-
-FC make_fc(const wm_grid &g) {
-  FC f;
-  f.f1 = g.c * g.delt / g.delx;
-  f.f2 = g.gfac * f.f1 * f.f1;
-  f.f3 = 4.0 * PI * g.delx / g.c;
-  const double t = g.delx / (g.c * g.delt * g.gfac);
-  f.f4 = 4.0 + t * t;
-  f.f5 = t * t;
-  f.gfac = g.gfac;
-  f.delt = g.delt;
-  return f;
-}
+using FC = SolveConst;
 
 // ------------------------------------------------------------ boundaries
 // boundary_periodic__curre (boundary_periodic.f90:357-506), row phase: one
@@ -88,7 +74,8 @@ __global__ void k_curre_cols(FieldGeom fg, double *uj) {
 // boundary_periodic__dfield (boundary_periodic.f90:263-345): ghost rows of
 // the interior columns x0 .. x0 + cnt - 1 (all of them, or the wall
 // families' active ones, boundary_shock.f90:326-392).
-__global__ void k_dfield_rows(FieldGeom fg, double *df, int ncomp, int x0, int cnt) {
+__global__ void k_dfield_rows(FieldGeom fg, double *df, int ncomp, int x0, int cnt, SolveGate gate) {
+  if (gate.closed()) return;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= cnt * ncomp) return;
   const int li = 2 + x0 + t % cnt, comp = t / cnt;
@@ -102,7 +89,8 @@ __global__ void k_dfield_rows(FieldGeom fg, double *df, int ncomp, int x0, int c
 }
 
 // boundary_periodic.f90:347-352: ghost columns of every row.
-__global__ void k_dfield_cols(FieldGeom fg, double *df, int ncomp) {
+__global__ void k_dfield_cols(FieldGeom fg, double *df, int ncomp, SolveGate gate) {
+  if (gate.closed()) return;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= fg.gy * ncomp) return;
   const int lj = t % fg.gy, comp = t / fg.gy;
@@ -119,7 +107,8 @@ __global__ void k_dfield_cols(FieldGeom fg, double *df, int ncomp) {
 // at nxs - 1/2, By, Bz, Ex even about column nxs, zero at nxe+1 -- or the
 // reconnection's (boundary_reconnection.f90:350-359), whose right wall is
 // the mirror image at nxe - 1/2 and rewrites column nxe of Bx, Ey, Ez.
-__global__ void k_dfield_walls(FieldGeom fg, double *df, XSide X) {
+__global__ void k_dfield_walls(FieldGeom fg, double *df, XSide X, SolveGate gate) {
+  if (gate.closed()) return;
   const int lj = blockIdx.x * blockDim.x + threadIdx.x;
   if (lj >= fg.gy) return;
   double *R = df + (size_t)lj * fg.gx;
@@ -191,9 +180,9 @@ __global__ void k_rhs(FieldGeom fg, FC f, XSide X, const double *__restrict__ uf
 
 // delta-E (field.f90:154-171), interior cells.
 __global__ void k_delta_e(FieldGeom fg, FC f, XSide X, const double *__restrict__ uf,
-                          const double *__restrict__ uj, double *__restrict__ df) {
+                          const double *__restrict__ uj, double *__restrict__ df, SolveGate gate) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= fg.nx * fg.ny) return;
+  if (t >= fg.nx * fg.ny || gate.closed()) return;
   const int ii = t % fg.nx, jj = t / fg.nx;
   if (ii < X.xa || ii > X.xb) return;
   const size_t gx = fg.gx, ps = fg.ps;
@@ -201,7 +190,7 @@ __global__ void k_delta_e(FieldGeom fg, FC f, XSide X, const double *__restrict_
   const double *dB1 = df, *dB2 = df + ps, *dB3 = df + 2 * ps;
   const double *B1 = uf, *B2 = uf + ps, *B3 = uf + 2 * ps;
   const double *J1 = uj, *J2 = uj + ps, *J3 = uj + 2 * ps;
-  const double fpt = 4. * PI * f.delt;
+  const double fpt = f.fpt;
   df[3 * ps + c] = f.f1 * (f.gfac * (-dB3[c] + dB3[c + gx]) + (-B3[c] + B3[c + gx])) - fpt * J1[c];
   df[4 * ps + c] = -f.f1 * (f.gfac * (-dB3[c] + dB3[c + 1]) + (-B3[c] + B3[c + 1])) - fpt * J2[c];
   df[5 * ps + c] = f.f1 * (f.gfac * (-dB2[c] + dB2[c + 1] + dB1[c] - dB1[c + gx]) +
@@ -210,17 +199,18 @@ __global__ void k_delta_e(FieldGeom fg, FC f, XSide X, const double *__restrict_
 }
 
 // uf += df over every cell including ghosts (field.f90:176-184).
-__global__ void k_add(size_t n, double *__restrict__ uf, const double *__restrict__ df) {
+__global__ void k_add(size_t n, double *__restrict__ uf, const double *__restrict__ df,
+                      SolveGate gate) {
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) uf[t] = uf[t] + df[t];
+  if (t < n && !gate.closed()) uf[t] = uf[t] + df[t];
 }
 // The same over columns nxs-2 .. nxe+2 only (an active range short of the
 // grid): ghost-inclusive columns xa .. xb + 4 of every row and component.
 __global__ void k_add_cols(FieldGeom fg, XSide X, double *__restrict__ uf,
-                           const double *__restrict__ df) {
+                           const double *__restrict__ df, SolveGate gate) {
   const int w = X.xb - X.xa + 5;
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)6 * fg.gy * w) return;
+  if (t >= (size_t)6 * fg.gy * w || gate.closed()) return;
   const int a = (int)(t % w);
   const size_t rc = t / w;                     // component * gy + row
   const size_t q = (rc / fg.gy) * fg.ps + (rc % fg.gy) * fg.gx + X.xa + a;
@@ -289,8 +279,6 @@ __device__ inline void partial_total(const double *partials, int nblk, double (*
 #pragma unroll
   for (int k = 0; k < NV; ++k) tot[k] = a[k];
 }
-
-__device__ inline int wrapm(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
 
 // XCD-aware workgroup order: the dispatcher deals workgroups round-robin to
 // the 8 XCDs; renumber them so that each XCD (own L2) sweeps a contiguous band
@@ -675,21 +663,22 @@ int wm_k_bc_curre(wm_ctx *ctx, double *uj) {
   return WM_OK;
 }
 
-int wm_k_bc_dfield(wm_ctx *ctx, double *df) {
+static int bc_dfield(wm_ctx *ctx, double *df, const SolveGate &gate) {
   const FieldGeom &fg = ctx->fg;
   const XSide X = wm_xside(ctx);
   const int cnt = X.xb - X.xa + 1;
   hipLaunchKernelGGL(k_dfield_rows, dim3(wm_cdiv(cnt * 6, 256)), dim3(256), 0, ctx->stream, fg, df,
-                     6, X.xa, cnt);
+                     6, X.xa, cnt, gate);
   if (X.wall)
     hipLaunchKernelGGL(k_dfield_walls, dim3(wm_cdiv(fg.gy, 256)), dim3(256), 0, ctx->stream, fg,
-                       df, X);
+                       df, X, gate);
   else
     hipLaunchKernelGGL(k_dfield_cols, dim3(wm_cdiv(fg.gy * 6, 256)), dim3(256), 0, ctx->stream, fg,
-                       df, 6);
+                       df, 6, gate);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }
+int wm_k_bc_dfield(wm_ctx *ctx, double *df) { return bc_dfield(ctx, df, SolveGate{}); }
 
 // phi(nxs-1:nxe+1, nys-1:nye+1) of component l on the device.
 int wm_k_bc_phi(wm_ctx *ctx, double *phi, int l) {
@@ -777,30 +766,70 @@ static int fcg_solve(wm_ctx *ctx, const CgArgs &A, int *its) {
   return WM_OK;
 }
 
-// RHS -> CG -> bc_dfield -> dE -> bc_dfield -> uf += df (field.f90:125-184).
-// The current uj must already be folded.
-int wm_k_field_solve(wm_ctx *ctx) {
+// delta E and uf += df with the boundaries' ghost cells (field.f90:150-184).
+static int field_update(wm_ctx *ctx, const SolveGate &gate) {
   const wm_grid &g = ctx->g;
   const FieldGeom &fg = ctx->fg;
   const FC f = make_fc(g);
   const int n = g.nx * g.ny;
   const XSide X = wm_xside(ctx);
-  hipLaunchKernelGGL(k_rhs, dim3(wm_cdiv(n, 256)), dim3(256), 0, ctx->stream, fg, f, X, ctx->uf,
-                     ctx->uj, ctx->gkl);
+  WM_TRY(bc_dfield(ctx, ctx->df, gate));
+  hipLaunchKernelGGL(k_delta_e, dim3(wm_cdiv(n, 256)), dim3(256), 0, ctx->stream, fg, f, X,
+                     ctx->uf, ctx->uj, ctx->df, gate);
   WM_HIP(hipGetLastError());
+  WM_TRY(bc_dfield(ctx, ctx->df, gate));
+  if (X.xa == 0 && X.xb == g.nx - 1) {
+    const size_t nall = 6 * fg.ps;
+    hipLaunchKernelGGL(k_add, dim3(wm_cdiv((long long)nall, 256)), dim3(256), 0, ctx->stream, nall,
+                       ctx->uf, ctx->df, gate);
+  } else {
+    const long long nadd = 6LL * fg.gy * (X.xb - X.xa + 5);
+    hipLaunchKernelGGL(k_add_cols, dim3(wm_cdiv(nadd, 256)), dim3(256), 0, ctx->stream, fg, X,
+                       ctx->uf, ctx->df, gate);
+  }
+  WM_HIP(hipGetLastError());
+  return WM_OK;
+}
 
+static CgArgs cg_args(const wm_ctx *ctx) {
+  const wm_grid &g = ctx->g;
+  const FC f = make_fc(g);
   CgArgs A;
-  A.nx = g.nx; A.ny = g.ny; A.gx = fg.gx; A.ps = fg.ps; A.n = (size_t)n;
+  A.nx = g.nx; A.ny = g.ny; A.gx = ctx->fg.gx; A.ps = ctx->fg.ps; A.n = (size_t)g.nx * g.ny;
   A.nbx = wm_cdiv(g.nx, CGB);
   A.nblk = A.nbx * g.ny;
   A.f4 = f.f4; A.f5 = f.f5; A.err = ctx->cg_err; A.ite_max = ctx->ite_max;
-  A.X = X;
+  A.X = wm_xside(ctx);
+  return A;
+}
+
+static int rhs(wm_ctx *ctx) {
+  hipLaunchKernelGGL(k_rhs, dim3(wm_cdiv((long long)ctx->g.nx * ctx->g.ny, 256)), dim3(256), 0,
+                     ctx->stream, ctx->fg, make_fc(ctx->g), wm_xside(ctx), ctx->uf, ctx->uj, ctx->gkl);
+  WM_HIP(hipGetLastError());
+  return WM_OK;
+}
+
+// Does the next solve begin with flexible CG?  The learned preconditioner was
+// trained on the periodic operator: the wall families solve with the
+// reference's plain CG.
+static bool flexible(const wm_ctx *ctx) {
+  return ctx->solver == WM_SOLVER_FCG && ctx->bcf == WM_BC_PERIODIC;
+}
+
+// Iteration counts of a solve: the plain solver's, after the flexible one's.
+static void solved(wm_ctx *ctx, const int *plain) {
+  for (int l = 0; l < 3; ++l) ctx->last_iters[l] = ctx->fcg_it[l] + plain[l];
+  if (flexible(ctx)) wm_pc_set_stats(ctx, ctx->fcg_it, plain);
+  ctx->cg_iters_total += ctx->last_iters[0] + ctx->last_iters[1] + ctx->last_iters[2];
+}
+
+// Plain CG by the streaming solver (gkl in place).
+static int stream_plain(wm_ctx *ctx) {
+  const CgArgs A = cg_args(ctx);
+  const XSide X = A.X;
   const dim3 grid(A.nblk, 3);
-  int fcg_it[3] = {0, 0, 0};
-  // the learned preconditioner was trained on the periodic operator: the
-  // wall families solve with the reference's plain CG
-  const bool fcg = ctx->solver == WM_SOLVER_FCG && !X.wall;
-  if (fcg) WM_TRY(fcg_solve(ctx, A, fcg_it));
+  const bool fcg = flexible(ctx);
   // the reference's plain CG; after flexible CG it recomputes the true
   // residual and only iterates if that misses the tolerance
   double *pbuf[2] = {ctx->cg_p[0], ctx->cg_p[1]};
@@ -854,27 +883,154 @@ int wm_k_field_solve(wm_ctx *ctx) {
   if (collect) WM_TRY(wm_pc_snapshot_fin(ctx));
   ctx->x0_fresh = x0 != nullptr && iters == 0;
   if (iters > 0) ctx->cg_hint = std::max(hs[0].ite, std::max(hs[1].ite, hs[2].ite));
-  for (int l = 0; l < 3; ++l) ctx->last_iters[l] = fcg_it[l] + hs[l].ite;
-  if (fcg) {
-    int fb[3] = {hs[0].ite, hs[1].ite, hs[2].ite};
-    wm_pc_set_stats(ctx, fcg_it, fb);
-  }
-  ctx->cg_iters_total += ctx->last_iters[0] + ctx->last_iters[1] + ctx->last_iters[2];
+  const int plain[3] = {hs[0].ite, hs[1].ite, hs[2].ite};
+  solved(ctx, plain);
+  return WM_OK;
+}
 
-  WM_TRY(wm_k_bc_dfield(ctx, ctx->df));
-  hipLaunchKernelGGL(k_delta_e, dim3(wm_cdiv(n, 256)), dim3(256), 0, ctx->stream, fg, f, X,
-                     ctx->uf, ctx->uj, ctx->df);
-  WM_HIP(hipGetLastError());
-  WM_TRY(wm_k_bc_dfield(ctx, ctx->df));
-  if (X.xa == 0 && X.xb == g.nx - 1) {
-    const size_t nall = 6 * fg.ps;
-    hipLaunchKernelGGL(k_add, dim3(wm_cdiv((long long)nall, 256)), dim3(256), 0, ctx->stream, nall,
-                       ctx->uf, ctx->df);
-  } else {
-    const long long nadd = 6LL * fg.gy * (X.xb - X.xa + 5);
-    hipLaunchKernelGGL(k_add_cols, dim3(wm_cdiv(nadd, 256)), dim3(256), 0, ctx->stream, fg, X,
-                       ctx->uf, ctx->df);
+// RHS, flexible CG if selected, then the reference's plain CG (field.f90:125-146,
+// 319-461), on chip where the grid fits.  The current uj must already be folded.
+int wm_field_launch(wm_ctx *ctx) {
+  const bool tiles = wm_tiles_fit(ctx), fcg = flexible(ctx);
+  for (int l = 0; l < 3; ++l) ctx->fcg_it[l] = 0;
+  if (fcg || !tiles) WM_TRY(rhs(ctx));
+  if (fcg) WM_TRY(fcg_solve(ctx, cg_args(ctx), ctx->fcg_it));
+  return tiles ? wm_k_tiles(ctx) : stream_plain(ctx);
+}
+
+int wm_field_update(wm_ctx *ctx) {
+  if (!wm_fused_update(ctx)) {
+    SolveGate gate;
+    if (ctx->tile_held) {
+      gate.abort_ = ctx->tile_abort;
+      gate.out = (const SolveOut *)ctx->tile_out;
+    }
+    WM_TRY(field_update(ctx, gate));
   }
+  return wm_k_update_report(ctx);
+}
+
+int wm_field_result(wm_ctx *ctx) {
+  if (!ctx->tile_held) return WM_OK;             // the streaming solver reported itself
+  bool gave_up = false;
+  int err = 0, ite[3];
+  WM_TRY(wm_tiles_result(ctx, &gave_up, &err, ite));
+  if (gave_up) {
+    WM_TRY(rhs(ctx));
+    WM_TRY(stream_plain(ctx));
+    WM_TRY(wm_field_update(ctx));
+    WM_HIP(hipStreamSynchronize(ctx->stream));
+    return WM_OK;
+  }
+  if (err) {
+    wm_set_error(ctx, WM_ERR_CG_ITEMAX, "********** stop at cgm after ite_max **********");
+    return WM_ERR_CG_ITEMAX;
+  }
+  ctx->x0_fresh = false;
+  solved(ctx, ite);
+  return WM_OK;
+}
+
+int wm_k_field_solve(wm_ctx *ctx) {
+  WM_TRY(wm_field_launch(ctx));
+  int st = wm_field_update(ctx);
+  if (st == WM_OK) {
+    WM_HIP(hipStreamSynchronize(ctx->stream));
+    st = wm_field_result(ctx);
+  }
+  wm_field_release(ctx);
+  return st;
+}
+
+// The deposit tiles (chunks of CHUNK cells, halo 2, [row][chunk][5][CHUNK +
+// 4][3]) summed into uj with the ghost cells folded and filled
+// (boundary_periodic.f90:357-506): a cell takes the tiles' values at its own
+// place and at its periodic images among the ghost-inclusive cells, and a
+// ghost cell what its image takes.  The walls fold in y only.  Per place:
+// source row offset ascending, chunk ascending.  FP32: also marks every
+// row's bins as awaiting the push's movers.  Bound by reading the tiles: 157 MB
+// at 1024 x 1024 in 16-cell chunks, 72 us (40 at a copy's rate); 5 us at 256 x
+// 64, where the gather and the folds were three launches.
+namespace {
+template <int CHUNK>
+__global__ __launch_bounds__(256) void k_current(FieldGeom fg, int nchunk, int wall,
+                                                 const double *__restrict__ part,
+                                                 double *__restrict__ uj, int *__restrict__ rowpend) {
+  constexpr int DW = CHUNK + 4, TILE = 5 * DW * 3;
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (rowpend && t < fg.ny) rowpend[t] = 1;
+  if (t >= fg.gx * fg.gy) return;
+  const int ny = fg.ny, nx = fg.nx;
+  const int li = t % fg.gx, lj = t / fg.gx;
+  // the rows and columns that fold here, the interior's own first
+  int row[4], nr = 0, colm[2], nc = 0;
+  if (ny == 1) {
+    // the reference's sequence of copies, each row its own neighbour
+    if (lj == 0 || lj == 4) {
+      row[nr++] = lj == 0 ? 1 : 3;
+      row[nr++] = lj;
+    } else {
+      row[nr++] = 2;
+      row[nr++] = 1;
+      row[nr++] = 3;
+    }
+  } else {
+    const int r0 = lj < 2 ? lj + ny : (lj >= ny + 2 ? lj - ny : lj);
+    row[nr++] = r0;
+    if (r0 - ny >= 0) row[nr++] = r0 - ny;
+    if (r0 + ny < fg.gy) row[nr++] = r0 + ny;
+  }
+  const int c0 = wall ? li : (li < 2 ? li + nx : (li >= nx + 2 ? li - nx : li));
+  colm[nc++] = c0;
+  if (!wall && c0 - nx >= 0) colm[nc++] = c0 - nx;
+  else if (!wall && c0 + nx < fg.gx) colm[nc++] = c0 + nx;
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+  for (int a = 0; a < nr; ++a)
+    for (int q = 0; q < nc; ++q) {
+      const int x = colm[q], y = row[a];
+      const int chi = min(x / CHUNK, nchunk - 1);
+      const int clo = chi > 0 && x - CHUNK * (chi - 1) < DW ? chi - 1 : chi;
+      // all loads before the first sum (rows off the grid read a neighbour's
+      // and add nothing)
+      double v[5][2][3];
+#pragma unroll
+      for (int b = 0; b < 5; ++b) {
+        const int jl = min(max(y - b, 0), ny - 1);   // source row: jl + (b - 2) = y - 2
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int c = k ? chi : clo;
+          const double *tp = part + ((size_t)jl * nchunk + c) * TILE +
+                             ((size_t)b * DW + min(x - CHUNK * c, DW - 1)) * 3;
+          v[b][k][0] = tp[0];
+          v[b][k][1] = tp[1];
+          v[b][k][2] = tp[2];
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < 5; ++b) {
+        if (y - b < 0 || y - b >= ny) continue;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          if (k == 0 && clo == chi) continue;
+          s0 += v[b][k][0];
+          s1 += v[b][k][1];
+          s2 += v[b][k][2];
+        }
+      }
+    }
+  uj[t] = s0;
+  uj[fg.ps + t] = s1;
+  uj[2 * fg.ps + t] = s2;
+}
+}  // namespace
+
+int wm_k_current(wm_ctx *ctx) {
+  const FieldGeom &fg = ctx->fg;
+  const int n = std::max(fg.gx * fg.gy, fg.ny);
+  const bool f32 = ctx->form == WM_FORM_FP32;
+  hipLaunchKernelGGL(f32 ? k_current<16> : k_current<32>, dim3(wm_cdiv(n, 256)), dim3(256), 0,
+                     ctx->stream, fg, wm_cdiv(fg.nx, f32 ? 16 : 32), ctx->bcf != WM_BC_PERIODIC,
+                     ctx->dep_part, ctx->uj, f32 ? ctx->rowpend : nullptr);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }

@@ -216,6 +216,7 @@ struct wm_ctx {
   hipEvent_t ev[32]{};
   bool ev_ready = false;
   int last_iters[3] = {0, 0, 0};
+  int fcg_it[3] = {0, 0, 0};     // flexible-CG iterations of the solve under way
   double phase_ms[8] = {0};
   int *cnt_scratch = nullptr;    // [nseg] counts for layout conversion
   // FP32 form: particles live in cell bins inside the row segments.  Bin
@@ -280,6 +281,18 @@ struct wm_ctx {
   // iterations queued before the first host check: the previous solve's
   // count, so a solve that converges as the last one did needs one check
   int fcg_hint = 2, cg_hint = 4;
+  // the solve on chip (wm_solve.hip): the other field planes its update
+  // writes, the workgroups' exchange buffers, tags used so far, its result
+  double *uf2 = nullptr;
+  unsigned long long *tile_sums = nullptr, *tile_edges = nullptr;
+  size_t tile_cap = 0;           // workgroups x groups the buffers hold
+  unsigned tile_tag = 1;
+  int *tile_abort = nullptr;
+  void *tile_out = nullptr;
+  int ncu = 0;                   // the device's CUs
+  int tile_rest = 0;             // solves to stream after one that gave up
+  int tile_held = 0;             // workgroups in flight (SolveSlots)
+  bool tile_swapped = false;     // uf and uf2 were exchanged for the update in flight
   bool x0_fresh = false;         // cg_x0 holds df's solution planes (the warm start)
   wm_pc *pc = nullptr;
   double *cg_z = nullptr, *cg_q = nullptr, *cg_x0 = nullptr;   // 3 planes nx*ny each
@@ -291,6 +304,7 @@ void wm_set_error(wm_ctx *ctx, int code, const char *fmt, ...);
 int wm_alloc_device(wm_ctx *ctx);
 int wm_check_derr(wm_ctx *ctx, const char *where);
 int wm_fetch_derr(wm_ctx *ctx, int *out);     // device error bits, cleared
+#define WM_PIN_REPORT 2048     // offset of the step's report in the pinned scratch
 int wm_report_derr(wm_ctx *ctx, int h, const char *where);
 
 // ---------------------------------------------------- kernel launch layer
@@ -299,13 +313,28 @@ int wm_k_cell_fields(wm_ctx *ctx);
 int wm_k_push(wm_ctx *ctx, int src, int dst);
 int wm_k_deposit(wm_ctx *ctx, int oldb, int newb);
 int wm_k_push_step(wm_ctx *ctx);   // the resident step's: push, deposit, particle_x, codes
-int wm_k_deposit_gather(wm_ctx *ctx);
 // Fields (wm_field.hip)
 int wm_k_bc_curre(wm_ctx *ctx, double *uj);
 XSide wm_xside(const wm_ctx *ctx);
 int wm_k_bc_dfield(wm_ctx *ctx, double *df);
 int wm_k_bc_phi(wm_ctx *ctx, double *phi, int l);   // phi(nxs-1:nxe+1, nys-1:nye+1)
-int wm_k_field_solve(wm_ctx *ctx);   // RHS .. uf += df (after the current is ready)
+int wm_k_current(wm_ctx *ctx);       // deposit tiles summed and folded into uj
+// RHS .. uf += df (after the current is ready).  A step launches the solve
+// and, once everything else of the step is ordered before it, the update with
+// the step's report; after the stream has been waited for it takes the result.
+// All three in one, waiting: wm_k_field_solve.
+int wm_field_launch(wm_ctx *ctx);
+int wm_field_update(wm_ctx *ctx);
+int wm_field_result(wm_ctx *ctx);
+void wm_field_release(wm_ctx *ctx);  // after an error: waits for the solve in flight
+int wm_k_field_solve(wm_ctx *ctx);
+// wm_solve.hip: the on-chip solve and, for the periodic box, its update
+bool wm_tiles_fit(wm_ctx *ctx);
+int wm_k_tiles(wm_ctx *ctx);
+bool wm_fused_update(const wm_ctx *ctx);
+int wm_k_update_report(wm_ctx *ctx);  // periodic; else the report alone
+int wm_tiles_result(wm_ctx *ctx, bool *gave_up, int *err, int *ite);
+struct SolveGate;
 int wm_k_energy(wm_ctx *ctx, int bank, double *out_host);
 // Particle boundaries (wm_bc.hip)
 int wm_k_particle_x(wm_ctx *ctx, int bank);
@@ -345,7 +374,6 @@ int wm_relayout(wm_ctx *ctx);        // listed blocks (segments) laid out anew, 
 int wm_k_cell_fields32(wm_ctx *ctx);
 int wm_k_push_deposit32(wm_ctx *ctx);   // in place on the bins (pending movers first)
 int wm_push32_pool();                     // movers one push workgroup lists
-int wm_k_deposit_gather32(wm_ctx *ctx);
 int wm_k_energy_kin32(wm_ctx *ctx, int bank, double *part, int nchunk);
 // Moment diagnostics (wm_mom.hip): CIC moments of bank 0 with cumcnt (FP64)
 // or of the settled bins (FP32) into ctx->mom (allocated by wm_mom_buffers on

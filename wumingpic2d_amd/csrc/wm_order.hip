@@ -448,6 +448,7 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
   const int64_t di0 = sub < D ? R.id[plane + de0.y] : 0;   // (the third)
   auto ballot16 = [&](bool b) { return (unsigned)(__ballot(b) >> gsh) & 0xFFFFu; };
   const unsigned below = (1u << sub) - 1u;
+  auto low16 = [](int n) { return n <= 0 ? 0u : n >= 16 ? 0xFFFFu : (1u << n) - 1u; };
   // displaced particles of a list (its first 16 in p) with slots below kb;
   // any inside [kb, ke)
   bool in = false;
@@ -467,6 +468,7 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
   int bR = sr + (o < nx - 1 ? (P.periodic && o + 1 == nx - 1 ? k0_.x : 0) : k0_.y + k1_.x) +
            lower(pR, dr0, Dr);
   int bL = sl + (o > 0 ? (o > 1 ? kll_.z : 0) + kl_.y : 0) + lower(pL, dl0, Dl);
+  int nbo = 0;             // stayers of the cell below this lane's displaced particle (the first 16)
   for (int k0 = kb; k0 < ke; k0 += PWIN * PG) {
     if (k0 > kb) fetch(k0);
 #pragma unroll
@@ -485,13 +487,28 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
         bR += __popc(mR);
         bL += __popc(mL);
       }
-      if (in && own_) {
-        const int f0 = moves ? (right ? dr0 : dl0) : d0, n = moves ? (right ? Dr : Dl) : D;
-        for (int i = 0; i < n; ++i) {
-          const int p = (int)dl[f0 + i].x;
-          dst += p >= kb && p < k;
+      if (in) {                                      // displaced slots among the cell's own
+        const bool stay = own_ && !moves;
+        for (int i = 0; i < min(D, PG); ++i) {
+          const int p = __shfl((int)de0.x, gsh + i, 64);
+          dst += stay && p >= kb && p < k;
         }
+        for (int i = 0; i < min(Dr, PG); ++i) {
+          const int p = __shfl(pR, gsh + i, 64);
+          dst += moves && right && p >= kb && p < k;
+        }
+        for (int i = 0; i < min(Dl, PG); ++i) {
+          const int p = __shfl(pL, gsh + i, 64);
+          dst += moves && !right && p >= kb && p < k;
+        }
+        const int f0 = moves ? (right ? dr0 : dl0) : d0, n = moves ? (right ? Dr : Dl) : D;
+        if (own_)
+          for (int i = PG; i < n; ++i) {
+            const int p = (int)dl[f0 + i].x;
+            dst += p >= kb && p < k;
+          }
       }
+      nbo += __popc(mS & low16((int)de0.x - (k - sub)));
       if (own_) {
         if (dst < newn) {
           R.perm[base + dst] = own + (unsigned)k;
@@ -521,22 +538,27 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
     // the row's own particles with lower slots, by the cell they come from: a
     // whole cell's count, or its codes up to the slot
     auto from = [&](int b, int e, int n) {
-      if (n == 0) return;
       if (mine && p >= e) dst += n;
-      unsigned todo = ballot16(mine && p > b && p < e);
-      while (todo) {
-        const int who = __ffs((int)todo) - 1;
-        todo &= todo - 1;
-        const int pw = __shfl(p, gsh + who, 64);
-        int m = 0;
-        for (int k = b + sub; k - sub < pw; k += PG) {
-          const unsigned c = k < pw ? cd[k] : 0xFFFFFFFFu;
-          m += __popc(ballot16(c == ((unsigned)o << 2 | WM_CODE_STAY)));
+      if (ballot16(mine && p > b && p < e) == 0u) return;
+      const unsigned way = (unsigned)o << 2 | WM_CODE_STAY;
+      const int upto = mine && p > b && p < e ? p : b;
+      for (int k0 = b; k0 < e; k0 += PWIN * PG) {
+        unsigned c[PWIN];
+#pragma unroll
+        for (int w = 0; w < PWIN; ++w) {
+          const int k = k0 + w * PG + sub;
+          c[w] = k < e ? cd[k] : 0xFFFFFFFFu;
         }
-        if (sub == who) dst += m;
+#pragma unroll
+        for (int w = 0; w < PWIN; ++w)
+          dst += __popc(ballot16(c[w] == way) & low16(upto - (k0 + w * PG)));
       }
     };
-    from(kb, ke, ko.y);
+    if (i0 == 0) {
+      if (mine) dst += p >= ke ? ko.y : (p > kb ? nbo : 0);
+    } else {
+      from(kb, ke, ko.y);
+    }
     if (fromL) from(max(0, co[l]), min(P.cap, co[l + 1]), fromL);
     if (fromR) from(max(0, co[r]), min(P.cap, co[r + 1]), fromR);
     if (mine) {
@@ -549,11 +571,6 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
     }
   }
   if (bad) atomicOr(derr, DERR_RANGE);
-}
-
-__global__ void k_order_clear(int *far, int n) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) far[t] = 0;
 }
 
 // The rows in their order: slot k of the result is what the index gives it.
@@ -591,8 +608,6 @@ int wm_k_order(wm_ctx *ctx, hipEvent_t mid) {
                 ctx->kind, ctx->disp, ctx->perm, ctx->id[ctx->idcur], ctx->id[1 - ctx->idcur]};
   hipLaunchKernelGGL(k_order_place, dim3(wm_cdiv(g.nx, PCELL), nseg), dim3(PT), 0, ctx->stream, P,
                      R, ctx->derr);
-  hipLaunchKernelGGL(k_order_clear, dim3(wm_cdiv(nseg, 256)), dim3(256), 0, ctx->stream, ctx->far,
-                     nseg);
   WM_HIP(hipGetLastError());
   ctx->idcur = 1 - ctx->idcur;
   std::swap(ctx->cumcnt, ctx->cumnew);

@@ -936,40 +936,13 @@ __global__ __launch_bounds__(256, 3) void k_push_step(PP P, const int *__restric
   }
 }
 
-// Sum of the deposit tiles into uj (ghost-inclusive), fixed order:
-// source row offset b ascending, chunk ascending.
-__global__ void k_deposit_gather(PP P, FieldGeom fg, const double *__restrict__ part,
-                                 double *__restrict__ uj) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n = fg.gx * fg.gy;
-  if (t >= n) return;
-  const int li = t % fg.gx, lj = t / fg.gx;     // ghost-inclusive local indices
-  // local column li <-> reference i = nxgs - 2 + li; tile column of chunk c:
-  // tcol = i - (nxgs + CHUNK*c) + 2 = li - CHUNK*c
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  const int chi = min(li / CHUNK, P.nchunk - 1);
-  for (int b = 0; b < 5; ++b) {
-    // source row jl with jl + (b - 2) = lj - 2  ->  jl = lj - b
-    const int jl = lj - b;
-    if (jl < 0 || jl >= P.ny) continue;
-    for (int c = max(0, chi - 1); c <= chi; ++c) {
-      const int tc = li - CHUNK * c;
-      if (tc < 0 || tc >= DW) continue;
-      const double *tp = part + ((size_t)jl * P.nchunk + c) * TILE + ((size_t)b * DW + tc) * 3;
-      s0 += tp[0];
-      s1 += tp[1];
-      s2 += tp[2];
-    }
-  }
-  uj[t] = s0;
-  uj[fg.ps + t] = s1;
-  uj[2 * fg.ps + t] = s2;
-}
-
 // Cell-centred fields, particle.f90:68-81, on cells nxs-1..nxe+1, nys-1..nye+1.
+// Also clears the rows' far marks for the push that follows.
 __global__ void k_cell_fields(FieldGeom fg, const double *__restrict__ uf,
-                              double *__restrict__ tmp, int TX, int TY, size_t tps) {
+                              double *__restrict__ tmp, int TX, int TY, size_t tps,
+                              int *__restrict__ far, int nseg) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < nseg) far[t] = 0;
   if (t >= TX * TY) return;
   const int a = t % TX, b = t / TX;
   // cell (i, j) = (nxs-1+a, nys-1+b) -> ghost-inclusive local (a+1, b+1)
@@ -1037,8 +1010,10 @@ size_t wm_deposit_part_elems(int nx, int ny) {
 int wm_k_cell_fields(wm_ctx *ctx) {
   const int TX = ctx->g.nx + 2, TY = ctx->g.ny + 2;
   const size_t tps = (size_t)TX * TY;
-  hipLaunchKernelGGL(k_cell_fields, dim3(wm_cdiv((long long)TX * TY, 256)), dim3(256), 0,
-                     ctx->stream, ctx->fg, ctx->uf, ctx->tmp, TX, TY, tps);
+  const int nseg = ctx->g.nsp * ctx->g.ny;
+  hipLaunchKernelGGL(k_cell_fields, dim3(wm_cdiv(std::max((long long)TX * TY, (long long)nseg), 256)),
+                     dim3(256), 0, ctx->stream, ctx->fg, ctx->uf, ctx->tmp, TX, TY, tps, ctx->far,
+                     nseg);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }
@@ -1069,14 +1044,5 @@ int wm_k_push_step(wm_ctx *ctx) {
                      ctx->tmp, TX, tps, ctx->bank[0], ctx->bank[1], O, ctx->dep_part, ctx->derr);
   WM_HIP(hipGetLastError());
   std::swap(ctx->bank[0], ctx->bank[1]);
-  return WM_OK;
-}
-
-int wm_k_deposit_gather(wm_ctx *ctx) {
-  PP P = make_pp(ctx);
-  const int n = ctx->fg.gx * ctx->fg.gy;
-  hipLaunchKernelGGL(k_deposit_gather, dim3(wm_cdiv(n, 256)), dim3(256), 0, ctx->stream, P,
-                     ctx->fg, ctx->dep_part, ctx->uj);
-  WM_HIP(hipGetLastError());
   return WM_OK;
 }

@@ -834,35 +834,6 @@ __global__ void k_cell_fields32(FieldGeom fg, const double *__restrict__ uf,
   tmp[5 * tps + t] = (float)E3[c0];
 }
 
-// Sum of the FP32 kernel's tiles into uj (ghost-inclusive), fixed order.
-// Also marks every row's bins as awaiting the push's movers.
-__global__ void k_deposit_gather32(int nx, int ny, int nchunk, FieldGeom fg,
-                                   const double *__restrict__ part, double *__restrict__ uj,
-                                   int *__restrict__ rowpend) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < ny) rowpend[t] = 1;
-  if (t >= fg.gx * fg.gy) return;
-  const int li = t % fg.gx, lj = t / fg.gx;
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  const int chi = min(li / CHUNK, nchunk - 1);
-  for (int b = 0; b < 5; ++b) {
-    const int jl = lj - b;
-    if (jl < 0 || jl >= ny) continue;
-    for (int c = max(0, chi - 1); c <= chi; ++c) {
-      const int tc = li - CHUNK * c;
-      if (tc < 0 || tc >= DW) continue;
-      const double *tp = part + ((size_t)jl * nchunk + c) * TILE + ((size_t)b * DW + tc) * 3;
-      s0 += tp[0];
-      s1 += tp[1];
-      s2 += tp[2];
-    }
-  }
-  (void)nx;
-  uj[t] = s0;
-  uj[fg.ps + t] = s1;
-  uj[2 * fg.ps + t] = s2;
-}
-
 // FP64 energy sums of FP32 momenta: per-workgroup partials.
 // Workgroup (x, seg) sums the bins of cells x, x + nchunk, ... of segment seg,
 // a wavefront per bin (wavefront w takes every fourth of them) and a lane
@@ -953,15 +924,6 @@ int wm_k_push_deposit32(wm_ctx *ctx) {
 }
 
 int wm_push32_pool() { return NPOOL; }
-
-int wm_k_deposit_gather32(wm_ctx *ctx) {
-  const int n = std::max(ctx->fg.gx * ctx->fg.gy, ctx->g.ny);
-  hipLaunchKernelGGL(k_deposit_gather32, dim3(wm_cdiv(n, 256)), dim3(256), 0, ctx->stream,
-                     ctx->g.nx, ctx->g.ny, wm_cdiv(ctx->g.nx, CHUNK), ctx->fg, ctx->dep_part,
-                     ctx->uj, ctx->rowpend);
-  WM_HIP(hipGetLastError());
-  return WM_OK;
-}
 
 int wm_k_energy_kin32(wm_ctx *ctx, int bank, double *part, int nchunk) {
   const int nseg = ctx->g.nsp * ctx->g.ny;

@@ -1,0 +1,46 @@
+// wm_solve.h -- what the two field solvers share: the streaming one
+// (wm_field.hip) and the one on chip (wm_solve.hip).
+#pragma once
+#include "wm_internal.h"
+
+struct SolveConst {      // field constants, field.f90:53-57
+  double f1, f2, f3, f4, f5, gfac, delt;
+  double fpt;            // 4 pi delt
+};
+
+static inline SolveConst make_fc(const wm_grid &g) {
+  const double pi = 3.141592653589793115997963468544185461590576171875;  // field.f90:13
+  SolveConst f;
+  f.f1 = g.c * g.delt / g.delx;
+  f.f2 = g.gfac * f.f1 * f.f1;
+  f.f3 = 4.0 * pi * g.delx / g.c;
+  const double t = g.delx / (g.c * g.delt * g.gfac);
+  f.f4 = 4.0 + t * t;
+  f.f5 = t * t;
+  f.gfac = g.gfac;
+  f.delt = g.delt;
+  f.fpt = 4. * pi * g.delt;
+  return f;
+}
+
+// The on-chip solve's result: iterations and ite_max reached, per component.
+struct SolveOut {
+  int ite[3], err[3];
+};
+// What a step's last kernel leaves in pinned host memory.
+struct SolveReport {
+  SolveOut out;
+  int abort_;            // the on-chip solve gave up
+  int derr;              // device error bits
+};
+// The field update's kernels skip when the on-chip solve before them gave up
+// or failed (null: after a streaming solve).
+struct SolveGate {
+  const int *abort_ = nullptr;
+  const SolveOut *out = nullptr;
+  __device__ bool closed() const {
+    return abort_ && (*abort_ || out->err[0] || out->err[1] || out->err[2]);
+  }
+};
+
+__device__ inline int wrapm(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
