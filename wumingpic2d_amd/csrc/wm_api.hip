@@ -656,7 +656,6 @@ int wm_alloc_device(wm_ctx *ctx) {
     WM_TRY(dmalloc(ctx, &ctx->rws.q, wslots));
     WM_TRY(dmalloc(ctx, &ctx->rws.uz, wslots));
     if (g.ndim >= 6) WM_TRY(dmalloc(ctx, &ctx->rws_id, wslots));
-    WM_TRY(dmalloc(ctx, &ctx->rws_bs, (size_t)ctx->relay_nws * 2 * (g.nx + 1)));
     WM_HIP(hipMemsetAsync(ctx->relay_ctl, 0, sizeof(int) * 4, ctx->stream));
     WM_HIP(hipMemsetAsync(ctx->blkflag, 0, sizeof(int) * nblk, ctx->stream));
     WM_HIP(hipMemsetAsync(ctx->segflag, 0, sizeof(int) * nseg, ctx->stream));
@@ -820,7 +819,7 @@ int wm_destroy(wm_ctx *ctx) {
                   ctx->pc_sc, ctx->fcg_s, ctx->mom, ctx->mom_part, ctx->bins.q, ctx->bins.uz,
                   ctx->bstart, ctx->pcnt, ctx->mfill[0], ctx->mfill[1], ctx->rowpend,
                   ctx->fstat, ctx->relay_ctl, ctx->relay_blocks, ctx->blkflag, ctx->relay_segs,
-                  ctx->segflag, ctx->rws.q, ctx->rws.uz, ctx->rws_id, ctx->rws_bs,
+                  ctx->segflag, ctx->rws.q, ctx->rws.uz, ctx->rws_id,
                   ctx->spill_l, ctx->spill_p, ctx->spill_q, ctx->sfill, ctx->perm, ctx->code,
                   ctx->kind, ctx->farcnt, ctx->far, ctx->lup, ctx->ldn, ctx->disp, ctx->dstart,
                   ctx->cumnew, ctx->nold, ctx->rowok, ctx->uf2, ctx->tile_sums,

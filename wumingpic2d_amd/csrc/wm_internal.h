@@ -263,7 +263,6 @@ struct wm_ctx {
   int *segflag = nullptr;        // [nseg]
   Bins32 rws;                    // workspace: relay_nwb blocks of relay_wsz slots, or
   int64_t *rws_id = nullptr;     // relay_nws segments of cap slots
-  int *rws_bs = nullptr;         // [relay_nws][2 (nx + 1)] a segment's new layout, count prefix
   int relay_wsz = 0, relay_nwb = 0, relay_nws = 0;
   double *fscratch = nullptr;    // 6 planes for the host-array boundary calls
   // restart files (paraio__init): the directory and the run's decomposition

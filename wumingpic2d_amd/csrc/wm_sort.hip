@@ -15,6 +15,7 @@
 // exactly the reference's stable scatter.  Keys are int(x) as in sort.f90:60
 // (the reference assumes delx = 1).
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 
 #include "wm_internal.h"
@@ -309,7 +310,6 @@ struct Relay {
   int *blocks, *segs, *blkflag, *segflag;
   Bins32 ws;
   int64_t *ws_id;
-  int *ws_bs;                    // per segment workgroup: new layout, count prefix
   int wsz;                       // slots per block workgroup
 };
 
@@ -371,34 +371,77 @@ __global__ __launch_bounds__(256) void k_fill_check(Mig G, int *__restrict__ pc,
   }
 }
 
-// Copies the n(j) particles of bins j < nb (old first slot ob(j), new first
-// slot nb_(j), count prefix pre(j)) of segment seg through the workspace W:
-// first all of them out, flat in prefix order, then all back at their new
+// Moves the pre[j + 1] - pre[j] particles of bins j < nb (old first slot
+// ob[j], new first slot nb_[j], count prefix pre) of segment seg to their new
 // places.  Bins move verbatim, holes included: slot k of a bin stays slot k.
-// Every thread of the workgroup calls it.
-template <class OB, class NB, class PRE>
-__device__ void move_bins(const SB &P, int seg, int nb, OB ob, NB nb_, PRE pre, Bins32 A,
-                          int64_t *ids, Bins32 W, int64_t *wid) {
-  const int T = pre(nb);
+// The particles are taken flat in prefix order, NT at a time, a thread finding
+// its particle's bin by bisection.  Up to MU each thread holds them all in
+// registers between reading and writing, all loads of an array in flight (a
+// re-layout is a chain of latencies: few rows or blocks are listed, each has
+// one workgroup); more go through the workspace W.  Every thread of the
+// workgroup calls it.
+template <int NT, int MU>
+__device__ void move_bins(const SB &P, int seg, int nb, const int *ob, const int *nb_,
+                          const int *pre, Bins32 A, int64_t *ids, Bins32 W, int64_t *wid) {
+  const int T = pre[nb], tid = threadIdx.x;
   const size_t s0 = seg_at(P, seg);
-  const int stride = blockDim.x;
-  // flat index f -> bin j: f grows by the block size, j follows it
-  int j = 0;
-  for (int f = threadIdx.x; f < T; f += stride) {
-    while (f >= pre(j + 1)) ++j;
-    const size_t src = s0 + ob(j) + (f - pre(j));
-    W.q[f] = A.q[src];
-    W.uz[f] = A.uz[src];
-    if (ids) wid[f] = ids[src];
-  }
-  __syncthreads();
-  j = 0;
-  for (int f = threadIdx.x; f < T; f += stride) {
-    while (f >= pre(j + 1)) ++j;
-    const size_t dst = s0 + nb_(j) + (f - pre(j));
-    A.q[dst] = W.q[f];
-    A.uz[dst] = W.uz[f];
-    if (ids) ids[dst] = wid[f];
+  const auto bin_of = [&](int f) {          // the bin with pre[j] <= f < pre[j + 1], f < T
+    int lo = 0, hi = nb - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (pre[mid] <= f) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+  };
+  if (T <= NT * MU) {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    v4 *const Aq = (v4 *)A.q;
+    int at[MU] = {}, to[MU] = {};
+#pragma unroll
+    for (int u = 0; u < MU; ++u)
+      if (u * NT < T) {
+        const int f = min(tid + u * NT, T - 1), j = bin_of(f), k = f - pre[j];
+        at[u] = ob[j] + k;
+        to[u] = nb_[j] + k;
+      }
+    const auto move = [&](auto *arr) {
+      std::remove_reference_t<decltype(*arr)> v[MU] = {};
+#pragma unroll
+      for (int u = 0; u < MU; ++u)
+        if (u * NT < T) v[u] = arr[s0 + at[u]];
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < MU; ++u)
+        if (tid + u * NT < T) arr[s0 + to[u]] = v[u];
+    };
+    move(Aq);
+    move(A.uz);
+    if (ids) move(ids);
+  } else {
+    constexpr int B = 4;                    // loads of a thread in flight
+    for (int f0 = tid; f0 < T; f0 += B * NT)
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const int f = f0 + u * NT;
+        if (f >= T) break;
+        const int j = bin_of(f);
+        const size_t src = s0 + ob[j] + (f - pre[j]);
+        W.q[f] = A.q[src];
+        W.uz[f] = A.uz[src];
+        if (ids) wid[f] = ids[src];
+      }
+    __syncthreads();
+    for (int f0 = tid; f0 < T; f0 += B * NT)
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const int f = f0 + u * NT;
+        if (f >= T) break;
+        const int j = bin_of(f);
+        const size_t dst = s0 + nb_[j] + (f - pre[j]);
+        A.q[dst] = W.q[f];
+        A.uz[dst] = W.uz[f];
+        if (ids) ids[dst] = wid[f];
+      }
   }
   __syncthreads();
 }
@@ -474,9 +517,7 @@ __global__ __launch_bounds__(RW) void k_relayout_blocks(SB P, Relay R, const int
     }
     __syncthreads();
     if (s_go) {
-      move_bins(
-          P, seg, nb, [&](int j) { return s_old[j]; }, [&](int j) { return s_new[j]; },
-          [&](int j) { return s_pre[j]; }, A, ids, W, wid);
+      move_bins<RW, 12>(P, seg, nb, s_old, s_new, s_pre, A, ids, W, wid);
       if (threadIdx.x < nb) bs[i0 + threadIdx.x] = s_new[threadIdx.x];
     }
     __syncthreads();
@@ -484,52 +525,101 @@ __global__ __launch_bounds__(RW) void k_relayout_blocks(SB P, Relay R, const int
 }
 
 // Step 2: each listed segment (a workgroup at a time) is laid out anew as a
-// whole (wm_bins::wave_layout on the same counts) and its bins moved through
-// a workspace of a segment's slots.  A segment whose counts do not fit is
-// the reference's memory over.
-__global__ __launch_bounds__(RW) void k_relayout_segs(SB P, Relay R, const int *__restrict__ cnt,
+// whole, by wm_bins' policy on the same counts over the segment's slots, as
+// wave_layout does it, and its bins moved.  LDS: counts, then new starts and
+// count prefix (nx + 1 each).  A segment whose counts do not fit is the
+// reference's memory over.
+constexpr int RS = 1024;  // threads of a segment's workgroup
+struct SegSums {
+  int a, b;
+};
+// Sums over the workgroup (in every thread); with excl also what the threads
+// before this one hold.
+__device__ inline SegSums seg_sums(SegSums v, SegSums *sh, SegSums *excl = nullptr) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  SegSums x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int a = __shfl_up(x.a, o, 64), b = __shfl_up(x.b, o, 64);
+    if (lane >= o) {
+      x.a += a;
+      x.b += b;
+    }
+  }
+  __syncthreads();                        // sh was read
+  if (lane == 63) sh[w] = x;
+  __syncthreads();
+  SegSums t{0, 0}, before{0, 0};
+#pragma unroll
+  for (int k = 0; k < RS / 64; ++k) {
+    if (k == w) before = t;
+    t.a += sh[k].a;
+    t.b += sh[k].b;
+  }
+  if (excl) *excl = SegSums{before.a + x.a - v.a, before.b + x.b - v.b};
+  return t;
+}
+__global__ __launch_bounds__(RS) void k_relayout_segs(SB P, Relay R, const int *__restrict__ cnt,
                                                       const int *__restrict__ pc,
                                                       int *__restrict__ bstart, Bins32 A,
                                                       int64_t *__restrict__ ids, int *derr) {
-  __shared__ int s_ok;
-  const int nlist = R.ctl[1];
+  extern __shared__ int s_lay[];
+  __shared__ SegSums s_sum[RS / 64];
+  const int nlist = R.ctl[1], nx = P.nx, tid = threadIdx.x;
   const size_t wsz = (size_t)P.cap;
   Bins32 W{R.ws.q + (size_t)blockIdx.x * wsz, R.ws.uz + (size_t)blockIdx.x * wsz};
   int64_t *wid = R.ws_id ? R.ws_id + (size_t)blockIdx.x * wsz : nullptr;
-  int *tb = R.ws_bs + (size_t)blockIdx.x * 2 * (P.nx + 1), *pre = tb + P.nx + 1;
+  int *tb = s_lay, *pre = s_lay + nx + 1;
+  const int per = (nx + RS - 1) / RS, lo = min(nx, tid * per), hi = min(nx, lo + per);
   for (int e = blockIdx.x; e < nlist; e += gridDim.x) {
     const int seg = R.segs[e];
-    const int *cn = cnt + (size_t)seg * P.nx, *pn = pc + (size_t)seg * P.nx;
-    int *bs = bstart + (size_t)seg * (P.nx + 1);
-    if (threadIdx.x < 64) {
-      const bool ok = wm_bins::wave_layout([&](int i) { return max(cn[i], pn[i]); }, P.nx, P.cap, tb);
-      // count prefix for the flat copy, 64 bins at a time
-      int run = 0;
-      for (int i0 = 0; i0 < P.nx; i0 += 64) {
-        const int i = i0 + threadIdx.x;
-        const int n = i < P.nx ? cn[i] : 0;
-        int incl = n;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const int v = __shfl_up(incl, o, 64);
-          if ((int)threadIdx.x >= o) incl += v;
-        }
-        if (i < P.nx) pre[i + 1] = run + incl;
-        run += __shfl(incl, 63, 64);
-      }
-      if (threadIdx.x == 0) {
-        pre[0] = 0;
-        s_ok = ok;
-        R.segflag[seg] = 0;
-        if (!ok) atomicOr(derr, DERR_NP_OVER);
-      }
+    const int *cn = cnt + (size_t)seg * nx, *pn = pc + (size_t)seg * nx;
+    int *bs = bstart + (size_t)seg * (nx + 1);
+    for (int i = tid; i < nx; i += RS) {
+      const int n = cn[i];
+      pre[i + 1] = n;
+      tb[i] = max(n, pn[i]);
     }
     __syncthreads();
-    if (s_ok) {
-      move_bins(
-          P, seg, P.nx, [&](int j) { return bs[j]; }, [&](int j) { return tb[j]; },
-          [&](int j) { return pre[j]; }, A, ids, W, wid);
-      for (int i = threadIdx.x; i <= P.nx; i += blockDim.x) bs[i] = tb[i];
+    SegSums v{0, 0};
+    for (int i = lo; i < hi; ++i) {
+      v.a += tb[i];
+      v.b += tb[i] > WM_BIN_MAX;
+    }
+    const SegSums c = seg_sums(v, s_sum);
+    v = SegSums{0, 0};
+    for (int i = lo; i < hi; ++i) {
+      v.a += wm_bins::need_of(tb[i], c.a / nx);
+      v.b += wm_bins::need_of(tb[i], 0);
+    }
+    const SegSums need = seg_sums(v, s_sum);
+    wm_bins::Policy pol;
+    const bool ok = wm_bins::make_policy(c.a, need.a, need.b, nx, P.cap, pol) && c.b == 0;
+    if (ok) {
+      v = SegSums{0, 0};
+      for (int i = lo; i < hi; ++i) {
+        v.a += wm_bins::need_of(tb[i], pol.floor);
+        v.b += pre[i + 1];
+      }
+      SegSums at;
+      seg_sums(v, s_sum, &at);
+      for (int i = lo; i < hi; ++i) {
+        const int nd = wm_bins::need_of(tb[i], pol.floor);
+        tb[i] = wm_bins::start_of(pol, at.a);
+        at.a += nd;
+        pre[i + 1] = at.b += pre[i + 1];
+      }
+    }
+    if (tid == 0) {
+      tb[nx] = P.cap;                     // the slack after the last block joins the last bin
+      pre[0] = 0;
+      R.segflag[seg] = 0;
+      if (!ok) atomicOr(derr, DERR_NP_OVER);
+    }
+    __syncthreads();
+    if (ok) {
+      move_bins<RS, 12>(P, seg, nx, bs, tb, pre, A, ids, W, wid);
+      for (int i = tid; i <= nx; i += RS) bs[i] = tb[i];
     }
     __syncthreads();
   }
@@ -699,7 +789,6 @@ Relay make_relay(const wm_ctx *ctx) {
   R.segflag = ctx->segflag;
   R.ws = ctx->rws;
   R.ws_id = ctx->rws_id;
-  R.ws_bs = ctx->rws_bs;
   R.wsz = ctx->relay_wsz;
   return R;
 }
@@ -723,7 +812,11 @@ int wm_relayout(wm_ctx *ctx) {
   const Relay R = make_relay(ctx);
   hipLaunchKernelGGL(k_relayout_blocks, dim3(ctx->relay_nwb), dim3(RW), 0, ctx->stream, P, R,
                      ctx->bin_cnt, ctx->pcnt, ctx->bstart, ctx->bins, ctx->id_bins);
-  hipLaunchKernelGGL(k_relayout_segs, dim3(ctx->relay_nws), dim3(RW), 0, ctx->stream, P, R,
+  const size_t lds = 2 * sizeof(int) * (P.nx + 1);
+  if (lds > 49152)
+    (void)hipFuncSetAttribute((const void *)k_relayout_segs,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL(k_relayout_segs, dim3(ctx->relay_nws), dim3(RS), lds, ctx->stream, P, R,
                      ctx->bin_cnt, ctx->pcnt, ctx->bstart, ctx->bins, ctx->id_bins, ctx->derr);
   hipLaunchKernelGGL(k_relayout_done, dim3(1), dim3(64), 0, ctx->stream, R, ctx->fstat);
   WM_HIP(hipGetLastError());
