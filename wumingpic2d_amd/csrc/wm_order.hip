@@ -10,8 +10,8 @@
 // them sorted.  A step so reads and writes each 48-byte record once, plus 8
 // bytes of codes and index, where pushing in place, scanning for leavers and
 // sorting moved 192 bytes a particle.  Measured at 2048 x 2048, 64 particles
-// per cell and species, beside the field solve: rows 0.9, merge 0.6, place
-// 5.5 ms, where pass 1 took 6.0 and pass 2 with the sort 16.7 ms.
+// per cell and species, beside the field solve: rows and merge 1.5, place
+// 4.6 ms, where pass 1 took 6.0 and pass 2 with the sort 16.7 ms.
 //
 // The order.  Pass 1 lists a row's leavers (up, down) and their slots, the
 // holes, in slot order.  Pass 2 puts arrival a (the neighbours' leavers,
@@ -376,24 +376,38 @@ __device__ bool place_wide(const OP &P, const Place &R, int seg, int c) {
 // that goes to cell c in {o-1, o, o+1} comes after the particles of lower
 // cells that go to c (counted by the push), after those of its own cell with
 // lower slots that go the same way, and after the displaced particles of c
-// with lower slots.  The latter are looked at one by one only if one of them
-// has a slot among the cell's own.
+// with lower slots.  Where some of the latter have slots among the cell's own
+// (near a row's ends), bitmaps of those slots are made in LDS, 512 slots at a
+// time, and each window adds the bits below it.
 //
 // The displaced particles of new cell o: after the row's own of the cell with
-// lower slots -- whole cells' counts, unless the slot lies inside one of the
-// three cells, whose codes are then searched -- and the displaced ones with
+// lower slots -- whole cells' counts, or the part of a cell before the slot
+// from the tables that its group left (per window: the particles that stay,
+// go right, go left, and how many before it) -- and the displaced ones with
 // lower slots.
 //
-// 2 B of code, 4 B of index and 16 B of ID per particle.
+// 2 B of code, 4 B of index and 16 B of ID per particle, three dependent round
+// trips to memory a cell, which bound it; six wavefronts a SIMD hide most.  Where
+// a plasma has pinched (256 x 64 cells, 407 particles in the densest at a mean
+// of 64) the longest cells set the time: 42 us, and 124 where every window
+// compared itself with each displaced particle and each of those searched the
+// codes again.
 constexpr int PG = 16;           // lanes of a cell
 constexpr int PT = 256;
 constexpr int PCELL = PT / PG;   // cells of a workgroup
 constexpr int PWIN = 4;          // windows of a cell in flight
-__global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
+constexpr int PD = 64;           // displaced particles of a cell ranked from LDS at a time
+constexpr int PWT = 32;          // windows of a cell in the tables and bitmaps
+__global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr) {
+  __shared__ __attribute__((aligned(16))) int slots[PCELL][PD];
+  __shared__ unsigned tab[3][PCELL][PWT];            // stay, right, left: count << 16 | lanes
+  __shared__ unsigned bits[3][PCELL][PWT / 2];       // displaced of o, r, l by slot - ks
+  constexpr int NONE = 0x7FFFFFFF;
   const int seg = blockIdx.y;
-  const int sub = threadIdx.x % PG, gsh = (threadIdx.x & 63) / PG * PG;
+  const int sub = threadIdx.x % PG, g = threadIdx.x / PG, gsh = (threadIdx.x & 63) / PG * PG;
   const int nx = P.nx, jl = seg % P.ny;
-  const int o = min(nx - 1, (int)blockIdx.x * PCELL + (int)threadIdx.x / PG);
+  const bool act = (int)blockIdx.x * PCELL + g < nx;
+  const int o = min(nx - 1, (int)blockIdx.x * PCELL + g);
   const size_t base = (size_t)seg * P.cap, plane = base - (size_t)jl * P.cap;
   const unsigned own = (unsigned)jl * (unsigned)P.cap;
   const uint16_t *cd = R.code + base;
@@ -407,7 +421,7 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
   const bool hasl = o > 0 || P.periodic, hasr = o + 1 < nx || P.periodic;
   const int l = o > 0 ? o - 1 : nx - 1, r = o + 1 < nx ? o + 1 : 0, ll = o > 1 ? o - 2 : 0;
   const int rowok = R.rowok[seg], far = R.far[seg], nold = R.nold[seg], newn = cn[nx];
-  const int kb = max(0, co[o]), ke = min(P.cap, co[o + 1]);
+  const int kb = max(0, co[o]), ke = act ? min(P.cap, co[o + 1]) : kb;
   const int start = cn[o], sl = cn[l], sr = cn[r];
   const int d0 = ds[o], d1 = ds[o + 1], dl0 = ds[l], dl1 = ds[l + 1], dr0 = ds[r], dr1 = ds[r + 1];
   const int4 ko = kd[o], kl_ = kd[l], kr_ = kd[r], kll_ = kd[ll], k0_ = kd[0], k1_ = kd[1];
@@ -420,11 +434,12 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
     if (bad) atomicOr(derr, DERR_RANGE);
     return;
   }
-  if ((int)blockIdx.x * PCELL + (int)threadIdx.x / PG >= nx) return;
   const int keep = min(nold, newn);
   const int toR = ko.z, toL = ko.x;                  // the cell's particles that go right, left
   const int fromL = hasl ? kl_.z : 0, fromR = hasr ? kr_.x : 0;   // the neighbours' that come here
-  const int D = d1 - d0, Dl = toL > 0 ? dl1 - dl0 : 0, Dr = toR > 0 ? dr1 - dr0 : 0;
+  const int D = act ? d1 - d0 : 0;
+  const int Dl = act && toL > 0 ? dl1 - dl0 : 0, Dr = act && toR > 0 ? dr1 - dr0 : 0;
+  const bool tabled = ke - kb <= PG * PWT;
   // second round trip: the first codes and IDs, the displaced particles (the
   // first 16 of each list in registers)
   unsigned cv[PWIN];
@@ -441,7 +456,6 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
       }
     }
   };
-  constexpr int NONE = 0x7FFFFFFF;
   const uint2 de0 = sub < D ? dl[d0 + sub] : make_uint2(NONE, 0u);
   const int pL = sub < Dl ? (int)dl[dl0 + sub].x : NONE, pR = sub < Dr ? (int)dl[dr0 + sub].x : NONE;
   fetch(kb);
@@ -449,17 +463,19 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
   auto ballot16 = [&](bool b) { return (unsigned)(__ballot(b) >> gsh) & 0xFFFFu; };
   const unsigned below = (1u << sub) - 1u;
   auto low16 = [](int n) { return n <= 0 ? 0u : n >= 16 ? 0xFFFFu : (1u << n) - 1u; };
-  // displaced particles of a list (its first 16 in p) with slots below kb;
-  // any inside [kb, ke)
+  // f(slot) for each displaced particle of a list (its first 16 in p)
+  auto each = [&](int p, int f0, int n, auto f) {
+    f(p);
+    for (int i0 = PG; i0 < n; i0 += PG) f(i0 + sub < n ? (int)dl[f0 + i0 + sub].x : NONE);
+  };
+  // how many of them have slots below kb; do any inside [kb, ke)
   bool in = false;
   auto lower = [&](int p, int f0, int n) {
-    int c = __popc(ballot16(p < kb));
-    in |= ballot16(p >= kb && p < ke) != 0u;
-    for (int i0 = PG; i0 < n; i0 += PG) {
-      const int q = i0 + sub < n ? (int)dl[f0 + i0 + sub].x : NONE;
+    int c = 0;
+    each(p, f0, n, [&](int q) {
       c += __popc(ballot16(q < kb));
       in |= ballot16(q >= kb && q < ke) != 0u;
-    }
+    });
     return c;
   };
   // first place of the cell's particles that stay, go right, go left
@@ -468,9 +484,25 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
   int bR = sr + (o < nx - 1 ? (P.periodic && o + 1 == nx - 1 ? k0_.x : 0) : k0_.y + k1_.x) +
            lower(pR, dr0, Dr);
   int bL = sl + (o > 0 ? (o > 1 ? kll_.z : 0) + kl_.y : 0) + lower(pL, dl0, Dl);
-  int nbo = 0;             // stayers of the cell below this lane's displaced particle (the first 16)
+  int cS = 0, cR = 0, cL = 0;                        // the cell's own so far
   for (int k0 = kb; k0 < ke; k0 += PWIN * PG) {
     if (k0 > kb) fetch(k0);
+    const int seg0 = (k0 - kb) & (PG * PWT - 1);     // within the bitmaps' 512 slots
+    if (in && seg0 == 0) {
+      __builtin_amdgcn_wave_barrier();               // what was there has been read
+      for (int i = sub; i < PWT / 2; i += PG) bits[0][g][i] = bits[1][g][i] = bits[2][g][i] = 0u;
+      __builtin_amdgcn_wave_barrier();
+      auto mark = [&](unsigned *b, int p, int f0, int n) {
+        each(p, f0, n, [&](int q) {
+          const int at = q - k0;
+          if (at >= 0 && at < PG * PWT && q < ke) atomicOr(b + (at >> 5), 1u << (at & 31));
+        });
+      };
+      mark(bits[0][g], (int)de0.x, d0, D);
+      mark(bits[1][g], pR, dr0, Dr);
+      mark(bits[2][g], pL, dl0, Dl);
+      __builtin_amdgcn_wave_barrier();
+    }
 #pragma unroll
     for (int w = 0; w < PWIN; ++w) {
       const int k = k0 + w * PG + sub;
@@ -479,36 +511,29 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
       const bool own_ = k < keep && (cv[w] & 3u) == WM_CODE_STAY;   // (none past ke: all bits set)
       const bool moves = own_ && c != o, right = c == r;
       const unsigned mS = ballot16(own_ && c == o), mM = ballot16(moves);
-      int dst = bS + __popc(mS & below);
-      bS += __popc(mS);
+      unsigned mR = 0, mL = 0;
+      int dst = bS + cS + __popc(mS & below);
       if (mM) {                                      // uniform over the group
-        const unsigned mR = ballot16(moves && right), mL = mM & ~mR;
-        if (moves) dst = right ? bR + __popc(mR & below) : bL + __popc(mL & below);
-        bR += __popc(mR);
-        bL += __popc(mL);
+        mR = ballot16(moves && right);
+        mL = mM & ~mR;
+        if (moves) dst = right ? bR + cR + __popc(mR & below) : bL + cL + __popc(mL & below);
       }
       if (in) {                                      // displaced slots among the cell's own
-        const bool stay = own_ && !moves;
-        for (int i = 0; i < min(D, PG); ++i) {
-          const int p = __shfl((int)de0.x, gsh + i, 64);
-          dst += stay && p >= kb && p < k;
-        }
-        for (int i = 0; i < min(Dr, PG); ++i) {
-          const int p = __shfl(pR, gsh + i, 64);
-          dst += moves && right && p >= kb && p < k;
-        }
-        for (int i = 0; i < min(Dl, PG); ++i) {
-          const int p = __shfl(pL, gsh + i, 64);
-          dst += moves && !right && p >= kb && p < k;
-        }
-        const int f0 = moves ? (right ? dr0 : dl0) : d0, n = moves ? (right ? Dr : Dl) : D;
-        if (own_)
-          for (int i = PG; i < n; ++i) {
-            const int p = (int)dl[f0 + i].x;
-            dst += p >= kb && p < k;
-          }
+        const int at = seg0 + w * PG;
+        unsigned d[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) d[q] = (bits[q][g][at >> 5] >> (at & 31)) & 0xFFFFu;
+        dst += __popc((!moves ? d[0] : (right ? d[1] : d[2])) & below);
+        bS += __popc(d[0]);
+        bR += __popc(d[1]);
+        bL += __popc(d[2]);
       }
-      nbo += __popc(mS & low16((int)de0.x - (k - sub)));
+      if (tabled && sub < 3)
+        tab[sub][g][(k - sub - kb) / PG] =
+            sub == 0 ? (unsigned)cS << 16 | mS : (sub == 1 ? (unsigned)cR << 16 | mR : (unsigned)cL << 16 | mL);
+      cS += __popc(mS);
+      cR += __popc(mR);
+      cL += __popc(mL);
       if (own_) {
         if (dst < newn) {
           R.perm[base + dst] = own + (unsigned)k;
@@ -519,7 +544,18 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
       }
     }
   }
-  // the displaced particles of cell o, 16 at a time
+  __syncthreads();                                   // the neighbours' tables
+  // the displaced particles of cell o, 16 at a time, each ranked among all
+  // (more than 16: their slots in LDS, PD at a time, padded to fours)
+  int *const sl_ = slots[g];
+  auto stage = [&](int f) {
+    __builtin_amdgcn_wave_barrier();                 // what was there has been read
+    for (int i = sub; i < min(PD, (D - f + 3) & ~3); i += PG)
+      sl_[i] = f + i < D ? (int)dl[d0 + f + i].x : NONE;
+    __builtin_amdgcn_wave_barrier();
+  };
+  if (D > PG && D <= PD) stage(0);
+  const int lb = max(0, co[l]), le = min(P.cap, co[l + 1]), rb = max(0, co[r]), re = min(P.cap, co[r + 1]);
   for (int i0 = 0; i0 < D; i0 += PG) {
     const bool mine = i0 + sub < D;
     uint2 de = de0;
@@ -533,15 +569,30 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
     if (D <= PG) {
       for (int i = 0; i < D; ++i) dst += __shfl(p, gsh + i, 64) < p;
     } else {
-      for (int i = 0; i < D; ++i) dst += (int)dl[d0 + i].x < p;
+      for (int f = 0; f < D; f += PD) {
+        if (D > PD) stage(f);
+        for (int i = 0; i < min(PD, D - f); i += 4) {
+          const int4 q = *(const int4 *)(sl_ + i);
+          dst += (q.x < p) + (q.y < p) + (q.z < p) + (q.w < p);
+        }
+      }
     }
-    // the row's own particles with lower slots, by the cell they come from: a
-    // whole cell's count, or its codes up to the slot
-    auto from = [&](int b, int e, int n) {
+    // the row's own particles with lower slots, by the cell [b, e) they come
+    // from: a whole cell's count n, or what its table t has up to the slot;
+    // without one (another workgroup's cell, a long one), its codes
+    auto from = [&](int b, int e, int n, const unsigned *t) {
+      const bool part = mine && p > b && p < e;
       if (mine && p >= e) dst += n;
-      if (ballot16(mine && p > b && p < e) == 0u) return;
+      if (ballot16(part) == 0u) return;
+      if (t && e - b <= PG * PWT) {
+        if (part) {
+          const unsigned q = t[(p - b) / PG];
+          dst += (int)(q >> 16) + __popc(q & low16((p - b) % PG));
+        }
+        return;
+      }
       const unsigned way = (unsigned)o << 2 | WM_CODE_STAY;
-      const int upto = mine && p > b && p < e ? p : b;
+      const int upto = part ? p : b;
       for (int k0 = b; k0 < e; k0 += PWIN * PG) {
         unsigned c[PWIN];
 #pragma unroll
@@ -554,13 +605,9 @@ __global__ __launch_bounds__(PT) void k_order_place(OP P, Place R, int *derr) {
           dst += __popc(ballot16(c[w] == way) & low16(upto - (k0 + w * PG)));
       }
     };
-    if (i0 == 0) {
-      if (mine) dst += p >= ke ? ko.y : (p > kb ? nbo : 0);
-    } else {
-      from(kb, ke, ko.y);
-    }
-    if (fromL) from(max(0, co[l]), min(P.cap, co[l + 1]), fromL);
-    if (fromR) from(max(0, co[r]), min(P.cap, co[r + 1]), fromR);
+    from(kb, ke, ko.y, tab[0][g]);
+    if (fromL) from(lb, le, fromL, g > 0 ? tab[1][g - 1] : nullptr);
+    if (fromR) from(rb, re, fromR, g + 1 < PCELL && o + 1 < nx ? tab[2][g + 1] : nullptr);
     if (mine) {
       if (dst < newn) {
         R.perm[base + dst] = de.y;
