@@ -1014,7 +1014,7 @@ int wm_field_fdtd_i(wm_ctx *ctx, double *uf, const double *up, const double *gp,
   WM_TRY(upload_cumcnt(ctx, cumcnt));
   WM_TRY(upload_field(ctx, uf, 6, ctx->uf));
   WM_TRY(wm_k_deposit(ctx, 0, 1));
-  WM_TRY(wm_k_current(ctx));
+  WM_TRY(wm_k_current(ctx, WM_CHUNK_HOST64));
   WM_TRY(wm_check_derr(ctx, "field__fdtd_i"));
   WM_TRY(wm_k_field_solve(ctx));
   WM_TRY(download_field(ctx, uf, 6, ctx->uf));
@@ -1393,7 +1393,7 @@ int wm_step(wm_ctx *ctx, int nsteps) {
       WM_TRY(wm_k_order(ctx, e[6]));
       WM_HIP(hipEventRecord(e[7], ctx->stream));
     }
-    WM_TRY(wm_k_current(ctx));                    // field.f90:121-122
+    WM_TRY(wm_k_current(ctx, f32 ? WM_CHUNK_STEP32 : WM_CHUNK_STEP64));   // field.f90:121-122
     WM_HIP(hipEventRecord(e[3], ctx->stream));
     WM_TRY(wm_field_launch(ctx));                 // field.f90:125-184
     WM_HIP(hipEventRecord(e[4], ctx->stream));

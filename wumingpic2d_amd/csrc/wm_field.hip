@@ -1024,13 +1024,16 @@ __global__ __launch_bounds__(256) void k_current(FieldGeom fg, int nchunk, int w
 }
 }  // namespace
 
-int wm_k_current(wm_ctx *ctx) {
+int wm_k_current(wm_ctx *ctx, int chunk) {
   const FieldGeom &fg = ctx->fg;
   const int n = std::max(fg.gx * fg.gy, fg.ny);
   const bool f32 = ctx->form == WM_FORM_FP32;
-  hipLaunchKernelGGL(f32 ? k_current<16> : k_current<32>, dim3(wm_cdiv(n, 256)), dim3(256), 0,
-                     ctx->stream, fg, wm_cdiv(fg.nx, f32 ? 16 : 32), ctx->bcf != WM_BC_PERIODIC,
-                     ctx->dep_part, ctx->uj, f32 ? ctx->rowpend : nullptr);
+  auto kernel = chunk == WM_CHUNK_STEP64   ? k_current<WM_CHUNK_STEP64>
+                : chunk == WM_CHUNK_STEP32 ? k_current<WM_CHUNK_STEP32>
+                                           : k_current<WM_CHUNK_HOST64>;
+  hipLaunchKernelGGL(kernel, dim3(wm_cdiv(n, 256)), dim3(256), 0, ctx->stream, fg,
+                     wm_cdiv(fg.nx, chunk), ctx->bcf != WM_BC_PERIODIC, ctx->dep_part, ctx->uj,
+                     f32 ? ctx->rowpend : nullptr);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }

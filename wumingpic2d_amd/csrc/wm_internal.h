@@ -126,6 +126,10 @@ struct __align__(32) BinSum {
 // full by the fill check, [6] blocks and [7] segments laid out anew (sums).
 #define WM_NSTAT 8
 #define WM_RB 64               // cells of a re-layout block
+// cells of a deposit tile: the resident step's (FP64, FP32), the host-array entry points'
+#define WM_CHUNK_STEP64 8
+#define WM_CHUNK_STEP32 16
+#define WM_CHUNK_HOST64 32
 
 using PBank = Rec64;
 
@@ -317,7 +321,7 @@ int wm_k_bc_curre(wm_ctx *ctx, double *uj);
 XSide wm_xside(const wm_ctx *ctx);
 int wm_k_bc_dfield(wm_ctx *ctx, double *df);
 int wm_k_bc_phi(wm_ctx *ctx, double *phi, int l);   // phi(nxs-1:nxe+1, nys-1:nye+1)
-int wm_k_current(wm_ctx *ctx);       // deposit tiles summed and folded into uj
+int wm_k_current(wm_ctx *ctx, int chunk);   // deposit tiles (of chunk cells) summed and folded into uj
 // RHS .. uf += df (after the current is ready).  A step launches the solve
 // and, once everything else of the step is ordered before it, the update with
 // the step's report; after the stream has been waited for it takes the result.

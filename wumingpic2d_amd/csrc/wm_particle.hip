@@ -26,7 +26,7 @@
 
 namespace {
 
-constexpr int CHUNK = 32;             // cells per workgroup
+constexpr int CHUNK = WM_CHUNK_HOST64;   // cells per workgroup
 constexpr int GROUP = 8;              // lanes per cell
 constexpr int TW = CHUNK + 2;         // push tile width (halo 1)
 constexpr int DW = CHUNK + 4;         // deposit tile width (halo 2)
@@ -87,6 +87,7 @@ __device__ inline void shape(double dh, double &sm, double &s0, double &sp) {
 
 // Cell-centred field tile: T[(k*3 + b)*TW + col], b = row j-1..j+1,
 // col = i - (i0 - 1).
+template <int TW>
 __device__ inline void load_tmp_tile(double *T, const double *tmp, int TX,
                                      size_t tps, int jl, int c0, int ncol) {
   // tmp planes hold cells (nxs-1 .. nxe+1) x (nys-1 .. nye+1); local column
@@ -342,7 +343,7 @@ __global__ __launch_bounds__(256, 3) void k_particle(
   const int j = P.nys + jl;
   const int i0 = P.nxgs + chunk * CHUNK;
   const int ncell = min(CHUNK, P.nx - chunk * CHUNK);
-  if (PUSH) load_tmp_tile(T, tmp, TX, tps, jl, chunk * CHUNK, min(TW, ncell + 2));
+  if (PUSH) load_tmp_tile<TW>(T, tmp, TX, tps, jl, chunk * CHUNK, min(TW, ncell + 2));
   if (DEPOSIT)
     for (int e = threadIdx.x; e < CHUNK * NACC; e += blockDim.x) cellbuf[e] = 0.0;
   __syncthreads();
@@ -501,29 +502,44 @@ __global__ __launch_bounds__(256, 3) void k_particle(
 // over the particles: read through the pending order (Order::perm), written
 // sorted, 40 bytes each way, plus 4 bytes of index and 2 of code.
 //
-// The decomposition is k_particle's, a group of 8 lanes per cell, with steps
-// of 8 consecutive particles (one per lane) from the 8-particle boundary at
-// or below the cell's first: a step's five loads were issued during the step
-// before it, its index one more step ahead.  Steps of 16 (two per lane) left
-// a third of the lanes idle at 64 particles per cell (a wavefront's eight
-// cells step together), steps of 8 leave a fifth.
+// A group of 16 lanes per cell, in steps of 16 consecutive particles.  Loads
+// run two steps ahead of their use and indexes four; a step's results wait in
+// registers and are stored in front of the next step's loads, since loads and
+// stores complete in order and whatever is waited for should have been issued
+// two steps ago.  A workgroup is two wavefronts of four cells each: with eight
+// wavefronts and 32 cells, more than half of the wavefronts' time went into
+// waiting for the densest cells of the workgroup at its end.
 //
-// Per cell, over all species: 21 stay-in-cell stencil values per lane
-// (wm: of the 27 values of the 3 x 3 cores, Jx's last column and Jy's last
-// row carry the sum of all three shape changes, which is zero), and a list of
-// the crossing particles in LDS, whose full stencils are summed at the end,
-// or whenever some cell's list could overflow in the next step.
+// Per cell, over all species: 21 stay-in-cell stencil values per lane (of the
+// 27 values of the 3 x 3 cores, Jx's last column and Jy's last row carry the
+// sum of all three shape changes, which is zero), and a list of the crossing
+// particles in LDS, summed when some cell's list could overflow in the next
+// two steps and at the end.  A hot plasma has a third of its particles cross a
+// cell's edge in a step, so the movers are half of the work: see mover_sums.
 //
 // The TSC gather of particle.f90:107-129 inside a cell is a biquadratic in
 // the in-cell offsets: nine coefficients per field and cell (LDS), 8 FMAs a
 // field.
-constexpr int MLC = 16;               // a cell's listed movers
+//
+// Two wavefronts a SIMD (197 registers): bound by FP64 operations (half of the
+// issue slots) and the memory path together; alone, loads and stores take 0.92
+// ms and the arithmetic 0.91 at 1024 x 512 cells with 32 per cell, both 1.1.
+// Measured, 8 lanes of one wavefront and 32 cells, 16 and 8 cells: 2048 x 2048,
+// 64 per cell: 18.9 -> 15.6 ms; 256 x 64, 64 per cell, pinched: 224 -> 128 us;
+// 1024 x 512, 32 per cell: 1.68 -> 1.51 ms.
+constexpr int PCH = WM_CHUNK_STEP64;  // cells of a workgroup
+constexpr int PG = 16;                // lanes of a cell
+constexpr int PTH = PCH * PG;         // threads: two wavefronts
+constexpr int PTW = PCH + 2, PDW = PCH + 4, PTILE = 5 * PDW * 3;
+constexpr int MLC = 47;               // a cell's listed movers
+constexpr int YN = 17;                // doubles of a mover's y side (mover_sums)
 constexpr int CFN = 10;               // doubles per field and cell (9 coefficients, padded)
 constexpr int NCORE = 21;
 
 // w-(o) = 1/2 - o + o^2/2, w0(o) = 1/2 + o - o^2, w+(o) = o^2/2:
 // sum_ab T(a, b) w_a(ox) w_b(oy) = sum_ij C_ij ox^i oy^j, C row i at 3 i.
 __device__ inline void cell_coeffs(double *cf, const double *Tk) {
+  constexpr int TW = PTW;
   double R[3][3];
 #pragma unroll
   for (int b = 0; b < 3; ++b) {
@@ -665,13 +681,13 @@ __device__ inline double dpp_f64(double v) {
   return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
 }
 
-// Sums of M values over the 8 lanes of a group, by halving: in each of three
+// Sums of 24 values over the 16 lanes of a group, by halving: in each of three
 // exchanges a lane keeps one half of the values and adds its partner's share
-// of them (partners: the mirrored lane, then lane xor 2, then lane xor 1).
-// Lane sub ends with the sums of values slot .. slot + M / 8 - 1 in v[0..],
-// slot = (sub >> 2) M / 2 + (sub >> 1 & 1) M / 4 + (sub & 1) M / 8.  About 6
-// instructions a value against 12 for a butterfly of each and one lane
-// writing them all.
+// of them (partners: lane xor 8, the mirrored lane of its eight, lane xor 2);
+// the last, with lane xor 1, adds the three that are left.  Lane sub ends with
+// the sums of values slot .. slot + 2 in v[0..2], slot = 12 (sub >> 3) +
+// 6 (sub >> 2 & 1) + 3 (sub >> 1 & 1).  About 6 instructions a value against
+// 15 for a butterfly of each.
 template <int M, int CTRL>
 __device__ inline void halve(double *v, bool up) {
 #pragma unroll
@@ -681,140 +697,300 @@ __device__ inline void halve(double *v, bool up) {
     v[e] = keep + dpp_f64<CTRL>(give);
   }
 }
-template <int M>
 __device__ inline int group_sums(double *v, int sub) {
-  static_assert(M % 8 == 0, "three halvings");
-  halve<M, 0x141>(v, sub & 4);           // row_half_mirror: lane 7 - sub
-  halve<M / 2, 0x4E>(v, sub & 2);        // quad_perm [2,3,0,1]
-  halve<M / 4, 0xB1>(v, sub & 1);        // quad_perm [1,0,3,2]
-  return ((sub >> 2) & 1) * (M / 2) + ((sub >> 1) & 1) * (M / 4) + (sub & 1) * (M / 8);
+  halve<24, 0x128>(v, sub & 8);          // row_ror:8: lane xor 8
+  halve<12, 0x141>(v, sub & 4);          // row_half_mirror: lane 7 - sub of its eight
+  halve<6, 0x4E>(v, sub & 2);            // quad_perm [2,3,0,1]
+#pragma unroll
+  for (int e = 0; e < 3; ++e) v[e] += dpp_f64<0xB1>(v[e]);   // quad_perm [1,0,3,2]
+  return ((sub >> 3) & 1) * 12 + ((sub >> 2) & 1) * 6 + ((sub >> 1) & 1) * 3;
 }
 
-// One current component of a cell's listed movers, added to its sums.
-template <int C>
-__device__ inline void mover_pass(double *cb, int sub, const double *L, const uint8_t *Ls, int nl,
-                                  int i, int j, const PP &P) {
-  constexpr int N = C == 2 ? 25 : 20, M = C == 2 ? 32 : 24;
-  double acc[M];
-#pragma unroll
-  for (int k = 0; k < M; ++k) acc[k] = 0.0;
-  for (int e = sub; e < nl; e += GROUP) {
-    Move m;
-    make_move(m, L[e], L[MLC + e], L[2 * MLC + e], L[3 * MLC + e], i, j, P);
-    stencil<C>(acc, m, P.q[Ls[e]] * P.qc_scale, L[4 * MLC + e]);
+// acc[a] += gx[a] V + dx[a] W with gx and dx those of lane N of the row of 16.
+// One instruction a product: the row broadcast is the multiply-add's own
+// operand modifier (the wait covers it after a write of gx or dx).
+template <int N>
+__device__ inline void add_outer(double (&acc)[5], const double (&gx)[5], const double (&dx)[5],
+                                 double V, double W) {
+#define WM_ROW "row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+  __asm__("s_nop 4\n\t"
+          "v_fmac_f64_dpp %0, %5, %15 " WM_ROW "v_fmac_f64_dpp %1, %6, %15 " WM_ROW
+          "v_fmac_f64_dpp %2, %7, %15 " WM_ROW "v_fmac_f64_dpp %3, %8, %15 " WM_ROW
+          "v_fmac_f64_dpp %4, %9, %15 " WM_ROW "v_fmac_f64_dpp %0, %10, %16 " WM_ROW
+          "v_fmac_f64_dpp %1, %11, %16 " WM_ROW "v_fmac_f64_dpp %2, %12, %16 " WM_ROW
+          "v_fmac_f64_dpp %3, %13, %16 " WM_ROW "v_fmac_f64_dpp %4, %14, %16 " WM_ROW
+          : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4])
+          : "v"(gx[0]), "v"(gx[1]), "v"(gx[2]), "v"(gx[3]), "v"(gx[4]), "v"(dx[0]), "v"(dx[1]),
+            "v"(dx[2]), "v"(dx[3]), "v"(dx[4]), "v"(V), "v"(W), "n"(N));
+#undef WM_ROW
+}
+
+// A lane's part in the sums of its cell's movers: one row of Jx, Jy or Jz, all
+// five columns.  With X = s0x + dx / 2, Y = s0y + dy / 2 and wy the
+// running sum of -q dy/dt dy, the three are sums over the movers of outer
+// products with X or dx (field.f90:274-298):
+//   Jy = X wy,  Jz = q vz (X Y + dx dy / 12),
+//   Jx = the running sum along x of -q dx/dt dx Y, taken at the end.
+// A lane's factors are V = y[p] y[s] (of X) and W = y[w] y[t] (of dx), y the
+// mover's y side in LDS: Y 0..4, wy 5..8, dy 9..13, then q vz, q vz / 12,
+// -q dx/dt; p or w -1: zero.
+struct Role {
+  int p, s, w, t, out;           // out: first of the cell's sums, -1: none
+};
+__device__ inline Role role_of(int lane16) {
+  Role r{-1, 0, -1, 0, -1};
+  if (lane16 < 5) {
+    r.w = lane16;
+    r.t = 16;
+    r.out = lane16;              // Jx: + 5 a
+  } else if (lane16 < 9) {
+    r.p = lane16;
+    r.out = 20 + lane16 - 5;     // Jy: + 4 a
+  } else if (lane16 < 14) {
+    r.p = lane16 - 9;
+    r.s = 14;
+    r.w = lane16;
+    r.t = 15;
+    r.out = 40 + lane16 - 9;     // Jz: + 5 a
   }
-  const int off = C == 0 ? 0 : (C == 1 ? 20 : 40), s0 = group_sums<M>(acc, sub);
+  return r;
+}
+
+// The listed movers' current, added to the lanes' sums.  Sixteen movers of a
+// cell at a time: lane sub prepares mover e0 + sub and keeps its x side, the y
+// sides go to LDS, and the cell's 16 lanes take the movers one after the
+// other.  No reduction: a lane's sums are its own.  All 64 lanes call it.
+// (One component after another over the list, a lane a mover, took three
+// passes over the shapes and 80 values through the lanes' reduction: 471
+// million vector instructions a step at 1024 x 512 against 339.)
+__device__ inline void outer_sums(double (&A)[5], const double (&gx)[5], const double (&dx)[5],
+                                  const double *Y, const Role &r, bool jy,
+                                  unsigned long long has) {
+  auto factors = [&](const double *y, double &V, double &W) {
+    const double p = y[r.p < 0 ? 0 : r.p], s = y[r.s], w = y[r.w < 0 ? 0 : r.w], t = y[r.t];
+    V = r.p < 0 ? 0.0 : (jy ? p : p * s);
+    W = r.w < 0 ? 0.0 : w * t;
+  };
+#define WM_PAIR(N0)                                     \
+  if (has & (0x0001000100010001ULL << (N0))) {          \
+    double V0, W0, V1, W1;                              \
+    factors(Y + (N0) * YN, V0, W0);                     \
+    factors(Y + ((N0) + 1) * YN, V1, W1);               \
+    add_outer<(N0)>(A, gx, dx, V0, W0);                 \
+    add_outer<(N0) + 1>(A, gx, dx, V1, W1);             \
+  }
+  WM_PAIR(0) WM_PAIR(2) WM_PAIR(4) WM_PAIR(6)
+  WM_PAIR(8) WM_PAIR(10) WM_PAIR(12) WM_PAIR(14)
+#undef WM_PAIR
+}
+__device__ inline void mover_sums(double (&A)[5], int sub, const double *L, const uint8_t *Ls,
+                                  double *Y, const Role &r, int nl, int i, int j, const PP &P,
+                                  const double *qcs) {
+  const bool jy = r.out >= 20 && r.out < 40;
+  for (int e0 = 0; __ballot(e0 < nl) != 0ULL; e0 += PG) {
+    const int e = e0 + sub;
+    const unsigned long long has = __ballot(e < nl);
+    double gx[5], dx[5], gy[5], dy[5], qv = 0.0, qc = 0.0;
+    if (e < nl) {
+      Move m;
+      make_move(m, L[e], L[MLC + e], L[2 * MLC + e], L[3 * MLC + e], i, j, P);
+      qv = L[4 * MLC + e];
+      qc = qcs[Ls[e]];
 #pragma unroll
-  for (int k = 0; k < M / 8; ++k)
-    if (s0 + k < N) cb[off + s0 + k] += acc[k];
+      for (int k = 0; k < 5; ++k) {
+        dx[k] = m.dsx[k];
+        dy[k] = m.dsy[k];
+        gx[k] = fma(0.5, dx[k], m.s0x[k]);
+        gy[k] = fma(0.5, dy[k], m.s0y[k]);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 5; ++k) gx[k] = dx[k] = gy[k] = dy[k] = 0.0;
+    }
+    double *y = Y + sub * YN, w = 0.0;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      y[k] = gy[k];
+      y[9 + k] = dy[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      w -= qc * dy[k];
+      y[5 + k] = w;
+    }
+    y[14] = qv;
+    y[15] = qv * (1.0 / 12.0);
+    y[16] = -qc;
+    __builtin_amdgcn_wave_barrier();
+    outer_sums(A, gx, dx, Y, r, jy, has);
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// A lane's mover sums of one cell into its 65 values.
+__device__ inline void put_sums(double *cb, const Role &r, const double (&v)[5]) {
+  if (r.out < 0) return;
+  if (r.out < 20) {
+    double t = 0.0;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      t += v[a];
+      cb[r.out + 5 * a] = t;
+    }
+  } else {
+    const int st = r.out < 40 ? 4 : 5;
+#pragma unroll
+    for (int a = 0; a < 5; ++a) cb[r.out + st * a] = v[a];
+  }
 }
 
 struct Part {
   double x, y, ux, uy, uz;
 };
 
-template <int SRC>
-__global__ __launch_bounds__(256, 3) void k_push_step(PP P, const int *__restrict__ cumcnt,
+// A loaded particle in registers of its own, so that the next load can have
+// the old ones: left to itself the compiler loads elsewhere and copies at the
+// end of the step, which waits for everything in flight.
+__device__ inline Part take(const Part &n) {
+  Part c;
+  __asm__ volatile("v_mov_b64 %0, %5\n\tv_mov_b64 %1, %6\n\tv_mov_b64 %2, %7\n\t"
+                   "v_mov_b64 %3, %8\n\tv_mov_b64 %4, %9"
+                   : "=&v"(c.x), "=&v"(c.y), "=&v"(c.ux), "=&v"(c.uy), "=&v"(c.uz)
+                   : "v"(n.x), "v"(n.y), "v"(n.ux), "v"(n.uy), "v"(n.uz));
+  return c;
+}
+
+template <int SRC, bool WALLS>
+__global__ __launch_bounds__(PTH, 2) void k_push_step(PP P, const int *__restrict__ cumcnt,
                                                       const double *__restrict__ tmp, int TX,
                                                       size_t tps, Rec64 A, Rec64 B, Order O,
                                                       double *__restrict__ part,
                                                       int *__restrict__ derr) {
-  __shared__ __attribute__((aligned(16))) double CF[CHUNK * 6 * CFN];
-  __shared__ double cellbuf[CHUNK * NACC];
-  // the movers' lists [x0 | y0 | x1 | y1 | q v_z][entry] per cell; before
-  // them, the chunk's cell-centred fields
-  __shared__ double mvl[CHUNK * 5 * MLC];
-  __shared__ uint8_t mvs[CHUNK * MLC];       // the entries' species
-  __shared__ int mk[CHUNK * 4];              // moves out of a cell: left, right, others
-  static_assert(6 * 3 * TW <= CHUNK * 5 * MLC, "the fields fit the lists' space");
-  double *T = mvl;
-  const int chunk = blockIdx.x;
-  const int jl = blockIdx.y;                 // row j = nys + jl
+  __shared__ __attribute__((aligned(16))) double CF[PCH * 6 * CFN];
+  // the movers' lists [x0 | y0 | x1 | y1 | q v_z][entry] per cell and their y
+  // sides; before them, the chunk's cell-centred fields, behind them the
+  // cells' sums
+  __shared__ double mvl[PCH * (5 * MLC + YN * PG)];
+  __shared__ uint8_t mvs[PCH * MLC];       // the entries' species
+  __shared__ int mk[PCH * 4];              // moves out of a cell: left, right, others
+  __shared__ double qcs[WM_MAXSP];         // q delx / dt of the species
+  static_assert(6 * 3 * PTW <= PCH * 5 * MLC && NACC <= 5 * MLC + YN * PG,
+                "the fields and the sums fit the lists' space");
+  double *T = mvl, *cellbuf = mvl;
+  // consecutive chunks on one XCD, which then has both parts of the lines that
+  // two of them share (workgroups go to the 8 XCDs in turn)
+  const unsigned nb = gridDim.x, per = nb / 8, cut = nb - per * 8;
+  const unsigned xcd = blockIdx.x % 8, at = xcd * per + min(xcd, cut) + blockIdx.x / 8;
+  const int chunk = at % P.nchunk;
+  const int jl = at / P.nchunk;              // row j = nys + jl
   const int j = P.nys + jl;
-  const int i0 = P.nxgs + chunk * CHUNK;
-  const int ncell = min(CHUNK, P.nx - chunk * CHUNK);
-  load_tmp_tile(T, tmp, TX, tps, jl, chunk * CHUNK, min(TW, ncell + 2));
-  for (int e = threadIdx.x; e < CHUNK * NACC; e += 256) cellbuf[e] = 0.0;
-  __syncthreads();
-  if (threadIdx.x < CHUNK * 6) {
-    const int c = threadIdx.x % CHUNK, k = threadIdx.x / CHUNK;
-    cell_coeffs(CF + (c * 6 + k) * CFN, T + k * 3 * TW + c);
+  const int i0 = P.nxgs + chunk * PCH;
+  const int ncell = min(PCH, P.nx - chunk * PCH);
+  const int g = threadIdx.x / PG;
+  const int sub = threadIdx.x % PG;
+  const int il = chunk * PCH + g, i = i0 + g;
+  // a species' slots of this group's cell (none beyond the row's cells)
+  int kb, ke, kbn = 0, ken = 0;                // this species, the next
+  auto slots = [&](int s, int &b, int &e) {
+    b = e = 0;
+    if (g < ncell && s < P.nsp) {
+      const int *cc = cumcnt + ((size_t)s * P.ny + jl) * (size_t)(P.nx + 1) + il;
+      b = max(0, cc[0]);
+      e = max(b, min(P.cap, cc[1]));
+    }
+  };
+  auto first = [&](int b, int e) { return b + sub; };
+  // the particle of slot q: where it is, and itself
+  auto src = [&](int s, int q, int b, int e) {
+    q = max(0, min(max(q, b), e - 1));
+    const unsigned p =
+        SRC == SRC_SLOT ? (unsigned)q : O.perm[((size_t)s * P.ny + jl) * (size_t)P.cap + q];
+    return b == e ? 0u : p;                    // an empty cell's is not read
+  };
+  auto load = [&](int s, unsigned p) {
+    const size_t sb = SRC == SRC_SLOT ? ((size_t)s * P.ny + jl) * (size_t)P.cap
+                                      : (size_t)s * P.ny * (size_t)P.cap;
+    const double *Xa = A.x + sb, *Ya = A.y + sb, *Uxa = A.ux + sb, *Uya = A.uy + sb, *Uza = A.uz + sb;
+    if (SRC == SRC_PERM64)
+      return Part{Xa[(size_t)p], Ya[(size_t)p], Uxa[(size_t)p], Uya[(size_t)p], Uza[(size_t)p]};
+    return Part{seg_ld(Xa, (int)p), seg_ld(Ya, (int)p), seg_ld(Uxa, (int)p), seg_ld(Uya, (int)p),
+                seg_ld(Uza, (int)p)};
+  };
+  // The chains of loads that start a species (slots, places, particles) run
+  // beside the fields' here, and the second species' beside the first's.
+  if (threadIdx.x < WM_MAXSP) qcs[threadIdx.x] = P.q[threadIdx.x] * P.qc_scale;
+  slots(0, kb, ke);
+  slots(1, kbn, ken);
+  load_tmp_tile<PTW>(T, tmp, TX, tps, jl, chunk * PCH, min(PTW, ncell + 2));
+  int k = first(kb, ke);
+  const unsigned p0 = src(0, k, kb, ke), p1 = src(0, k + PG, kb, ke);
+  // where the particles of the two steps after those in n0 and n1 come from
+  unsigned f0 = src(0, k + 2 * PG, kb, ke), f1 = src(0, k + 3 * PG, kb, ke);
+  const int kn = first(kbn, ken);
+  unsigned q0 = 0, q1 = 0, q2 = 0, q3 = 0;
+  if (P.nsp > 1) {
+    q0 = src(1, kn, kbn, ken);
+    q1 = src(1, kn + PG, kbn, ken);
+    q2 = src(1, kn + 2 * PG, kbn, ken);
+    q3 = src(1, kn + 3 * PG, kbn, ken);
   }
   __syncthreads();
-  const int g = threadIdx.x / GROUP;
-  const int sub = threadIdx.x % GROUP;
-  const int il = chunk * CHUNK + g, i = i0 + g;
+  Part n0 = load(0, p0), n1 = load(0, p1);     // the next two steps' particles
+  if (threadIdx.x < PCH * 6) {
+    const int c = threadIdx.x % PCH, k = threadIdx.x / PCH;
+    cell_coeffs(CF + (c * 6 + k) * CFN, T + k * 3 * PTW + c);
+  }
+  __syncthreads();
   double *cb = cellbuf + g * NACC;
   double *L = mvl + g * 5 * MLC;
+  double *Ys = mvl + PCH * 5 * MLC;
   uint8_t *Ls = mvs + g * MLC;
   const double2 *cf = (const double2 *)(CF + g * 6 * CFN);
-  const int wg = (threadIdx.x & 63) / GROUP;   // the group's place in its wavefront
+  const int wg = (threadIdx.x & 63) / PG;   // the group's place in its wavefront
+  const Role role = role_of(threadIdx.x & 15);
   int bad = 0;
-  if (g < ncell) {
-    double core[24];
-    int mcnt = 0;                              // the list's entries
-    int kb = 0, ke = 0, k = 0;
-    unsigned pn = 0;                           // the source of the step after next's particle
-    Part nxt{};                                // the next step's particle
-    const double *Xa = nullptr, *Ya = nullptr, *Uxa = nullptr, *Uya = nullptr, *Uza = nullptr;
-    const unsigned *Pm = nullptr;
-    auto src = [&](int q) {
-      q = min(max(q, kb), ke - 1);
-      return SRC == SRC_SLOT ? (unsigned)q : Pm[q];
-    };
-    auto load = [&](unsigned p) {
-      if (SRC == SRC_PERM64)
-        return Part{Xa[(size_t)p], Ya[(size_t)p], Uxa[(size_t)p], Uya[(size_t)p], Uza[(size_t)p]};
-      return Part{seg_ld(Xa, (int)p), seg_ld(Ya, (int)p), seg_ld(Uxa, (int)p), seg_ld(Uya, (int)p),
-                  seg_ld(Uza, (int)p)};
-    };
-    bool fresh = true, empty = true;
-    for (int s = 0;;) {
-      if (empty) {
+  double core[24], mv[5];               // the cell's own sums, its movers'
 #pragma unroll
-        for (int e = 0; e < 24; ++e) core[e] = 0.0;
-        empty = false;
-      }
+  for (int e = 0; e < 24; ++e) core[e] = 0.0;
+#pragma unroll
+  for (int e = 0; e < 5; ++e) mv[e] = 0.0;
+  {
+    // The step's results wait in registers and are stored at the top of the
+    // next, in front of its loads: loads and stores complete in order, and
+    // whatever is waited for was issued a whole step earlier.
+    Part out{};
+    unsigned ocd = 0;
+    int ok = -1;                               // their slot, -1: none
+    int mcnt = 0;                              // the list's entries
+    if (sub < 4) mk[g * 4 + sub] = 0;
+    for (int s = 0;;) {
       const size_t seg = (size_t)s * P.ny + jl, base = seg * (size_t)P.cap;
       const double q = P.q[s], r = P.r[s];
       const double fac1 = q / r * 0.5 * P.delt;
       const double txxx = fac1 * fac1;
       const double fac2 = q * P.delt / r;
       const double qc = q * P.qc_scale;
-      if (fresh) {
-        const int *cc = cumcnt + seg * (size_t)(P.nx + 1) + il;
-        kb = max(0, cc[0]);
-        ke = min(P.cap, cc[1]);
-        if (kb >= ke) ke = kb;
-        k = kb - kb % GROUP + sub;
-        const size_t sb = SRC == SRC_SLOT ? base : (size_t)s * P.ny * (size_t)P.cap;
-        Xa = A.x + sb;
-        Ya = A.y + sb;
-        Uxa = A.ux + sb;
-        Uya = A.uy + sb;
-        Uza = A.uz + sb;
-        Pm = O.perm + base;
-        if (sub < 4) mk[g * 4 + sub] = 0;
-        if (kb == ke) k = ke + sub;
-        fresh = false;
-      }
-      if (k - sub < ke) {
-        nxt = load(src(k));
-        pn = src(k + GROUP);
-      }
-      double *Xb = B.x + base, *Yb = B.y + base;
-      double *Uxb = B.ux + base, *Uyb = B.uy + base, *Uzb = B.uz + base;
-      uint16_t *Cd = O.code + base;
-      for (; k - sub < ke && __ballot(mcnt > MLC - GROUP) == 0ULL; k += GROUP) {
-        const Part c = nxt;
-        nxt = load(pn);
-        pn = src(k + 2 * GROUP);
+      auto put = [&] {
+        if (ok < 0) return;
+        O.code[base + ok] = (uint16_t)ocd;
+        seg_st(B.x + base, ok, out.x);
+        seg_st(B.y + base, ok, out.y);
+        seg_st(B.ux + base, ok, out.ux);
+        seg_st(B.uy + base, ok, out.uy);
+        seg_st(B.uz + base, ok, out.uz);
+        ok = -1;
+      };
+      auto step = [&](Part &n, unsigned &f) {
+        const Part c = take(n);
+        put();
+        n = load(s, f);
+        f = src(s, k + 4 * PG, kb, ke);
         bool cross = false;
         double qv = 0.0, x1 = 0.0, y1 = 0.0;
         if (k >= kb && k < ke) {
           const double ox = c.x * P.d_delx - i, oy = c.y * P.d_delx - j;
           PushOut o = boris_coeffs(cf, ox, oy, c.x, c.y, c.ux, c.uy, c.uz, P, fac1, txxx, fac2);
-          if (P.inj) injection_edge(o.x, o.ux, o.uy, o.uz, P);
+          if (WALLS && P.inj) injection_edge(o.x, o.ux, o.uy, o.uz, P);
           x1 = o.x;
           y1 = o.y;
           const int i2 = (int)(x1 * P.d_delx), j2 = (int)(y1 * P.d_delx);
@@ -822,19 +998,19 @@ __global__ __launch_bounds__(256, 3) void k_push_step(PP P, const int *__restric
           // field.f90:270's v_z = u_z / gamma with the push's 1 / gamma of the
           // same u, except where the shock's injection edge may have
           // reflected it
-          const double gvz = !P.inj ? o.uz * o.ig
+          const double gvz = !(WALLS && P.inj) ? o.uz * o.ig
                                     : o.uz / sqrt(1.0 + (o.ux * o.ux + o.uy * o.uy + o.uz * o.uz) /
                                                             (P.c * P.c));
           qv = q * gvz;
           if (!cross) core_add(core, ox, oy, x1 * P.d_delx - i, y1 * P.d_delx - j, qc, qv);
           unsigned cd = (unsigned)il << 2;
-          if (cross || P.xmode == 2) {
+          if (cross || (WALLS && P.xmode == 2)) {
             // particle_x and particle_y of the stored state (the deposit takes
             // the unwrapped one), as boundary_periodic.f90 and the wall
             // families' particle_x write them
             if (!(i2 - i >= -1 && i2 - i <= 1)) bad |= DERR_JUMP;
             int inew = i2;
-            if (P.xmode == 1) {
+            if (!WALLS) {
               if (i2 < P.nxgs) o.x = wm_edges::add_rd(o.x, P.spanx);
               else if (i2 >= P.nxgs + P.nx) o.x = wm_edges::add_rd(o.x, -P.spanx);
               inew = (int)o.x;
@@ -858,7 +1034,7 @@ __global__ __launch_bounds__(256, 3) void k_push_step(PP P, const int *__restric
             }
             if (d < -1 || d > 1) bad |= DERR_JUMP;
             int dc = cn - il;
-            if (P.xmode == 1) dc = dc == P.nx - 1 ? -1 : (dc == 1 - P.nx ? 1 : dc);
+            if (!WALLS) dc = dc == P.nx - 1 ? -1 : (dc == 1 - P.nx ? 1 : dc);
             const bool out = d == 1 || d == -1, far = !out && (dc < -1 || dc > 1);
             cd = (unsigned)cn << 2 | (out ? (d == 1 ? WM_CODE_UP : WM_CODE_DOWN)
                                           : (far ? WM_CODE_FAR : WM_CODE_STAY));
@@ -868,16 +1044,13 @@ __global__ __launch_bounds__(256, 3) void k_push_step(PP P, const int *__restric
             }
             if (out || dc != 0) atomicAdd(&mk[g * 4 + (out || far ? 2 : (dc < 0 ? 0 : 1))], 1);
           }
-          Cd[k] = (uint16_t)cd;
-          seg_st(Xb, k, o.x);
-          seg_st(Yb, k, o.y);
-          seg_st(Uxb, k, o.ux);
-          seg_st(Uyb, k, o.uy);
-          seg_st(Uzb, k, o.uz);
+          out = Part{o.x, o.y, o.ux, o.uy, o.uz};
+          ocd = cd;
+          ok = k;
         }
         // a crossing particle goes to the cell's list in (step, lane) order,
         // ranked by a ballot over the group
-        const unsigned gb = (unsigned)(__ballot(cross) >> (GROUP * wg)) & 0xFFu;
+        const unsigned gb = (unsigned)(__ballot(cross) >> (PG * wg)) & 0xFFFFu;
         if (cross) {
           const int e = mcnt + __popc(gb & ((1u << sub) - 1u));
           L[e] = c.x;
@@ -888,47 +1061,63 @@ __global__ __launch_bounds__(256, 3) void k_push_step(PP P, const int *__restric
           Ls[e] = (uint8_t)s;
         }
         mcnt += __popc(gb);
+        k += PG;
+      };
+      for (; k - sub < ke && __ballot(mcnt > MLC - 2 * PG) == 0ULL;) {
+        step(n0, f0);
+        if (__ballot(k - sub < ke) == 0ULL) break;   // (the next species' loads start anew)
+        step(n1, f1);
       }
+      put();
       if (__ballot(k - sub < ke) == 0ULL) {    // every cell's particles of this species are done
         __builtin_amdgcn_wave_barrier();
-        if (sub == 0) {
+        if (sub == 0 && g < ncell) {
           const int l = mk[g * 4], rr = mk[g * 4 + 1], o = mk[g * 4 + 2];
           O.kind[seg * P.nx + il] = make_int4(l, ke - kb - l - rr - o, rr, o);
         }
         __builtin_amdgcn_wave_barrier();
         if (++s < P.nsp) {
-          fresh = true;
+          if (sub < 4) mk[g * 4 + sub] = 0;
+          kb = kbn;
+          ke = ken;
+          k = first(kb, ke);
+          if (s > 1) {
+            q0 = src(s, k, kb, ke);
+            q1 = src(s, k + PG, kb, ke);
+            q2 = src(s, k + 2 * PG, kb, ke);
+            q3 = src(s, k + 3 * PG, kb, ke);
+          }
+          n0 = load(s, q0);
+          n1 = load(s, q1);
+          f0 = q2;
+          f1 = q3;
+          slots(s + 1, kbn, ken);
           continue;
         }
       }
-      // the cell's sums so far (its accumulators are free for the lists then)
-      {
-        const int s0 = group_sums<24>(core, sub);
-#pragma unroll
-        for (int e = 0; e < 3; ++e)
-          if (s0 + e < NCORE) cb[core_at(s0 + e)] += core[e];
-        empty = true;
-      }
       __builtin_amdgcn_wave_barrier();         // the group reads what its lanes listed
-      if (__ballot(mcnt > 0)) {
-        // full 5x5 stencils, one component at a time
-        mover_pass<0>(cb, sub, L, Ls, mcnt, i, j, P);
-        mover_pass<1>(cb, sub, L, Ls, mcnt, i, j, P);
-        mover_pass<2>(cb, sub, L, Ls, mcnt, i, j, P);
-        mcnt = 0;
-      }
-      __builtin_amdgcn_wave_barrier();         // the list is read before it is filled again
+      mover_sums(mv, sub, L, Ls, Ys + g * (YN * PG), role, mcnt, i, j, P, qcs);
+      mcnt = 0;
       if (s == P.nsp) break;
     }
   }
   if (bad) atomicOr(derr, bad);
+  __syncthreads();                             // the lists' space is free
+  put_sums(cb, role, mv);
+  __builtin_amdgcn_wave_barrier();
+  const int s0 = group_sums(core, sub);
+  if ((sub & 1) == 0) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (s0 + e < NCORE) cb[core_at(s0 + e)] += core[e];
+  }
   __syncthreads();
   // assemble the workgroup tile [b][t][comp] in a fixed order
-  double *out = part + ((size_t)jl * P.nchunk + chunk) * TILE;
-  for (int e = threadIdx.x; e < TILE; e += 256) {
+  double *out = part + ((size_t)jl * P.nchunk + chunk) * PTILE;
+  for (int e = threadIdx.x; e < PTILE; e += PTH) {
     const int comp = e % 3;
-    const int t = (e / 3) % DW;
-    const int b = e / (3 * DW);
+    const int t = (e / 3) % PDW;
+    const int b = e / (3 * PDW);
     double sum = 0.0;
     const int glo = max(0, t - 4), ghi = min(ncell - 1, t);
     for (int gg = glo; gg <= ghi; ++gg) sum += acc_at(cellbuf + gg * NACC, comp, t - gg, b);
@@ -1004,7 +1193,7 @@ int launch_particle(wm_ctx *ctx, int a, int b) {
 }  // namespace
 
 size_t wm_deposit_part_elems(int nx, int ny) {
-  return (size_t)ny * (size_t)wm_cdiv(nx, CHUNK) * (size_t)TILE;
+  return (size_t)ny * std::max((size_t)wm_cdiv(nx, CHUNK) * TILE, (size_t)wm_cdiv(nx, PCH) * PTILE);
 }
 
 int wm_k_cell_fields(wm_ctx *ctx) {
@@ -1037,10 +1226,18 @@ int wm_k_push_step(wm_ctx *ctx) {
   const size_t tps = (size_t)TX * (size_t)(ctx->g.ny + 2);
   const Order O{ctx->perm, ctx->code, ctx->kind, ctx->farcnt, ctx->far};
   // a species' plane below 4 GB is addressed by 32-bit byte offsets
-  auto kernel = !ctx->perm_valid                              ? k_push_step<SRC_SLOT>
-                : (size_t)P.ny * P.cap <= (size_t)1 << 29 ? k_push_step<SRC_PERM32>
-                                                              : k_push_step<SRC_PERM64>;
-  hipLaunchKernelGGL(kernel, dim3(P.nchunk, P.ny), dim3(256), 0, ctx->stream, P, ctx->cumcnt,
+  const int src = !ctx->perm_valid                          ? SRC_SLOT
+                  : (size_t)P.ny * P.cap <= (size_t)1 << 29 ? SRC_PERM32
+                                                            : SRC_PERM64;
+  auto kernel = P.xmode == 1
+                    ? (src == SRC_SLOT     ? k_push_step<SRC_SLOT, false>
+                       : src == SRC_PERM32 ? k_push_step<SRC_PERM32, false>
+                                           : k_push_step<SRC_PERM64, false>)
+                    : (src == SRC_SLOT     ? k_push_step<SRC_SLOT, true>
+                       : src == SRC_PERM32 ? k_push_step<SRC_PERM32, true>
+                                           : k_push_step<SRC_PERM64, true>);
+  P.nchunk = wm_cdiv(P.nx, PCH);
+  hipLaunchKernelGGL(kernel, dim3(P.nchunk * P.ny), dim3(PTH), 0, ctx->stream, P, ctx->cumcnt,
                      ctx->tmp, TX, tps, ctx->bank[0], ctx->bank[1], O, ctx->dep_part, ctx->derr);
   WM_HIP(hipGetLastError());
   std::swap(ctx->bank[0], ctx->bank[1]);

@@ -19,7 +19,7 @@
 
 namespace {
 
-constexpr int CHUNK = 16;             // cells per workgroup
+constexpr int CHUNK = WM_CHUNK_STEP32;             // cells per workgroup
 constexpr int GROUP = 16;             // lanes per cell
 constexpr int TW = CHUNK + 2;         // push tile width (halo 1)
 constexpr int DW = CHUNK + 4;         // deposit tile width (halo 2)
