@@ -10,6 +10,7 @@
 
 #include "wm_internal.h"
 #include "wm_solve.h"
+#include "wm_xfer.h"
 
 size_t wm_deposit_part_elems(int nx, int ny);
 size_t wm_deposit_part_elems32(int nx, int ny);
@@ -192,6 +193,20 @@ int ensure_mover_lists(wm_ctx *ctx) {
   return dmalloc(ctx, &ctx->mvid_dn, ms);
 }
 
+// The rows s0 .. s1 - 1 of a reference-layout particle array (cnt records
+// each), in a buffer of rows of w records.
+std::vector<WmSpan> row_spans(const wm_ctx *ctx, const double *up, const int *cnt, int s0, int s1,
+                              int w) {
+  const size_t rec = sizeof(double) * ctx->g.ndim;
+  std::vector<WmSpan> v;
+  v.reserve(s1 - s0);
+  for (int s = s0; s < s1; ++s)
+    if (cnt[s] > 0)
+      v.push_back({(const char *)up + (size_t)s * ctx->g.np * rec, (size_t)(s - s0) * w * rec,
+                   cnt[s] * rec});
+  return v;
+}
+
 // Upload the active records (cnt[seg] per segment) of a reference-layout
 // particle array into bank `b` and the current ID array.
 int upload_particles(wm_ctx *ctx, const double *up, const int *cnt_host, int b) {
@@ -215,13 +230,8 @@ int upload_particles(wm_ctx *ctx, const double *up, const int *cnt_host, int b) 
   ctx->perm_valid = false;                 // rows as given
   const size_t elems = (size_t)nseg * w * g.ndim;
   WM_TRY(ensure_stage(ctx, elems));
-  std::vector<double> h(elems);
-  for (int s = 0; s < nseg; ++s)
-    memcpy(&h[(size_t)s * w * g.ndim], up + (size_t)s * g.np * g.ndim,
-           sizeof(double) * (size_t)cnt_host[s] * g.ndim);
   int *dcnt = ctx->cnt_scratch;
-  WM_HIP(hipMemcpyAsync(ctx->stage, h.data(), sizeof(double) * elems, hipMemcpyHostToDevice,
-                        ctx->stream));
+  WM_TRY(wm_to_device(ctx, ctx->stage, row_spans(ctx, up, cnt_host, 0, nseg, w)));
   WM_HIP(hipMemcpyAsync(dcnt, cnt_host, sizeof(int) * nseg, hipMemcpyHostToDevice, ctx->stream));
   hipLaunchKernelGGL(k_aos_to_soa, dim3(std::min(64, wm_cdiv(w, 256)), nseg), dim3(256), 0,
                      ctx->stream, g.ndim, w, ctx->cap, dcnt, ctx->stage, ctx->bank[b],
@@ -250,21 +260,9 @@ int download_particles(wm_ctx *ctx, double *up, const int *cnt_host, int b, int 
                      ctx->stream, g.ndim, w, ctx->cap, dcnt, ctx->stage, ctx->bank[b],
                      ctx->id[ctx->idcur]);
   WM_HIP(hipGetLastError());
-  std::vector<double> h(elems);
-  WM_HIP(hipMemcpyAsync(h.data(), ctx->stage, sizeof(double) * elems, hipMemcpyDeviceToHost,
-                        ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
-  if (ncomp > 0 && ncomp < g.ndim) {      // the first ncomp components of each record only
-    for (int s = 0; s < nseg; ++s)
-      for (int k = 0; k < cnt_host[s]; ++k)
-        memcpy(up + ((size_t)s * g.np + k) * g.ndim, &h[((size_t)s * w + k) * g.ndim],
-               sizeof(double) * ncomp);
-    return WM_OK;
-  }
-  for (int s = 0; s < nseg; ++s)
-    memcpy(up + (size_t)s * g.np * g.ndim, &h[(size_t)s * w * g.ndim],
-           sizeof(double) * (size_t)cnt_host[s] * g.ndim);
-  return WM_OK;
+  const size_t rec = sizeof(double) * g.ndim;       // ncomp: the first components only
+  return wm_to_host(ctx, ctx->stage, row_spans(ctx, up, cnt_host, 0, nseg, w), rec,
+                    ncomp > 0 ? sizeof(double) * std::min(ncomp, g.ndim) : rec);
 }
 
 // FP32 form: the reference's rows <-> cell bins, through the staging buffer
@@ -302,12 +300,7 @@ int upload_bins(wm_ctx *ctx, const double *up, const int *cnt_host) {
     const int s1 = wm_batch_end(ctx, cnt_host, s0, &w);
     const size_t elems = (size_t)(s1 - s0) * w * g.ndim;
     WM_TRY(ensure_stage(ctx, elems));
-    std::vector<double> h(elems);
-    for (int s = s0; s < s1; ++s)
-      memcpy(&h[(size_t)(s - s0) * w * g.ndim], up + (size_t)s * g.np * g.ndim,
-             sizeof(double) * (size_t)cnt_host[s] * g.ndim);
-    WM_HIP(hipMemcpyAsync(ctx->stage, h.data(), sizeof(double) * elems, hipMemcpyHostToDevice,
-                          ctx->stream));
+    WM_TRY(wm_to_device(ctx, ctx->stage, row_spans(ctx, up, cnt_host, s0, s1, w)));
     WM_HIP(hipMemcpyAsync(ctx->cnt_scratch, cnt_host + s0, sizeof(int) * (s1 - s0),
                           hipMemcpyHostToDevice, ctx->stream));
     WM_TRY(wm_k_stage_to_bins(ctx, s0, s1 - s0, w));
@@ -333,13 +326,7 @@ int download_bins(wm_ctx *ctx, double *up, const int *cnt_host) {
     const size_t elems = (size_t)(s1 - s0) * w * g.ndim;
     WM_TRY(ensure_stage(ctx, elems));
     WM_TRY(wm_k_bins_to_stage(ctx, s0, s1 - s0, w));
-    std::vector<double> h(elems);
-    WM_HIP(hipMemcpyAsync(h.data(), ctx->stage, sizeof(double) * elems, hipMemcpyDeviceToHost,
-                          ctx->stream));
-    WM_HIP(hipStreamSynchronize(ctx->stream));
-    for (int s = s0; s < s1; ++s)
-      memcpy(up + (size_t)s * g.np * g.ndim, &h[(size_t)(s - s0) * w * g.ndim],
-             sizeof(double) * (size_t)cnt_host[s] * g.ndim);
+    WM_TRY(wm_to_host(ctx, ctx->stage, row_spans(ctx, up, cnt_host, s0, s1, w)));
     s0 = s1;
   }
   return WM_OK;
@@ -360,8 +347,7 @@ int fresh_bins(wm_ctx *ctx) {
 int upload_field(wm_ctx *ctx, const double *a, int ncomp, double *planes) {
   const size_t n = (size_t)ctx->fg.gx * ctx->fg.gy;
   WM_TRY(ensure_stage(ctx, n * ncomp));
-  WM_HIP(hipMemcpyAsync(ctx->stage, a, sizeof(double) * n * ncomp, hipMemcpyHostToDevice,
-                        ctx->stream));
+  WM_TRY(wm_to_device(ctx, ctx->stage, a, sizeof(double) * n * ncomp));
   hipLaunchKernelGGL(k_aos_to_planes, dim3(wm_cdiv((long long)n, 256)), dim3(256), 0, ctx->stream,
                      ncomp, n, ctx->fg.ps, ctx->stage, planes);
   WM_HIP(hipGetLastError());
@@ -373,10 +359,7 @@ int download_field(wm_ctx *ctx, double *a, int ncomp, const double *planes) {
   hipLaunchKernelGGL(k_planes_to_aos, dim3(wm_cdiv((long long)n, 256)), dim3(256), 0, ctx->stream,
                      ncomp, n, ctx->fg.ps, ctx->stage, planes);
   WM_HIP(hipGetLastError());
-  WM_HIP(hipMemcpyAsync(a, ctx->stage, sizeof(double) * n * ncomp, hipMemcpyDeviceToHost,
-                        ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
-  return WM_OK;
+  return wm_to_host(ctx, ctx->stage, a, sizeof(double) * n * ncomp);
 }
 
 // cumcnt as the device reads it: the wall families' entries outside
@@ -420,10 +403,7 @@ int upload_cumcnt(wm_ctx *ctx, const int *cumcnt_in) {
       return WM_ERR_RANGE;
     }
   }
-  WM_HIP(hipMemcpyAsync(ctx->cumcnt, cumcnt, sizeof(int) * n, hipMemcpyHostToDevice, ctx->stream));
-  // the copy reads act before this scope ends
-  WM_HIP(hipStreamSynchronize(ctx->stream));
-  return WM_OK;
+  return wm_to_device(ctx, ctx->cumcnt, cumcnt, sizeof(int) * n);
 }
 
 // The particles a cumcnt table hands out: the largest entry of the active
@@ -830,6 +810,7 @@ int wm_destroy(wm_ctx *ctx) {
   for (int k = 0; k < 32; ++k) (void)hipEventDestroy(ctx->ev[k]);
   (void)hipStreamDestroy(ctx->stream);
   (void)hipStreamDestroy(ctx->stream2);
+  wm_xfer_free(ctx);
   if (ctx->h_pin) (void)hipHostFree(ctx->h_pin);
   delete ctx;
   return WM_OK;
@@ -985,10 +966,8 @@ int wm_particle_solv(wm_ctx *ctx, double *gp, const double *up, const double *uf
   WM_TRY(wm_check_derr(ctx, "particle__solv"));
   WM_TRY(download_particles(ctx, gp, cnt.data(), 1));
   // gp(6,:,:,:) = up(6,:,:,:) over the whole capacity (particle.f90:171-175)
-  if (ctx->g.ndim == 6) {
-    const size_t n = (size_t)ctx->g.np * ctx->g.ny * ctx->g.nsp;
-    for (size_t t = 0; t < n; ++t) gp[6 * t + 5] = up[6 * t + 5];
-  }
+  // (the downloaded records hold it)
+  if (ctx->g.ndim == 6) wm_copy_field6(gp, up, cnt.data(), ctx->g.np, nseg_of(ctx));
   return WM_OK;
 }
 
@@ -1076,9 +1055,7 @@ int wm_sort_bucket(wm_ctx *ctx, double *gp, const double *up, int *cumcnt, const
   WM_TRY(wm_check_derr(ctx, "sort__bucket"));
   const int w = ctx->g.nx + 1;
   std::vector<int> cc((size_t)nseg * w);
-  WM_HIP(hipMemcpyAsync(cc.data(), ctx->cumcnt, sizeof(int) * cc.size(), hipMemcpyDeviceToHost,
-                        ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
+  WM_TRY(wm_to_host(ctx, ctx->cumcnt, cc.data(), sizeof(int) * cc.size()));
   // sort.f90:66-69 writes cumcnt(nxs:nxe+1) only
   const int a = nxs - ctx->g.nxgs, b = nxe + 1 - ctx->g.nxgs;
   for (int sg = 0; sg < nseg; ++sg)
@@ -1293,10 +1270,9 @@ int wm_state_download(wm_ctx *ctx, double *up, int *np2, int *cumcnt, double *uf
   if (up) WM_TRY(wm_order_apply(ctx));
   std::vector<int> n2(nseg);
   WM_HIP(hipMemcpyAsync(n2.data(), ctx->np2, sizeof(int) * nseg, hipMemcpyDeviceToHost, ctx->stream));
-  if (cumcnt)
-    WM_HIP(hipMemcpyAsync(cumcnt, ctx->cumcnt, sizeof(int) * (size_t)nseg * (ctx->g.nx + 1),
-                          hipMemcpyDeviceToHost, ctx->stream));
   WM_HIP(hipStreamSynchronize(ctx->stream));
+  if (cumcnt)
+    WM_TRY(wm_to_host(ctx, ctx->cumcnt, cumcnt, sizeof(int) * (size_t)nseg * (ctx->g.nx + 1)));
   if (f32) WM_TRY(wm_check_derr(ctx, "state download"));
   if (np2) memcpy(np2, n2.data(), sizeof(int) * nseg);
   if (up) WM_TRY(f32 ? download_bins(ctx, up, n2.data()) : download_particles(ctx, up, n2.data(), 0));
@@ -1472,10 +1448,7 @@ int wm_mom_calc_nvt(wm_ctx *ctx, double *mom, const double *up, const int *np2) 
   WM_TRY(wm_k_sort(ctx, 1, 0));
   WM_TRY(wm_k_moments(ctx, false));
   WM_TRY(wm_check_derr(ctx, "mom_calc__nvt"));
-  WM_HIP(hipMemcpyAsync(mom, ctx->mom, sizeof(double) * wm_mom_elems(ctx), hipMemcpyDeviceToHost,
-                        ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
-  return WM_OK;
+  return wm_to_host(ctx, ctx->mom, mom, sizeof(double) * wm_mom_elems(ctx));
 }
 
 int wm_bcp_mom(wm_ctx *ctx, double *mom) {
@@ -1507,16 +1480,14 @@ int wm_moments(wm_ctx *ctx, double *mom) {
   WM_HIP(hipEventRecord(e[1], ctx->stream));
   WM_TRY(wm_k_bc_mom(ctx, ctx->mom));
   WM_HIP(hipEventRecord(e[2], ctx->stream));
+  wm_touch(mom, sizeof(double) * wm_mom_elems(ctx));
   WM_TRY(wm_check_derr(ctx, "mom_calc__nvt"));
   float ms = 0.f;
   WM_HIP(hipEventElapsedTime(&ms, e[0], e[1]));
   ctx->phase_ms[WM_NPHASE] = ms;
   WM_HIP(hipEventElapsedTime(&ms, e[1], e[2]));
   ctx->phase_ms[WM_NPHASE + 1] = ms;
-  WM_HIP(hipMemcpyAsync(mom, ctx->mom, sizeof(double) * wm_mom_elems(ctx), hipMemcpyDeviceToHost,
-                        ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
-  return WM_OK;
+  return wm_to_host(ctx, ctx->mom, mom, sizeof(double) * wm_mom_elems(ctx));
 }
 
 int wm_cg_iters(wm_ctx *ctx, int *iters3) {

@@ -211,6 +211,7 @@ struct wm_ctx {
   double *diag = nullptr;  // diagnostics scratch
   int *derr = nullptr;     // device error bits
   void *h_pin = nullptr;   // pinned host scratch for small read-backs (WM_PIN_BYTES)
+  struct wm_xfer *xfer = nullptr;   // pinned buffers of the host arrays' copies
 
   // host staging (drop-in host-array entry points)
   double *stage = nullptr; size_t stage_elems = 0;
