@@ -28,7 +28,14 @@
 namespace {
 constexpr size_t SLOT = (size_t)4 << 20;
 constexpr int WORKERS = 8;
-constexpr size_t SHARE = (size_t)1 << 20;   // bytes worth a thread (starting one costs about 20 us)
+// Threads for a copy: one up to 8 MB, then one per MB.  Starting one costs
+// about 20 us, and now and then milliseconds where the process has used up its
+// share of the processors (its other threads may be waiting actively); 5 MB by
+// one thread take 0.30 ms, as by four.
+int threads_for(size_t bytes) {
+  constexpr size_t ALONE = (size_t)8 << 20, SHARE = (size_t)1 << 20;
+  return bytes < ALONE ? 1 : (int)std::min<size_t>(WORKERS, bytes / SHARE);
+}
 
 // f(worker) on `n` threads, the caller's as worker 0; fewer if the system
 // gives no more.
@@ -48,7 +55,7 @@ void on_threads(int n, F f) {
 struct wm_xfer {
   void *pin[WORKERS] = {};
   hipEvent_t ev[WORKERS] = {};
-  bool busy[WORKERS] = {};                  // the device may still read it
+  bool busy[WORKERS] = {};                     // the device may still read it
 };
 
 void wm_xfer_free(wm_ctx *ctx) {
@@ -93,8 +100,11 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
   if (total == 0) return WM_OK;
   if (!ctx->xfer) ctx->xfer = new wm_xfer;
   wm_xfer &x = *ctx->xfer;
-  const int want = (int)std::min<size_t>(WORKERS, std::max<size_t>(1, total / SHARE));
-  const size_t most = std::min(SLOT, std::max<size_t>(total / want + rec, 256 << 10)) / rec * rec;
+  const int want = threads_for(total);
+  // one thread alone has two buffers, and copies a chunk while the next is on
+  // its way
+  const size_t most =
+      std::min(SLOT, std::max<size_t>(total / (want > 1 ? want : 3) + rec, (size_t)1 << 20)) / rec * rec;
   std::vector<WmSpan> piece;
   std::vector<Chunk> chunk;
   for (const WmSpan &s : spans)
@@ -112,37 +122,49 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
   const int device = ctx->device;
   on_threads((int)std::min<size_t>(want, chunk.size()), [&](int w) {
     hipError_t e = w > 0 ? hipSetDevice(device) : hipSuccess;   // (a thread's own)
-    if (e == hipSuccess) e = slot_of(x, w);
+    size_t last = chunk.size();               // down: the chunk on its way
+    const int other = want > 1 ? 0 : 1;
+    int buf = w;
+    auto land = [&](size_t c, int b) {        // chunk c, in buffer b, to its place
+      const Chunk &h = chunk[c];
+      for (size_t k = h.s0; k < h.s1; ++k) touch(piece[k].host, piece[k].bytes);
+      const hipError_t r = hipEventSynchronize(x.ev[b]);
+      if (r != hipSuccess) return r;
+      x.busy[b] = false;
+      for (size_t k = h.s0; k < h.s1; ++k) {
+        char *d = const_cast<char *>(piece[k].host);
+        const char *s = (const char *)x.pin[b] + (piece[k].at - piece[h.s0].at);
+        if (keep == rec) {
+          memcpy(d, s, piece[k].bytes);
+        } else {
+          for (size_t o = 0; o < piece[k].bytes; o += rec) memcpy(d + o, s + o, keep);
+        }
+      }
+      return r;
+    };
     for (size_t c; e == hipSuccess && err.load() == (int)hipSuccess && (c = next++) < chunk.size();) {
       const Chunk &h = chunk[c];
       const size_t at = piece[h.s0].at, len = piece[h.s1 - 1].at + piece[h.s1 - 1].bytes - at;
-      char *pin = (char *)x.pin[w];
-      if (x.busy[w]) e = hipEventSynchronize(x.ev[w]);
+      e = slot_of(x, buf);
+      if (e == hipSuccess && x.busy[buf]) e = hipEventSynchronize(x.ev[buf]);
       if (e != hipSuccess) break;
-      x.busy[w] = true;
+      x.busy[buf] = true;
+      char *pin = (char *)x.pin[buf];
       if (up) {
         for (size_t k = h.s0; k < h.s1; ++k) memcpy(pin + (piece[k].at - at), piece[k].host, piece[k].bytes);
         e = hipMemcpyAsync(dev + at, pin, len, hipMemcpyHostToDevice, st);
-        if (e == hipSuccess) e = hipEventRecord(x.ev[w], st);
       } else {
         e = hipMemcpyAsync(pin, dev + at, len, hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipEventRecord(x.ev[w], st);
-        if (e != hipSuccess) break;
-        for (size_t k = h.s0; k < h.s1; ++k) touch(piece[k].host, piece[k].bytes);
-        e = hipEventSynchronize(x.ev[w]);
-        if (e != hipSuccess) break;
-        x.busy[w] = false;
-        for (size_t k = h.s0; k < h.s1; ++k) {
-          char *d = const_cast<char *>(piece[k].host);
-          const char *s = pin + (piece[k].at - at);
-          if (keep == rec) {
-            memcpy(d, s, piece[k].bytes);
-          } else {
-            for (size_t o = 0; o < piece[k].bytes; o += rec) memcpy(d + o, s + o, keep);
-          }
-        }
       }
+      if (e == hipSuccess) e = hipEventRecord(x.ev[buf], st);
+      if (e == hipSuccess && !up) {
+        if (other == 0) e = land(c, buf);
+        else if (last < chunk.size()) e = land(last, buf ^ 1);
+        last = c;
+      }
+      buf ^= other;
     }
+    if (!up && other && e == hipSuccess && last < chunk.size()) e = land(last, buf ^ 1);
     int ok = (int)hipSuccess;
     if (e != hipSuccess) err.compare_exchange_strong(ok, (int)e);
   });
@@ -166,8 +188,7 @@ int wm_to_host(wm_ctx *ctx, const void *dev, void *host, size_t bytes) {
 }
 
 void wm_touch(void *host, size_t bytes) {
-  const int n = (int)std::min<size_t>(WORKERS, bytes / (2 * SHARE));
-  if (n < 1) return;
+  const int n = threads_for(bytes);
   on_threads(n, [&](int k) {
     const size_t a = bytes * k / n, b = bytes * (k + 1) / n;
     touch((const char *)host + a, b - a);
@@ -176,7 +197,7 @@ void wm_touch(void *host, size_t bytes) {
 
 void wm_copy_field6(double *dst, const double *src, const int *from, size_t np, int nrow) {
   const size_t bytes = (size_t)nrow * np * 96;
-  const int want = (int)std::min<size_t>(WORKERS, std::max<size_t>(1, bytes / (2 * SHARE)));
+  const int want = threads_for(bytes / 2);
   std::atomic<int> next{0};
   on_threads(std::min(want, nrow), [&](int) {
     for (int s; (s = next++) < nrow;)
