@@ -22,9 +22,15 @@
 // floating-point atomics).
 #include "wm_internal.h"
 #include "wm_edges.h"
+#include "wm_mover.h"
 #include "wm_order.h"
 
 namespace {
+
+using wm_mover::put_sums;
+using wm_mover::Role;
+using wm_mover::role_of;
+using wm_mover::YN;
 
 constexpr int CHUNK = WM_CHUNK_HOST64;   // cells per workgroup
 constexpr int GROUP = 8;              // lanes per cell
@@ -532,7 +538,6 @@ constexpr int PG = 16;                // lanes of a cell
 constexpr int PTH = PCH * PG;         // threads: two wavefronts
 constexpr int PTW = PCH + 2, PDW = PCH + 4, PTILE = 5 * PDW * 3;
 constexpr int MLC = 47;               // a cell's listed movers
-constexpr int YN = 17;                // doubles of a mover's y side (mover_sums)
 constexpr int CFN = 10;               // doubles per field and cell (9 coefficients, padded)
 constexpr int NCORE = 21;
 
@@ -725,37 +730,6 @@ __device__ inline void add_outer(double (&acc)[5], const double (&gx)[5], const 
 #undef WM_ROW
 }
 
-// A lane's part in the sums of its cell's movers: one row of Jx, Jy or Jz, all
-// five columns.  With X = s0x + dx / 2, Y = s0y + dy / 2 and wy the
-// running sum of -q dy/dt dy, the three are sums over the movers of outer
-// products with X or dx (field.f90:274-298):
-//   Jy = X wy,  Jz = q vz (X Y + dx dy / 12),
-//   Jx = the running sum along x of -q dx/dt dx Y, taken at the end.
-// A lane's factors are V = y[p] y[s] (of X) and W = y[w] y[t] (of dx), y the
-// mover's y side in LDS: Y 0..4, wy 5..8, dy 9..13, then q vz, q vz / 12,
-// -q dx/dt; p or w -1: zero.
-struct Role {
-  int p, s, w, t, out;           // out: first of the cell's sums, -1: none
-};
-__device__ inline Role role_of(int lane16) {
-  Role r{-1, 0, -1, 0, -1};
-  if (lane16 < 5) {
-    r.w = lane16;
-    r.t = 16;
-    r.out = lane16;              // Jx: + 5 a
-  } else if (lane16 < 9) {
-    r.p = lane16;
-    r.out = 20 + lane16 - 5;     // Jy: + 4 a
-  } else if (lane16 < 14) {
-    r.p = lane16 - 9;
-    r.s = 14;
-    r.w = lane16;
-    r.t = 15;
-    r.out = 40 + lane16 - 9;     // Jz: + 5 a
-  }
-  return r;
-}
-
 // The listed movers' current, added to the lanes' sums.  Sixteen movers of a
 // cell at a time: lane sub prepares mover e0 + sub and keeps its x side, the y
 // sides go to LDS, and the cell's 16 lanes take the movers one after the
@@ -824,23 +798,6 @@ __device__ inline void mover_sums(double (&A)[5], int sub, const double *L, cons
     __builtin_amdgcn_wave_barrier();
     outer_sums(A, gx, dx, Y, r, jy, has);
     __builtin_amdgcn_wave_barrier();
-  }
-}
-
-// A lane's mover sums of one cell into its 65 values.
-__device__ inline void put_sums(double *cb, const Role &r, const double (&v)[5]) {
-  if (r.out < 0) return;
-  if (r.out < 20) {
-    double t = 0.0;
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      t += v[a];
-      cb[r.out + 5 * a] = t;
-    }
-  } else {
-    const int st = r.out < 40 ? 4 : 5;
-#pragma unroll
-    for (int a = 0; a < 5; ++a) cb[r.out + st * a] = v[a];
   }
 }
 

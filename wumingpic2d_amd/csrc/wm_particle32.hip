@@ -16,6 +16,8 @@
 // grid size.
 #include "wm_internal.h"
 #include "wm_migrate.h"
+#include "wm_mover.h"
+#include <type_traits>
 
 namespace {
 
@@ -192,32 +194,14 @@ __device__ inline void core32(float *core, float ox0, float oy0, float ox1, floa
   }
 }
 
-// A cell's stencil sums: the movers' sums, 65 per cell (Jx 0..19 as
-// (a-1)*5 + b with tile offset a >= 1, Jy 20..39 as 20 + a*4 + (b-1) with
-// b >= 1, Jz 40..64 as 40 + a*5 + b), and the stayers' 21 core sums where
-// the core has the offset (Jx a = 2..3, Jy b = 2..3, offsets 1..3
-// otherwise; the layout of core32).  Both are FP32 sums of the group's
-// lanes; after the movers' deposit each group adds its cell's pair in FP64
-// (csum, which takes the place of the movers' list offsets in LDS) for the
-// tile assembly.
-constexpr int CCS = 24;               // floats per cell of the core sums (21, padded)
-constexpr int CMS = 68;               // floats per cell of the movers' sums (65, padded)
-__shared__ float ccore[CHUNK * CCS];
-__shared__ float cmov[CHUNK * CMS];
-__device__ inline int core_of(int comp, int a, int b) {
-  if (comp == 0) return (a >= 2 && a <= 3 && b >= 1 && b <= 3) ? (a - 2) * 3 + (b - 1) : -1;
-  if (comp == 1) return (a >= 1 && a <= 3 && b >= 2 && b <= 3) ? 6 + (a - 1) * 2 + (b - 2) : -1;
-  return (a >= 1 && a <= 3 && b >= 1 && b <= 3) ? 12 + (a - 1) * 3 + (b - 1) : -1;
-}
-// Entry e of the 65 sums in FP64: core + movers (the core term first).
-__device__ inline double cell_sum(int cell, int e) {
-  const int comp = e < 20 ? 0 : (e < 40 ? 1 : 2);
-  const int a = comp == 0 ? e / 5 + 1 : (comp == 1 ? (e - 20) / 4 : (e - 40) / 5);
-  const int b = comp == 0 ? e % 5 : (comp == 1 ? (e - 20) % 4 + 1 : (e - 40) % 5);
-  const int c = core_of(comp, a, b);
-  const double mv = (double)cmov[cell * CMS + e];
-  const double cv = (double)ccore[cell * CCS + (c < 0 ? 0 : c)];
-  return c < 0 ? mv : cv + mv;
+// A cell's stencil sums (csum): 65 in FP64 (Jx 0..19 as (a-1)*5 + b with tile
+// offset a >= 1, Jy 20..39 as 20 + a*4 + (b-1) with b >= 1, Jz 40..64 as
+// 40 + a*5 + b), the movers' and, where the core has the offset, the stayers'
+// FP32 sums of the group's lanes.
+__device__ inline int core_at(int e) {             // slot of core value e (core32)
+  if (e < 6) return (1 + e / 3) * 5 + 1 + e % 3;
+  if (e < 12) return 20 + (1 + (e - 6) / 2) * 4 + 1 + (e - 6) % 2;
+  return 40 + (1 + (e - 12) / 3) * 5 + 1 + (e - 12) % 3;
 }
 // Sum of component comp at tile offset (a, b) of a cell, from csum.
 __device__ inline double acc_at(const double *csum, int cell, int comp, int a, int b) {
@@ -227,27 +211,34 @@ __device__ inline double acc_at(const double *csum, int cell, int comp, int a, i
   return none ? 0.0 : v;
 }
 
-// Sum over the 16 lanes of one DPP row (a group): quad butterflies, then
-// rotations by 4 and 8 within the row.  Every lane ends with the total; the
-// callers use lane 0's, whose association order is fixed.  The callers run
-// it with every lane of the row active, so each DPP source lane is valid;
-// written as update_dpp with bound_ctrl (zero for an invalid source), each
-// step compiles to a single v_add_f32_dpp.
+// Sums of 24 values over the 16 lanes of a group, by halving: in each of three
+// exchanges a lane keeps one half of the values and adds its partner's share
+// of them (partners: lane xor 8, the mirrored lane of its eight, lane xor 2);
+// the last, with lane xor 1, adds the three that are left.  Lane sub ends with
+// the sums of values slot .. slot + 2 in v[0..2], slot = 12 (sub >> 3) +
+// 6 (sub >> 2 & 1) + 3 (sub >> 1 & 1).  66 instructions, where a butterfly of
+// each of the 21 takes 84 and one lane writes them all.
 template <int CTRL>
-__device__ inline float dpp_add(float v) {
-  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+__device__ inline float dpp_of(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
-__device__ inline float row_sum16(float v) {
-  v = dpp_add<0xB1>(v);         // quad_perm [1,0,3,2]
-  v = dpp_add<0x4E>(v);         // quad_perm [2,3,0,1]
-  v = dpp_add<0x124>(v);        // row_ror 4
-  v = dpp_add<0x128>(v);        // row_ror 8
-  __asm__ volatile("" : "+v"(v));   // the last add stays fused, not sunk into the caller's branch
-  return v;
+template <int M, int CTRL>
+__device__ inline void halve(float *v, bool up) {
+#pragma unroll
+  for (int e = 0; e < M / 2; ++e) {
+    const float a = v[e], b = v[M / 2 + e];
+    const float keep = up ? b : a, give = up ? a : b;
+    v[e] = keep + dpp_of<CTRL>(give);
+  }
 }
-
-
-
+__device__ inline int group_sums(float *v, int sub) {
+  halve<24, 0x128>(v, sub & 8);          // row_ror:8: lane xor 8
+  halve<12, 0x141>(v, sub & 4);          // row_half_mirror: lane 7 - sub of its eight
+  halve<6, 0x4E>(v, sub & 2);            // quad_perm [2,3,0,1]
+#pragma unroll
+  for (int e = 0; e < 3; ++e) v[e] += dpp_of<0xB1>(v[e]);   // quad_perm [1,0,3,2]
+  return ((sub >> 3) & 1) * 12 + ((sub >> 2) & 1) * 6 + ((sub >> 1) & 1) * 3;
+}
 
 // Bin of (species s, row jl, cell i).
 __device__ inline size_t bin_of(int s, int jl, int i, int ny, int nx) {
@@ -269,8 +260,10 @@ constexpr int MAXB = 64;              // spill blocks of one cell's list
 constexpr int HCN = NPOOL * 4 / (NT / 8);   // migration prologue: holes cached per bin group
 
 // The push kernel's LDS (file scope, so device functions address it directly).
+__shared__ float4 CF4[CHUNK * CFS / 4];           // per-cell gather coefficients; then the
+                                                  // movers' y sides, YH of a cell at a time
 __shared__ float T[6 * 3 * TW];                   // cell-centred fields of the chunk
-__shared__ float4 CF4[CHUNK * CFS / 4];           // per-cell gather coefficients
+__shared__ float ccore[CHUNK * 24];               // stayers' sums per cell (21, padded)
 __shared__ int xl[NPOOL];                         // movers: species << 28 | dir << 20 | slot
 __shared__ float4 xpl[NPOOL];                     // movers' offsets before and after
 __shared__ float xql[NPOOL];                      // movers' charge times v_z
@@ -312,14 +305,6 @@ __device__ inline float xql_at(int e, const Spill &X) {
   return e < NPOOL ? xql[e] : X.q[X.base + (e - NPOOL)];
 }
 
-// The deposit of one cell's movers j = p, p + MQ, ... (part p of MQ) into
-// the 65 stencil sums of the cell (Jx a < 4 at a*5 + b, Jy b < 4 at
-// 20 + a*4 + b, Jz at 40 + a*5 + b): field.f90:224-268's Esirkepov weights
-// with s0 the old and ds the new minus the old 5-point shapes, in FP32,
-// summed over the part's movers in FP32.  Jz uses
-// s0x s0y + ds_x s0y / 2 + s0x ds_y / 2 + ds_x ds_y / 3 = X Y + ds_x ds_y / 12
-// with X = s0x + ds_x / 2, Y = s0y + ds_y / 2.
-constexpr int MQ = 16;
 // The 5-point old shape (support at 1..3) and new shape (support at
 // 1 + inc .. 3 + inc): ds = new - old and X = old + ds / 2.  Selects on
 // three flags rather than on inc's value, which the compiler would turn into
@@ -336,42 +321,113 @@ __device__ inline void place5(float sm, float s0, float sp, float nm, float n0, 
     X[k] = o[k] + 0.5f * ds[k];
   }
 }
-__device__ inline void mover_part(float *acc, int p, int nm, int mc, const Spill &X) {
-  const float twelfth = 1.0f / 12.0f;
-  for (int j = p; j < nm; j += MQ) {
-    const int e = xent(mc, j);
-    const float4 v = xpl_at(e, X);
-    const float qv = xql_at(e, X);
-    const int xv = xl_at(e, X);
-    const int dir = (xv >> 20) & 0xF;
-    const int dy = dir / 3 - 1, dx = dir - 3 * (dy + 1) - 1;
-    const float qc = sqc[xv >> 28];
-    float xm, x0, xp_, ym, y0, yp, nxm, nx0, nxp, nym, ny0, nyp;
-    shapef(v.x - 0.5f, xm, x0, xp_);
-    shapef(v.y - 0.5f, ym, y0, yp);
-    shapef(v.z - 0.5f, nxm, nx0, nxp);
-    shapef(v.w - 0.5f, nym, ny0, nyp);
-    float X[5], dX[5], Y[5], dY[5];
-    place5(xm, x0, xp_, nxm, nx0, nxp, dx, X, dX);
-    place5(ym, y0, yp, nym, ny0, nyp, dy, Y, dY);
-    // Jx (a, b) = w_a Y_b, w_a = -qc sum_{a' <= a} ds_x[a']; Jy likewise in y
-    float wx = 0.0f, wy[4];
+
+// acc[a] += gx[a] V + dx[a] W with gx and dx those of lane N of the group: the
+// row broadcast is the multiply-add's own operand modifier (the wait covers it
+// after a write of gx or dx).
+template <int N>
+__device__ inline void add_outer(float (&acc)[5], const float (&gx)[5], const float (&dx)[5],
+                                 float V, float W) {
+#define WM_ROW "row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+  __asm__("s_nop 4\n\t"
+          "v_fmac_f32_dpp %0, %5, %15 " WM_ROW "v_fmac_f32_dpp %1, %6, %15 " WM_ROW
+          "v_fmac_f32_dpp %2, %7, %15 " WM_ROW "v_fmac_f32_dpp %3, %8, %15 " WM_ROW
+          "v_fmac_f32_dpp %4, %9, %15 " WM_ROW "v_fmac_f32_dpp %0, %10, %16 " WM_ROW
+          "v_fmac_f32_dpp %1, %11, %16 " WM_ROW "v_fmac_f32_dpp %2, %12, %16 " WM_ROW
+          "v_fmac_f32_dpp %3, %13, %16 " WM_ROW "v_fmac_f32_dpp %4, %14, %16 " WM_ROW
+          : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4])
+          : "v"(gx[0]), "v"(gx[1]), "v"(gx[2]), "v"(gx[3]), "v"(gx[4]), "v"(dx[0]), "v"(dx[1]),
+            "v"(dx[2]), "v"(dx[3]), "v"(dx[4]), "v"(V), "v"(W), "n"(N));
+#undef WM_ROW
+}
+
+// The current of a cell's movers (field.f90:224-298's Esirkepov weights, s0
+// the old and ds the new minus the old 5-point shapes), as the lanes' sums of
+// outer products (wm_mover.h).  Sixteen at a time: lane sub prepares mover
+// e0 + sub and keeps its x side, the y sides go to LDS (Y, room for YH), and
+// the cell's lanes take the movers one after the other.  Products and the sums
+// of sixteen are FP32, the totals FP64.  All 64 lanes call it.  (A lane a
+// mover, with all 65 values in its registers and 4 instructions each to sum
+// them over the lanes, was a tenth of the push's instructions at 64 particles
+// per cell.  The push is bound by these, 82% of the issue slots: 2.36 -> 2.16 ms
+// at 1024 x 1024 cells, with the halving of the stayers' sums above.)
+constexpr int YH = 4;
+constexpr int YN = wm_mover::YN;
+static_assert(YH * YN * 4 <= CFS * 4, "the y sides take a cell's coefficients' place");
+template <int H>
+__device__ inline void outer_part(float (&acc)[5], const float (&gx)[5], const float (&dx)[5],
+                                  const float *Y, const wm_mover::Role &r, bool jy,
+                                  unsigned long long has) {
+  auto factors = [&](const float *y, float &V, float &W) {
+    const float p = y[r.p < 0 ? 0 : r.p], s = y[r.s], w = y[r.w < 0 ? 0 : r.w], t = y[r.t];
+    V = r.p < 0 ? 0.0f : (jy ? p : p * s);
+    W = r.w < 0 ? 0.0f : w * t;
+  };
+#define WM_PAIR(E)                                                  \
+  if (has & (0x0001000100010001ULL << (YH * H + (E)))) {            \
+    float V0, W0, V1, W1;                                           \
+    factors(Y + (E) * YN, V0, W0);                                  \
+    factors(Y + ((E) + 1) * YN, V1, W1);                            \
+    add_outer<YH * H + (E)>(acc, gx, dx, V0, W0);                   \
+    add_outer<YH * H + (E) + 1>(acc, gx, dx, V1, W1);               \
+  }
+  WM_PAIR(0) WM_PAIR(2)
+#undef WM_PAIR
+}
+__device__ inline void mover_sums(double (&sum)[5], int sub, int nm, int mc, float *Y,
+                                  const wm_mover::Role &r, const Spill &X) {
+  const bool jy = r.out >= 20 && r.out < 40;
+  for (int e0 = 0; __ballot(e0 < nm) != 0ULL; e0 += GROUP) {
+    const unsigned long long has = __ballot(e0 + sub < nm);
+    float gx[5], dx[5], gy[5], dy[5], wy[4], qv = 0.0f, qc = 0.0f;
+    if (e0 + sub < nm) {
+      const int e = xent(mc, e0 + sub);
+      const float4 v = xpl_at(e, X);
+      const int xv = xl_at(e, X);
+      qv = xql_at(e, X);
+      qc = sqc[xv >> 28];
+      const int dir = (xv >> 20) & 0xF;
+      const int iy = dir / 3 - 1, ix = dir - 3 * (iy + 1) - 1;
+      float xm, x0, xp_, ym, y0, yp, nxm, nx0, nxp, nym, ny0, nyp;
+      shapef(v.x - 0.5f, xm, x0, xp_);
+      shapef(v.y - 0.5f, ym, y0, yp);
+      shapef(v.z - 0.5f, nxm, nx0, nxp);
+      shapef(v.w - 0.5f, nym, ny0, nyp);
+      place5(xm, x0, xp_, nxm, nx0, nxp, ix, gx, dx);
+      place5(ym, y0, yp, nym, ny0, nyp, iy, gy, dy);
+    } else {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) wy[k] = (k ? wy[k - 1] : 0.0f) - qc * dY[k];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      wx -= qc * dX[a];
-#pragma unroll
-      for (int b = 0; b < 5; ++b) acc[a * 5 + b] += wx * Y[b];
+      for (int k = 0; k < 5; ++k) gx[k] = dx[k] = gy[k] = dy[k] = 0.0f;
     }
 #pragma unroll
-    for (int a = 0; a < 5; ++a) {
+    for (int k = 0; k < 4; ++k) wy[k] = (k ? wy[k - 1] : 0.0f) - qc * dy[k];
+    float acc[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    auto part = [&](auto h) {
+      constexpr int H = decltype(h)::value;
+      if ((has & (0x000F000F000F000FULL << (YH * H))) == 0ULL) return;
+      __builtin_amdgcn_wave_barrier();               // the last ones were read
+      if (sub / YH == H) {
+        float *y = Y + (sub % YH) * YN;
 #pragma unroll
-      for (int b = 0; b < 4; ++b) acc[20 + a * 4 + b] += X[a] * wy[b];
-      const float za = qv * X[a], zb = (qv * twelfth) * dX[a];
+        for (int k = 0; k < 5; ++k) {
+          y[k] = gy[k];
+          y[9 + k] = dy[k];
+        }
 #pragma unroll
-      for (int b = 0; b < 5; ++b) acc[40 + a * 5 + b] += za * Y[b] + zb * dY[b];
-    }
+        for (int k = 0; k < 4; ++k) y[5 + k] = wy[k];
+        y[14] = qv;
+        y[15] = qv * (1.0f / 12.0f);
+        y[16] = -qc;
+      }
+      __builtin_amdgcn_wave_barrier();
+      outer_part<H>(acc, gx, dx, Y, r, jy, has);
+    };
+    part(std::integral_constant<int, 0>{});
+    part(std::integral_constant<int, 1>{});
+    part(std::integral_constant<int, 2>{});
+    part(std::integral_constant<int, 3>{});
+#pragma unroll
+    for (int a = 0; a < 5; ++a) sum[a] += (double)acc[a];
   }
 }
 
@@ -669,9 +725,9 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
   L.xcnt = 0;
   L.ok = true;
   L.lost = false;
-  float core[NCORE];
+  float core[24];
 #pragma unroll
-  for (int k = 0; k < NCORE; ++k) core[k] = 0.0f;
+  for (int k = 0; k < 24; ++k) core[k] = 0.0f;
   if (g < ncell) {
     // the next species' windows load while this one is pushed
     if (PAIR) {
@@ -693,11 +749,13 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
       push_species<false>(L, core, win, sc, sn, P, A, X);
       if (sub == 0) gsb[(P.nsp - 1) * CHUNK + g] = L.xcnt;
     }
-    // stay-in-cell stencils of every species, summed over the group once
+  }
+  // stay-in-cell stencils of every species, summed over the group once
+  {
+    const int s0 = group_sums(core, sub);
+    if ((sub & 1) == 0) {
 #pragma unroll
-    for (int c = 0; c < NCORE; ++c) {
-      const float v = row_sum16(core[c]);
-      if (sub == 0) ccore[g * CCS + c] = v;
+      for (int e = 0; e < 3; ++e) ccore[g * 24 + s0 + e] = core[e];
     }
   }
   if (!L.ok) atomicOr(derr, DERR_JUMP);
@@ -706,10 +764,7 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
   __syncthreads();                                   // the lists, and the movers' new state in
                                                      // their slots
   // the workgroup's records in the row's pool (one atomic), while every
-  // cell's group deposits the cell's movers: lane sub takes movers j = sub,
-  // sub + MQ, ... (a dense cell of the nonlinear phase loses a hundred
-  // particles a step), and the group sums its lanes in a fixed order
-  static_assert(CHUNK * MQ == NT && MQ == GROUP, "the movers' deposit runs on every cell group");
+  // cell's group deposits the cell's movers
   if (threadIdx.x == 0) {
     int tot = 0;
     for (int c = 0; c < CHUNK; ++c) tot += gcnt[c];
@@ -721,18 +776,9 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
     rfirst = f;
     atomicMax(stats + 2, tot);
   }
-  {
-    float acc[NACC];
-#pragma unroll
-    for (int e = 0; e < NACC; ++e) acc[e] = 0.0f;
-    mover_part(acc, sub, g < ncell ? gcnt[g] : 0, g, X);
-    const bool lead = sub == 0 && g < ncell;
-#pragma unroll
-    for (int e = 0; e < NACC; ++e) {
-      const float v = row_sum16(acc[e]);
-      if (lead) cmov[g * CMS + e] = v;
-    }
-  }
+  double mv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  const wm_mover::Role role = wm_mover::role_of(sub);
+  mover_sums(mv, sub, g < ncell ? gcnt[g] : 0, g, (float *)CF4 + g * CFS, role, X);
   __syncthreads();
   const int rf = rfirst;
   double *csum = (double *)xpl;                      // the list offsets are read by now
@@ -755,7 +801,9 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
                           __int_as_float((int)(uint32_t)id), __int_as_float((int)(id >> 32)));
     }
     // the cell's sums in FP64 for the tile assembly
-    for (int e = sub; e < NACC; e += GROUP) csum[g * NACC + e] = cell_sum(g, e);
+    wm_mover::put_sums(csum + g * NACC, role, mv);
+    __builtin_amdgcn_wave_barrier();
+    for (int e = sub; e < NCORE; e += GROUP) csum[g * NACC + core_at(e)] += (double)ccore[g * 24 + e];
     // per bin: movers in total and per direction
     for (int s = 0; s < P.nsp; ++s) {
       const int j0 = s ? gsb[(s - 1) * CHUNK + g] : 0;
