@@ -697,6 +697,11 @@ int wm_alloc_device(wm_ctx *ctx) {
   WM_TRY(dmalloc(ctx, &ctx->cg_p[0], 3 * n));
   WM_TRY(dmalloc(ctx, &ctx->cg_p[1], 3 * n));
   WM_TRY(dmalloc(ctx, &ctx->cg_s, 4));
+  WM_TRY(dmalloc(ctx, &ctx->ts, 8));
+  WM_HIP(hipMemsetAsync(ctx->ts, 0, 8 * sizeof(*ctx->ts), ctx->stream));
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device) == hipSuccess && khz > 0)
+    ctx->clock_khz = khz;
   WM_TRY(dmalloc(ctx, &ctx->red, wm_cg_partials(g.nx, g.ny)));
   WM_TRY(dmalloc(ctx, &ctx->red_cnt, 8));
   ctx->dep_part_elems = ctx->form == WM_FORM_FP32 ? wm_deposit_part_elems32(g.nx, g.ny)
@@ -770,13 +775,15 @@ int wm_create(wm_ctx **out, int device) {
   }
   // small device-to-host read-backs (solver scalars, error flags) land in
   // pinned memory: a copy to pageable memory is staged by the runtime
-  if (hipHostMalloc(&ctx->h_pin, WM_PIN_BYTES, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&ctx->h_pin, WM_PIN_BYTES, hipHostMallocCoherent) != hipSuccess) {
     (void)hipStreamDestroy(ctx->stream);
     (void)hipStreamDestroy(ctx->stream2);
     delete ctx;
     return WM_ERR_NODEV;
   }
+  memset(ctx->h_pin, 0, WM_PIN_BYTES);
   for (int k = 0; k < 32; ++k) (void)hipEventCreate(&ctx->ev[k]);
+  for (hipEvent_t &e : ctx->join) (void)hipEventCreateWithFlags(&e, hipEventDisableTiming);
   *out = ctx;
   return WM_OK;
 }
@@ -803,11 +810,12 @@ int wm_destroy(wm_ctx *ctx) {
                   ctx->spill_l, ctx->spill_p, ctx->spill_q, ctx->sfill, ctx->perm, ctx->code,
                   ctx->kind, ctx->farcnt, ctx->far, ctx->lup, ctx->ldn, ctx->disp, ctx->dstart,
                   ctx->cumnew, ctx->nold, ctx->rowok, ctx->uf2, ctx->tile_sums,
-                  ctx->tile_edges, ctx->tile_abort, ctx->tile_out};
+                  ctx->tile_edges, ctx->tile_abort, ctx->tile_out, ctx->ts};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   wm_pc_free(ctx);
   for (int k = 0; k < 32; ++k) (void)hipEventDestroy(ctx->ev[k]);
+  for (hipEvent_t e : ctx->join) (void)hipEventDestroy(e);
   (void)hipStreamDestroy(ctx->stream);
   (void)hipStreamDestroy(ctx->stream2);
   wm_xfer_free(ctx);
@@ -1333,63 +1341,55 @@ int wm_step(wm_ctx *ctx, int nsteps) {
   }
   WM_TRY(wm_alloc_device(ctx));
   double acc[WM_NPHASE] = {0};
+  const bool f32 = ctx->form == WM_FORM_FP32;
   for (int it = 0; it < nsteps; ++it) {
-    hipEvent_t *e = ctx->ev;
     StepScope scope{ctx, false};
-    WM_HIP(hipEventRecord(e[0], ctx->stream));
     // particle__solv + ele_cur (proj/weibel/app.f90:102, field.f90:121)
-    const bool f32 = ctx->form == WM_FORM_FP32;
     WM_TRY(f32 ? wm_k_cell_fields32(ctx) : wm_k_cell_fields(ctx));
-    WM_HIP(hipEventRecord(e[1], ctx->stream));
-    if (f32) {
-      // Cell bins: the push wraps x itself, and moves the last push's movers
-      // into their bins before it pushes (the particle boundaries and the
-      // sort of app.f90:104-106 reduce to that).  Beside the solve, on the
-      // second stream, the fill check lists the blocks of cells whose bins
-      // would overflow with this push's movers and they are laid out anew.
-      WM_TRY(wm_k_push_deposit32(ctx));
-      WM_HIP(hipEventRecord(e[2], ctx->stream));
-      WM_HIP(hipStreamWaitEvent(ctx->stream2, e[2], 0));
+    WM_TRY(f32 ? wm_k_push_deposit32(ctx) : wm_k_push_step(ctx));
+    WM_HIP(hipEventRecord(ctx->join[0], ctx->stream));
+    // On the second stream, beside the current and the field solve, which read
+    // only the deposit and the fields (the next step waits for both):
+    // FP64: the row order (particle_y and the sort, app.f90:105-106), from what
+    // the push left.
+    // FP32: cell bins.  The push wraps x itself, and moves the last push's
+    // movers into their bins before it pushes (the particle boundaries and the
+    // sort of app.f90:104-106 reduce to that).  The fill check lists the blocks
+    // of cells whose bins would overflow with this push's movers and they are
+    // laid out anew.
+    const auto second = [&]() -> int {
+      WM_HIP(hipStreamWaitEvent(ctx->stream2, ctx->join[0], 0));
       StreamSwap on2(ctx, ctx->stream2);
-      WM_HIP(hipEventRecord(e[5], ctx->stream));
-      WM_TRY(wm_k_fill_check(ctx));
-      WM_HIP(hipEventRecord(e[6], ctx->stream));
-      WM_TRY(wm_relayout(ctx));
-      WM_HIP(hipEventRecord(e[7], ctx->stream));
-    } else {
-      // The row order (particle_y and the sort, app.f90:105-106) reads only
-      // what the push left, and the field solve (app.f90:103) only the
-      // current and the fields: they run concurrently, the order on the
-      // second stream, and the next step waits for both.
-      WM_TRY(wm_k_push_step(ctx));
-      WM_HIP(hipEventRecord(e[2], ctx->stream));
-      WM_HIP(hipStreamWaitEvent(ctx->stream2, e[2], 0));
-      StreamSwap on2(ctx, ctx->stream2);
-      WM_HIP(hipEventRecord(e[5], ctx->stream));
-      WM_TRY(wm_k_order(ctx, e[6]));
-      WM_HIP(hipEventRecord(e[7], ctx->stream));
-    }
+      if (f32) {
+        WM_TRY(wm_k_fill_check(ctx));
+        WM_TRY(wm_relayout(ctx));
+      } else {
+        WM_TRY(wm_k_order(ctx));
+      }
+      WM_HIP(hipEventRecord(ctx->join[1], ctx->stream));
+      return WM_OK;
+    };
+    // whichever the host can enqueue without waiting comes first: the solve's
+    // few kernels are a small step's longest chain, a streaming solve is watched
+    const bool enqueues = wm_field_enqueues(ctx);
+    if (!enqueues) WM_TRY(second());
     WM_TRY(wm_k_current(ctx, f32 ? WM_CHUNK_STEP32 : WM_CHUNK_STEP64));   // field.f90:121-122
-    WM_HIP(hipEventRecord(e[3], ctx->stream));
     WM_TRY(wm_field_launch(ctx));                 // field.f90:125-184
-    WM_HIP(hipEventRecord(e[4], ctx->stream));
-    WM_HIP(hipStreamWaitEvent(ctx->stream, e[7], 0));
+    if (enqueues) WM_TRY(second());
+    WM_HIP(hipStreamWaitEvent(ctx->stream, ctx->join[1], 0));
     WM_TRY(wm_field_update(ctx));                 // and the step's report
-    WM_HIP(hipEventRecord(e[8], ctx->stream));
-    WM_HIP(hipEventSynchronize(e[8]));
+    if (it + 1 == nsteps) WM_HIP(hipStreamSynchronize(ctx->stream));
+    WM_TRY(wm_report_wait(ctx));
     scope.ended = true;
-    // phases: [0..3] on the first stream (e0..e4), [4] particle boundaries
-    // (e5..e6) and [5] the places (e6..e7) on the second (FP64; in the FP32 form
-    // the push holds them, and [4] is the fill check, [5] the re-layout)
+    // phases: [0..3] on the first stream, [4] particle boundaries and [5] the
+    // places on the second (FP64; in the FP32 form the push holds them, and [4]
+    // is the fill check, [5] the re-layout)
+    const SolveReport r = *(const SolveReport *)((const char *)ctx->h_pin + WM_PIN_REPORT);
     const int from[WM_NPHASE] = {0, 1, 2, 3, 5, 6}, to[WM_NPHASE] = {1, 2, 3, 4, 6, 7};
-    for (int k = 0; k < WM_NPHASE; ++k) {
-      float ms = 0.f;
-      WM_HIP(hipEventElapsedTime(&ms, e[from[k]], e[to[k]]));
-      acc[k] += ms;
-    }
+    for (int k = 0; k < WM_NPHASE; ++k)
+      acc[k] += (double)std::max(0LL, (long long)(r.ts[to[k]] - r.ts[from[k]])) / ctx->clock_khz;
     WM_TRY(wm_field_result(ctx));
-    const int bits = ((const SolveReport *)((const char *)ctx->h_pin + WM_PIN_REPORT))->derr;
-    if (bits) WM_TRY(wm_check_derr(ctx, "step"));
+    if (r.derr) WM_TRY(wm_check_derr(ctx, "step"));
   }
   for (int k = 0; k < WM_NPHASE; ++k) ctx->phase_ms[k] = acc[k];
   return WM_OK;

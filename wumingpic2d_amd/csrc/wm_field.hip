@@ -154,8 +154,11 @@ __global__ void k_phi_walls(int nx, int ny, double *phi, int l) {
 
 // ----------------------------------------------------------- RHS, dE, +=
 // gkl (field.f90:125-146), interior cells, gkl planes nx x ny.
+__global__ void k_stamp(unsigned long long *ts, int k) { wm_stamp(ts, k); }
 __global__ void k_rhs(FieldGeom fg, FC f, XSide X, const double *__restrict__ uf,
-                      const double *__restrict__ uj, double *__restrict__ gkl) {
+                      const double *__restrict__ uj, double *__restrict__ gkl,
+                      unsigned long long *ts) {
+  wm_stamp(ts, 3);
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= fg.nx * fg.ny) return;
   const int ii = t % fg.nx, jj = t / fg.nx;
@@ -805,7 +808,8 @@ static CgArgs cg_args(const wm_ctx *ctx) {
 
 static int rhs(wm_ctx *ctx) {
   hipLaunchKernelGGL(k_rhs, dim3(wm_cdiv((long long)ctx->g.nx * ctx->g.ny, 256)), dim3(256), 0,
-                     ctx->stream, ctx->fg, make_fc(ctx->g), wm_xside(ctx), ctx->uf, ctx->uj, ctx->gkl);
+                     ctx->stream, ctx->fg, make_fc(ctx->g), wm_xside(ctx), ctx->uf, ctx->uj, ctx->gkl,
+                     ctx->ts);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }
@@ -895,8 +899,15 @@ int wm_field_launch(wm_ctx *ctx) {
   for (int l = 0; l < 3; ++l) ctx->fcg_it[l] = 0;
   if (fcg || !tiles) WM_TRY(rhs(ctx));
   if (fcg) WM_TRY(fcg_solve(ctx, cg_args(ctx), ctx->fcg_it));
-  return tiles ? wm_k_tiles(ctx) : stream_plain(ctx);
+  if (tiles) return wm_k_tiles(ctx, !fcg);
+  WM_TRY(stream_plain(ctx));
+  hipLaunchKernelGGL(k_stamp, dim3(1), dim3(1), 0, ctx->stream, ctx->ts, 4);
+  WM_HIP(hipGetLastError());
+  return WM_OK;
 }
+
+// Does wm_field_launch only enqueue (no looking at the residual meanwhile)?
+bool wm_field_enqueues(wm_ctx *ctx) { return wm_tiles_fit(ctx, true) && !flexible(ctx); }
 
 int wm_field_update(wm_ctx *ctx) {
   if (!wm_fused_update(ctx)) {
@@ -955,7 +966,9 @@ namespace {
 template <int CHUNK>
 __global__ __launch_bounds__(256) void k_current(FieldGeom fg, int nchunk, int wall,
                                                  const double *__restrict__ part,
-                                                 double *__restrict__ uj, int *__restrict__ rowpend) {
+                                                 double *__restrict__ uj, int *__restrict__ rowpend,
+                                                 unsigned long long *ts) {
+  wm_stamp(ts, 2);
   constexpr int DW = CHUNK + 4, TILE = 5 * DW * 3;
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (rowpend && t < fg.ny) rowpend[t] = 1;
@@ -1033,7 +1046,7 @@ int wm_k_current(wm_ctx *ctx, int chunk) {
                                            : k_current<WM_CHUNK_HOST64>;
   hipLaunchKernelGGL(kernel, dim3(wm_cdiv(n, 256)), dim3(256), 0, ctx->stream, fg,
                      wm_cdiv(fg.nx, chunk), ctx->bcf != WM_BC_PERIODIC, ctx->dep_part, ctx->uj,
-                     f32 ? ctx->rowpend : nullptr);
+                     f32 ? ctx->rowpend : nullptr, ctx->ts);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }

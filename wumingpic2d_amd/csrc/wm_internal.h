@@ -135,6 +135,11 @@ using PBank = Rec64;
 
 struct wm_pc;   // learned preconditioner (wm_pc.hip)
 
+// The first thread of a launch leaves the device clock at ts[k].
+__device__ inline void wm_stamp(unsigned long long *ts, int k) {
+  if ((blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) == 0) ts[k] = wall_clock64();
+}
+
 struct wm_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -219,6 +224,13 @@ struct wm_ctx {
 
   // timing (per-phase HIP events of the last wm_step call)
   hipEvent_t ev[32]{};
+  hipEvent_t join[2]{};    // between the streams of a step: the push done, the second stream's end
+  // a step's kernels leave the device clock here as they start (wm_stamp): cell
+  // fields, push, current, solve, solve's end; on the second stream row order
+  // (fill check), places (re-layout), its end
+  unsigned long long *ts = nullptr;
+  unsigned seq = 0;        // reports asked for
+  int clock_khz = 100000;
   bool ev_ready = false;
   int last_iters[3] = {0, 0, 0};
   int fcg_it[3] = {0, 0, 0};     // flexible-CG iterations of the solve under way
@@ -328,13 +340,15 @@ int wm_k_current(wm_ctx *ctx, int chunk);   // deposit tiles (of chunk cells) su
 // the step's report; after the stream has been waited for it takes the result.
 // All three in one, waiting: wm_k_field_solve.
 int wm_field_launch(wm_ctx *ctx);
+bool wm_field_enqueues(wm_ctx *ctx);
 int wm_field_update(wm_ctx *ctx);
 int wm_field_result(wm_ctx *ctx);
 void wm_field_release(wm_ctx *ctx);  // after an error: waits for the solve in flight
 int wm_k_field_solve(wm_ctx *ctx);
 // wm_solve.hip: the on-chip solve and, for the periodic box, its update
-bool wm_tiles_fit(wm_ctx *ctx);
-int wm_k_tiles(wm_ctx *ctx);
+bool wm_tiles_fit(wm_ctx *ctx, bool peek = false);
+int wm_k_tiles(wm_ctx *ctx, bool begins);
+int wm_report_wait(wm_ctx *ctx);
 bool wm_fused_update(const wm_ctx *ctx);
 int wm_k_update_report(wm_ctx *ctx);  // periodic; else the report alone
 int wm_tiles_result(wm_ctx *ctx, bool *gave_up, int *err, int *ite);
@@ -345,7 +359,7 @@ int wm_k_particle_x(wm_ctx *ctx, int bank);
 int wm_k_particle_y(wm_ctx *ctx, int bank);
 // The resident step's particle_y and sort, as the order of the rows in
 // bank 0; mid is recorded before the last kernel (wm_order.hip)
-int wm_k_order(wm_ctx *ctx, hipEvent_t mid);
+int wm_k_order(wm_ctx *ctx);
 int wm_order_apply(wm_ctx *ctx);   // bank 0 in that order, if one is pending
 int wm_k_injection(wm_ctx *ctx, int bank, double u0);   // boundary_shock__injection
 double wm_injection_xend(const wm_ctx *ctx, double u0);

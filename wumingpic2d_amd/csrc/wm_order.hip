@@ -84,7 +84,8 @@ __global__ __launch_bounds__(RT) void k_order_rows(OP P, const int *__restrict__
                                                    uint2 *__restrict__ lup, uint2 *__restrict__ ldn,
                                                    int *__restrict__ hole, int *__restrict__ nhole,
                                                    int *__restrict__ nup, int *__restrict__ ndn,
-                                                   int *derr) {
+                                                   int *derr, unsigned long long *ts) {
+  wm_stamp(ts, 5);
   __shared__ int su[RW], sd[RW];
   const int seg = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int n = np2[seg];
@@ -398,7 +399,9 @@ constexpr int PCELL = PT / PG;   // cells of a workgroup
 constexpr int PWIN = 4;          // windows of a cell in flight
 constexpr int PD = 64;           // displaced particles of a cell ranked from LDS at a time
 constexpr int PWT = 32;          // windows of a cell in the tables and bitmaps
-__global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr) {
+__global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr,
+                                                     unsigned long long *ts) {
+  wm_stamp(ts, 6);
   __shared__ __attribute__((aligned(16))) int slots[PCELL][PD];
   __shared__ unsigned tab[3][PCELL][PWT];            // stay, right, left: count << 16 | lanes
   __shared__ unsigned bits[3][PCELL][PWT / 2];       // displaced of o, r, l by slot - ks
@@ -618,6 +621,10 @@ __global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr)
     }
   }
   if (bad) atomicOr(derr, DERR_RANGE);
+  // the end: of a row's last workgroup, every 16th row's and the last's
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 &&
+      ((blockIdx.y & 15) == 15 || blockIdx.y == gridDim.y - 1))
+    atomicMax(ts + 7, (unsigned long long)wall_clock64());
 }
 
 // The rows in their order: slot k of the result is what the index gives it.
@@ -634,8 +641,8 @@ __global__ __launch_bounds__(256) void k_order_apply(int cap, int ny, const int 
 
 // particle_y and the sort of the pushed rows (bank 0, in the slots the push
 // read them from): the order of the rows into ctx->perm, the IDs, cumcnt and
-// np2 moved on.  mid is recorded before the last kernel.
-int wm_k_order(wm_ctx *ctx, hipEvent_t mid) {
+// np2 moved on.
+int wm_k_order(wm_ctx *ctx) {
   const wm_grid &g = ctx->g;
   const OP P{g.nx, g.ny, ctx->cap, ctx->mcap, ctx->bcf == WM_BC_PERIODIC};
   const int nseg = g.nsp * g.ny;
@@ -645,16 +652,16 @@ int wm_k_order(wm_ctx *ctx, hipEvent_t mid) {
     return WM_ERR_ARG;
   }
   hipLaunchKernelGGL(k_order_rows, dim3(nseg), dim3(RT), 0, ctx->stream, P, ctx->np2, ctx->code,
-                     ctx->lup, ctx->ldn, ctx->hole, ctx->nhole, ctx->nup, ctx->ndn, ctx->derr);
+                     ctx->lup, ctx->ldn, ctx->hole, ctx->nhole, ctx->nup, ctx->ndn, ctx->derr,
+                     ctx->ts);
   hipLaunchKernelGGL(k_order_merge, dim3(nseg), dim3(RT), lds, ctx->stream, P, ctx->np2, ctx->nold,
                      ctx->code, ctx->kind, ctx->farcnt, ctx->far, ctx->lup, ctx->ldn, ctx->hole,
                      ctx->nhole, ctx->nup, ctx->ndn, ctx->cumnew, ctx->disp, ctx->dstart,
                      ctx->rowok, ctx->derr);
-  if (mid) WM_HIP(hipEventRecord(mid, ctx->stream));
   const Place R{ctx->nold, ctx->rowok, ctx->cumcnt, ctx->cumnew, ctx->far, ctx->dstart, ctx->code,
                 ctx->kind, ctx->disp, ctx->perm, ctx->id[ctx->idcur], ctx->id[1 - ctx->idcur]};
   hipLaunchKernelGGL(k_order_place, dim3(wm_cdiv(g.nx, PCELL), nseg), dim3(PT), 0, ctx->stream, P,
-                     R, ctx->derr);
+                     R, ctx->derr, ctx->ts);
   WM_HIP(hipGetLastError());
   ctx->idcur = 1 - ctx->idcur;
   std::swap(ctx->cumcnt, ctx->cumnew);

@@ -1086,7 +1086,9 @@ __global__ __launch_bounds__(PTH, 2) void k_push_step(PP P, const int *__restric
 // Also clears the rows' far marks for the push that follows.
 __global__ void k_cell_fields(FieldGeom fg, const double *__restrict__ uf,
                               double *__restrict__ tmp, int TX, int TY, size_t tps,
-                              int *__restrict__ far, int nseg) {
+                              int *__restrict__ far, int nseg, unsigned long long *ts) {
+  wm_stamp(ts, 0);
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) ts[1] = wall_clock64();
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < nseg) far[t] = 0;
   if (t >= TX * TY) return;
@@ -1159,7 +1161,7 @@ int wm_k_cell_fields(wm_ctx *ctx) {
   const int nseg = ctx->g.nsp * ctx->g.ny;
   hipLaunchKernelGGL(k_cell_fields, dim3(wm_cdiv(std::max((long long)TX * TY, (long long)nseg), 256)),
                      dim3(256), 0, ctx->stream, ctx->fg, ctx->uf, ctx->tmp, TX, TY, tps, ctx->far,
-                     nseg);
+                     nseg, ctx->ts);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }

@@ -862,7 +862,10 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
 // follows.
 __global__ void k_cell_fields32(FieldGeom fg, const double *__restrict__ uf,
                                 float *__restrict__ tmp, int TX, int TY, size_t tps,
-                                int *__restrict__ mfill, int *__restrict__ sfill, int ny) {
+                                int *__restrict__ mfill, int *__restrict__ sfill, int ny,
+                                unsigned long long *ts) {
+  wm_stamp(ts, 0);
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) ts[1] = wall_clock64();
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < ny) {
     mfill[t] = 0;
@@ -946,7 +949,7 @@ int wm_k_cell_fields32(wm_ctx *ctx) {
   const int out = ctx->mv_pending ? 1 - ctx->mv_last : ctx->mv_last;
   hipLaunchKernelGGL(k_cell_fields32, dim3(wm_cdiv((long long)std::max(TX * TY, ctx->g.ny), 256)),
                      dim3(256), 0, ctx->stream, ctx->fg, ctx->uf, ctx->tmp32, TX, TY, tps,
-                     ctx->mfill[out], ctx->sfill, ctx->g.ny);
+                     ctx->mfill[out], ctx->sfill, ctx->g.ny, ctx->ts);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }

@@ -32,7 +32,20 @@ struct SolveReport {
   SolveOut out;
   int abort_;            // the on-chip solve gave up
   int derr;              // device error bits
+  unsigned long long ts[8];   // wm_ctx::ts
+  unsigned seq;          // written last: which report this is
 };
+// One thread leaves the report (abort_ null: the solve streamed).
+__device__ inline void leave_report(SolveReport *host, const SolveOut &out, int given,
+                                    const int *derr, const unsigned long long *ts, unsigned seq) {
+  host->out = out;
+  host->abort_ = given;
+  host->derr = *derr;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) host->ts[k] = ts[k];
+  __threadfence_system();
+  __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // The field update's kernels skip when the on-chip solve before them gave up
 // or failed (null: after a streaming solve).
 struct SolveGate {

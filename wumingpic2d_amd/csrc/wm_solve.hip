@@ -35,6 +35,7 @@
 // Bound by the exchanges: about 4 us an iteration at 256 x 64 (40 us a solve of
 // 7), of which the sweeps are 1.6; at 1024 x 1024 by the sweeps of 16 rows a
 // lane, one component after another (163 us).
+#include <chrono>
 #include <condition_variable>
 #include <mutex>
 
@@ -138,6 +139,8 @@ struct SArgs {
   unsigned tag0;
   int *abort_;
   SolveOut *out;
+  unsigned long long *ts;
+  bool stamp;                     // the solve begins here
 };
 
 // f5 gkl of component l at interior cell (ii, jj): field.f90:125-146.
@@ -180,6 +183,7 @@ __device__ inline double phi_at(const SArgs &A, int l, int a, int b, int wx) {
 __global__ __launch_bounds__(256) void k_tile_start(SArgs A) {
   const int t = blockIdx.x * 256 + threadIdx.x, l = blockIdx.y;
   const int nx = A.fg.nx, n = nx * A.fg.ny;
+  if (A.stamp) wm_stamp(A.ts, 3);
   if (t >= n) return;
   const int ii = t % nx, jj = t / nx;
   if (ii < A.X.xa || ii > A.X.xb) return;
@@ -395,6 +399,7 @@ __global__ __launch_bounds__(NTH) void k_cg_tiles(SArgs A) {
     if (me == 0 && tid == 0) {
       A.out->ite[l] = ite;
       A.out->err[l] = err;
+      atomicMax(A.ts + 4, (unsigned long long)wall_clock64());
     }
     __syncthreads();                                   // P is filled again
   }
@@ -414,15 +419,12 @@ __global__ __launch_bounds__(256) void k_field_update(FieldGeom fg, SolveConst f
                                                       const double *__restrict__ df,
                                                       double *__restrict__ un, const int *abort_,
                                                       const SolveOut *out, const int *derr,
+                                                      const unsigned long long *ts, unsigned seq,
                                                       SolveReport *host) {
   const int t = blockIdx.x * 256 + threadIdx.x;
   const int given = abort_ ? *abort_ : 0;
   const SolveOut o = abort_ ? *out : SolveOut{};
-  if (t == 0) {
-    host->out = o;
-    host->abort_ = given;
-    host->derr = *derr;
-  }
+  if (t == 0) leave_report(host, o, given, derr, ts, seq);
   if (given || o.err[0] || o.err[1] || o.err[2] || t >= fg.gx * fg.gy) return;
   const int li = t % fg.gx, lj = t / fg.gx;
   const int ci = wrapm(li - 2, fg.nx);
@@ -527,14 +529,8 @@ void launch_tiles(const Plan &p, const SArgs &A, hipStream_t st) {
 namespace {
 // One thread: the step's status for the host, where no update kernel leaves it.
 __global__ void k_report(const int *abort_, const SolveOut *out, const int *derr,
-                         SolveReport *host) {
-  SolveReport r{};
-  if (abort_) {
-    r.out = *out;
-    r.abort_ = *abort_;
-  }
-  r.derr = *derr;
-  *host = r;
+                         const unsigned long long *ts, unsigned seq, SolveReport *host) {
+  leave_report(host, abort_ ? *out : SolveOut{}, abort_ ? *abort_ : 0, derr, ts, seq);
 }
 
 SolveReport *report_of(wm_ctx *ctx) { return (SolveReport *)((char *)ctx->h_pin + WM_PIN_REPORT); }
@@ -558,7 +554,7 @@ void release(wm_ctx *ctx) {
 
 // Plain CG on a grid whose tiles run side by side; the recording of
 // preconditioner pairs needs the iterates, so it streams.
-bool wm_tiles_fit(wm_ctx *ctx) {
+bool wm_tiles_fit(wm_ctx *ctx, bool peek) {
   if (ctx->solver == WM_SOLVER_CG && ctx->bcf == WM_BC_PERIODIC && wm_pc_collecting(ctx))
     return false;
   if (ctx->device < 0 || ctx->device >= MAX_DEV) return false;
@@ -569,13 +565,13 @@ bool wm_tiles_fit(wm_ctx *ctx) {
     ctx->ncu = n;
   }
   if (ctx->tile_rest > 0) {
-    --ctx->tile_rest;
+    if (!peek) --ctx->tile_rest;
     return false;
   }
   return plan_of(ctx).R > 0;
 }
 
-int wm_k_tiles(wm_ctx *ctx) {
+int wm_k_tiles(wm_ctx *ctx, bool begins) {
   const Plan p = plan_of(ctx);
   const size_t n = (size_t)p.workgroups();
   if (n > ctx->tile_cap) {
@@ -616,6 +612,8 @@ int wm_k_tiles(wm_ctx *ctx) {
   ctx->tile_tag += need;
   A.abort_ = ctx->tile_abort;
   A.out = (SolveOut *)ctx->tile_out;
+  A.ts = ctx->ts;
+  A.stamp = begins;
   {
     Slots &s = slots[ctx->device];
     std::unique_lock<std::mutex> lk(s.m);
@@ -642,22 +640,42 @@ bool wm_fused_update(const wm_ctx *ctx) { return ctx->bcf == WM_BC_PERIODIC && c
 int wm_k_update_report(wm_ctx *ctx) {
   const FieldGeom &fg = ctx->fg;
   const int *abort_ = ctx->tile_held ? ctx->tile_abort : nullptr;
+  ++ctx->seq;
   if (wm_fused_update(ctx)) {
     if (!ctx->uf2) WM_HIP(hipMalloc((void **)&ctx->uf2, sizeof(double) * 6 * fg.ps));
     hipLaunchKernelGGL(k_field_update, dim3(wm_cdiv((long long)fg.gx * fg.gy, 256)), dim3(256), 0,
                        ctx->stream, fg, make_fc(ctx->g), ctx->uf, ctx->uj, ctx->df, ctx->uf2,
-                       abort_, (const SolveOut *)ctx->tile_out, ctx->derr, report_of(ctx));
+                       abort_, (const SolveOut *)ctx->tile_out, ctx->derr, ctx->ts, ctx->seq,
+                       report_of(ctx));
     std::swap(ctx->uf, ctx->uf2);
     ctx->tile_swapped = ctx->tile_held != 0;
   } else {
     hipLaunchKernelGGL(k_report, dim3(1), dim3(1), 0, ctx->stream, abort_,
-                       (const SolveOut *)ctx->tile_out, ctx->derr, report_of(ctx));
+                       (const SolveOut *)ctx->tile_out, ctx->derr, ctx->ts, ctx->seq, report_of(ctx));
   }
   WM_HIP(hipGetLastError());
   return WM_OK;
 }
 
-// After the stream has been waited for.
+// Waits for the last report asked for.  For a while by looking at it: a small
+// grid's step is over in a tenth of a millisecond, of which waiting for the
+// stream would take a tenth again.
+int wm_report_wait(wm_ctx *ctx) {
+  const SolveReport *r = report_of(ctx);
+  const auto there = [&] { return __atomic_load_n(&r->seq, __ATOMIC_ACQUIRE) == ctx->seq; };
+  const auto t0 = std::chrono::steady_clock::now();
+  while (!there()) {
+    for (int k = 0; k < 64 && !there(); ++k) __builtin_ia32_pause();
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) break;
+  }
+  if (there()) return WM_OK;
+  WM_HIP(hipStreamSynchronize(ctx->stream));
+  if (there()) return WM_OK;
+  wm_set_error(ctx, WM_ERR_HIP, "the step's report did not arrive");
+  return WM_ERR_HIP;
+}
+
+// After the report has been waited for.
 int wm_tiles_result(wm_ctx *ctx, bool *gave_up, int *err, int *ite) {
   release(ctx);
   const SolveReport r = *report_of(ctx);

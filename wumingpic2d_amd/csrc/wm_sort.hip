@@ -321,7 +321,9 @@ struct Relay {
 __global__ __launch_bounds__(256) void k_fill_check(Mig G, int *__restrict__ pc, Relay R,
                                                     const int *__restrict__ mfill,
                                                     const int *__restrict__ sfill,
-                                                    int *__restrict__ stats, int *derr) {
+                                                    int *__restrict__ stats, int *derr,
+                                                    unsigned long long *ts) {
+  wm_stamp(ts, 5);
   const size_t d = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   int cnew = 0, mout = 0;
   bool over = false;
@@ -456,7 +458,9 @@ constexpr int RW = 256;   // threads of a re-layout workgroup
 __global__ __launch_bounds__(RW) void k_relayout_blocks(SB P, Relay R, const int *__restrict__ cnt,
                                                         const int *__restrict__ pc,
                                                         int *__restrict__ bstart, Bins32 A,
-                                                        int64_t *__restrict__ ids) {
+                                                        int64_t *__restrict__ ids,
+                                                        unsigned long long *ts) {
+  wm_stamp(ts, 6);
   __shared__ int s_old[WM_RB], s_new[WM_RB], s_pre[WM_RB + 1];
   __shared__ int s_go;
   const int nblk = (P.nx + WM_RB - 1) / WM_RB;
@@ -629,8 +633,9 @@ __global__ __launch_bounds__(RS) void k_relayout_segs(SB P, Relay R, const int *
 }
 
 // Step 3: the lists' totals into the statistics, the lists emptied.
-__global__ void k_relayout_done(Relay R, int *__restrict__ stats) {
+__global__ void k_relayout_done(Relay R, int *__restrict__ stats, unsigned long long *ts) {
   if (threadIdx.x == 0) {
+    ts[7] = wall_clock64();
     stats[6] += R.ctl[0];
     stats[7] += R.ctl[1];
     R.ctl[0] = 0;
@@ -802,7 +807,7 @@ int wm_k_fill_check(wm_ctx *ctx) {
   const size_t nthr = std::max(G.nbin, (size_t)ctx->g.ny);
   hipLaunchKernelGGL(k_fill_check, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, ctx->stream,
                      G, ctx->pcnt, make_relay(ctx), ctx->mfill[ctx->mv_last], ctx->sfill,
-                     ctx->fstat, ctx->derr);
+                     ctx->fstat, ctx->derr, ctx->ts);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }
@@ -814,14 +819,14 @@ int wm_relayout(wm_ctx *ctx) {
   const SB P = make_sb(ctx);
   const Relay R = make_relay(ctx);
   hipLaunchKernelGGL(k_relayout_blocks, dim3(ctx->relay_nwb), dim3(RW), 0, ctx->stream, P, R,
-                     ctx->bin_cnt, ctx->pcnt, ctx->bstart, ctx->bins, ctx->id_bins);
+                     ctx->bin_cnt, ctx->pcnt, ctx->bstart, ctx->bins, ctx->id_bins, ctx->ts);
   const size_t lds = 2 * sizeof(int) * (P.nx + 1);
   if (lds > 49152)
     (void)hipFuncSetAttribute((const void *)k_relayout_segs,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   hipLaunchKernelGGL(k_relayout_segs, dim3(ctx->relay_nws), dim3(RS), lds, ctx->stream, P, R,
                      ctx->bin_cnt, ctx->pcnt, ctx->bstart, ctx->bins, ctx->id_bins, ctx->derr);
-  hipLaunchKernelGGL(k_relayout_done, dim3(1), dim3(64), 0, ctx->stream, R, ctx->fstat);
+  hipLaunchKernelGGL(k_relayout_done, dim3(1), dim3(64), 0, ctx->stream, R, ctx->fstat, ctx->ts);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }
