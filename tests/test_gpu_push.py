@@ -56,3 +56,34 @@ def test_walled_push_over_tile_edges(bc, nx, ny, ppc, vth):
     n = np.zeros_like(np2)
     ctx.state_download(np2=n)
     assert np.array_equal(n, np2)
+
+
+@pytest.mark.parametrize("nx,ny,ppc,vth,nsp,bc", [
+    (4099, 9, 30, 1.0, 1, None),            # lists filled over and over, three wraps of 8 cells
+    (193, 170, 1, 0.5, 3, None),            # odd and even cells of a row, empty ones
+    (250, 132, 3, 0.4, 2, BC_SHOCK), (259, 127, 2, 0.6, 2, BC_RECONNECTION),
+])
+def test_push_with_eight_lanes_a_cell(nx, ny, ppc, vth, nsp, bc):
+    """More than 32768 cells of at most 36 particles a species: eight lanes a
+    cell, two cells' movers in each row of sixteen."""
+    if bc is None:
+        p, up, np2, cc, uf = state(nx, ny, ppc, 83, vth=vth, nsp=nsp)
+        random_fields(uf, 83, amp=0.05)
+        ctx = make_ctx(p)
+        s = slice(2, -2)
+    else:
+        p, up, np2, cc, uf = wall_state(bc, nx, ny, ppc, 83, vth=vth, extra=6)
+        ctx = make_wall_ctx(p)
+        ctx.set_walls(p["nxs"], p["nxe"], p["u0"])
+        s = slice(p["nxs"] - p["nxgs"] + 2, p["nxe"] - p["nxgs"] + 3)
+    assert p["nx"] * ny > 32768
+    ctx.state_upload(up, np2, cc, uf)
+    orc = Oracle(p)
+    gp, guf = up.copy(order="F"), np.zeros_like(uf)
+    for _ in range(2):
+        orc.step(up, gp, uf, cc, np2)
+        ctx.step(1)
+        ctx.state_download(uf=guf)
+        assert np.abs(guf - uf)[:, s, 2:-2].max() <= 1e-12 * np.abs(uf[:, s]).max()
+    if bc is None:
+        _same(p, ctx, up, np2, cc)

@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <numeric>
 #include <vector>
 
 #include "wm_internal.h"
@@ -550,6 +551,7 @@ int wm_rows_done(wm_ctx *ctx, const int *np2_host) {
   }
   WM_HIP(hipStreamSynchronize(ctx->stream));
   WM_TRY(wm_check_derr(ctx, "state rows"));
+  ctx->npart = std::accumulate(np2_host, np2_host + nseg_of(ctx), 0LL);
   ctx->resident = true;
   return WM_OK;
 }
@@ -1260,6 +1262,7 @@ int wm_state_upload(wm_ctx *ctx, const double *up, const int *np2, const int *cu
   WM_TRY(upload_field(ctx, uf, 6, ctx->uf));
   WM_HIP(hipStreamSynchronize(ctx->stream));
   WM_TRY(wm_check_derr(ctx, "state upload"));
+  ctx->npart = std::accumulate(np2, np2 + nseg, 0LL);
   ctx->resident = true;
   return WM_OK;
 }
@@ -1306,6 +1309,7 @@ int wm_state_init_weibel(wm_ctx *ctx, uint64_t seed, int ppc, double vth, double
   }
   WM_TRY(fill_zero(ctx, ctx->uf, 6 * ctx->fg.ps));
   WM_TRY(wm_check_derr(ctx, "initial state"));
+  ctx->npart = (long long)ppc * ctx->g.nx * ctx->g.ny * ctx->g.nsp;
   ctx->resident = true;
   return WM_OK;
 }

@@ -190,6 +190,7 @@ struct wm_ctx {
   // perm[seg * cap + k] of its species' plane (row * cap + slot); np2, cumcnt
   // and the IDs are the ordered rows'.
   bool perm_valid = false;
+  long long npart = 0;           // particles of the resident state (their number stays)
   unsigned *perm = nullptr;      // [nseg*cap]
   uint16_t *code = nullptr;      // [nseg*cap] the push's code per particle (wm_order.h)
   int4 *kind = nullptr;          // [nseg*nx] moves out of a cell by kind

@@ -508,13 +508,14 @@ __global__ __launch_bounds__(256, 3) void k_particle(
 // over the particles: read through the pending order (Order::perm), written
 // sorted, 40 bytes each way, plus 4 bytes of index and 2 of code.
 //
-// A group of 16 lanes per cell, in steps of 16 consecutive particles.  Loads
-// run two steps ahead of their use and indexes four; a step's results wait in
-// registers and are stored in front of the next step's loads, since loads and
-// stores complete in order and whatever is waited for should have been issued
-// two steps ago.  A workgroup is two wavefronts of four cells each: with eight
-// wavefronts and 32 cells, more than half of the wavefronts' time went into
-// waiting for the densest cells of the workgroup at its end.
+// A group of 8 or 16 lanes per cell (wm_k_push_step), in steps of as many
+// consecutive particles.  Loads run two steps ahead of their use and indexes
+// four; a step's results wait in registers and are stored in front of the next
+// step's loads, since loads and stores complete in order and whatever is waited
+// for should have been issued two steps ago.  A workgroup is 8 cells, one
+// wavefront or two: with eight wavefronts and 32 cells, more than half of the
+// wavefronts' time went into waiting for the densest cells of the workgroup at
+// its end.
 //
 // Per cell, over all species: 21 stay-in-cell stencil values per lane (of the
 // 27 values of the 3 x 3 cores, Jx's last column and Jy's last row carry the
@@ -527,17 +528,15 @@ __global__ __launch_bounds__(256, 3) void k_particle(
 // the in-cell offsets: nine coefficients per field and cell (LDS), 8 FMAs a
 // field.
 //
-// Two wavefronts a SIMD (197 registers): bound by FP64 operations (half of the
+// Two wavefronts a SIMD (197 and 224 registers): bound by FP64 operations (half of the
 // issue slots) and the memory path together; alone, loads and stores take 0.92
 // ms and the arithmetic 0.91 at 1024 x 512 cells with 32 per cell, both 1.1.
-// Measured, 8 lanes of one wavefront and 32 cells, 16 and 8 cells: 2048 x 2048,
-// 64 per cell: 18.9 -> 15.6 ms; 256 x 64, 64 per cell, pinched: 224 -> 128 us;
-// 1024 x 512, 32 per cell: 1.68 -> 1.51 ms.
+// Measured against 8 lanes a cell, 32 cells and lists summed component by
+// component: 2048 x 2048, 64 per cell: 18.9 -> 15.6 ms; 256 x 64, 64 per cell,
+// pinched: 224 -> 128 us; 1024 x 512, 32 per cell: 1.68 -> 1.37 ms; 499 x 309, 21
+// per cell: 424 -> 325 us.
 constexpr int PCH = WM_CHUNK_STEP64;  // cells of a workgroup
-constexpr int PG = 16;                // lanes of a cell
-constexpr int PTH = PCH * PG;         // threads: two wavefronts
 constexpr int PTW = PCH + 2, PDW = PCH + 4, PTILE = 5 * PDW * 3;
-constexpr int MLC = 47;               // a cell's listed movers
 constexpr int CFN = 10;               // doubles per field and cell (9 coefficients, padded)
 constexpr int NCORE = 21;
 
@@ -686,13 +685,13 @@ __device__ inline double dpp_f64(double v) {
   return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
 }
 
-// Sums of 24 values over the 16 lanes of a group, by halving: in each of three
-// exchanges a lane keeps one half of the values and adds its partner's share
-// of them (partners: lane xor 8, the mirrored lane of its eight, lane xor 2);
-// the last, with lane xor 1, adds the three that are left.  Lane sub ends with
-// the sums of values slot .. slot + 2 in v[0..2], slot = 12 (sub >> 3) +
-// 6 (sub >> 2 & 1) + 3 (sub >> 1 & 1).  About 6 instructions a value against
-// 15 for a butterfly of each.
+// Sums of 24 values over the 8 or 16 lanes of a group, by halving: in each
+// exchange a lane keeps one half of the values and adds its partner's share of
+// them (partners: lane xor 8, the mirrored lane of its eight, lane xor 2, and
+// lane xor 1; of 16 lanes the last adds the three that are left).  Lane sub
+// ends with the sums of values slot .. slot + 2, which it returns, in v[0..2];
+// of 16 lanes the odd ones have what the even ones have.  About 6
+// instructions a value against 12 or 15 for a butterfly of each.
 template <int M, int CTRL>
 __device__ inline void halve(double *v, bool up) {
 #pragma unroll
@@ -702,12 +701,19 @@ __device__ inline void halve(double *v, bool up) {
     v[e] = keep + dpp_f64<CTRL>(give);
   }
 }
+template <int PG>
 __device__ inline int group_sums(double *v, int sub) {
+  if (PG == 8) {
+    halve<24, 0x141>(v, sub & 4);        // row_half_mirror: lane 7 - sub of its eight
+    halve<12, 0x4E>(v, sub & 2);         // quad_perm [2,3,0,1]
+    halve<6, 0xB1>(v, sub & 1);          // quad_perm [1,0,3,2]
+    return ((sub >> 2) & 1) * 12 + ((sub >> 1) & 1) * 6 + (sub & 1) * 3;
+  }
   halve<24, 0x128>(v, sub & 8);          // row_ror:8: lane xor 8
-  halve<12, 0x141>(v, sub & 4);          // row_half_mirror: lane 7 - sub of its eight
-  halve<6, 0x4E>(v, sub & 2);            // quad_perm [2,3,0,1]
+  halve<12, 0x141>(v, sub & 4);
+  halve<6, 0x4E>(v, sub & 2);
 #pragma unroll
-  for (int e = 0; e < 3; ++e) v[e] += dpp_f64<0xB1>(v[e]);   // quad_perm [1,0,3,2]
+  for (int e = 0; e < 3; ++e) v[e] += dpp_f64<0xB1>(v[e]);
   return ((sub >> 3) & 1) * 12 + ((sub >> 2) & 1) * 6 + ((sub >> 1) & 1) * 3;
 }
 
@@ -730,36 +736,42 @@ __device__ inline void add_outer(double (&acc)[5], const double (&gx)[5], const 
 #undef WM_ROW
 }
 
-// The listed movers' current, added to the lanes' sums.  Sixteen movers of a
-// cell at a time: lane sub prepares mover e0 + sub and keeps its x side, the y
-// sides go to LDS, and the cell's 16 lanes take the movers one after the
-// other.  No reduction: a lane's sums are its own.  All 64 lanes call it.
+// The listed movers' current, added to the lanes' sums (with 8 lanes a cell A
+// and B are those of the row's two cells; with 16 A).  PG movers of a cell at a
+// time: lane sub prepares its cell's mover e0 + sub and keeps its x side, the y
+// sides go to LDS (Y: the cell's; Ya, Yb: the row's first and second cell's),
+// and the row's 16 lanes take the movers of its cells one after the other.
+// No reduction: a lane's sums are its own.  All 64 lanes call it.
 // (One component after another over the list, a lane a mover, took three
 // passes over the shapes and 80 values through the lanes' reduction: 471
 // million vector instructions a step at 1024 x 512 against 339.)
-__device__ inline void outer_sums(double (&A)[5], const double (&gx)[5], const double (&dx)[5],
-                                  const double *Y, const Role &r, bool jy,
-                                  unsigned long long has) {
+template <int PG>
+__device__ inline void outer_sums(double (&A)[5], double (&B)[5], const double (&gx)[5],
+                                  const double (&dx)[5], const double *Ya, const double *Yb,
+                                  const Role &r, bool jy, unsigned long long has) {
   auto factors = [&](const double *y, double &V, double &W) {
     const double p = y[r.p < 0 ? 0 : r.p], s = y[r.s], w = y[r.w < 0 ? 0 : r.w], t = y[r.t];
     V = r.p < 0 ? 0.0 : (jy ? p : p * s);
     W = r.w < 0 ? 0.0 : w * t;
   };
-#define WM_PAIR(N0)                                     \
-  if (has & (0x0001000100010001ULL << (N0))) {          \
-    double V0, W0, V1, W1;                              \
-    factors(Y + (N0) * YN, V0, W0);                     \
-    factors(Y + ((N0) + 1) * YN, V1, W1);               \
-    add_outer<(N0)>(A, gx, dx, V0, W0);                 \
-    add_outer<(N0) + 1>(A, gx, dx, V1, W1);             \
+#define WM_PAIR(N0)                                                                 \
+  if (has & (0x0001000100010001ULL << (N0))) {                                      \
+    double V0, W0, V1, W1;                                                          \
+    const double *y = (PG == 8 && (N0) >= 8 ? Yb : Ya) + ((N0) & (PG - 1)) * YN;    \
+    factors(y, V0, W0);                                                             \
+    factors(y + YN, V1, W1);                                                        \
+    add_outer<(N0)>(PG == 8 && (N0) >= 8 ? B : A, gx, dx, V0, W0);                  \
+    add_outer<(N0) + 1>(PG == 8 && (N0) >= 8 ? B : A, gx, dx, V1, W1);              \
   }
   WM_PAIR(0) WM_PAIR(2) WM_PAIR(4) WM_PAIR(6)
   WM_PAIR(8) WM_PAIR(10) WM_PAIR(12) WM_PAIR(14)
 #undef WM_PAIR
 }
-__device__ inline void mover_sums(double (&A)[5], int sub, const double *L, const uint8_t *Ls,
-                                  double *Y, const Role &r, int nl, int i, int j, const PP &P,
-                                  const double *qcs) {
+template <int PG, int MLC>
+__device__ inline void mover_sums(double (&A)[5], double (&B)[5], int sub, const double *L,
+                                  const uint8_t *Ls, double *Y, const double *Ya,
+                                  const double *Yb, const Role &r, int nl, int i, int j,
+                                  const PP &P, const double *qcs) {
   const bool jy = r.out >= 20 && r.out < 40;
   for (int e0 = 0; __ballot(e0 < nl) != 0ULL; e0 += PG) {
     const int e = e0 + sub;
@@ -796,7 +808,7 @@ __device__ inline void mover_sums(double (&A)[5], int sub, const double *L, cons
     y[15] = qv * (1.0 / 12.0);
     y[16] = -qc;
     __builtin_amdgcn_wave_barrier();
-    outer_sums(A, gx, dx, Y, r, jy, has);
+    outer_sums<PG>(A, B, gx, dx, Ya, Yb, r, jy, has);
     __builtin_amdgcn_wave_barrier();
   }
 }
@@ -817,12 +829,14 @@ __device__ inline Part take(const Part &n) {
   return c;
 }
 
-template <int SRC, bool WALLS>
-__global__ __launch_bounds__(PTH, 2) void k_push_step(PP P, const int *__restrict__ cumcnt,
+template <int SRC, bool WALLS, int PG>
+__global__ __launch_bounds__(PCH * PG, 2) void k_push_step(PP P, const int *__restrict__ cumcnt,
                                                       const double *__restrict__ tmp, int TX,
                                                       size_t tps, Rec64 A, Rec64 B, Order O,
                                                       double *__restrict__ part,
                                                       int *__restrict__ derr) {
+  constexpr int PTH = PCH * PG;
+  constexpr int MLC = PG == 8 ? 23 : 47;       // a cell's listed movers
   __shared__ __attribute__((aligned(16))) double CF[PCH * 6 * CFN];
   // the movers' lists [x0 | y0 | x1 | y1 | q v_z][entry] per cell and their y
   // sides; before them, the chunk's cell-centred fields, behind them the
@@ -906,11 +920,12 @@ __global__ __launch_bounds__(PTH, 2) void k_push_step(PP P, const int *__restric
   const int wg = (threadIdx.x & 63) / PG;   // the group's place in its wavefront
   const Role role = role_of(threadIdx.x & 15);
   int bad = 0;
-  double core[24], mv[5];               // the cell's own sums, its movers'
+  double core[24], mv[5], mw[5];               // the cell's own sums, its movers' (8 lanes: the
+                                               // row's two cells' movers')
 #pragma unroll
   for (int e = 0; e < 24; ++e) core[e] = 0.0;
 #pragma unroll
-  for (int e = 0; e < 5; ++e) mv[e] = 0.0;
+  for (int e = 0; e < 5; ++e) mv[e] = mw[e] = 0.0;
   {
     // The step's results wait in registers and are stored at the top of the
     // next, in front of its loads: loads and stores complete in order, and
@@ -1007,7 +1022,7 @@ __global__ __launch_bounds__(PTH, 2) void k_push_step(PP P, const int *__restric
         }
         // a crossing particle goes to the cell's list in (step, lane) order,
         // ranked by a ballot over the group
-        const unsigned gb = (unsigned)(__ballot(cross) >> (PG * wg)) & 0xFFFFu;
+        const unsigned gb = (unsigned)(__ballot(cross) >> (PG * wg)) & ((1u << PG) - 1u);
         if (cross) {
           const int e = mcnt + __popc(gb & ((1u << sub) - 1u));
           L[e] = c.x;
@@ -1053,17 +1068,24 @@ __global__ __launch_bounds__(PTH, 2) void k_push_step(PP P, const int *__restric
         }
       }
       __builtin_amdgcn_wave_barrier();         // the group reads what its lanes listed
-      mover_sums(mv, sub, L, Ls, Ys + g * (YN * PG), role, mcnt, i, j, P, qcs);
+      const int ga = PG == 8 ? g & ~1 : g, gb = PG == 8 ? g | 1 : g;
+      mover_sums<PG, MLC>(mv, mw, sub, L, Ls, Ys + g * (YN * PG), Ys + ga * (YN * PG),
+                          Ys + gb * (YN * PG), role, mcnt, i, j, P, qcs);
       mcnt = 0;
       if (s == P.nsp) break;
     }
   }
   if (bad) atomicOr(derr, bad);
   __syncthreads();                             // the lists' space is free
-  put_sums(cb, role, mv);
+  if (PG == 8) {
+    put_sums(cellbuf + (g & ~1) * NACC, role, mv);
+    put_sums(cellbuf + (g | 1) * NACC, role, mw);
+  } else {
+    put_sums(cb, role, mv);
+  }
   __builtin_amdgcn_wave_barrier();
-  const int s0 = group_sums(core, sub);
-  if ((sub & 1) == 0) {
+  const int s0 = group_sums<PG>(core, sub);
+  if (PG == 8 || (sub & 1) == 0) {
 #pragma unroll
     for (int e = 0; e < 3; ++e)
       if (s0 + e < NCORE) cb[core_at(s0 + e)] += core[e];
@@ -1188,15 +1210,26 @@ int wm_k_push_step(wm_ctx *ctx) {
   const int src = !ctx->perm_valid                          ? SRC_SLOT
                   : (size_t)P.ny * P.cap <= (size_t)1 << 29 ? SRC_PERM32
                                                             : SRC_PERM64;
-  auto kernel = P.xmode == 1
-                    ? (src == SRC_SLOT     ? k_push_step<SRC_SLOT, false>
-                       : src == SRC_PERM32 ? k_push_step<SRC_PERM32, false>
-                                           : k_push_step<SRC_PERM64, false>)
-                    : (src == SRC_SLOT     ? k_push_step<SRC_SLOT, true>
-                       : src == SRC_PERM32 ? k_push_step<SRC_PERM32, true>
-                                           : k_push_step<SRC_PERM64, true>);
+  // Lanes of a cell: steps of 16 waste lanes on few particles, steps of 8 take
+  // the longer over many, and over the dense cells of a small grid whose
+  // wavefronts are all resident.  16 against 8, time ratio after 10 and 200
+  // steps of a two-stream plasma, 1024 x 1024 cells: 1.47 and 1.42 at 8
+  // particles per cell and species, 1.24 and 1.19 at 24, 1.08 and 1.12 at 32,
+  // 0.95 and 1.05 at 40, 0.88 and 1.00 at 48; 512 x 512: 1.10 and 1.08 at 32,
+  // 0.98 and 1.04 at 40, 0.86 and 0.91 at 64; 256 x 64: 1.33 and 0.83 at 24,
+  // 1.25 and 0.86 at 32.
+  const long long cells = (long long)P.nx * P.ny;
+  const bool eight = cells > 32768 && ctx->npart <= 36 * cells * P.nsp;
+#define WM_PUSH(S, W) (eight ? k_push_step<S, W, 8> : k_push_step<S, W, 16>)
+  auto kernel = P.xmode == 1 ? (src == SRC_SLOT     ? WM_PUSH(SRC_SLOT, false)
+                                : src == SRC_PERM32 ? WM_PUSH(SRC_PERM32, false)
+                                                    : WM_PUSH(SRC_PERM64, false))
+                             : (src == SRC_SLOT     ? WM_PUSH(SRC_SLOT, true)
+                                : src == SRC_PERM32 ? WM_PUSH(SRC_PERM32, true)
+                                                    : WM_PUSH(SRC_PERM64, true));
+#undef WM_PUSH
   P.nchunk = wm_cdiv(P.nx, PCH);
-  hipLaunchKernelGGL(kernel, dim3(P.nchunk * P.ny), dim3(PTH), 0, ctx->stream, P, ctx->cumcnt,
+  hipLaunchKernelGGL(kernel, dim3(P.nchunk * P.ny), dim3(PCH * (eight ? 8 : 16)), 0, ctx->stream, P, ctx->cumcnt,
                      ctx->tmp, TX, tps, ctx->bank[0], ctx->bank[1], O, ctx->dep_part, ctx->derr);
   WM_HIP(hipGetLastError());
   std::swap(ctx->bank[0], ctx->bank[1]);
