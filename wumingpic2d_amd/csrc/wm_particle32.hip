@@ -203,14 +203,6 @@ __device__ inline int core_at(int e) {             // slot of core value e (core
   if (e < 12) return 20 + (1 + (e - 6) / 2) * 4 + 1 + (e - 6) % 2;
   return 40 + (1 + (e - 12) / 3) * 5 + 1 + (e - 12) % 3;
 }
-// Sum of component comp at tile offset (a, b) of a cell, from csum.
-__device__ inline double acc_at(const double *csum, int cell, int comp, int a, int b) {
-  const int idx = comp == 0 ? (a - 1) * 5 + b : (comp == 1 ? 20 + a * 4 + (b - 1) : 40 + a * 5 + b);
-  const bool none = (comp == 0 && a == 0) || (comp == 1 && b == 0);
-  const double v = csum[cell * NACC + (none ? 0 : idx)];
-  return none ? 0.0 : v;
-}
-
 // Sums of 24 values over the 16 lanes of a group, by halving: in each of three
 // exchanges a lane keeps one half of the values and adds its partner's share
 // of them (partners: lane xor 8, the mirrored lane of its eight, lane xor 2);
@@ -804,39 +796,62 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
     wm_mover::put_sums(csum + g * NACC, role, mv);
     __builtin_amdgcn_wave_barrier();
     for (int e = sub; e < NCORE; e += GROUP) csum[g * NACC + core_at(e)] += (double)ccore[g * 24 + e];
-    // per bin: movers in total and per direction
+    // per bin: movers in total and per direction (index 0..7: directions 0..8
+    // without 4), sixteen of the list at a time by ballots; a bin with more
+    // movers than its summary lists has its records of each direction
+    // together, in list order, at perm[first + (counts of the directions
+    // before) + rank]
     for (int s = 0; s < P.nsp; ++s) {
       const int j0 = s ? gsb[(s - 1) * CHUNK + g] : 0;
       const int m = gsb[s * CHUNK + g] - j0;
       BinSum *bs = msum + bin_of(s, jl, il, P.ny, P.nx);
-      // lane sub < 8 of the cell's group: direction index sub (directions
-      // 0..8 without 4); its count, and (a bin with more movers than its
-      // summary lists) the bin's records of that direction in list order at
-      // perm[first + (counts of the directions before) + rank]
-      const int d = sub < 4 ? sub : sub + 1;
+      const int gsh = (int)(threadIdx.x & 63) & ~(GROUP - 1);
+      auto dir_of = [&](int q, int &xv) {
+        xv = q < m ? xl_at(xent(g, j0 + q), X) : 0;
+        const int d = (xv >> 20) & 0xF;
+        return q < m ? d - (d > 4) : -1;
+      };
+      // lane sub < 8: the count of direction index sub
       int c = 0;
-      if (sub < 8)
-        for (int q = 0; q < m; ++q) c += ((xl_at(xent(g, j0 + q), X) >> 20) & 0xF) == d;
-      int pre = c;
+      for (int q0 = 0; q0 < m; q0 += GROUP) {
+        int xv;
+        const int d = dir_of(q0 + sub, xv);
 #pragma unroll
-      for (int o = 1; o < 8; o <<= 1) {
-        const int v = __shfl_up(pre, o, 8);
-        if (sub >= o) pre += v;
+        for (int e = 0; e < 8; ++e) {
+          const int n = __popc((unsigned)(__ballot(d == e) >> gsh) & 0xFFFFu);
+          c += sub == e ? n : 0;
+        }
+        if (q0 == 0 && sub < min(m, WM_SUM_MV))
+          bs->mv[sub] = (uint16_t)((xv & 0xFFFFF) | (d << WM_SLOT_BITS));
       }
-      pre -= c;
       if (sub < 8) {
         if (c > 255) atomicOr(derr, DERR_MOVER_OVER);
         bs->cnt[sub] = (uint8_t)min(c, 255);
-        if (rf >= 0 && c > 0 && m > WM_SUM_MV) {       // else the summary lists them
-          int *pp = M.perm + (size_t)jl * mrow + rf + before + j0 + pre;
-          for (int q = 0, r = 0; r < c; ++q)
-            if (((xl_at(xent(g, j0 + q), X) >> 20) & 0xF) == d) pp[r++] = q;
-        }
       }
-      if (sub < min(m, WM_SUM_MV)) {
-        const int xv = xl_at(xent(g, j0 + sub), X);
-        const int dir = (xv >> 20) & 0xF;
-        bs->mv[sub] = (uint16_t)((xv & 0xFFFFF) | ((dir - (dir > 4)) << WM_SLOT_BITS));
+      if (rf >= 0 && m > WM_SUM_MV) {                  // else the summary lists them
+        int pre = c;
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) {
+          const int v = __shfl_up(pre, o, 8);
+          if ((sub & 7) >= o) pre += v;
+        }
+        pre -= c;                                      // lane e: where direction e's begin
+        int *pp = M.perm + (size_t)jl * mrow + rf + before + j0;
+        for (int q0 = 0; q0 < m; q0 += GROUP) {
+          int xv;
+          const int d = dir_of(q0 + sub, xv);
+          unsigned same = 0;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const unsigned b = (unsigned)(__ballot(d == e) >> gsh) & 0xFFFFu;
+            same = d == e ? b : same;
+            const int n = __popc(b);
+            if (sub == e) c = n;
+          }
+          const int at = __shfl(pre, gsh + max(d, 0), 64);
+          if (d >= 0) pp[at + __popc(same & ((1u << sub) - 1u))] = q0 + sub;
+          if (sub < 8) pre += c;
+        }
       }
       if (sub == 0) {
         bs->first = (uint32_t)(max(rf, 0) + before + j0);
@@ -845,14 +860,21 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
     }
   }
   __syncthreads();                                   // every cell's FP64 sums
+  // tile value (b, t, comp): the cells t - a, a = 4 .. 0, at tile offset (a, b)
+  // (csum's layout: Jx (a-1)*5 + b, Jy 20 + a*4 + (b-1), Jz 40 + a*5 + b)
   double *out = part + ((size_t)jl * P.nchunk + chunk) * TILE;
   for (int e = threadIdx.x; e < TILE; e += NT) {
-    const int comp = e % 3;
-    const int t = (e / 3) % DW;
-    const int b = e / (3 * DW);
+    const int comp = e % 3, bt = e / 3, t = bt % DW, b = bt / DW;
+    const int st = comp == 1 ? 4 : 5;
+    const int at = t * NACC + (comp == 0 ? b - 5 : (comp == 1 ? 19 + b : 40 + b));
+    const bool row = comp != 1 || b > 0;
     double sum = 0.0;
-    const int glo = max(0, t - 4), ghi = min(ncell - 1, t);
-    for (int gg = glo; gg <= ghi; ++gg) sum += acc_at(csum, gg, comp, t - gg, b);
+#pragma unroll
+    for (int a = 4; a >= 0; --a) {
+      const bool on = row && (unsigned)(t - a) < (unsigned)ncell && (a > 0 || comp != 0);
+      const double v = csum[on ? at + a * (st - NACC) : 0];
+      sum += on ? v : 0.0;
+    }
     out[e] = sum;
   }
 }
