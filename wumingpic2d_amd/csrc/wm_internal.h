@@ -175,7 +175,9 @@ struct wm_ctx {
   float *tmp32 = nullptr;  // cell-centred fields of the FP32 push
   Rec64 b64(int k) const { return bank[k]; }
   int64_t *id[2]{};
-  int idcur = 0;           // which id array goes with bank 0 / bank 1 data
+  int idcur = 0;           // which id array goes with bank 0 / bank 1 data (the other holds
+                           // the row order's ID indexes, oidcur the current half, with perm_valid)
+  int oidcur = 0;
   int *np2 = nullptr;      // [nseg]
   int *cumcnt = nullptr;   // [nseg*(nx+1)]
 

@@ -310,8 +310,8 @@ struct Place {
   const int4 *kind;
   const uint2 *disp;
   unsigned *perm;
-  const int64_t *id;
-  int64_t *idd;
+  const unsigned *oid;           // whose ID each slot's particle has (null: its own)
+  unsigned *oidd;
 };
 
 // A row with particles that crossed more than one cell (mirrored by a wall
@@ -349,7 +349,7 @@ __device__ bool place_wide(const OP &P, const Place &R, int seg, int c) {
         for (int i = 0; i < D; ++i) dst += (int)dl[d0 + i].x < k;
         if (dst < newn) {
           R.perm[base + dst] = own + (unsigned)k;
-          R.idd[base + dst] = R.id[base + k];
+          R.oidd[base + dst] = R.oid ? R.oid[base + k] : own + (unsigned)k;
         } else {
           bad = true;
         }
@@ -361,7 +361,7 @@ __device__ bool place_wide(const OP &P, const Place &R, int seg, int c) {
       for (int i = 0; i < D; ++i) dst += (int)dl[d0 + i].x < (int)de.x;
       if (dst < newn) {
         R.perm[base + dst] = de.y;
-        R.idd[base + dst] = R.id[plane + de.y];
+        R.oidd[base + dst] = R.oid ? R.oid[plane + de.y] : de.y;
       } else {
         bad = true;
       }
@@ -370,8 +370,9 @@ __device__ bool place_wide(const OP &P, const Place &R, int seg, int c) {
   return bad;
 }
 
-// The place of every particle, as the index it comes from, and its ID, which
-// moves here.  A group of 16 lanes per cell o, in two parts.
+// The place of every particle, as the index it comes from, and whose ID it has
+// (an index into the IDs, which stay where they are until the rows are read as
+// rows).  A group of 16 lanes per cell o, in two parts.
 //
 // The row's own particles of old cell o (16 codes at a time, ballots): one
 // that goes to cell c in {o-1, o, o+1} comes after the particles of lower
@@ -387,7 +388,7 @@ __device__ bool place_wide(const OP &P, const Place &R, int seg, int c) {
 // go right, go left, and how many before it) -- and the displaced ones with
 // lower slots.
 //
-// 2 B of code, 4 B of index and 16 B of ID per particle, three dependent round
+// 2 B of code, 4 B of index and 8 B of ID index per particle, three dependent round
 // trips to memory a cell, which bound it; six wavefronts a SIMD hide most.  Where
 // a plasma has pinched (256 x 64 cells, 407 particles in the densest at a mean
 // of 64) the longest cells set the time: 42 us, and 124 where every window
@@ -418,7 +419,6 @@ __global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr,
   const int *ds = R.dstart + (size_t)seg * (nx + 1);
   const int4 *kd = R.kind + (size_t)seg * nx;
   const uint2 *dl = R.disp + 2 * (size_t)seg * P.mcap;
-  const int64_t *id = R.id + base;
   // first round trip: everything about the cell and its neighbours (walls
   // have none beyond the ends: their counts are zero)
   const bool hasl = o > 0 || P.periodic, hasr = o + 1 < nx || P.periodic;
@@ -445,8 +445,7 @@ __global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr,
   const bool tabled = ke - kb <= PG * PWT;
   // second round trip: the first codes and IDs, the displaced particles (the
   // first 16 of each list in registers)
-  unsigned cv[PWIN];
-  int64_t iv[PWIN];
+  unsigned cv[PWIN], iv[PWIN];
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int w = 0; w < PWIN; ++w) {
@@ -455,14 +454,14 @@ __global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr,
       iv[w] = 0;
       if (k < ke) {
         cv[w] = cd[k];
-        iv[w] = id[k];
+        iv[w] = R.oid ? R.oid[base + k] : own + (unsigned)k;
       }
     }
   };
   const uint2 de0 = sub < D ? dl[d0 + sub] : make_uint2(NONE, 0u);
   const int pL = sub < Dl ? (int)dl[dl0 + sub].x : NONE, pR = sub < Dr ? (int)dl[dr0 + sub].x : NONE;
   fetch(kb);
-  const int64_t di0 = sub < D ? R.id[plane + de0.y] : 0;   // (the third)
+  const unsigned di0 = sub < D && R.oid ? R.oid[plane + de0.y] : de0.y;   // (the third)
   auto ballot16 = [&](bool b) { return (unsigned)(__ballot(b) >> gsh) & 0xFFFFu; };
   const unsigned below = (1u << sub) - 1u;
   auto low16 = [](int n) { return n <= 0 ? 0u : n >= 16 ? 0xFFFFu : (1u << n) - 1u; };
@@ -540,7 +539,7 @@ __global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr,
       if (own_) {
         if (dst < newn) {
           R.perm[base + dst] = own + (unsigned)k;
-          R.idd[base + dst] = iv[w];
+          R.oidd[base + dst] = iv[w];
         } else {
           bad = true;
         }
@@ -562,10 +561,10 @@ __global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr,
   for (int i0 = 0; i0 < D; i0 += PG) {
     const bool mine = i0 + sub < D;
     uint2 de = de0;
-    int64_t v = di0;
+    unsigned v = di0;
     if (i0 > 0) {
       de = mine ? dl[d0 + i0 + sub] : make_uint2(NONE, 0u);
-      v = mine ? R.id[plane + de.y] : 0;
+      v = mine && R.oid ? R.oid[plane + de.y] : de.y;
     }
     const int p = (int)de.x;
     int dst = start;
@@ -614,7 +613,7 @@ __global__ __launch_bounds__(PT, 6) void k_order_place(OP P, Place R, int *derr,
     if (mine) {
       if (dst < newn) {
         R.perm[base + dst] = de.y;
-        R.idd[base + dst] = v;
+        R.oidd[base + dst] = v;
       } else {
         bad = true;
       }
@@ -635,6 +634,26 @@ __global__ __launch_bounds__(256) void k_order_apply(int cap, int ny, const int 
   const size_t base = (size_t)seg * cap, plane = (size_t)(seg / ny) * ny * cap;
   for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += 256 * gridDim.x)
     B.store(base + k, A.load(plane + perm[base + k]));
+}
+// Their IDs: gathered (an index that a row without a place left is kept inside
+// the plane), then put in place.
+__global__ __launch_bounds__(256) void k_ids_gather(int cap, int ny, const int *__restrict__ np2,
+                                                    const unsigned *__restrict__ oid,
+                                                    const int64_t *__restrict__ id,
+                                                    int64_t *__restrict__ to) {
+  const int seg = blockIdx.y, n = np2[seg];
+  const size_t len = (size_t)ny * cap;
+  const size_t base = (size_t)seg * cap, plane = (size_t)(seg / ny) * len;
+  for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += 256 * gridDim.x)
+    to[base + k] = id[plane + min((size_t)oid[base + k], len - 1)];
+}
+__global__ __launch_bounds__(256) void k_ids_put(int cap, const int *__restrict__ np2,
+                                                 const int64_t *__restrict__ from,
+                                                 int64_t *__restrict__ id) {
+  const int seg = blockIdx.y, n = np2[seg];
+  const size_t base = (size_t)seg * cap;
+  for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += 256 * gridDim.x)
+    id[base + k] = from[base + k];
 }
 
 }  // namespace
@@ -658,12 +677,17 @@ int wm_k_order(wm_ctx *ctx) {
                      ctx->code, ctx->kind, ctx->farcnt, ctx->far, ctx->lup, ctx->ldn, ctx->hole,
                      ctx->nhole, ctx->nup, ctx->ndn, ctx->cumnew, ctx->disp, ctx->dstart,
                      ctx->rowok, ctx->derr);
+  // the IDs' indexes of this order and the last share the spare ID array
+  unsigned *const o = (unsigned *)ctx->id[1 - ctx->idcur];
+  const size_t slots = (size_t)nseg * ctx->cap;
+  const int now = ctx->perm_valid ? ctx->oidcur : 1;
   const Place R{ctx->nold, ctx->rowok, ctx->cumcnt, ctx->cumnew, ctx->far, ctx->dstart, ctx->code,
-                ctx->kind, ctx->disp, ctx->perm, ctx->id[ctx->idcur], ctx->id[1 - ctx->idcur]};
+                ctx->kind, ctx->disp, ctx->perm, ctx->perm_valid ? o + now * slots : nullptr,
+                o + (1 - now) * slots};
   hipLaunchKernelGGL(k_order_place, dim3(wm_cdiv(g.nx, PCELL), nseg), dim3(PT), 0, ctx->stream, P,
                      R, ctx->derr, ctx->ts);
   WM_HIP(hipGetLastError());
-  ctx->idcur = 1 - ctx->idcur;
+  ctx->oidcur = 1 - now;
   std::swap(ctx->cumcnt, ctx->cumnew);
   ctx->perm_valid = true;
   return WM_OK;
@@ -673,10 +697,17 @@ int wm_k_order(wm_ctx *ctx) {
 int wm_order_apply(wm_ctx *ctx) {
   if (!ctx->perm_valid) return WM_OK;
   const wm_grid &g = ctx->g;
-  hipLaunchKernelGGL(k_order_apply, dim3(std::max(1, std::min(64, wm_cdiv(ctx->cap, 1024))),
-                                         g.nsp * g.ny),
-                     dim3(256), 0, ctx->stream, ctx->cap, g.ny, ctx->np2, ctx->perm, ctx->bank[0],
-                     ctx->bank[1]);
+  const dim3 grid(std::max(1, std::min(64, wm_cdiv(ctx->cap, 1024))), g.nsp * g.ny);
+  hipLaunchKernelGGL(k_order_apply, grid, dim3(256), 0, ctx->stream, ctx->cap, g.ny, ctx->np2,
+                     ctx->perm, ctx->bank[0], ctx->bank[1]);
+  // (bank 0's records have moved: its space holds the IDs on their way)
+  const unsigned *oid = (const unsigned *)ctx->id[1 - ctx->idcur] +
+                        (size_t)ctx->oidcur * g.nsp * g.ny * ctx->cap;
+  int64_t *const tmp = (int64_t *)ctx->bank[0].x;
+  hipLaunchKernelGGL(k_ids_gather, grid, dim3(256), 0, ctx->stream, ctx->cap, g.ny, ctx->np2, oid,
+                     ctx->id[ctx->idcur], tmp);
+  hipLaunchKernelGGL(k_ids_put, grid, dim3(256), 0, ctx->stream, ctx->cap, ctx->np2, tmp,
+                     ctx->id[ctx->idcur]);
   WM_HIP(hipGetLastError());
   std::swap(ctx->bank[0], ctx->bank[1]);
   ctx->perm_valid = false;
