@@ -452,6 +452,97 @@ __global__ __launch_bounds__(256) void k_field_update(FieldGeom fg, SolveConst f
   un[5 * ps + t] = uf[5 * ps + t] + e3;
 }
 
+// The same between conducting walls (active columns L .. E of the
+// ghost-inclusive planes, boundary_shock.f90:326-405,
+// boundary_reconnection.f90:280-359): rows wrap, then Bx, Ey, Ez are odd about
+// the left wall and By, Bz, Ex even; right of the shock's box is zero, the
+// reconnection's right wall is the mirror image and rewrites column E of Bx,
+// Ey and Ez.  delta E at a cell that takes another's is worked out there.  What
+// no rule writes (two columns out, and E + 1 of the reconnection's odd
+// components) is added as it stands, and df is left as the separate kernels
+// leave it: the walls may move.  Columns outside L - 2 .. E + 2 are copied.
+// One launch for seven, 32 us of a step at 256 x 128.
+struct WallField {
+  const double *df;
+  size_t ps;
+  int L, E;
+  bool shock;
+  // delta B of component k at column li (L - 1 .. E + 1) of the interior row
+  // that begins at ro
+  __device__ double dB(int k, int li, size_t ro) const {
+    const double *R = df + (size_t)k * ps + ro;
+    if (li == L - 1) return k == 0 ? -R[L] : R[L + 1];
+    if (li == E && k == 0 && !shock) return -R[E - 1];
+    if (li == E + 1) return shock ? 0.0 : (k == 0 ? R[li] : R[E - 1]);
+    return R[li];
+  }
+};
+__global__ __launch_bounds__(256) void k_walls_update(FieldGeom fg, SolveConst f, XSide X,
+                                                      const double *__restrict__ uf,
+                                                      const double *__restrict__ uj, double *df,
+                                                      double *__restrict__ un, const int *abort_,
+                                                      const SolveOut *out, const int *derr,
+                                                      const unsigned long long *ts, unsigned seq,
+                                                      SolveReport *host) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  const int given = abort_ ? *abort_ : 0;
+  const SolveOut o = abort_ ? *out : SolveOut{};
+  if (t == 0) leave_report(host, o, given, derr, ts, seq);
+  if (given || o.err[0] || o.err[1] || o.err[2] || t >= fg.gx * fg.gy) return;
+  const int li = t % fg.gx, lj = t / fg.gx;
+  const size_t gx = fg.gx, ps = fg.ps;
+  const WallField W{df, ps, X.xa + 2, X.xb + 2, X.wall == WM_BC_SHOCK};
+  double d[6];
+  if (li < W.L - 1 || li > W.E + 1) {
+    const bool add = li == W.L - 2 || li == W.E + 2;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) d[k] = add ? df[k * ps + t] : 0.0;
+  } else {
+    int j = (lj - 2) % fg.ny;
+    if (j < 0) j += fg.ny;
+    const size_t ro = gx * (size_t)(j + 2), rn = gx * (size_t)(wrapm(j + 1, fg.ny) + 2);
+    const double *B1 = uf, *B2 = uf + ps, *B3 = uf + 2 * ps;
+    auto dE = [&](int k, int col) {            // field.f90:154-171
+      const size_t c = (size_t)col + ro;
+      if (k == 3)
+        return f.f1 * (f.gfac * (-W.dB(2, col, ro) + W.dB(2, col, rn)) + (-B3[c] + B3[c + gx])) -
+               f.fpt * uj[c];
+      if (k == 4)
+        return -f.f1 * (f.gfac * (-W.dB(2, col, ro) + W.dB(2, col + 1, ro)) + (-B3[c] + B3[c + 1])) -
+               f.fpt * uj[ps + c];
+      return f.f1 * (f.gfac * (-W.dB(1, col, ro) + W.dB(1, col + 1, ro) + W.dB(0, col, ro) -
+                               W.dB(0, col, rn)) +
+                     (-B2[c] + B2[c + 1] + B1[c] - B1[c + gx])) -
+             f.fpt * uj[2 * ps + c];
+    };
+    const bool left = li == W.L - 1, right = li == W.E + 1, stale = right && !W.shock;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) d[k] = stale && k == 0 ? df[t] : W.dB(k, li, ro);
+    if (right && W.shock) {
+      d[3] = d[4] = d[5] = 0.0;
+    } else {
+      d[3] = dE(3, left ? W.L + 1 : (right ? W.E - 1 : li));
+      const bool odd = left || (li == W.E && !W.shock);
+      const int col = left ? W.L : (odd ? W.E - 1 : li);
+#pragma unroll
+      for (int k = 4; k < 6; ++k) {
+        if (stale) {
+          d[k] = df[k * ps + t];
+        } else {
+          const double v = dE(k, col);
+          d[k] = odd ? -v : v;
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k)                // (delta B inside the box is there)
+      if (k >= 3 || left || right || li == W.E || lj < 2 || lj >= fg.ny + 2)
+        if (!(stale && (k == 0 || k > 3))) df[k * ps + t] = d[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) un[k * ps + t] = uf[k * ps + t] + d[k];
+}
+
 // The device's CUs shared by the contexts of this process: a solve in flight
 // holds as many as it has workgroups.
 struct Slots {
@@ -634,8 +725,8 @@ int wm_k_tiles(wm_ctx *ctx, bool begins) {
 
 // A single row is its own neighbour above and below: its ghost rows hold what
 // the reference's sequence of copies leaves there, which takes the separate
-// kernels, as the walls do.
-bool wm_fused_update(const wm_ctx *ctx) { return ctx->bcf == WM_BC_PERIODIC && ctx->g.ny > 1; }
+// kernels.
+bool wm_fused_update(const wm_ctx *ctx) { return ctx->g.ny > 1; }
 
 int wm_k_update_report(wm_ctx *ctx) {
   const FieldGeom &fg = ctx->fg;
@@ -643,10 +734,18 @@ int wm_k_update_report(wm_ctx *ctx) {
   ++ctx->seq;
   if (wm_fused_update(ctx)) {
     if (!ctx->uf2) WM_HIP(hipMalloc((void **)&ctx->uf2, sizeof(double) * 6 * fg.ps));
-    hipLaunchKernelGGL(k_field_update, dim3(wm_cdiv((long long)fg.gx * fg.gy, 256)), dim3(256), 0,
-                       ctx->stream, fg, make_fc(ctx->g), ctx->uf, ctx->uj, ctx->df, ctx->uf2,
-                       abort_, (const SolveOut *)ctx->tile_out, ctx->derr, ctx->ts, ctx->seq,
-                       report_of(ctx));
+    const dim3 grid(wm_cdiv((long long)fg.gx * fg.gy, 256));
+    const XSide X = wm_xside(ctx);
+    if (X.wall)
+      hipLaunchKernelGGL(k_walls_update, grid, dim3(256), 0, ctx->stream, fg, make_fc(ctx->g), X,
+                         ctx->uf, ctx->uj, ctx->df, ctx->uf2, abort_,
+                         (const SolveOut *)ctx->tile_out, ctx->derr, ctx->ts, ctx->seq,
+                         report_of(ctx));
+    else
+      hipLaunchKernelGGL(k_field_update, grid, dim3(256), 0, ctx->stream, fg, make_fc(ctx->g),
+                         ctx->uf, ctx->uj, ctx->df, ctx->uf2, abort_,
+                         (const SolveOut *)ctx->tile_out, ctx->derr, ctx->ts, ctx->seq,
+                         report_of(ctx));
     std::swap(ctx->uf, ctx->uf2);
     ctx->tile_swapped = ctx->tile_held != 0;
   } else {
