@@ -12,7 +12,7 @@ synthetic state generated on the device.
 Prints one JSON line.  ``value`` is the headline form's rate (FP32
 particles, flexible CG with the learned preconditioner) over the timed steps
 after the warm-up; ``roofline`` covers the dominant kernel (fused
-push+deposit), timed with HIP events on the library's stream; ``cpu_baseline``
+push+deposit), timed by the device's clock; ``cpu_baseline``
 is the FP64 CPU restatement timed on this host's cores on a bounded sample
 (256 x 256 cells at the same density), with the reference's own OpenMP build
 of the push and the sort timed beside the restatement's where it was built.
@@ -464,7 +464,7 @@ def main() -> int:
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic,
-                "kernel": ("k_particle<PUSH,DEPOSIT>" if args.form == "fp64" else "k_push_deposit32")
+                "kernel": ("k_push_step" if args.form == "fp64" else "k_push_deposit32")
                 + " (fused push+deposit)",
                 "bytes_per_particle": bpp, "launches_per_step": launches,
                 "launch_ms": round(launch_ms, 4),

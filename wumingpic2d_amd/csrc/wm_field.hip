@@ -735,7 +735,7 @@ static int fcg_solve(wm_ctx *ctx, const CgArgs &A, int *its) {
   // partial pair per 16x16 tile
   CgArgs AT = A;
   AT.nblk = wm_pc_dot_tiles(A.nx, A.ny);
-  static_assert(3 * sizeof(FcgScal) <= WM_PIN_BYTES, "pinned scratch too small");
+  static_assert(3 * sizeof(FcgScal) <= WM_PIN_REPORT, "pinned scratch too small");
   FcgScal *hs = (FcgScal *)ctx->h_pin;
   int cur = 0;
   int batch = std::max(1, ctx->fcg_hint);
@@ -845,7 +845,7 @@ static int stream_plain(wm_ctx *ctx) {
   hipLaunchKernelGGL(k_cg_fin, dim3(3), dim3(CGB), 0, ctx->stream, A, 0, ctx->red, ctx->cg_s);
   WM_HIP(hipGetLastError());
   const bool collect = ctx->solver == WM_SOLVER_CG && !X.wall && wm_pc_collecting(ctx);
-  static_assert(3 * sizeof(CgScal) <= WM_PIN_BYTES, "pinned scratch too small");
+  static_assert(3 * sizeof(CgScal) <= WM_PIN_REPORT, "pinned scratch too small");
   CgScal *hs = (CgScal *)ctx->h_pin;
   int iters = 0, cur = 0;
   int batch = collect ? 1 : std::max(1, ctx->cg_hint);
@@ -961,7 +961,8 @@ int wm_k_field_solve(wm_ctx *ctx) {
 // source row offset ascending, chunk ascending.  FP32: also marks every
 // row's bins as awaiting the push's movers.  Bound by reading the tiles: 157 MB
 // at 1024 x 1024 in 16-cell chunks, 72 us (40 at a copy's rate); 5 us at 256 x
-// 64, where the gather and the folds were three launches.
+// 64, where the gather and the folds were three launches.  (The FP64 step's
+// tiles, of 8 cells, hold a fifth more.)
 namespace {
 template <int CHUNK>
 __global__ __launch_bounds__(256) void k_current(FieldGeom fg, int nchunk, int wall,

@@ -6,7 +6,8 @@
 //   the reference's particle index ii = k+1 of row j (proj/weibel/app.f90:281
 //   up(ndim,np,nys:nye,nsp)), so row-local orders, np2 and cumcnt keep the
 //   reference's meaning exactly.  Two position/momentum banks: bank 0 plays
-//   `up`, bank 1 plays `gp`.  IDs live in their own ping-pong pair.
+//   `up`, bank 1 plays `gp`; between steps of the resident run the rows' order
+//   may be an index into bank 0 (perm).  IDs live in arrays of their own.
 //   Fields: one plane per component, x fastest, ghost-inclusive
 //   (nx+4) x (ny+4) for uf/df/uj (the reference's nxgs-2:nxge+2,
 //   nys-2:nye+2 bounds), planes of (nx+2) x (ny+2) for the cell-centred
@@ -175,8 +176,9 @@ struct wm_ctx {
   float *tmp32 = nullptr;  // cell-centred fields of the FP32 push
   Rec64 b64(int k) const { return bank[k]; }
   int64_t *id[2]{};
-  int idcur = 0;           // which id array goes with bank 0 / bank 1 data (the other holds
-                           // the row order's ID indexes, oidcur the current half, with perm_valid)
+  int idcur = 0;           // which id array goes with bank 0 / bank 1 data.  With perm_valid the
+                           // IDs lie as they did when the order began and the other array holds
+                           // every slot's ID index (32 bits; two halves, oidcur the current one)
   int oidcur = 0;
   int *np2 = nullptr;      // [nseg]
   int *cumcnt = nullptr;   // [nseg*(nx+1)]
@@ -189,8 +191,8 @@ struct wm_ctx {
   // The resident step's row order (wm_order.hip).  With perm_valid, bank 0
   // holds the last push's output in the slots it read its particles from
   // (nold per segment), and slot k of a row is the particle at index
-  // perm[seg * cap + k] of its species' plane (row * cap + slot); np2, cumcnt
-  // and the IDs are the ordered rows'.
+  // perm[seg * cap + k] of its species' plane (row * cap + slot); np2 and cumcnt
+  // are the ordered rows'.
   bool perm_valid = false;
   long long npart = 0;           // particles of the resident state (their number stays)
   unsigned *perm = nullptr;      // [nseg*cap]

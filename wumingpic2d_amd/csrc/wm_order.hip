@@ -7,11 +7,13 @@
 // three kernels below turn the codes into the order the reference's
 // particle_x, particle_y and sort__bucket would leave, as one 32-bit source
 // index per new slot; the next push reads its particles through it and writes
-// them sorted.  A step so reads and writes each 48-byte record once, plus 8
-// bytes of codes and index, where pushing in place, scanning for leavers and
-// sorting moved 192 bytes a particle.  Measured at 2048 x 2048, 64 particles
-// per cell and species, beside the field solve: rows and merge 1.5, place
-// 4.6 ms, where pass 1 took 6.0 and pass 2 with the sort 16.7 ms.
+// them sorted.  The IDs stay where they are until someone asks for them; a
+// second index says which goes with which slot.  A step so reads and writes
+// the 40 bytes of each particle's state once, plus about 20 of codes and
+// indexes, where pushing in place, scanning for leavers and sorting moved 192
+// bytes a particle.  Measured at 2048 x 2048, 64 particles per cell and
+// species, beside the field solve: rows and merge 1.5, place 4.0 ms, where
+// pass 1 took 6.0 and pass 2 with the sort 16.7 ms.
 //
 // The order.  Pass 1 lists a row's leavers (up, down) and their slots, the
 // holes, in slot order.  Pass 2 puts arrival a (the neighbours' leavers,

@@ -1,7 +1,8 @@
 // wm_particle.hip -- Buneman-Boris push and Esirkepov deposit (FP64 form).
 //
-// Work decomposition (the same for the push, the deposit and the fused
-// push+deposit kernel): one workgroup per (row j, chunk of CHUNK cells); the
+// The resident step's kernel, push and deposit in one, is k_push_step below.
+// The host-array entry points push and deposit apart, in k_particle.  Its work
+// decomposition: one workgroup per (row j, chunk of CHUNK cells); the
 // workgroup's 256 lanes form 32 groups of 8 lanes, group g owns cell
 // i0+g and its 8 lanes stride through that cell's particles of every species
 // (the reference's cell -> species -> particle loop, particle.f90:85-94 and
@@ -391,14 +392,14 @@ __global__ __launch_bounds__(256, 3) void k_particle(
       auto one = [&](int k, double x0, double y0, double cux, double cuy, double cuz, double &x1,
                      double &y1, double &qv) {
         if (k < kb || k >= ke) return false;   // before or after the cell
-        double ux, uy, uz, ig = 0.0;
+        double ux, uy, uz;
         // keep the 54 tile values in LDS instead of hoisting them into
         // registers for the whole cell loop (occupancy)
         __asm__ volatile("" ::: "memory");
         int i2, j2;
         if (PUSH) {
           PushOut o = boris(T, g, x0, y0, cux, cuy, cuz, i, j, P, fac1, txxx, fac2);
-          x1 = o.x; y1 = o.y; ux = o.ux; uy = o.uy; uz = o.uz; ig = o.ig;
+          x1 = o.x; y1 = o.y;
           i2 = (int)(x1 * P.d_delx);
           j2 = (int)(y1 * P.d_delx);
           seg_st(Xb, k, o.x); seg_st(Yb, k, o.y);
@@ -411,8 +412,7 @@ __global__ __launch_bounds__(256, 3) void k_particle(
         }
         if (DEPOSIT) {
           // v_z = u_z / gamma, field.f90:270
-          const double gvz = PUSH ? uz * ig
-                                  : uz / sqrt(1.0 + (ux * ux + uy * uy + uz * uz) / (P.c * P.c));
+          const double gvz = uz / sqrt(1.0 + (ux * ux + uy * uy + uz * uz) / (P.c * P.c));
           if (i2 == i && j2 == j) {
             stencil_core(core, x0, y0, x1, y1, gvz, i, j, q, P);
           } else {

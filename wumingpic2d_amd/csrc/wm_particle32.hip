@@ -1,7 +1,7 @@
 // wm_particle32.hip -- Buneman-Boris push and Esirkepov deposit in the FP32
 // form (int32 cell index + FP32 in-cell offsets + FP32 momenta).
 //
-// Same decomposition as the FP64 kernel: one workgroup per (row, chunk of
+// One workgroup per (row, chunk of
 // CHUNK cells), a group of GROUP lanes per cell striding through the cell's
 // particles in windows of GROUP consecutive particles.  The push and
 // the per-lane deposit run in FP32; the group's stencils are summed in FP32
