@@ -7,15 +7,18 @@
 // eight threads each own a pinned buffer and take pieces of the array in turn:
 // while one waits for its piece the others copy theirs, and a destination's
 // pages are touched while its piece is on the way.  202 MB of fields: 11.7 ->
-// 4.7 ms; pieces of 1 MB took 7.0, of 2 MB 5.3.
+// 4.7 ms; pieces of 1 MB took 7.0, of 2 MB 5.3.  Arrays below 64 MB go in pieces
+// of up to 2 MB, the 30 MB of moments as fast as in pieces of 4 MB (2.04 and 2.03
+// ms a call) and a context's first call, which makes the buffers, faster (3.15
+// and 3.9 ms).
 //
 // Rows of particles are gathered from and scattered to the caller's arrays in
 // the same pass; they used to go through a vector of the whole state, zeroed,
 // filled and copied on one thread (35 MB of rows in an array of 176: 9.7 -> 1.1
 // ms).
 //
-// The threads live as long as the call; the pinned buffers (4 MB each, made
-// when first needed) as long as the context.
+// The threads live as long as the call; the pinned buffers (2 or 4 MB each,
+// made when first needed) as long as the context.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -26,7 +29,8 @@
 #include "wm_xfer.h"
 
 namespace {
-constexpr size_t SLOT = (size_t)4 << 20;
+// The largest piece of a copy, and the size of the buffers it needs.
+size_t slot_for(size_t bytes) { return bytes < (size_t)64 << 20 ? (size_t)2 << 20 : (size_t)4 << 20; }
 constexpr int WORKERS = 8;
 // Threads for a copy: one up to 8 MB, then one per MB.  Starting one costs
 // about 20 us, and now and then milliseconds where the process has used up its
@@ -54,6 +58,7 @@ void on_threads(int n, F f) {
 
 struct wm_xfer {
   void *pin[WORKERS] = {};
+  size_t size[WORKERS] = {};
   hipEvent_t ev[WORKERS] = {};
   bool busy[WORKERS] = {};                     // the device may still read it
 };
@@ -69,11 +74,20 @@ void wm_xfer_free(wm_ctx *ctx) {
 }
 
 namespace {
-hipError_t slot_of(wm_xfer &x, int k) {
-  if (x.pin[k]) return hipSuccess;
+// Buffer k, of `size` bytes at least and not in use.
+hipError_t slot_of(wm_xfer &x, int k, size_t size) {
   hipError_t e = hipSuccess;
   if (!x.ev[k]) e = hipEventCreateWithFlags(&x.ev[k], hipEventDisableTiming);
-  if (e == hipSuccess) e = hipHostMalloc(&x.pin[k], SLOT, hipHostMallocDefault);
+  if (e == hipSuccess && x.busy[k]) {
+    e = hipEventSynchronize(x.ev[k]);
+    x.busy[k] = e != hipSuccess;
+  }
+  if (e != hipSuccess || x.size[k] >= size) return e;
+  if (x.pin[k]) e = hipHostFree(x.pin[k]);
+  x.pin[k] = nullptr;
+  x.size[k] = 0;
+  if (e == hipSuccess) e = hipHostMalloc(&x.pin[k], size, hipHostMallocDefault);
+  if (e == hipSuccess) x.size[k] = size;
   return e;
 }
 
@@ -103,8 +117,9 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
   const int want = threads_for(total);
   // one thread alone has two buffers, and copies a chunk while the next is on
   // its way
+  const size_t slot = slot_for(total);
   const size_t most =
-      std::min(SLOT, std::max<size_t>(total / (want > 1 ? want : 3) + rec, (size_t)1 << 20)) / rec * rec;
+      std::min(slot, std::max<size_t>(total / (want > 1 ? want : 3) + rec, (size_t)1 << 20)) / rec * rec;
   std::vector<WmSpan> piece;
   std::vector<Chunk> chunk;
   for (const WmSpan &s : spans)
@@ -145,8 +160,7 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
     for (size_t c; e == hipSuccess && err.load() == (int)hipSuccess && (c = next++) < chunk.size();) {
       const Chunk &h = chunk[c];
       const size_t at = piece[h.s0].at, len = piece[h.s1 - 1].at + piece[h.s1 - 1].bytes - at;
-      e = slot_of(x, buf);
-      if (e == hipSuccess && x.busy[buf]) e = hipEventSynchronize(x.ev[buf]);
+      e = slot_of(x, buf, slot);
       if (e != hipSuccess) break;
       x.busy[buf] = true;
       char *pin = (char *)x.pin[buf];
