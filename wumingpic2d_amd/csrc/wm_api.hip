@@ -674,7 +674,10 @@ int wm_alloc_device(wm_ctx *ctx) {
     WM_TRY(dmalloc(ctx, &ctx->cumnew, (size_t)nseg * (g.nx + 1)));
     WM_TRY(dmalloc(ctx, &ctx->nold, nseg));
     WM_TRY(dmalloc(ctx, &ctx->rowok, nseg));
+    // A slot that no cell of cumcnt covers (counts that do not belong together:
+    // an error of the step) keeps the code it has: always a cell of the row.
     WM_HIP(hipMemsetAsync(ctx->perm, 0, sizeof(unsigned) * slots, ctx->stream));
+    WM_HIP(hipMemsetAsync(ctx->code, 0, sizeof(uint16_t) * slots, ctx->stream));
     WM_HIP(hipMemsetAsync(ctx->farcnt, 0, sizeof(int) * (size_t)nseg * g.nx, ctx->stream));
     WM_HIP(hipMemsetAsync(ctx->far, 0, sizeof(int) * nseg, ctx->stream));
     WM_HIP(hipMemsetAsync(ctx->cumnew, 0, sizeof(int) * (size_t)nseg * (g.nx + 1), ctx->stream));
