@@ -1,0 +1,11 @@
+"""The test suite's way to what no program needs (csrc/wm_debug.h)."""
+import ctypes
+
+SOLVE_SLOTS = 1      # CUs held by solves in flight on the device; value is added
+SOLVE_FAILS = 2      # on-chip solves that fail to launch
+
+
+def debug(ctx, key, value=0):
+    f = ctx._lib.wm_debug
+    f.argtypes, f.restype = [ctypes.c_void_p, ctypes.c_int, ctypes.c_longlong], ctypes.c_longlong
+    return f(ctx._h, key, value)

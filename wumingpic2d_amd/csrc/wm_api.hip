@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "wm_internal.h"
+#include "wm_debug.h"
 #include "wm_solve.h"
 #include "wm_xfer.h"
 
@@ -1639,6 +1640,15 @@ int wm_solve_stats(wm_ctx *ctx, int *fcg3, int *plain3) {
     }
   }
   return WM_OK;
+}
+
+long long wm_debug(wm_ctx *ctx, int key, long long value) {
+  if (!ctx) return -1;
+  switch (key) {
+    case WM_DEBUG_SOLVE_SLOTS: return wm_debug_slots(ctx, (int)value);
+    case WM_DEBUG_SOLVE_FAILS: return ctx->solve_fails = (int)value;
+    default: return -1;
+  }
 }
 
 }  // extern "C"

@@ -899,7 +899,12 @@ int wm_field_launch(wm_ctx *ctx) {
   for (int l = 0; l < 3; ++l) ctx->fcg_it[l] = 0;
   if (fcg || !tiles) WM_TRY(rhs(ctx));
   if (fcg) WM_TRY(fcg_solve(ctx, cg_args(ctx), ctx->fcg_it));
-  if (tiles) return wm_k_tiles(ctx, !fcg);
+  if (tiles) {
+    bool ran = false;
+    WM_TRY(wm_k_tiles(ctx, !fcg, &ran));
+    if (ran) return WM_OK;
+    if (!fcg) WM_TRY(rhs(ctx));
+  }
   WM_TRY(stream_plain(ctx));
   hipLaunchKernelGGL(k_stamp, dim3(1), dim3(1), 0, ctx->stream, ctx->ts, 4);
   WM_HIP(hipGetLastError());
@@ -943,14 +948,14 @@ int wm_field_result(wm_ctx *ctx) {
 }
 
 int wm_k_field_solve(wm_ctx *ctx) {
+  struct Scope {                                 // what the solve holds, on every way out
+    wm_ctx *c;
+    ~Scope() { wm_field_release(c); }
+  } scope{ctx};
   WM_TRY(wm_field_launch(ctx));
-  int st = wm_field_update(ctx);
-  if (st == WM_OK) {
-    WM_HIP(hipStreamSynchronize(ctx->stream));
-    st = wm_field_result(ctx);
-  }
-  wm_field_release(ctx);
-  return st;
+  WM_TRY(wm_field_update(ctx));
+  WM_HIP(hipStreamSynchronize(ctx->stream));
+  return wm_field_result(ctx);
 }
 
 // The deposit tiles (chunks of CHUNK cells, halo 2, [row][chunk][5][CHUNK +

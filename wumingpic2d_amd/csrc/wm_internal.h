@@ -313,6 +313,7 @@ struct wm_ctx {
   int ncu = 0;                   // the device's CUs
   int tile_rest = 0;             // solves to stream after one that gave up
   int tile_held = 0;             // workgroups in flight (SolveSlots)
+  int solve_fails = 0;           // on-chip launches to fail (wm_debug.h)
   bool tile_swapped = false;     // uf and uf2 were exchanged for the update in flight
   bool x0_fresh = false;         // cg_x0 holds df's solution planes (the warm start)
   wm_pc *pc = nullptr;
@@ -352,7 +353,7 @@ void wm_field_release(wm_ctx *ctx);  // after an error: waits for the solve in f
 int wm_k_field_solve(wm_ctx *ctx);
 // wm_solve.hip: the on-chip solve and, for the periodic box, its update
 bool wm_tiles_fit(wm_ctx *ctx, bool peek = false);
-int wm_k_tiles(wm_ctx *ctx, bool begins);
+int wm_k_tiles(wm_ctx *ctx, bool begins, bool *ran);
 int wm_report_wait(wm_ctx *ctx);
 bool wm_fused_update(const wm_ctx *ctx);
 int wm_k_update_report(wm_ctx *ctx);  // periodic; else the report alone

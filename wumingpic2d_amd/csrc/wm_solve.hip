@@ -40,6 +40,7 @@
 #include <mutex>
 
 #include "wm_internal.h"
+#include "wm_debug.h"
 #include "wm_solve.h"
 
 namespace {
@@ -626,6 +627,9 @@ __global__ void k_report(const int *abort_, const SolveOut *out, const int *derr
 
 SolveReport *report_of(wm_ctx *ctx) { return (SolveReport *)((char *)ctx->h_pin + WM_PIN_REPORT); }
 
+// How long a solve waits for others of this process to end before it streams.
+constexpr auto SLOT_WAIT = std::chrono::seconds(1);
+
 Plan plan_of(const wm_ctx *ctx) {
   const XSide X = wm_xside(ctx);
   return make_plan(X.xb - X.xa + 1, ctx->g.ny, ctx->ncu);
@@ -662,9 +666,12 @@ bool wm_tiles_fit(wm_ctx *ctx, bool peek) {
   return plan_of(ctx).R > 0;
 }
 
-int wm_k_tiles(wm_ctx *ctx, bool begins) {
+// *ran: false where other contexts' solves hold too much of the device for too
+// long (nothing is launched then).
+int wm_k_tiles(wm_ctx *ctx, bool begins, bool *ran) {
   const Plan p = plan_of(ctx);
   const size_t n = (size_t)p.workgroups();
+  *ran = false;
   if (n > ctx->tile_cap) {
     if (ctx->tile_sums) (void)hipFree(ctx->tile_sums);
     if (ctx->tile_edges) (void)hipFree(ctx->tile_edges);
@@ -708,9 +715,14 @@ int wm_k_tiles(wm_ctx *ctx, bool begins) {
   {
     Slots &s = slots[ctx->device];
     std::unique_lock<std::mutex> lk(s.m);
-    s.cv.wait(lk, [&] { return s.used + (int)n <= ctx->ncu; });
+    if (!s.cv.wait_for(lk, SLOT_WAIT, [&] { return s.used + (int)n <= ctx->ncu; })) return WM_OK;
     s.used += (int)n;
     ctx->tile_held = (int)n;
+  }
+  if (ctx->solve_fails > 0) {
+    --ctx->solve_fails;
+    wm_set_error(ctx, WM_ERR_HIP, "the field solve's launch failed");
+    return WM_ERR_HIP;
   }
   hipLaunchKernelGGL(k_tile_start, dim3(wm_cdiv((long long)ctx->g.nx * ctx->g.ny, 256), 3),
                      dim3(256), 0, ctx->stream, A);
@@ -720,6 +732,7 @@ int wm_k_tiles(wm_ctx *ctx, bool begins) {
     default: launch_tiles<16>(p, A, ctx->stream); break;
   }
   WM_HIP(hipGetLastError());
+  *ran = true;
   return WM_OK;
 }
 
@@ -800,4 +813,16 @@ void wm_field_release(wm_ctx *ctx) {
     ctx->tile_swapped = false;
   }
   release(ctx);
+}
+
+long long wm_debug_slots(wm_ctx *ctx, int add) {
+  if (ctx->device < 0 || ctx->device >= MAX_DEV) return -1;
+  Slots &s = slots[ctx->device];
+  long long used;
+  {
+    std::lock_guard<std::mutex> lk(s.m);
+    used = s.used += add;
+  }
+  if (add < 0) s.cv.notify_all();
+  return used;
 }
