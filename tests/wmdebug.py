@@ -3,6 +3,8 @@ import ctypes
 
 SOLVE_SLOTS = 1      # CUs held by solves in flight on the device; value is added
 SOLVE_FAILS = 2      # on-chip solves that fail to launch
+SOLVE_GIVES_UP = 3   # on-chip solves that wait for nothing and give up
+SOLVE_REST = 4       # solves to come that stream (-1 ends that)
 
 
 def debug(ctx, key, value=0):

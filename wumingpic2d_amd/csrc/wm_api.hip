@@ -1647,6 +1647,8 @@ long long wm_debug(wm_ctx *ctx, int key, long long value) {
   switch (key) {
     case WM_DEBUG_SOLVE_SLOTS: return wm_debug_slots(ctx, (int)value);
     case WM_DEBUG_SOLVE_FAILS: return ctx->solve_fails = (int)value;
+    case WM_DEBUG_SOLVE_GIVES_UP: return ctx->solve_gives_up = (int)value;
+    case WM_DEBUG_SOLVE_REST: return value == -1 ? ctx->tile_rest = 0 : ctx->tile_rest;
     default: return -1;
   }
 }

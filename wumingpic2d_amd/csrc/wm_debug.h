@@ -11,6 +11,10 @@ enum {
   WM_DEBUG_SOLVE_SLOTS = 1,
   // the next value on-chip solves fail to launch
   WM_DEBUG_SOLVE_FAILS = 2,
+  // the next value on-chip solves wait for nothing and are taken to have given up
+  WM_DEBUG_SOLVE_GIVES_UP = 3,
+  // solves to come that stream; value -1 ends that
+  WM_DEBUG_SOLVE_REST = 4,
 };
 
 // The quantity, after value has been put in place; -1 for an unknown key.

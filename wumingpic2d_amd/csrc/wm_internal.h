@@ -311,9 +311,11 @@ struct wm_ctx {
   int *tile_abort = nullptr;
   void *tile_out = nullptr;
   int ncu = 0;                   // the device's CUs
-  int tile_rest = 0;             // solves to stream after one that gave up
-  int tile_held = 0;             // workgroups in flight (SolveSlots)
-  int solve_fails = 0;           // on-chip launches to fail (wm_debug.h)
+  int tile_rest = 0;             // solves to stream after one that gave up,
+  int tile_rest_next = 0;        // and after the next that does
+  int tile_held = 0;             // workgroups in flight (wm_solve.hip's Slots)
+  int solve_fails = 0;           // on-chip launches to fail, solves to give up
+  int solve_gives_up = 0;        // (wm_debug.h)
   bool tile_swapped = false;     // uf and uf2 were exchanged for the update in flight
   bool x0_fresh = false;         // cg_x0 holds df's solution planes (the warm start)
   wm_pc *pc = nullptr;

@@ -27,10 +27,13 @@
 //
 // Every workgroup has to run at the same time as the others.  The launch has
 // at most as many as the device has CUs, contexts of this process share that
-// number (SolveSlots), and whatever else occupies the CUs ends without waiting
-// for this kernel.  Should they still not meet within a second (another
-// process on the same GPU), the kernel gives up, leaves phi as it was, and the
-// host runs the streaming solver.
+// number (Slots), and whatever else occupies the CUs ends without waiting
+// for this kernel.  Should they still not meet within a tenth of a second
+// (another process on the same GPU, say), the kernel gives up and the host runs
+// the streaming solver, from whatever df holds by then: the old change, or the
+// new one where a component or a workgroup had come to its end.  The solves
+// after it stream, a thousand the first time and twice as many each further
+// time, so that what the waits cost stays below what the streaming does.
 //
 // Bound by the exchanges: about 4 us an iteration at 256 x 64 (40 us a solve of
 // 7), of which the sweeps are 1.6; at 1024 x 1024 by the sweeps of 16 rows a
@@ -47,7 +50,8 @@ namespace {
 
 constexpr int NTH = 512;          // threads of a workgroup: 8 wavefronts
 constexpr int TXC = 128;          // columns of a tile that has others beside it
-constexpr long long PATIENCE = 100000000;   // ticks of the 100 MHz clock: 1 s
+constexpr long long PATIENCE_MS = 100;
+constexpr int REST_FIRST = 1000, REST_MOST = 1 << 30;   // solves to stream after giving up
 
 typedef unsigned long long u64;
 
@@ -138,7 +142,9 @@ struct SArgs {
   double *b, *r;                  // f5 gkl and the initial residual, nx x ny planes
   u64 *sums, *edges;              // [group][2][W][8 words], [group][2][W][512][2 words]
   unsigned tag0;
+  long long patience;             // of a wait, in ticks of the clock
   int *abort_;
+  int abort0;                     // what it begins with
   SolveOut *out;
   unsigned long long *ts;
   bool stamp;                     // the solve begins here
@@ -180,11 +186,13 @@ __device__ inline double phi_at(const SArgs &A, int l, int a, int b, int wx) {
   return s * A.df[(size_t)l * A.fg.ps + (size_t)(A.X.xa + a + 2) + (size_t)A.fg.gx * (size_t)(b + 2)];
 }
 
-// b = f5 gkl and r = b - A phi (field.f90:350-385) of every active cell.
+// b = f5 gkl and r = b - A phi (field.f90:350-385) of every active cell; also
+// clears the mark of a solve that gave up.
 __global__ __launch_bounds__(256) void k_tile_start(SArgs A) {
   const int t = blockIdx.x * 256 + threadIdx.x, l = blockIdx.y;
   const int nx = A.fg.nx, n = nx * A.fg.ny;
   if (A.stamp) wm_stamp(A.ts, 3);
+  if (t == 0 && l == 0) *A.abort_ = A.abort0;
   if (t >= n) return;
   const int ii = t % nx, jj = t / nx;
   if (ii < A.X.xa || ii > A.X.xb) return;
@@ -251,7 +259,7 @@ __global__ __launch_bounds__(NTH) void k_cg_tiles(SArgs A) {
   const u64 *hsrc = edges + ((size_t)nb * 512 + (side ^ 1) * 128 + at) * 2;
   u64 *mine = edges + (size_t)me * 1024;
   const size_t ebuf = (size_t)W * 1024, sbuf = (size_t)W * 8;
-  const Wait wait{A.abort_, (long long)wall_clock64() + PATIENCE};
+  const Wait wait{A.abort_, (long long)wall_clock64() + A.patience};
   unsigned ex = 0;                // exchanges so far
   const double f4 = A.f.f4;
 
@@ -686,7 +694,6 @@ int wm_k_tiles(wm_ctx *ctx, bool begins, bool *ran) {
   if (!ctx->tile_abort) {
     WM_HIP(hipMalloc((void **)&ctx->tile_abort, sizeof(int)));
     WM_HIP(hipMalloc(&ctx->tile_out, sizeof(SolveOut)));
-    WM_HIP(hipMemsetAsync(ctx->tile_abort, 0, sizeof(int), ctx->stream));
     WM_HIP(hipMemsetAsync(ctx->tile_out, 0, sizeof(SolveOut), ctx->stream));
   }
   SArgs A;
@@ -708,7 +715,11 @@ int wm_k_tiles(wm_ctx *ctx, bool begins, bool *ran) {
   if (ctx->tile_tag > 0xFFFFFFFFu - need) ctx->tile_tag = 1;
   A.tag0 = ctx->tile_tag;
   ctx->tile_tag += need;
+  const bool forced = ctx->solve_gives_up > 0;
+  if (forced) --ctx->solve_gives_up;
+  A.patience = forced ? 0 : PATIENCE_MS * ctx->clock_khz;
   A.abort_ = ctx->tile_abort;
+  A.abort0 = forced;
   A.out = (SolveOut *)ctx->tile_out;
   A.ts = ctx->ts;
   A.stamp = begins;
@@ -797,9 +808,8 @@ int wm_tiles_result(wm_ctx *ctx, bool *gave_up, int *err, int *ite) {
   if ((*gave_up || *err) && ctx->tile_swapped) std::swap(ctx->uf, ctx->uf2);
   ctx->tile_swapped = false;
   if (*gave_up) {
-    ctx->tile_rest = 1000;
-    WM_HIP(hipMemsetAsync(ctx->tile_abort, 0, sizeof(int), ctx->stream));
-    WM_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->tile_rest = std::max(REST_FIRST, ctx->tile_rest_next);
+    ctx->tile_rest_next = std::min(2 * (long long)ctx->tile_rest, (long long)REST_MOST);
   }
   return WM_OK;
 }
