@@ -564,16 +564,17 @@ __device__ inline void cell_coeffs(double *cf, const double *Tk) {
 
 // 1 / sqrt(a), a > 0 normal: the hardware's estimate (to about 2^-23) and two
 // Newton steps in FMAs, within an ulp.  Where a has overflowed (a momentum above
-// 1e154) the estimate is zero, as the quotient is, and stays so: its corrections
-// are no numbers, of which fmax takes the other argument.
+// 1e154) the estimate is zero, as the quotient is; the steps, on the largest
+// number instead, leave it there.
 __device__ inline double rsqrt64(double a) {
   double y = __builtin_amdgcn_rsq(a);
+  a = fmin(a, 0x1.fffffffffffffp1023);
   double h = 0.5 * y;
-  double e = fmax(fma(-a * y, h, 0.5), -0.5);   // 1/2 - a y^2 / 2
+  double e = fma(-a * y, h, 0.5);      // 1/2 - a y^2 / 2
   y = fma(y, e, y);
   h = 0.5 * y;
   const double g = a * y;              // sqrt(a) to twice the estimate's bits
-  e = fmax(fma(-g, h, 0.5), -0.5);
+  e = fma(-g, h, 0.5);
   return fma(y, e, y);
 }
 
@@ -600,7 +601,7 @@ __device__ inline PushOut boris_coeffs(const double2 *cf, double ox, double oy, 
   double uvm3 = uz + fac1 * epz;
   const double g2 = P.c * P.c + uvm1 * uvm1 + uvm2 * uvm2 + uvm3 * uvm3;
   const double igam = rsqrt64(g2);
-  const double g1 = g2 * igam;
+  const double g1 = g2 * igam;         // (no number where g2 is infinite, as the root is)
   const double gam = fmin(fma(fma(-g1, g1, g2), 0.5 * igam, g1), INFINITY);   // sqrt(g2)
   const double fac1r = fac1 * igam;
   const double fac2r = fac2 / (gam + txxx * (bpx * bpx + bpy * bpy + bpz * bpz) * igam);
