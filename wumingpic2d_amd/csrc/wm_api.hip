@@ -1649,6 +1649,7 @@ long long wm_debug(wm_ctx *ctx, int key, long long value) {
     case WM_DEBUG_SOLVE_FAILS: return ctx->solve_fails = (int)value;
     case WM_DEBUG_SOLVE_GIVES_UP: return ctx->solve_gives_up = (int)value;
     case WM_DEBUG_SOLVE_REST: return value == -1 ? ctx->tile_rest = 0 : ctx->tile_rest;
+    case WM_DEBUG_SOLVE_TAG: return value ? ctx->tile_tag = (unsigned)value : ctx->tile_tag;
     default: return -1;
   }
 }

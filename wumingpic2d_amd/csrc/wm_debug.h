@@ -15,6 +15,8 @@ enum {
   WM_DEBUG_SOLVE_GIVES_UP = 3,
   // solves to come that stream; value -1 ends that
   WM_DEBUG_SOLVE_REST = 4,
+  // the next on-chip solve's first tag, if value is not 0
+  WM_DEBUG_SOLVE_TAG = 5,
 };
 
 // The quantity, after value has been put in place; -1 for an unknown key.

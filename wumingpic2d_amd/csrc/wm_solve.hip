@@ -712,7 +712,13 @@ int wm_k_tiles(wm_ctx *ctx, bool begins, bool *ran) {
   A.sums = ctx->tile_sums;
   A.edges = ctx->tile_edges;
   const unsigned need = 3u * (unsigned)(ctx->ite_max + 4);
-  if (ctx->tile_tag > 0xFFFFFFFFu - need) ctx->tile_tag = 1;
+  if (ctx->tile_tag > 0xFFFFFFFFu - need) {
+    // the tags begin again: words that still carry one of them must not pass
+    // for this solve's
+    WM_HIP(hipMemsetAsync(ctx->tile_sums, 0, sizeof(u64) * ctx->tile_cap * 2 * 8, ctx->stream));
+    WM_HIP(hipMemsetAsync(ctx->tile_edges, 0, sizeof(u64) * ctx->tile_cap * 2 * 1024, ctx->stream));
+    ctx->tile_tag = 1;
+  }
   A.tag0 = ctx->tile_tag;
   ctx->tile_tag += need;
   const bool forced = ctx->solve_gives_up > 0;
