@@ -6,6 +6,7 @@ SOLVE_FAILS = 2      # on-chip solves that fail to launch
 SOLVE_GIVES_UP = 3   # on-chip solves that wait for nothing and give up
 SOLVE_REST = 4       # solves to come that stream (-1 ends that)
 SOLVE_TAG = 5        # the next on-chip solve's first tag (if not 0)
+PLANE32 = 6          # largest plane the FP64 push addresses in 32 bits (if not 0)
 
 
 def debug(ctx, key, value=0):

@@ -1650,6 +1650,9 @@ long long wm_debug(wm_ctx *ctx, int key, long long value) {
     case WM_DEBUG_SOLVE_GIVES_UP: return ctx->solve_gives_up = (int)value;
     case WM_DEBUG_SOLVE_REST: return value == -1 ? ctx->tile_rest = 0 : ctx->tile_rest;
     case WM_DEBUG_SOLVE_TAG: return value ? ctx->tile_tag = (unsigned)value : ctx->tile_tag;
+    case WM_DEBUG_PLANE32:
+      if (value > 0 && value <= 1LL << 29) ctx->plane32 = (size_t)value;
+      return (long long)ctx->plane32;
     default: return -1;
   }
 }

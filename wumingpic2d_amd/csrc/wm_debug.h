@@ -17,6 +17,9 @@ enum {
   WM_DEBUG_SOLVE_REST = 4,
   // the next on-chip solve's first tag, if value is not 0
   WM_DEBUG_SOLVE_TAG = 5,
+  // slots of the largest species plane the FP64 push addresses by 32-bit byte
+  // offsets, if value is not 0
+  WM_DEBUG_PLANE32 = 6,
 };
 
 // The quantity, after value has been put in place; -1 for an unknown key.

@@ -196,6 +196,7 @@ struct wm_ctx {
   bool perm_valid = false;
   long long npart = 0;           // particles of the resident state (their number stays)
   unsigned *perm = nullptr;      // [nseg*cap]
+  size_t plane32 = (size_t)1 << 29;   // slots of a plane below 4 GB an array (wm_debug.h)
   uint16_t *code = nullptr;      // [nseg*cap] the push's code per particle (wm_order.h)
   int4 *kind = nullptr;          // [nseg*nx] moves out of a cell by kind
   int *farcnt = nullptr, *far = nullptr;   // [nseg*nx], [nseg]; zero between steps

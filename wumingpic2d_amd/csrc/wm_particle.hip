@@ -1214,7 +1214,7 @@ int wm_k_push_step(wm_ctx *ctx) {
   const Order O{ctx->perm, ctx->code, ctx->kind, ctx->farcnt, ctx->far};
   // a species' plane below 4 GB is addressed by 32-bit byte offsets
   const int src = !ctx->perm_valid                          ? SRC_SLOT
-                  : (size_t)P.ny * P.cap <= (size_t)1 << 29 ? SRC_PERM32
+                  : (size_t)P.ny * P.cap <= ctx->plane32    ? SRC_PERM32
                                                             : SRC_PERM64;
   // Lanes of a cell: steps of 16 waste lanes on few particles, steps of 8 take
   // the longer over many, and over the dense cells of a small grid whose
