@@ -7,6 +7,7 @@ SOLVE_GIVES_UP = 3   # on-chip solves that wait for nothing and give up
 SOLVE_REST = 4       # solves to come that stream (-1 ends that)
 SOLVE_TAG = 5        # the next on-chip solve's first tag (if not 0)
 PLANE32 = 6          # largest plane the FP64 push addresses in 32 bits (if not 0)
+XFER_BUFFERS = 7     # pinned buffers of the host arrays' copies
 
 
 def debug(ctx, key, value=0):

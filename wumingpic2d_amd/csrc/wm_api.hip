@@ -1653,6 +1653,7 @@ long long wm_debug(wm_ctx *ctx, int key, long long value) {
     case WM_DEBUG_PLANE32:
       if (value > 0 && value <= 1LL << 29) ctx->plane32 = (size_t)value;
       return (long long)ctx->plane32;
+    case WM_DEBUG_XFER_BUFFERS: return wm_xfer_buffers(ctx);
     default: return -1;
   }
 }

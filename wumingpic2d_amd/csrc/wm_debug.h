@@ -20,6 +20,8 @@ enum {
   // slots of the largest species plane the FP64 push addresses by 32-bit byte
   // offsets, if value is not 0
   WM_DEBUG_PLANE32 = 6,
+  // pinned buffers of the host arrays' copies
+  WM_DEBUG_XFER_BUFFERS = 7,
 };
 
 // The quantity, after value has been put in place; -1 for an unknown key.

@@ -27,6 +27,7 @@ int wm_to_host(wm_ctx *ctx, const void *dev, void *host, size_t bytes);
 // device works.
 void wm_touch(void *host, size_t bytes);
 void wm_xfer_free(wm_ctx *ctx);
+int wm_xfer_buffers(const wm_ctx *ctx);   // pinned buffers it has
 
 // Component 6 of the records from[s] .. np - 1 of every row s (np records).
 void wm_copy_field6(double *dst, const double *src, const int *from, size_t np, int nrow);

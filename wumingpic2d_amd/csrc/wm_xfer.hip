@@ -9,10 +9,9 @@
 // pages are touched while its piece is on the way.  202 MB of fields: 11.7 ->
 // 4.7 ms; pieces of 1 MB took 7.0, of 2 MB 5.3.  Arrays below 64 MB go in pieces
 // of up to 2 MB, the 30 MB of moments as fast as in pieces of 4 MB (2.04 and 2.03
-// ms a call) and a context's first call, which makes the buffers, faster (3.15
-// and 3.9 ms).  Arrays below 8 MB, by one thread, go in pieces of 1 MB: a buffer
-// takes 0.08 ms to make, one of 2 MB 0.33, and laying out a state of 192000
-// particles 11.6 ms instead of 13.1; later copies take as long.
+// ms a call; 1 MB: 1.75 where 2 MB take 1.53 on a grid of 4 per cell).  Arrays
+// below 8 MB, by one thread, go in pieces of 1 MB, whose two buffers take half as
+// long to make; later copies take as long.
 //
 // Rows of particles are gathered from and scattered to the caller's arrays in
 // the same pass; they used to go through a vector of the whole state, zeroed,
@@ -46,6 +45,13 @@ int threads_for(size_t bytes) {
   return bytes < ALONE ? 1 : (int)std::min<size_t>(WORKERS, bytes / SHARE);
 }
 
+// The buffers a copy may make anew.  One takes 0.05 to 0.15 ms and the process
+// makes one at a time, so eight of them cost a context's first copies more than
+// eight threads save: 9 MB of particles, first copy of a context, 1.08 ms by the
+// runtime's staging, 1.56 with eight new buffers and 1.08 with two (then two more
+// a call); 29 MB 2.5, 2.3 and 1.9 ms; later copies are the same.
+int new_buffers(size_t bytes) { return (int)std::max<size_t>(2, bytes >> 24); }
+
 // f(worker) on `n` threads, the caller's as worker 0; fewer if the system
 // gives no more.
 template <class F>
@@ -76,6 +82,13 @@ void wm_xfer_free(wm_ctx *ctx) {
   }
   delete ctx->xfer;
   ctx->xfer = nullptr;
+}
+
+int wm_xfer_buffers(const wm_ctx *ctx) {
+  int n = 0;
+  if (ctx->xfer)
+    for (size_t s : ctx->xfer->size) n += s > 0;
+  return n;
 }
 
 namespace {
@@ -119,12 +132,13 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
   if (total == 0) return WM_OK;
   if (!ctx->xfer) ctx->xfer = new wm_xfer;
   wm_xfer &x = *ctx->xfer;
-  const int want = threads_for(total);
-  // one thread alone has two buffers, and copies a chunk while the next is on
-  // its way
   const size_t slot = slot_for(total);
-  const size_t most =
-      std::min(slot, std::max<size_t>(total / (want > 1 ? want : 3) + rec, (size_t)1 << 20)) / rec * rec;
+  int have = 0;
+  for (size_t s : x.size) have += s >= slot;
+  const int want = std::min(threads_for(total), have + new_buffers(total));
+  // (one thread alone has two buffers, and copies a chunk while the next is on
+  // its way)
+  const size_t most = std::min(slot, std::max<size_t>(total / want + rec, (size_t)1 << 20)) / rec * rec;
   std::vector<WmSpan> piece;
   std::vector<Chunk> chunk;
   for (const WmSpan &s : spans)
