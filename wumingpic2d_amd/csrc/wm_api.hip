@@ -1481,7 +1481,6 @@ int wm_moments(wm_ctx *ctx, double *mom) {
     return WM_ERR_NOT_INIT;
   }
   if (ctx->form == WM_FORM_FP32) WM_TRY(wm_settle_movers(ctx));
-  WM_TRY(wm_order_apply(ctx));
   hipEvent_t *e = ctx->ev + 20;
   WM_HIP(hipEventRecord(e[0], ctx->stream));
   WM_TRY(wm_k_moments(ctx, true));

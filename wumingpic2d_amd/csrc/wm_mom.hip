@@ -52,7 +52,27 @@ struct Src64 {
     ke = min(P.cap, cc[i + 1]);
     base = seg * (size_t)P.cap;
   }
+  static constexpr bool INDEXED = false;
   __device__ Pt load(size_t p, int, int) const { return Pt{x[p], y[p], ux[p], uy[p], uz[p]}; }
+};
+
+// The same between steps of the resident run, while the rows' order is an index
+// into the species' planes (wm_order.hip).  Putting the rows in order first, as
+// every other reader of whole rows does, moves 120 bytes a particle: a call after
+// a step 1.93 ms at 512 x 512 with 64 per cell and species, 2.78 with that and 1.91
+// where the rows lie in order (the index costs the kernel 0.64 to 0.62 ms).
+struct Order64 {
+  Src64 s;
+  const unsigned *perm;
+  size_t plane;                  // slots of a species' plane
+  size_t seg0 = 0;               // the plane of the species at hand
+  static constexpr bool INDEXED = true;
+  __device__ void range(const MP &P, int sp, int jl, int i, size_t &base, int &kb, int &ke) {
+    seg0 = sp * plane;
+    s.range(P, sp, jl, i, base, kb, ke);
+  }
+  __device__ unsigned at(size_t p) const { return perm[p]; }
+  __device__ Pt load(unsigned q, int i, int j) const { return s.load(seg0 + q, i, j); }
 };
 
 // FP32 form: the cell's bin.  The position is the cell's index plus the
@@ -68,6 +88,7 @@ struct Src32 {
     ke = cnt[seg * P.nx + i];
     base = seg * (size_t)P.cap + bstart[seg * (P.nx + 1) + i];
   }
+  static constexpr bool INDEXED = false;
   __device__ Pt load(size_t p, int iabs, int jabs) const {
     const float4 v = q[p];
     return Pt{(double)iabs + (double)v.x, (double)jabs + (double)v.y, (double)v.z, (double)v.w,
@@ -271,14 +292,25 @@ __global__ __launch_bounds__(MC * MG, 4) void k_mom(MP P, FieldGeom fg,
       double C[9];
       if (ACCL) coeffs(C, F + (min(sub, 5) * MH + rl) * MW + g);
       // rounds of sixteen particles, one per lane; the next round's particle
-      // is loaded while this one is computed
+      // is loaded while this one is computed, and where the one after that is
       int k = kb + sub;
       Pt nxt{0, 0, 0, 0, 0};
-      if (k < ke) nxt = src.load(base + (size_t)k, iabs, jabs);
+      unsigned at = 0;
+      if constexpr (S::INDEXED) {
+        if (k < ke) nxt = src.load(src.at(base + (size_t)k), iabs, jabs);
+        if (k + MG < ke) at = src.at(base + (size_t)(k + MG));
+      } else {
+        if (k < ke) nxt = src.load(base + (size_t)k, iabs, jabs);
+      }
       for (int k0 = kb; __ballot(k0 < ke) != 0ULL; k0 += MG, k += MG) {
         const Pt v = nxt;
         const bool live = k < ke;
-        if (k + MG < ke) nxt = src.load(base + (size_t)(k + MG), iabs, jabs);
+        if constexpr (S::INDEXED) {
+          if (k + MG < ke) nxt = src.load(at, iabs, jabs);
+          if (k + 2 * MG < ke) at = src.at(base + (size_t)(k + 2 * MG));
+        } else {
+          if (k + MG < ke) nxt = src.load(base + (size_t)(k + MG), iabs, jabs);
+        }
         double ux = v.ux, uy = v.uy, uz = v.uz;
         if (ACCL) {
           const double ox = v.x * P.d_delx - iabs, oy = v.y * P.d_delx - jabs;
@@ -469,7 +501,10 @@ int wm_k_moments(wm_ctx *ctx, bool accl) {
   } else {
     const PBank &A = ctx->bank[0];
     const Src64 src{A.x, A.y, A.ux, A.uy, A.uz, ctx->cumcnt};
-    if (accl)
+    if (accl && ctx->perm_valid)
+      WM_TRY((launch_mom<Order64, true>(
+          ctx, P, Order64{src, ctx->perm, (size_t)ctx->g.ny * ctx->cap})));
+    else if (accl)
       WM_TRY((launch_mom<Src64, true>(ctx, P, src)));
     else
       WM_TRY((launch_mom<Src64, false>(ctx, P, src)));
