@@ -1,6 +1,6 @@
-"""A context's first copies make two pinned buffers a call (one for each 16 MB of
-larger arrays), later ones as many more until eight threads have one each; what
-they copy is right at every number of them."""
+"""A context's first copies make two pinned buffers (from 16 MB on one for each 4 MB
+beyond 8 MB), later ones of such arrays more until eight threads have one each;
+what they copy is right at every number of them."""
 import numpy as np
 import pytest
 
@@ -11,12 +11,12 @@ from wmhelpers import bits, make_ctx, state
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,ny,ppc,most", [
-    (250, 24, 20, 2),            # 11.5 MB of particles, then small arrays
-    (600, 500, 1, 4),            # 29 MB of particles, 15 MB of fields
-    (1500, 1203, 1, 13),         # 173 MB and 87 MB: ten and five at once
+@pytest.mark.parametrize("nx,ny,ppc,first,end", [
+    (250, 24, 20, 2, 2),         # 11 MB of particles, then small arrays
+    (600, 500, 1, 4, 8),         # 27.5 MB of particles, 14 MB of fields
+    (1500, 1203, 1, 8, 8),       # 165 MB
 ])
-def test_buffers_grow_with_the_calls(nx, ny, ppc, most):
+def test_buffers_grow_with_the_calls(nx, ny, ppc, first, end):
     p, up, np2, cc, uf = state(nx, ny, ppc, 96, vth=0.2)
     uf[...] = np.random.default_rng(96).normal(size=uf.shape)
     ctx = make_ctx(p, form=wm.FORM_FP64)
@@ -26,7 +26,7 @@ def test_buffers_grow_with_the_calls(nx, ny, ppc, most):
         n = debug(ctx, XFER_BUFFERS)
         assert last <= n <= 8
         if call == 0:
-            assert n <= most
+            assert n == first
         last = n
         got = [np.zeros_like(a) for a in (up, np2, cc, uf)]
         ctx.state_download(*got)
@@ -35,4 +35,4 @@ def test_buffers_grow_with_the_calls(nx, ny, ppc, most):
             for jl in range(0, ny, 7):
                 m = np2[jl, s]
                 assert np.array_equal(bits(up[:, :m, jl, s]), bits(got[0][:, :m, jl, s]))
-    assert last == 8
+    assert last == end

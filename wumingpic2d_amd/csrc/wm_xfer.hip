@@ -6,12 +6,13 @@
 // 1.8 ms (2.9 into fresh pages), of which the link needs 0.56.  Here up to
 // eight threads each own a pinned buffer and take pieces of the array in turn:
 // while one waits for its piece the others copy theirs, and a destination's
-// pages are touched while its piece is on the way.  202 MB of fields: 11.7 ->
-// 4.7 ms; pieces of 1 MB took 7.0, of 2 MB 5.3.  Arrays below 64 MB go in pieces
-// of up to 2 MB, the 30 MB of moments as fast as in pieces of 4 MB (2.04 and 2.03
-// ms a call; 1 MB: 1.75 where 2 MB take 1.53 on a grid of 4 per cell).  Arrays
-// below 8 MB, by one thread, go in pieces of 1 MB, whose two buffers take half as
-// long to make; later copies take as long.
+// pages are touched while its piece is on the way.  202 MB of fields in pieces of
+// 4 MB: 11.7 -> 4.7 ms.  Arrays below 64 MB go up in pieces of 2 MB (58 MB 1.9 ms,
+// by the runtime 14.7) and down in pieces of 1 MB, as fast as 2 MB and the buffers
+// made sooner: 30 MB of moments on 512 x 512 with 64 per cell and species, a
+// context's first call 2.7 ms, later ones 1.9; by the runtime 3.1 and 2.95, with
+// eight buffers of 2 MB and the runtime's copies 3.4 and, by turns, 2.0 and 3.6.
+// Arrays below 8 MB go by one thread with two buffers of 1 MB.
 //
 // Rows of particles are gathered from and scattered to the caller's arrays in
 // the same pass; they used to go through a vector of the whole state, zeroed,
@@ -23,6 +24,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <numeric>
 #include <system_error>
 #include <thread>
 
@@ -31,9 +33,9 @@
 
 namespace {
 // The largest piece of a copy, and the size of the buffers it needs.
-size_t slot_for(size_t bytes) {
+size_t slot_for(size_t bytes, bool up) {
   constexpr size_t MB = (size_t)1 << 20;
-  return bytes < 8 * MB ? MB : bytes < 64 * MB ? 2 * MB : 4 * MB;
+  return bytes < 8 * MB ? MB : bytes < 64 * MB ? (up ? 2 * MB : MB) : 4 * MB;
 }
 constexpr int WORKERS = 8;
 // Threads for a copy: one up to 8 MB, then one per MB.  Starting one costs
@@ -45,12 +47,15 @@ int threads_for(size_t bytes) {
   return bytes < ALONE ? 1 : (int)std::min<size_t>(WORKERS, bytes / SHARE);
 }
 
-// The buffers a copy may make anew.  One takes 0.05 to 0.15 ms and the process
-// makes one at a time, so eight of them cost a context's first copies more than
-// eight threads save: 9 MB of particles, first copy of a context, 1.08 ms by the
-// runtime's staging, 1.56 with eight new buffers and 1.08 with two (then two more
-// a call); 29 MB 2.5, 2.3 and 1.9 ms; later copies are the same.
-int new_buffers(size_t bytes) { return (int)std::max<size_t>(2, bytes >> 24); }
+// The buffers a copy may make anew, beyond two.  One of 1 MB takes 0.05 to 0.15
+// ms, and the process makes one at a time, so that eight cost a context's first
+// copies of a few MB more than eight threads save: a state of 9 MB goes up in
+// 1.4 ms by the runtime's staging, 1.8 with eight new buffers, 1.1 with two.  Two
+// serve it as well as eight, later too.
+int new_buffers(size_t bytes) {
+  constexpr size_t MB = (size_t)1 << 20;
+  return bytes < 16 * MB ? 0 : (int)((bytes - 8 * MB) >> 22);
+}
 
 // f(worker) on `n` threads, the caller's as worker 0; fewer if the system
 // gives no more.
@@ -104,7 +109,7 @@ hipError_t slot_of(wm_xfer &x, int k, size_t size) {
   if (x.pin[k]) e = hipHostFree(x.pin[k]);
   x.pin[k] = nullptr;
   x.size[k] = 0;
-  if (e == hipSuccess) e = hipHostMalloc(&x.pin[k], size, hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc(&x.pin[k], size, hipHostMallocCoherent);
   if (e == hipSuccess) x.size[k] = size;
   return e;
 }
@@ -112,6 +117,34 @@ hipError_t slot_of(wm_xfer &x, int k, size_t size) {
 struct Chunk {
   size_t s0, s1;                            // pieces
 };
+
+// n bytes (both ends on 8-byte boundaries) to a pinned buffer.  Copies that the
+// runtime is asked for while others are on their way go to several DMA engines:
+// making one's queue takes a millisecond of a context's first call, and some
+// move 12 GB/s where others move 41, so that 30 MB took 1.5 ms in two calls of
+// three and 3.1 in the third.  By this kernel 1.4 to 1.6 ms.  (Uploads have shown
+// neither, and from new buffers a kernel reads more slowly than they.)
+__global__ __launch_bounds__(256) void k_to_pinned(const char *src, char *dst, size_t n) {
+  const double *s = (const double *)src;
+  double *d = (double *)dst;
+  const size_t n8 = n / 8, st = (size_t)gridDim.x * 256;
+  size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  for (; i + 3 * st < n8; i += 4 * st) {
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = s[i + k * st];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) d[i + k * st] = v[k];
+  }
+  for (; i < n8; i += st) d[i] = s[i];
+  if (blockIdx.x == 0 && threadIdx.x < n % 8) dst[8 * n8 + threadIdx.x] = src[8 * n8 + threadIdx.x];
+}
+hipError_t to_pinned(char *pin, const char *dev, size_t n, hipStream_t st) {
+  if ((size_t)dev % 8 != 0) return hipMemcpyAsync(pin, dev, n, hipMemcpyDeviceToHost, st);
+  const size_t blocks = std::max<size_t>(1, std::min<size_t>(64, n / 2048));
+  hipLaunchKernelGGL(k_to_pinned, dim3((unsigned)blocks), dim3(256), 0, st, dev, pin, n);
+  return hipGetLastError();
+}
 
 // Has the pages of memory that is about to be written faulted in (their
 // contents stay).
@@ -132,13 +165,14 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
   if (total == 0) return WM_OK;
   if (!ctx->xfer) ctx->xfer = new wm_xfer;
   wm_xfer &x = *ctx->xfer;
-  const size_t slot = slot_for(total);
+  const size_t slot = slot_for(total, up);
   int have = 0;
   for (size_t s : x.size) have += s >= slot;
-  const int want = std::min(threads_for(total), have + new_buffers(total));
+  const int want = std::min(threads_for(total), std::max(2, have + new_buffers(total)));
   // (one thread alone has two buffers, and copies a chunk while the next is on
   // its way)
-  const size_t most = std::min(slot, std::max<size_t>(total / want + rec, (size_t)1 << 20)) / rec * rec;
+  const size_t unit = std::lcm(rec, (size_t)16);
+  const size_t most = std::min(slot, std::max<size_t>(total / want + rec, (size_t)1 << 20)) / unit * unit;
   std::vector<WmSpan> piece;
   std::vector<Chunk> chunk;
   for (const WmSpan &s : spans)
@@ -187,7 +221,7 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
         for (size_t k = h.s0; k < h.s1; ++k) memcpy(pin + (piece[k].at - at), piece[k].host, piece[k].bytes);
         e = hipMemcpyAsync(dev + at, pin, len, hipMemcpyHostToDevice, st);
       } else {
-        e = hipMemcpyAsync(pin, dev + at, len, hipMemcpyDeviceToHost, st);
+        e = to_pinned(pin, dev + at, len, st);
       }
       if (e == hipSuccess) e = hipEventRecord(x.ev[buf], st);
       if (e == hipSuccess && !up) {
