@@ -840,7 +840,9 @@ __global__ __launch_bounds__(PCH * PG, 2) void k_push_step(PP P, const int *__re
                                                       const double *__restrict__ tmp, int TX,
                                                       size_t tps, Rec64 A, Rec64 B, Order O,
                                                       double *__restrict__ part,
-                                                      int *__restrict__ derr) {
+                                                      int *__restrict__ derr,
+                                                      unsigned long long *ts) {
+  wm_stamp(ts, 1);
   constexpr int PTH = PCH * PG;
   constexpr int MLC = PG == 8 ? 23 : 47;       // a cell's listed movers
   __shared__ __attribute__((aligned(16))) double CF[PCH * 6 * CFN];
@@ -1116,7 +1118,6 @@ __global__ void k_cell_fields(FieldGeom fg, const double *__restrict__ uf,
                               double *__restrict__ tmp, int TX, int TY, size_t tps,
                               int *__restrict__ far, int nseg, unsigned long long *ts) {
   wm_stamp(ts, 0);
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) ts[1] = wall_clock64();
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < nseg) far[t] = 0;
   if (t >= TX * TY) return;
@@ -1236,7 +1237,8 @@ int wm_k_push_step(wm_ctx *ctx) {
 #undef WM_PUSH
   P.nchunk = wm_cdiv(P.nx, PCH);
   hipLaunchKernelGGL(kernel, dim3(P.nchunk * P.ny), dim3(PCH * (eight ? 8 : 16)), 0, ctx->stream, P, ctx->cumcnt,
-                     ctx->tmp, TX, tps, ctx->bank[0], ctx->bank[1], O, ctx->dep_part, ctx->derr);
+                     ctx->tmp, TX, tps, ctx->bank[0], ctx->bank[1], O, ctx->dep_part, ctx->derr,
+                     ctx->ts);
   WM_HIP(hipGetLastError());
   std::swap(ctx->bank[0], ctx->bank[1]);
   return WM_OK;

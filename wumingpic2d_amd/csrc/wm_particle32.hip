@@ -644,7 +644,8 @@ __global__ __launch_bounds__(256, 4) void k_push_deposit32(
     PP32 P, const float *__restrict__ tmp, int TX, size_t tps, Bins32 A, int64_t *ids,
     wm_mig::Mig G, Movers Mp, const int *__restrict__ rowpend, Movers M, int *__restrict__ mfill,
     int mrow, Spill X, BinSum *__restrict__ msum, double *__restrict__ part,
-    int *__restrict__ stats, int *__restrict__ derr) {
+    int *__restrict__ stats, int *__restrict__ derr, unsigned long long *ts) {
+  wm_stamp(ts, 1);
   const int chunk = blockIdx.x;
   const int jl = blockIdx.y;
   const int i0 = chunk * CHUNK;                      // cell index relative to nxgs
@@ -887,7 +888,6 @@ __global__ void k_cell_fields32(FieldGeom fg, const double *__restrict__ uf,
                                 int *__restrict__ mfill, int *__restrict__ sfill, int ny,
                                 unsigned long long *ts) {
   wm_stamp(ts, 0);
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) ts[1] = wall_clock64();
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < ny) {
     mfill[t] = 0;
@@ -989,7 +989,7 @@ int wm_k_push_deposit32(wm_ctx *ctx) {
                      ctx->bins, ctx->id_bins, G, ctx->mv[in], ctx->rowpend, ctx->mv[out],
                      ctx->mfill[out], ctx->mrow,
                      Spill{ctx->spill_l, ctx->spill_p, ctx->spill_q, 0, ctx->sfill, ctx->srow / MB},
-                     ctx->bin_sum[out], ctx->dep_part, ctx->fstat, ctx->derr);
+                     ctx->bin_sum[out], ctx->dep_part, ctx->fstat, ctx->derr, ctx->ts);
   WM_HIP(hipGetLastError());
   ctx->mv_last = out;
   ctx->mv_pending = true;
