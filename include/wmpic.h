@@ -220,14 +220,16 @@ int wm_energy(wm_ctx *ctx, double *out);
 /* CG iterations per component (l = 1..3) of the last field solve. */
 int wm_cg_iters(wm_ctx *ctx, int *iters3);
 /* GPU time (ms) of each phase of the last wm_step call, summed over its
- * steps, by the device's clock as the phases' kernels start: [0] cell-centred
- * fields, [1] push+deposit, [2] current gather+fold, [3] field solve; beside
+ * steps, by the device's clock as the phases' kernels start and the last ends:
+ * [0] cell-centred fields, [1] push+deposit, [2] current gather+fold, [3] field
+ * solve and update (not what the update waits for the second stream); beside
  * them, on a second stream, [4] particle boundaries (the rows' leavers and
- * arrivals), [5] sort (every particle's place).  In the FP32 form the push places the last push's
- * movers (the particle boundaries and the sort reduce to that); [4] is the
- * bins' fill check beside the solve and [5] the re-layouts of rows whose
- * bins would overflow.  [6] and [7] hold the last wm_moments call's fused
- * moment pass and its fold.  Returns the number written. */
+ * arrivals), [5] sort (every particle's place).  In the FP32 form the push
+ * places the last push's movers (the particle boundaries and the sort reduce
+ * to that); [4] is the bins' fill check beside the solve and [5] the
+ * re-layouts of rows whose bins would overflow.  [6] and [7] hold the last
+ * wm_moments call's fused moment pass and its fold.  Returns the number
+ * written. */
 int wm_phase_times(wm_ctx *ctx, double *ms, int n);
 /* Total active particles (sum of np2). */
 int wm_particle_count(wm_ctx *ctx, long long *count);

@@ -703,8 +703,8 @@ int wm_alloc_device(wm_ctx *ctx) {
   WM_TRY(dmalloc(ctx, &ctx->cg_p[0], 3 * n));
   WM_TRY(dmalloc(ctx, &ctx->cg_p[1], 3 * n));
   WM_TRY(dmalloc(ctx, &ctx->cg_s, 4));
-  WM_TRY(dmalloc(ctx, &ctx->ts, 8));
-  WM_HIP(hipMemsetAsync(ctx->ts, 0, 8 * sizeof(*ctx->ts), ctx->stream));
+  WM_TRY(dmalloc(ctx, &ctx->ts, 9));
+  WM_HIP(hipMemsetAsync(ctx->ts, 0, 9 * sizeof(*ctx->ts), ctx->stream));
   int khz = 0;
   if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device) == hipSuccess && khz > 0)
     ctx->clock_khz = khz;
@@ -1350,6 +1350,11 @@ int wm_step(wm_ctx *ctx, int nsteps) {
   WM_TRY(wm_alloc_device(ctx));
   double acc[WM_NPHASE] = {0};
   const bool f32 = ctx->form == WM_FORM_FP32;
+  const auto add = [&](int phase, unsigned long long from, unsigned long long to) {
+    acc[phase] += (double)std::max(0LL, (long long)(to - from)) / ctx->clock_khz;
+  };
+  unsigned long long update_from = 0;        // the last step's field update
+  unsigned update_seq = 0;
   for (int it = 0; it < nsteps; ++it) {
     StepScope scope{ctx, false};
     // particle__solv + ele_cur (proj/weibel/app.f90:102, field.f90:121)
@@ -1391,14 +1396,19 @@ int wm_step(wm_ctx *ctx, int nsteps) {
     scope.ended = true;
     // phases: [0..3] on the first stream, [4] particle boundaries and [5] the
     // places on the second (FP64; in the FP32 form the push holds them, and [4]
-    // is the fill check, [5] the re-layout)
+    // is the fill check, [5] the re-layout).  [3] has two parts, the solve and,
+    // once both streams are there, the update.  The report comes as that begins;
+    // when it ended, the next step's report tells.
     const SolveReport r = *(const SolveReport *)((const char *)ctx->h_pin + WM_PIN_REPORT);
-    const int from[WM_NPHASE] = {0, 1, 2, 3, 5, 6}, to[WM_NPHASE] = {1, 2, 3, 4, 6, 7};
-    for (int k = 0; k < WM_NPHASE; ++k)
-      acc[k] += (double)std::max(0LL, (long long)(r.ts[to[k]] - r.ts[from[k]])) / ctx->clock_khz;
+    for (int k = 0; k < 4; ++k) add(k, r.ts[k], r.ts[k + 1]);
+    for (int k = 4; k < WM_NPHASE; ++k) add(k, r.ts[k + 1], r.ts[k + 2]);
+    if (it > 0) add(3, update_from, wm_update_end(ctx, update_seq));
     WM_TRY(wm_field_result(ctx));
+    update_from = r.begin;
+    update_seq = ctx->seq;
     if (r.derr) WM_TRY(wm_check_derr(ctx, "step"));
   }
+  if (nsteps > 0) add(3, update_from, wm_update_end(ctx, update_seq));
   for (int k = 0; k < WM_NPHASE; ++k) ctx->phase_ms[k] = acc[k];
   return WM_OK;
 }

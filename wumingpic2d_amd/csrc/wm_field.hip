@@ -74,7 +74,9 @@ __global__ void k_curre_cols(FieldGeom fg, double *uj) {
 // boundary_periodic__dfield (boundary_periodic.f90:263-345): ghost rows of
 // the interior columns x0 .. x0 + cnt - 1 (all of them, or the wall
 // families' active ones, boundary_shock.f90:326-392).
-__global__ void k_dfield_rows(FieldGeom fg, double *df, int ncomp, int x0, int cnt, SolveGate gate) {
+__global__ void k_dfield_rows(FieldGeom fg, double *df, int ncomp, int x0, int cnt, SolveGate gate,
+                              unsigned long long *ts) {
+  if (ts) wm_stamp(ts, 8);
   if (gate.closed()) return;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= cnt * ncomp) return;
@@ -666,12 +668,12 @@ int wm_k_bc_curre(wm_ctx *ctx, double *uj) {
   return WM_OK;
 }
 
-static int bc_dfield(wm_ctx *ctx, double *df, const SolveGate &gate) {
+static int bc_dfield(wm_ctx *ctx, double *df, const SolveGate &gate, unsigned long long *ts = nullptr) {
   const FieldGeom &fg = ctx->fg;
   const XSide X = wm_xside(ctx);
   const int cnt = X.xb - X.xa + 1;
   hipLaunchKernelGGL(k_dfield_rows, dim3(wm_cdiv(cnt * 6, 256)), dim3(256), 0, ctx->stream, fg, df,
-                     6, X.xa, cnt, gate);
+                     6, X.xa, cnt, gate, ts);
   if (X.wall)
     hipLaunchKernelGGL(k_dfield_walls, dim3(wm_cdiv(fg.gy, 256)), dim3(256), 0, ctx->stream, fg,
                        df, X, gate);
@@ -776,7 +778,7 @@ static int field_update(wm_ctx *ctx, const SolveGate &gate) {
   const FC f = make_fc(g);
   const int n = g.nx * g.ny;
   const XSide X = wm_xside(ctx);
-  WM_TRY(bc_dfield(ctx, ctx->df, gate));
+  WM_TRY(bc_dfield(ctx, ctx->df, gate, ctx->ts));
   hipLaunchKernelGGL(k_delta_e, dim3(wm_cdiv(n, 256)), dim3(256), 0, ctx->stream, fg, f, X,
                      ctx->uf, ctx->uj, ctx->df, gate);
   WM_HIP(hipGetLastError());

@@ -233,7 +233,8 @@ struct wm_ctx {
   hipEvent_t join[2]{};    // between the streams of a step: the push done, the second stream's end
   // a step's kernels leave the device clock here as they start (wm_stamp): cell
   // fields, push, current, solve, solve's end; on the second stream row order
-  // (fill check), places (re-layout), its end
+  // (fill check), places (re-layout), its end; last the update, where it has
+  // several kernels
   unsigned long long *ts = nullptr;
   unsigned seq = 0;        // reports asked for
   int clock_khz = 100000;
@@ -358,6 +359,7 @@ int wm_k_field_solve(wm_ctx *ctx);
 bool wm_tiles_fit(wm_ctx *ctx, bool peek = false);
 int wm_k_tiles(wm_ctx *ctx, bool begins, bool *ran);
 int wm_report_wait(wm_ctx *ctx);
+unsigned long long wm_update_end(const wm_ctx *ctx, unsigned seq);
 bool wm_fused_update(const wm_ctx *ctx);
 int wm_k_update_report(wm_ctx *ctx);  // periodic; else the report alone
 int wm_tiles_result(wm_ctx *ctx, bool *gave_up, int *err, int *ite);

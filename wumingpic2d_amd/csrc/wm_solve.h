@@ -33,18 +33,29 @@ struct SolveReport {
   int abort_;            // the on-chip solve gave up
   int derr;              // device error bits
   unsigned long long ts[8];   // wm_ctx::ts
+  unsigned long long begin;   // the clock as the update began
   unsigned seq;          // written last: which report this is
+  // the clock as the update's last workgroup ends, of this report and the last
+  // (by seq's lowest bit): there once the stream's next kernel has begun
+  unsigned long long end[2];
 };
 // One thread leaves the report (abort_ null: the solve streamed).
 __device__ inline void leave_report(SolveReport *host, const SolveOut &out, int given,
-                                    const int *derr, const unsigned long long *ts, unsigned seq) {
+                                    const int *derr, const unsigned long long *ts,
+                                    unsigned long long begin, unsigned seq) {
   host->out = out;
   host->abort_ = given;
   host->derr = *derr;
 #pragma unroll
   for (int k = 0; k < 8; ++k) host->ts[k] = ts[k];
+  host->begin = begin;
   __threadfence_system();
   __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// One thread of the update's last workgroup leaves the clock.
+__device__ inline void leave_end(SolveReport *host, unsigned seq) {
+  __hip_atomic_store(&host->end[seq & 1], (unsigned long long)wall_clock64(), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // The field update's kernels skip when the on-chip solve before them gave up
 // or failed (null: after a streaming solve).

@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256) void k_field_update(FieldGeom fg, SolveConst f
   const int t = blockIdx.x * 256 + threadIdx.x;
   const int given = abort_ ? *abort_ : 0;
   const SolveOut o = abort_ ? *out : SolveOut{};
-  if (t == 0) leave_report(host, o, given, derr, ts, seq);
+  if (t == 0) leave_report(host, o, given, derr, ts, wall_clock64(), seq);
   if (given || o.err[0] || o.err[1] || o.err[2] || t >= fg.gx * fg.gy) return;
   const int li = t % fg.gx, lj = t / fg.gx;
   const int ci = wrapm(li - 2, fg.nx);
@@ -459,6 +459,7 @@ __global__ __launch_bounds__(256) void k_field_update(FieldGeom fg, SolveConst f
   un[3 * ps + t] = uf[3 * ps + t] + e1;
   un[4 * ps + t] = uf[4 * ps + t] + e2;
   un[5 * ps + t] = uf[5 * ps + t] + e3;
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) leave_end(host, seq);
 }
 
 // The same between conducting walls (active columns L .. E of the
@@ -496,7 +497,7 @@ __global__ __launch_bounds__(256) void k_walls_update(FieldGeom fg, SolveConst f
   const int t = blockIdx.x * 256 + threadIdx.x;
   const int given = abort_ ? *abort_ : 0;
   const SolveOut o = abort_ ? *out : SolveOut{};
-  if (t == 0) leave_report(host, o, given, derr, ts, seq);
+  if (t == 0) leave_report(host, o, given, derr, ts, wall_clock64(), seq);
   if (given || o.err[0] || o.err[1] || o.err[2] || t >= fg.gx * fg.gy) return;
   const int li = t % fg.gx, lj = t / fg.gx;
   const size_t gx = fg.gx, ps = fg.ps;
@@ -550,6 +551,7 @@ __global__ __launch_bounds__(256) void k_walls_update(FieldGeom fg, SolveConst f
   }
 #pragma unroll
   for (int k = 0; k < 6; ++k) un[k * ps + t] = uf[k * ps + t] + d[k];
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) leave_end(host, seq);
 }
 
 // The device's CUs shared by the contexts of this process: a solve in flight
@@ -630,7 +632,8 @@ namespace {
 // One thread: the step's status for the host, where no update kernel leaves it.
 __global__ void k_report(const int *abort_, const SolveOut *out, const int *derr,
                          const unsigned long long *ts, unsigned seq, SolveReport *host) {
-  leave_report(host, abort_ ? *out : SolveOut{}, abort_ ? *abort_ : 0, derr, ts, seq);
+  leave_end(host, seq);
+  leave_report(host, abort_ ? *out : SolveOut{}, abort_ ? *abort_ : 0, derr, ts, ts[8], seq);
 }
 
 SolveReport *report_of(wm_ctx *ctx) { return (SolveReport *)((char *)ctx->h_pin + WM_PIN_REPORT); }
@@ -802,6 +805,12 @@ int wm_report_wait(wm_ctx *ctx) {
   if (there()) return WM_OK;
   wm_set_error(ctx, WM_ERR_HIP, "the step's report did not arrive");
   return WM_ERR_HIP;
+}
+
+// The clock as the update of report seq ended (this or the last report's).
+unsigned long long wm_update_end(const wm_ctx *ctx, unsigned seq) {
+  const SolveReport *r = (const SolveReport *)((const char *)ctx->h_pin + WM_PIN_REPORT);
+  return __atomic_load_n(&r->end[seq & 1], __ATOMIC_ACQUIRE);
 }
 
 // After the report has been waited for.
