@@ -21,8 +21,6 @@
 // order.  Tiles go to a partial buffer that a gather
 // kernel sums in a fixed order, so the deposit is deterministic (no
 // floating-point atomics).
-#include <math.h>
-
 #include "wm_internal.h"
 #include "wm_edges.h"
 #include "wm_mover.h"
@@ -562,13 +560,18 @@ __device__ inline void cell_coeffs(double *cf, const double *Tk) {
   }
 }
 
+// A square that has overflowed (a momentum above 1e154) as one of the largest
+// numbers, by one 32-bit operation (a NaN becomes a number too: the momentum it
+// comes from is none).
+__device__ inline double below_inf(double a) {
+  return __hiloint2double((int)min((unsigned)__double2hiint(a), 0x7FEFFFFFu), __double2loint(a));
+}
 // 1 / sqrt(a), a > 0 normal: the hardware's estimate (to about 2^-23) and two
-// Newton steps in FMAs, within an ulp.  Where a has overflowed (a momentum above
-// 1e154) the estimate is zero, as the quotient is; the steps, on the largest
-// number instead, leave it there.
+// Newton steps in FMAs, within an ulp.  At infinity the estimate is zero, as the
+// quotient is, and the steps leave it there.
 __device__ inline double rsqrt64(double a) {
   double y = __builtin_amdgcn_rsq(a);
-  a = fmin(a, 0x1.fffffffffffffp1023);
+  a = below_inf(a);
   double h = 0.5 * y;
   double e = fma(-a * y, h, 0.5);      // 1/2 - a y^2 / 2
   y = fma(y, e, y);
@@ -599,12 +602,12 @@ __device__ inline PushOut boris_coeffs(const double2 *cf, double ox, double oy, 
   double uvm1 = ux + fac1 * epx;
   double uvm2 = uy + fac1 * epy;
   double uvm3 = uz + fac1 * epz;
-  const double g2 = P.c * P.c + uvm1 * uvm1 + uvm2 * uvm2 + uvm3 * uvm3;
-  const double igam = rsqrt64(g2);
-  const double g1 = g2 * igam;         // (no number where g2 is infinite, as the root is)
-  const double gam = fmin(fma(fma(-g1, g1, g2), 0.5 * igam, g1), INFINITY);   // sqrt(g2)
+  // fac2 / (gam + txxx b^2 / gam) by igam alone, which is zero where gam has
+  // overflowed
+  const double igam = rsqrt64(P.c * P.c + uvm1 * uvm1 + uvm2 * uvm2 + uvm3 * uvm3);
   const double fac1r = fac1 * igam;
-  const double fac2r = fac2 / (gam + txxx * (bpx * bpx + bpy * bpy + bpz * bpz) * igam);
+  const double fac2r =
+      fac2 * igam / fma(txxx * (bpx * bpx + bpy * bpy + bpz * bpz) * igam, igam, 1.0);
   const double uvm4 = uvm1 + fac1r * (uvm2 * bpz - uvm3 * bpy);
   const double uvm5 = uvm2 + fac1r * (uvm3 * bpx - uvm1 * bpz);
   const double uvm6 = uvm3 + fac1r * (uvm1 * bpy - uvm2 * bpx);
