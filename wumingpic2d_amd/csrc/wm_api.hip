@@ -1326,7 +1326,8 @@ struct StreamSwap {
   StreamSwap(wm_ctx *ctx, hipStream_t s) : c(ctx), saved(ctx->stream) { ctx->stream = s; }
   ~StreamSwap() { c->stream = saved; }
 };
-// What a step that ends early has in flight on both streams is waited for.
+// A step that ends early: the second stream is waited for, and the first where a
+// solve on chip is in flight (whatever else it has, the next call's work follows).
 struct StepScope {
   wm_ctx *c;
   bool ended;

@@ -199,7 +199,8 @@ struct wm_ctx {
   size_t plane32 = (size_t)1 << 29;   // slots of a plane below 4 GB an array (wm_debug.h)
   uint16_t *code = nullptr;      // [nseg*cap] the push's code per particle (wm_order.h)
   int4 *kind = nullptr;          // [nseg*nx] moves out of a cell by kind
-  int *farcnt = nullptr, *far = nullptr;   // [nseg*nx], [nseg]; zero between steps
+  int *farcnt = nullptr, *far = nullptr;   // [nseg*nx], zero between steps; [nseg], cleared
+                                           // by the next step's first kernel
   uint2 *lup = nullptr, *ldn = nullptr;    // [nseg*mcap] a row's leavers
   uint2 *disp = nullptr;         // [nseg*2*mcap] displaced particles by new cell
   int *dstart = nullptr;         // [nseg*(nx+1)]
@@ -355,13 +356,13 @@ int wm_field_update(wm_ctx *ctx);
 int wm_field_result(wm_ctx *ctx);
 void wm_field_release(wm_ctx *ctx);  // after an error: waits for the solve in flight
 int wm_k_field_solve(wm_ctx *ctx);
-// wm_solve.hip: the on-chip solve and, for the periodic box, its update
+// wm_solve.hip: the on-chip solve, the update in one launch, the step's report
 bool wm_tiles_fit(wm_ctx *ctx, bool peek = false);
 int wm_k_tiles(wm_ctx *ctx, bool begins, bool *ran);
 int wm_report_wait(wm_ctx *ctx);
 unsigned long long wm_update_end(const wm_ctx *ctx, unsigned seq);
 bool wm_fused_update(const wm_ctx *ctx);
-int wm_k_update_report(wm_ctx *ctx);  // periodic; else the report alone
+int wm_k_update_report(wm_ctx *ctx);  // update and report; a single row's report alone
 int wm_tiles_result(wm_ctx *ctx, bool *gave_up, int *err, int *ite);
 struct SolveGate;
 int wm_k_energy(wm_ctx *ctx, int bank, double *out_host);
@@ -369,7 +370,7 @@ int wm_k_energy(wm_ctx *ctx, int bank, double *out_host);
 int wm_k_particle_x(wm_ctx *ctx, int bank);
 int wm_k_particle_y(wm_ctx *ctx, int bank);
 // The resident step's particle_y and sort, as the order of the rows in
-// bank 0; mid is recorded before the last kernel (wm_order.hip)
+// bank 0 (wm_order.hip)
 int wm_k_order(wm_ctx *ctx);
 int wm_order_apply(wm_ctx *ctx);   // bank 0 in that order, if one is pending
 int wm_k_injection(wm_ctx *ctx, int bank, double u0);   // boundary_shock__injection

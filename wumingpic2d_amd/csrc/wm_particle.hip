@@ -528,7 +528,7 @@ __global__ __launch_bounds__(256, 3) void k_particle(
 // the in-cell offsets: nine coefficients per field and cell (LDS), 8 FMAs a
 // field.
 //
-// Two wavefronts a SIMD (197 and 224 registers): bound by FP64 operations (half of the
+// Two wavefronts a SIMD (197 registers with 16 lanes a cell, 224 with 8): bound by FP64 operations (half of the
 // issue slots) and the memory path together; alone, loads and stores take 0.92
 // ms and the arithmetic 0.91 at 1024 x 512 cells with 32 per cell, both 1.1.
 // Measured against 8 lanes a cell, 32 cells and lists summed component by
@@ -881,7 +881,6 @@ __global__ __launch_bounds__(PCH * PG, 2) void k_push_step(PP P, const int *__re
       e = max(b, min(P.cap, cc[1]));
     }
   };
-  auto first = [&](int b, int e) { return b + sub; };
   // the particle of slot q: where it is, and itself
   auto src = [&](int s, int q, int b, int e) {
     q = max(0, min(max(q, b), e - 1));
@@ -904,11 +903,11 @@ __global__ __launch_bounds__(PCH * PG, 2) void k_push_step(PP P, const int *__re
   slots(0, kb, ke);
   slots(1, kbn, ken);
   load_tmp_tile<PTW>(T, tmp, TX, tps, jl, chunk * PCH, min(PTW, ncell + 2));
-  int k = first(kb, ke);
+  int k = kb + sub;
   const unsigned p0 = src(0, k, kb, ke), p1 = src(0, k + PG, kb, ke);
   // where the particles of the two steps after those in n0 and n1 come from
   unsigned f0 = src(0, k + 2 * PG, kb, ke), f1 = src(0, k + 3 * PG, kb, ke);
-  const int kn = first(kbn, ken);
+  const int kn = kbn + sub;
   unsigned q0 = 0, q1 = 0, q2 = 0, q3 = 0;
   if (P.nsp > 1) {
     q0 = src(1, kn, kbn, ken);
@@ -1063,7 +1062,7 @@ __global__ __launch_bounds__(PCH * PG, 2) void k_push_step(PP P, const int *__re
           if (sub < 4) mk[g * 4 + sub] = 0;
           kb = kbn;
           ke = ken;
-          k = first(kb, ke);
+          k = kb + sub;
           if (s > 1) {
             q0 = src(s, k, kb, ke);
             q1 = src(s, k + PG, kb, ke);
@@ -1226,8 +1225,12 @@ int wm_k_push_step(wm_ctx *ctx) {
   // steps of a two-stream plasma, 1024 x 1024 cells: 1.47 and 1.42 at 8
   // particles per cell and species, 1.24 and 1.19 at 24, 1.08 and 1.12 at 32,
   // 0.95 and 1.05 at 40, 0.88 and 1.00 at 48; 512 x 512: 1.10 and 1.08 at 32,
-  // 0.98 and 1.04 at 40, 0.86 and 0.91 at 64; 256 x 64: 1.33 and 0.83 at 24,
-  // 1.25 and 0.86 at 32.
+  // 0.98 and 1.04 at 40, 0.86 and 0.91 at 64; 256 x 256: 1.13 and 1.01 at 24, 1.02
+  // and 0.91 at 32; 256 x 192: 1.11 and 0.98, 1.06 and 0.94; 256 x 128: 1.17 and
+  // 0.91, 1.05 and 0.83; 256 x 64: 1.31 and 0.89, 1.24 and 0.73; 128 x 64: 0.87 and
+  // 0.63, 0.83 and 0.59.  So the line lies where a run's pinched part, the longer
+  // one, begins to lose more than its first steps gain.  At 8 per cell eight lanes
+  // are the faster from 16384 cells on (1.5 and 1.06).
   const long long cells = (long long)P.nx * P.ny;
   const bool eight = cells > 32768 && ctx->npart <= 36 * cells * P.nsp;
 #define WM_PUSH(S, W) (eight ? k_push_step<S, W, 8> : k_push_step<S, W, 16>)

@@ -35,9 +35,10 @@
 // after it stream, a thousand the first time and twice as many each further
 // time, so that what the waits cost stays below what the streaming does.
 //
-// Bound by the exchanges: about 4 us an iteration at 256 x 64 (40 us a solve of
-// 7), of which the sweeps are 1.6; at 1024 x 1024 by the sweeps of 16 rows a
-// lane, one component after another (163 us).
+// Bound by the exchanges: about 4 us an iteration at 256 x 64 (the kernel 36 us
+// for 7), of which the sweeps are 1.6; at 1024 x 1024 by the sweeps of 16 rows a
+// lane, two components and then the third (161 us; the right-hand side before it
+// takes 40).
 #include <chrono>
 #include <condition_variable>
 #include <mutex>
@@ -571,10 +572,10 @@ struct Plan {
 };
 
 // The tile, and how many of the three components run side by side: the least
-// estimate of an iteration's time in microseconds, from the solve phase's time
-// at 7 iterations measured for every plan: a row of cells 0.4 (alone on its CU
+// estimate of an iteration's time in microseconds, from the time of both kernels
+// at 7 iterations, launches and all, measured for every plan: a row of cells 0.4 (alone on its CU
 // 0.2), an exchange 3 and 0.08 a workgroup that takes part, a component that
-// waits for another's end a whole iteration more.  Solve phase in us at 4, 8 and
+// waits for another's end a whole iteration more.  Both kernels, us, at 4, 8 and
 // 16 rows a lane: 256 x 64: 44, 52, 69; 512 x 128: 49, 55, 76; 499 x 309: 84,
 // 69, 85; 1024 x 256: 158 (two turns), 79, 92.  One workgroup a component
 // against several: 250 x 24: 35 and 42; 128 x 64: 35 and 40; 500 x 16: 39 and
