@@ -42,7 +42,7 @@ def test_the_field_phase_holds_the_update():
     ctx = _run(wm.FORM_FP32, n, 8, 1e10, steps)
     assert not ctx.cg_iters().any()
     short = []
-    for _ in range(6):
+    for _ in range(20):
         t = time.perf_counter()
         ctx.step(steps)
         short.append(((time.perf_counter() - t) - ctx.phase_times()[:4].sum() * 1e-3) / steps)
