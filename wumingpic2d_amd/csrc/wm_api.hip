@@ -1540,7 +1540,7 @@ int wm_particle_count(wm_ctx *ctx, long long *count) {
 int wm_id_checksum(wm_ctx *ctx, unsigned long long *sum_xor) {
   if (!ctx || !sum_xor) return WM_ERR_ARG;
   if (!ctx->alloc_done) return WM_ERR_NOT_INIT;
-  WM_TRY(ctx->form == WM_FORM_FP32 ? wm_settle_movers(ctx) : wm_order_apply(ctx));
+  if (ctx->form == WM_FORM_FP32) WM_TRY(wm_settle_movers(ctx));
   unsigned long long *d = nullptr;
   WM_HIP(hipMalloc((void **)&d, 2 * sizeof(unsigned long long)));
   int st = WM_OK;

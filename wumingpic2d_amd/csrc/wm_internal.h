@@ -373,6 +373,7 @@ int wm_k_particle_y(wm_ctx *ctx, int bank);
 // bank 0 (wm_order.hip)
 int wm_k_order(wm_ctx *ctx);
 int wm_order_apply(wm_ctx *ctx);   // bank 0 in that order, if one is pending
+const unsigned *wm_order_ids(const wm_ctx *ctx);   // its ID indexes (null: none is pending)
 int wm_k_injection(wm_ctx *ctx, int bank, double u0);   // boundary_shock__injection
 double wm_injection_xend(const wm_ctx *ctx, double u0);
 // Sort (wm_sort.hip)

@@ -695,6 +695,14 @@ int wm_k_order(wm_ctx *ctx) {
   return WM_OK;
 }
 
+// Where the particles' IDs are (species-plane indexes by slot) while the IDs lie
+// as they did when the order began.
+const unsigned *wm_order_ids(const wm_ctx *ctx) {
+  if (!ctx->perm_valid) return nullptr;
+  return (const unsigned *)ctx->id[1 - ctx->idcur] +
+         (size_t)ctx->oidcur * ctx->g.nsp * ctx->g.ny * ctx->cap;
+}
+
 // Bank 0 put in its order (for whoever reads the rows as rows).
 int wm_order_apply(wm_ctx *ctx) {
   if (!ctx->perm_valid) return WM_OK;
@@ -703,8 +711,7 @@ int wm_order_apply(wm_ctx *ctx) {
   hipLaunchKernelGGL(k_order_apply, grid, dim3(256), 0, ctx->stream, ctx->cap, g.ny, ctx->np2,
                      ctx->perm, ctx->bank[0], ctx->bank[1]);
   // (bank 0's records have moved: its space holds the IDs on their way)
-  const unsigned *oid = (const unsigned *)ctx->id[1 - ctx->idcur] +
-                        (size_t)ctx->oidcur * g.nsp * g.ny * ctx->cap;
+  const unsigned *oid = wm_order_ids(ctx);
   int64_t *const tmp = (int64_t *)ctx->bank[0].x;
   hipLaunchKernelGGL(k_ids_gather, grid, dim3(256), 0, ctx->stream, ctx->cap, g.ny, ctx->np2, oid,
                      ctx->id[ctx->idcur], tmp);

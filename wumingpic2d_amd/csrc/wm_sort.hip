@@ -672,11 +672,14 @@ __global__ __launch_bounds__(256) void k_migrate(Mig G, Movers M, Bins32 A,
 
 // The IDs of the active particles of one segment per workgroup, summed and
 // xor-ed (64-bit integer wrap: the order does not matter): bins of the FP32
-// form (bs, cnt) or rows of the FP64 form (np2).
+// form (bs, cnt) or rows of the FP64 form (np2), there through the pending
+// order's ID indexes (oid) into the species' planes if there is one: 12 bytes a
+// particle, where putting the rows in order first moves 120.
 __global__ __launch_bounds__(256) void k_id_checksum(const int64_t *__restrict__ ids, int nx,
                                                      int cap, const int *__restrict__ bstart,
                                                      const int *__restrict__ cnt,
                                                      const int *__restrict__ np2,
+                                                     const unsigned *__restrict__ oid, int ny,
                                                      unsigned long long *out) {
   const int seg = blockIdx.x;
   unsigned long long sum = 0, x = 0;
@@ -691,8 +694,12 @@ __global__ __launch_bounds__(256) void k_id_checksum(const int64_t *__restrict__
         x ^= v;
       }
   } else {
+    const size_t plane = (size_t)ny * cap;
+    const int64_t *of = ids + (size_t)(seg / ny) * plane;
+    const unsigned *o = oid ? oid + (size_t)seg * cap : nullptr;
     for (int k = threadIdx.x; k < np2[seg]; k += blockDim.x) {
-      const unsigned long long v = (unsigned long long)row[k];
+      const unsigned long long v =
+          (unsigned long long)(o ? of[min((size_t)o[k], plane - 1)] : row[k]);
       sum += v;
       x ^= v;
     }
@@ -840,7 +847,8 @@ int wm_k_id_checksum(wm_ctx *ctx, unsigned long long *out_dev) {
   }
   hipLaunchKernelGGL(k_id_checksum, dim3(ctx->g.nsp * ctx->g.ny), dim3(256), 0, ctx->stream, ids,
                      ctx->g.nx, ctx->cap, f32 ? ctx->bstart : nullptr,
-                     f32 ? ctx->bin_cnt : nullptr, ctx->np2, out_dev);
+                     f32 ? ctx->bin_cnt : nullptr, ctx->np2, f32 ? nullptr : wm_order_ids(ctx),
+                     ctx->g.ny, out_dev);
   WM_HIP(hipGetLastError());
   return WM_OK;
 }
