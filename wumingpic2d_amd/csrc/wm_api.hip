@@ -1179,11 +1179,9 @@ int bc_mom(wm_ctx *ctx, int family, double *mom) {
   WM_TRY(wm_alloc_device(ctx));
   WM_TRY(wm_mom_buffers(ctx));
   const size_t n = wm_mom_elems(ctx);
-  WM_HIP(hipMemcpyAsync(ctx->mom, mom, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream));
+  WM_TRY(wm_to_device(ctx, ctx->mom, mom, sizeof(double) * n));
   WM_TRY(wm_k_bc_mom(ctx, ctx->mom));
-  WM_HIP(hipMemcpyAsync(mom, ctx->mom, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
-  return WM_OK;
+  return wm_to_host(ctx, ctx->mom, mom, sizeof(double) * n);
 }
 }  // namespace
 
@@ -1476,11 +1474,9 @@ int wm_bcp_mom(wm_ctx *ctx, double *mom) {
   WM_TRY(wm_alloc_device(ctx));
   WM_TRY(wm_mom_buffers(ctx));
   const size_t n = wm_mom_elems(ctx);
-  WM_HIP(hipMemcpyAsync(ctx->mom, mom, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream));
+  WM_TRY(wm_to_device(ctx, ctx->mom, mom, sizeof(double) * n));
   WM_TRY(wm_k_bc_mom(ctx, ctx->mom));
-  WM_HIP(hipMemcpyAsync(mom, ctx->mom, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
-  return WM_OK;
+  return wm_to_host(ctx, ctx->mom, mom, sizeof(double) * n);
 }
 
 int wm_moments(wm_ctx *ctx, double *mom) {
