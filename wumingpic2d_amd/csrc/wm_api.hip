@@ -1282,8 +1282,7 @@ int wm_state_download(wm_ctx *ctx, double *up, int *np2, int *cumcnt, double *uf
   }
   if (up) WM_TRY(wm_order_apply(ctx));
   std::vector<int> n2(nseg);
-  WM_HIP(hipMemcpyAsync(n2.data(), ctx->np2, sizeof(int) * nseg, hipMemcpyDeviceToHost, ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
+  WM_TRY(wm_to_host(ctx, ctx->np2, n2.data(), sizeof(int) * nseg));
   if (cumcnt)
     WM_TRY(wm_to_host(ctx, ctx->cumcnt, cumcnt, sizeof(int) * (size_t)nseg * (ctx->g.nx + 1)));
   if (f32) WM_TRY(wm_check_derr(ctx, "state download"));
@@ -1524,9 +1523,7 @@ int wm_particle_count(wm_ctx *ctx, long long *count) {
   const bool f32 = ctx->form == WM_FORM_FP32;
   const size_t n = f32 ? (size_t)nseg_of(ctx) * ctx->g.nx : (size_t)nseg_of(ctx);
   std::vector<int> c(n);
-  WM_HIP(hipMemcpyAsync(c.data(), f32 ? ctx->bin_cnt : ctx->np2, sizeof(int) * n,
-                        hipMemcpyDeviceToHost, ctx->stream));
-  WM_HIP(hipStreamSynchronize(ctx->stream));
+  WM_TRY(wm_to_host(ctx, f32 ? ctx->bin_cnt : ctx->np2, c.data(), sizeof(int) * n));
   long long t = 0;
   for (int v : c) t += v;
   *count = t;
