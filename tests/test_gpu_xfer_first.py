@@ -1,6 +1,7 @@
-"""A context's first copies make two pinned buffers (from 16 MB on one for each 4 MB
-beyond 8 MB), later ones of such arrays more until eight threads have one each;
-what they copy is right at every number of them."""
+"""A context's first copies make two pinned buffers, or four on the way down (from
+16 MB on one for each 4 MB beyond 8 MB, if that is more), later ones of such arrays
+more until eight threads have one each; what they copy is right at every number of
+them."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nx,ny,ppc,first,end", [
-    (250, 24, 20, 2, 2),         # 11 MB of particles, then small arrays
+    (512, 8, 12, 2, 2),          # 4.5 MB of particles: one thread
+    (250, 24, 20, 2, 4),         # 11 MB of particles, then small arrays
     (600, 500, 1, 4, 8),         # 27.5 MB of particles, 14 MB of fields
     (1500, 1203, 1, 8, 8),       # 165 MB
 ])

@@ -47,7 +47,7 @@ int threads_for(size_t bytes) {
   return bytes < ALONE ? 1 : (int)std::min<size_t>(WORKERS, bytes / SHARE);
 }
 
-// The buffers a copy may make anew, beyond two.  One of 1 MB takes 0.05 to 0.15
+// The buffers a copy may make anew, beyond `few`.  One of 1 MB takes 0.05 to 0.15
 // ms, and the process makes one at a time, so that eight cost a context's first
 // copies of a few MB more than eight threads save: a state of 9 MB goes up in
 // 1.4 ms by the runtime's staging, 1.8 with eight new buffers, 1.1 with two.  Two
@@ -56,6 +56,14 @@ int new_buffers(size_t bytes) {
   constexpr size_t MB = (size_t)1 << 20;
   return bytes < 16 * MB ? 0 : (int)((bytes - 8 * MB) >> 22);
 }
+
+// Threads with a buffer each that a copy has at once.  Down four: the caller's
+// pages, often fresh ones, are touched and filled on the way.  A moments call whose
+// result is 15.5 MB takes 1.05 ms by four, 1.18 by two and 1.15 by eight and the
+// runtime's copies; two steps and 12.6 MB of particles to the host 0.72, 0.87 and
+// 0.90.  Eight would give 0.02 more, for four calls of 0.3 more to make their
+// buffers.
+int few(bool up) { return up ? 2 : 4; }
 
 // f(worker) on `n` threads, the caller's as worker 0; fewer if the system
 // gives no more.
@@ -124,6 +132,11 @@ struct Chunk {
 // move 12 GB/s where others move 41, so that 30 MB took 1.5 ms in two calls of
 // three and 3.1 in the third.  By this kernel 1.4 to 1.6 ms.  (Uploads have shown
 // neither, and from new buffers a kernel reads more slowly than they.)
+// One array of more than a piece by one thread (`plain`) stays with the runtime,
+// whose copies then follow one another: a moments call of 5.5 MB 0.48 to 0.50 ms,
+// by the kernel 0.50 to 0.53.  Arrays of several parts and single pieces are faster
+// by the kernel: two steps and 6.3 MB of particles to the host 0.52 ms, by the
+// runtime 0.57.
 __global__ __launch_bounds__(256) void k_to_pinned(const char *src, char *dst, size_t n) {
   const double *s = (const double *)src;
   double *d = (double *)dst;
@@ -139,8 +152,8 @@ __global__ __launch_bounds__(256) void k_to_pinned(const char *src, char *dst, s
   for (; i < n8; i += st) d[i] = s[i];
   if (blockIdx.x == 0 && threadIdx.x < n % 8) dst[8 * n8 + threadIdx.x] = src[8 * n8 + threadIdx.x];
 }
-hipError_t to_pinned(char *pin, const char *dev, size_t n, hipStream_t st) {
-  if ((size_t)dev % 8 != 0) return hipMemcpyAsync(pin, dev, n, hipMemcpyDeviceToHost, st);
+hipError_t to_pinned(char *pin, const char *dev, size_t n, hipStream_t st, bool plain) {
+  if (plain || (size_t)dev % 8 != 0) return hipMemcpyAsync(pin, dev, n, hipMemcpyDeviceToHost, st);
   const size_t blocks = std::max<size_t>(1, std::min<size_t>(64, n / 2048));
   hipLaunchKernelGGL(k_to_pinned, dim3((unsigned)blocks), dim3(256), 0, st, dev, pin, n);
   return hipGetLastError();
@@ -168,9 +181,10 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
   const size_t slot = slot_for(total, up);
   int have = 0;
   for (size_t s : x.size) have += s >= slot;
-  const int want = std::min(threads_for(total), std::max(2, have + new_buffers(total)));
+  const int want = std::min(threads_for(total), std::max(few(up), have + new_buffers(total)));
   // (one thread alone has two buffers, and copies a chunk while the next is on
   // its way)
+  const bool plain = want == 1 && spans.size() == 1 && total > slot;
   const size_t unit = std::lcm(rec, (size_t)16);
   const size_t most = std::min(slot, std::max<size_t>(total / want + rec, (size_t)1 << 20)) / unit * unit;
   std::vector<WmSpan> piece;
@@ -221,7 +235,7 @@ int move(wm_ctx *ctx, char *dev, const std::vector<WmSpan> &spans, bool up, size
         for (size_t k = h.s0; k < h.s1; ++k) memcpy(pin + (piece[k].at - at), piece[k].host, piece[k].bytes);
         e = hipMemcpyAsync(dev + at, pin, len, hipMemcpyHostToDevice, st);
       } else {
-        e = to_pinned(pin, dev + at, len, st);
+        e = to_pinned(pin, dev + at, len, st, plain);
       }
       if (e == hipSuccess) e = hipEventRecord(x.ev[buf], st);
       if (e == hipSuccess && !up) {
